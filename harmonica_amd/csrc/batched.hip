@@ -10,7 +10,8 @@
 // Kernel: a grid sized to the device's resident capacity; each workgroup
 // takes the next item from an atomic counter until the list is exhausted
 // (every workgroup reaches the exit), evaluates its tile against its chunk
-// (prisms staged in LDS, FP64 closed form) and stores 256 partial sums at
+// (prisms staged in LDS, far or closed form as prism_gz_kernel) and stores
+// 256 partial sums at
 // the item's slot.
 // Reduce: each point sums its model's chunk partials in chunk order
 // (deterministic), applies harmonica's sign and mGal.
@@ -19,61 +20,49 @@
 #include <vector>
 
 #include "hmx_internal.h"
-#include "prism_device.h"
+#include "prism_far.h"
 
 namespace hmx {
 namespace {
 
 constexpr int kItemWords = 5;  // model, tile, p0, p1, slot
 
-struct alignas(16) BPrism {
-    double w, e, s, n, b, t, grho;
-    int skip, share;  // never set: batched models are not marked for edge sharing
-};
+// Workgroups (of kGzThreads, one point per lane) that share an item.
+constexpr int kItemParts = kObsPerBlock / dev::kGzThreads;
+static_assert(kItemParts * dev::kGzThreads == kObsPerBlock, "parts cover an item");
 
-static_assert(kTile <= 128, "tile_pairs marks at most 128 prisms");
-
-__global__ __launch_bounds__(kObsPerBlock) void batched_gz_kernel(
+__global__ __launch_bounds__(dev::kGzThreads, 4) void batched_gz_kernel(
     const double *__restrict__ oe, const double *__restrict__ on, const double *__restrict__ ou,
     const int64_t *__restrict__ obs_off, const double *__restrict__ prisms,
     const double *__restrict__ density, const int64_t *__restrict__ items, int64_t n_items,
     double *__restrict__ partial, unsigned long long *__restrict__ counter) {
-    __shared__ BPrism tile[kTile];
-    __shared__ dm::Tables tables;
+    __shared__ dev::GzShared sh;
     __shared__ long long item_id;
-    dm::load_tables(&tables);
+    dm::load_tables(&sh.tables);
+    const dev::GzExplicit src{prisms, density};
     for (;;) {
         __syncthreads();
         if (threadIdx.x == 0) item_id = (long long)atomicAdd(counter, 1ull);
         __syncthreads();
-        const long long k = item_id;
+        const long long k = item_id / kItemParts;
         if (k >= n_items) break;
+        const int local = (int)(item_id % kItemParts) * dev::kGzThreads + threadIdx.x;
         const int64_t *it = items + kItemWords * k;
         const int64_t b = it[0], T = it[1], p0 = it[2], p1 = it[3], slot = it[4];
-        const int64_t first = obs_off[b], end = obs_off[b + 1];
-        const int64_t i = first + T * kObsPerBlock + threadIdx.x;
-        const bool valid = i < end;
-        const int64_t ii = valid ? i : end - 1;
-        const double e = oe[ii], n = on[ii], u = ou[ii];
-        double acc[1] = {0.0};
-        uint32_t sflags = 0;
-        for (int64_t t0 = p0; t0 < p1; t0 += kTile) {
-            const int cnt = (int)(p1 - t0 < kTile ? p1 - t0 : kTile);
-            __syncthreads();
-            double *flat = reinterpret_cast<double *>(tile);
-            for (int idx = threadIdx.x; idx < 6 * cnt; idx += blockDim.x) {
-                const int q = idx / 6, c = idx - 6 * q;
-                flat[8 * q + c] = prisms[6 * t0 + idx];
-            }
-            for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
-                tile[q].grho = dev::kG * density[t0 + q];
-                tile[q].skip = 0;
-                tile[q].share = 0;
-            }
-            __syncthreads();
-            dev::tile_pairs<0x8u, false>(tile, cnt, e, n, u, acc, sflags, tables);
+        const int64_t first = obs_off[b] + T * kObsPerBlock, end = obs_off[b + 1];
+        const int64_t i = first + local, ii = i < end ? i : end - 1;
+        dev::GzPoint pt{oe[ii], on[ii], ou[ii], 0.0, 0.0, oe[first], on[first]};
+        pt.x = pt.e - pt.xo;
+        pt.y = pt.n - pt.yo;
+        if (p0 < p1) dev::gz_table(src, p0, sh);
+        dev::gz_box(pt, sh);
+        double acc = 0.0;
+        for (int64_t t0 = p0; t0 < p1; t0 += dev::kGzTile) {
+            const int cnt = (int)(p1 - t0 < dev::kGzTile ? p1 - t0 : dev::kGzTile);
+            dev::gz_stage(src, t0, cnt, pt.xo, pt.yo, sh);
+            dev::gz_tile(cnt, pt, acc, sh);
         }
-        partial[slot * kObsPerBlock + threadIdx.x] = valid ? acc[0] : 0.0;
+        partial[slot * kObsPerBlock + local] = i < end ? acc : 0.0;
     }
 }
 
@@ -208,8 +197,9 @@ int hmx_batched_prism_gz(const double *easting, const double *northing, const do
     hipLaunchKernelGGL(zero_counter_kernel, dim3(1), dim3(64), 0, s, counter);
     HMX_LAUNCHED("zero_counter_kernel");
     if (n_items > 0) {
-        const int64_t grid64 = std::min<int64_t>((int64_t)cu * blocks_per_cu, n_items);
-        hipLaunchKernelGGL(batched_gz_kernel, dim3((unsigned)grid64), dim3(kObsPerBlock), 0, s,
+        // blocks_per_cu counts workgroups of four waves; these have two
+        const int64_t grid64 = std::min<int64_t>((int64_t)cu * blocks_per_cu * 2, n_items * kItemParts);
+        hipLaunchKernelGGL(batched_gz_kernel, dim3((unsigned)grid64), dim3(dev::kGzThreads), 0, s,
                            easting, northing, upward, obs_offsets, prisms, density, items, n_items,
                            partial, counter);
         HMX_LAUNCHED("batched_gz_kernel");

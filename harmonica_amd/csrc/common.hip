@@ -75,7 +75,8 @@ int hmx_forward_workspace_bytes(int64_t n_obs, int64_t n_sources, uint32_t field
         return hmx::fail(HMX_ERR_ARG, "invalid field mask 0x%x", field_mask);
     int cu = hmx::device_cu_count();
     if (cu < 0) return cu;
-    int64_t chunks = hmx::forward_chunks(n_obs, n_sources, cu);
+    int64_t chunks = hmx::prism_chunks(n_obs, n_sources, cu);
+    // (the point masses' chunks are at most as many)
     *bytes = (size_t)chunks * (size_t)nf * (size_t)n_obs * sizeof(double);
     // the prism paths' point order, after the partial sums
     if (hmx::use_point_order(n_obs, n_sources))

@@ -67,6 +67,21 @@ inline int64_t forward_chunks(int64_t n_obs, int64_t n_src, int n_cu) {
     return chunks;
 }
 
+// forward_chunks for the prism field kernels, whose pairs differ several
+// times in cost (far and closed forms): chunks down to 32 prisms even out the
+// workgroups, and calls that cannot give every CU a workgroup that way split
+// down to 8 prisms (24 bodies at 501 points, the pair kernel: 29 -> 16 us).
+inline int64_t prism_chunks(int64_t n_obs, int64_t n_src, int n_cu) {
+    const int64_t obs_blocks = n_obs > kObsPerBlock ? (n_obs + kObsPerBlock - 1) / kObsPerBlock : 1;
+    const int64_t cu = n_cu > 0 ? n_cu : 256;
+    int64_t chunks = (40 * cu + obs_blocks - 1) / obs_blocks;
+    int64_t max_by_src = (n_src + 31) / 32;
+    if (obs_blocks * max_by_src < cu) max_by_src = (n_src + 7) / 8;
+    if (chunks > max_by_src) chunks = max_by_src;
+    if (chunks > 1024) chunks = 1024;
+    return chunks < 1 ? 1 : chunks;
+}
+
 inline int popcount10(uint32_t m) { return __builtin_popcount(m & HMX_ALL_FIELDS); }
 
 // Wavefront-coherent point order of the prism kernels (point_order.hip):
@@ -77,12 +92,25 @@ struct PointOrder {
     const int *perm;
 };
 
+// Points one workgroup orders in one launch.
+constexpr int kSmallOrder = 8192;
+
 // Whether a prism call sorts its points: enough points for the strips to
-// matter and enough pairs that the sort's dozen small launches are
-// negligible next to the pair loop.
+// matter and enough pairs that the sort costs little next to the pair loop:
+// one launch of 25-30 us up to kSmallOrder points, a dozen launches (0.1 ms)
+// beyond.  Scattered points over 20,000 bodies, g_z with and without the
+// sort: 1000 points 165 / 170 us, 3000 points 352 / 417 us, 8000 points 794 /
+// 992 us; over 2000 bodies 3000 points 73 / 57 us.
 inline bool use_point_order(int64_t n_obs, int64_t n_src) {
-    // n_obs * n_src >= 2^30, without forming the product
-    return n_obs >= 2048 && n_src >= ((((int64_t)1 << 30) + n_obs - 1) / n_obs);
+    const int64_t pairs = n_obs <= kSmallOrder ? (int64_t)1 << 25 : (int64_t)1 << 28;
+    // n_obs * n_src >= pairs, without forming the product
+    return n_obs >= 512 && n_src >= (pairs + n_obs - 1) / n_obs;
+}
+
+// Whether a call with a workspace too small for the order is refused; below
+// this it evaluates the points in the caller's order.
+inline bool need_point_order(int64_t n_obs, int64_t n_src) {
+    return n_obs >= 2048 && n_src >= (((int64_t)1 << 30) + n_obs - 1) / n_obs;
 }
 
 // Bytes of the order's workspace region for n_obs points.

@@ -268,9 +268,10 @@ int hmx_prism_magnetic(const double *easting, const double *northing, const doub
     if (cu < 0) return cu;
     const int64_t chunks = hmx::forward_chunks(n_obs, n_prisms, cu);
     const size_t partial_bytes = (size_t)chunks * (size_t)nc * (size_t)n_obs * sizeof(double);
-    const bool order = hmx::use_point_order(n_obs, n_prisms);
     const size_t order_at = hmx::point_order_offset(partial_bytes);
-    const size_t need = order ? order_at + hmx::point_order_bytes(n_obs) : partial_bytes;
+    const size_t with_order = order_at + hmx::point_order_bytes(n_obs);
+    const size_t need = hmx::need_point_order(n_obs, n_prisms) ? with_order : partial_bytes;
+    const bool order = hmx::use_point_order(n_obs, n_prisms) && workspace_bytes >= with_order;
     if (!workspace || workspace_bytes < need)
         return hmx::fail(HMX_ERR_ARG, "workspace too small: %zu < %zu bytes", workspace_bytes,
                          need);

@@ -66,11 +66,12 @@ struct OrderLayout {
 
 // Bounding box of the points (NaN coordinates ignored) and the strip and
 // cell counts: ns * nc <= cells, cells of height h = span_n / ns and width
-// w = span_e / nc with h ~ 4 w.  One workgroup.
-__global__ __launch_bounds__(kBoundsThreads) void order_bounds_kernel(
-    const double *__restrict__ e, const double *__restrict__ n, int64_t n_obs, int64_t cells,
-    OrderParams *__restrict__ par) {
-    __shared__ double red[4][kBoundsThreads];
+// w = span_e / nc with h ~ 4 w.  By a workgroup of kBoundsThreads; thread 0
+// writes *par (global memory or LDS).
+__device__ __forceinline__ void order_bounds(const double *__restrict__ e,
+                                             const double *__restrict__ n, int64_t n_obs,
+                                             int64_t cells, double (&red)[4][kBoundsThreads],
+                                             OrderParams *par) {
     double emin = INFINITY, emax = -INFINITY, nmin = INFINITY, nmax = -INFINITY;
     for (int64_t i = threadIdx.x; i < n_obs; i += kBoundsThreads) {
         const double x = e[i], y = n[i];
@@ -117,11 +118,26 @@ __global__ __launch_bounds__(kBoundsThreads) void order_bounds_kernel(
     par->nc = nc;
 }
 
+__global__ __launch_bounds__(kBoundsThreads) void order_bounds_kernel(
+    const double *__restrict__ e, const double *__restrict__ n, int64_t n_obs, int64_t cells,
+    OrderParams *__restrict__ par) {
+    __shared__ double red[4][kBoundsThreads];
+    order_bounds(e, n, n_obs, cells, red, par);
+}
+
 // Cell index in [0, cnt) of v on a row of cnt cells starting at lo (0 for
 // NaN, clamped at the ends).
 __device__ __forceinline__ int64_t cell_of(double v, double lo, double inv, int64_t cnt) {
     const double f = floor((v - lo) * inv);
     return f >= 0.0 ? (f < (double)cnt ? (int64_t)f : cnt - 1) : 0;
+}
+
+// Boustrophedon cell index of a point.
+__device__ __forceinline__ uint32_t order_key(double e, double n, const OrderParams &p) {
+    const int64_t s = cell_of(n, p.nmin, p.inv_h, p.ns);
+    int64_t c = cell_of(e, p.emin, p.inv_w, p.nc);
+    if (s & 1) c = p.nc - 1 - c;
+    return (uint32_t)(s * p.nc + c);
 }
 
 // keys[i] = boustrophedon cell index of point i, vals[i] = i.
@@ -130,11 +146,7 @@ __global__ void order_keys_kernel(const double *__restrict__ e, const double *__
                                   uint32_t *__restrict__ keys, int *__restrict__ vals) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n_obs) return;
-    const OrderParams p = *par;
-    const int64_t s = cell_of(n[i], p.nmin, p.inv_h, p.ns);
-    int64_t c = cell_of(e[i], p.emin, p.inv_w, p.nc);
-    if (s & 1) c = p.nc - 1 - c;
-    keys[i] = (uint32_t)(s * p.nc + c);
+    keys[i] = order_key(e[i], n[i], *par);
     vals[i] = (int)i;
 }
 
@@ -258,6 +270,116 @@ __global__ void order_gather_kernel(const double *__restrict__ e, const double *
     ou[i] = u[k];
 }
 
+// The whole order of at most kSmallOrder points in one launch of one
+// workgroup: bounding box, keys, two stable radix passes of 6 bits in LDS
+// (at most n / 4 = 2048 cells, 11 bits) and the gather.  The permutation is
+// that of the separate kernels, whose ten launches take about 60 us for so
+// few points; this one takes 25-30 us, bound by the latency of its barriers.
+constexpr int kSmallThreads = kBoundsThreads;
+constexpr int kSmallItems = kSmallOrder / kSmallThreads;
+constexpr int kSmallBits = 6;
+constexpr int kSmallBins = 1 << kSmallBits;
+static_assert(kSmallOrder / 4 <= 1 << (2 * kSmallBits), "two passes cover the cells");
+static_assert(kSmallOrder <= 1 << 16, "keys and indices are 16-bit");
+
+__global__ __launch_bounds__(kSmallThreads) void order_small_kernel(
+    const double *__restrict__ e, const double *__restrict__ n, const double *__restrict__ u,
+    int n_obs, int64_t cells, int *__restrict__ perm, double *__restrict__ oe,
+    double *__restrict__ on, double *__restrict__ ou) {
+    constexpr int kWaves = kSmallThreads / 64, kGroups = kSmallItems * kWaves;
+    constexpr int kPer = kSmallBins * kGroups / kSmallThreads;  // counters per thread
+    __shared__ union {
+        double red[4][kBoundsThreads];
+        struct {
+            uint16_t cnt[kSmallBins][kGroups];  // keys per digit and (slot, wave) group
+            uint16_t key[kSmallOrder], val[kSmallOrder];
+            uint32_t wave_sum[kWaves];
+        } s;
+    } sh;
+    __shared__ OrderParams par;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    order_bounds(e, n, n_obs, cells, sh.red, &par);
+    __syncthreads();
+    uint32_t key[kSmallItems], val[kSmallItems];
+#pragma unroll
+    for (int j = 0; j < kSmallItems; ++j) {
+        const int i = j * kSmallThreads + threadIdx.x;
+        val[j] = i;
+        key[j] = i < n_obs ? order_key(e[i], n[i], par) : 0u;
+    }
+    for (int pass = 0; pass < 2; ++pass) {
+        const int shift = pass * kSmallBits;
+        uint32_t *zero = reinterpret_cast<uint32_t *>(&sh.s.cnt[0][0]);
+        for (int k = threadIdx.x; k < kSmallBins * kGroups / 2; k += kSmallThreads) zero[k] = 0u;
+        __syncthreads();
+        int rank[kSmallItems];
+#pragma unroll
+        for (int j = 0; j < kSmallItems; ++j) {
+            const bool ok = j * kSmallThreads + (int)threadIdx.x < n_obs;
+            const uint32_t d = (key[j] >> shift) & (kSmallBins - 1);
+            uint64_t same = __ballot(ok);
+#pragma unroll
+            for (int b = 0; b < kSmallBits; ++b) {
+                const bool bit = (d >> b) & 1u;
+                const uint64_t on_bit = __ballot(bit);
+                same &= bit ? on_bit : ~on_bit;
+            }
+            rank[j] = ok ? __popcll(same & ((1ull << lane) - 1ull)) : -1;
+            if (rank[j] == 0) sh.s.cnt[d][j * kWaves + wave] = (uint16_t)__popcll(same);
+        }
+        __syncthreads();
+        // exclusive prefix sums over (digit, group)
+        uint16_t *mine = &sh.s.cnt[0][0] + threadIdx.x * kPer;
+        uint32_t c[kPer], total = 0;
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            c[k] = total;
+            total += mine[k];
+        }
+        uint32_t incl = total;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t v = __shfl_up(incl, o);
+            if (lane >= o) incl += v;
+        }
+        if (lane == 63) sh.s.wave_sum[wave] = incl;
+        __syncthreads();
+        uint32_t before = incl - total;
+        for (int w = 0; w < wave; ++w) before += sh.s.wave_sum[w];
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) mine[k] = (uint16_t)(before + c[k]);
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kSmallItems; ++j) {
+            if (rank[j] < 0) continue;
+            const uint32_t d = (key[j] >> shift) & (kSmallBins - 1);
+            const uint32_t pos = sh.s.cnt[d][j * kWaves + wave] + (uint32_t)rank[j];
+            sh.s.key[pos] = (uint16_t)key[j];
+            sh.s.val[pos] = (uint16_t)val[j];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kSmallItems; ++j) {
+            const int i = j * kSmallThreads + threadIdx.x;
+            if (i < n_obs) {
+                key[j] = sh.s.key[i];
+                val[j] = sh.s.val[i];
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int j = 0; j < kSmallItems; ++j) {
+        const int i = j * kSmallThreads + threadIdx.x;
+        if (i >= n_obs) continue;
+        const uint32_t k = val[j];
+        perm[i] = (int)k;
+        oe[i] = e[k];
+        on[i] = n[k];
+        ou[i] = u[k];
+    }
+}
+
 }  // namespace
 
 size_t point_order_bytes(int64_t n_obs) { return OrderLayout(n_obs).total; }
@@ -275,6 +397,16 @@ int point_order(const double *e, const double *n, const double *u, int64_t n_obs
     auto *on = reinterpret_cast<double *>(base + L.n);
     auto *ou = reinterpret_cast<double *>(base + L.u);
     const int64_t cells = order_cells(n_obs), nblocks = sort_blocks(n_obs);
+    if (n_obs <= kSmallOrder) {
+        hipLaunchKernelGGL(order_small_kernel, dim3(1), dim3(kSmallThreads), 0, s, e, n, u,
+                           (int)n_obs, cells, vals[0], oe, on, ou);
+        HMX_LAUNCHED("order_small_kernel");
+        po->e = oe;
+        po->n = on;
+        po->u = ou;
+        po->perm = vals[0];
+        return HMX_OK;
+    }
     int bits = 0;
     while (bits < 32 && ((uint64_t)(cells - 1) >> bits) != 0) ++bits;
     const int passes = (bits + kDigitBits - 1) / kDigitBits;

@@ -11,17 +11,17 @@
 
 #include "hmx_internal.h"
 #include "prism_device.h"
+#include "prism_far.h"
 
 namespace hmx {
 namespace {
 
 using dev::FieldSet;
 
-// One staged prism (64 bytes): bounds, G * density, skip flag and the edge
-// it shares with the previous prism of the tile (dev::shared_edge).
+// One staged prism (64 bytes): bounds, G * density and skip flag.
 struct alignas(16) StagedPrism {
     double w, e, s, n, b, t, grho;
-    int skip, share;
+    int skip, pad;
 };
 
 // Stage prisms [t0, t0 + cnt) of an (m, 6) row-major array.
@@ -37,7 +37,6 @@ __device__ __forceinline__ void stage_prisms(StagedPrism *tile, const double *__
     for (int p = threadIdx.x; p < cnt; p += blockDim.x) {
         tile[p].grho = dev::kG * density[t0 + p];
         tile[p].skip = 0;
-        tile[p].share = 0;
     }
 }
 
@@ -69,13 +68,13 @@ __device__ __forceinline__ void stage_layer(StagedPrism *tile, const double *__r
         sp.t = t;
         sp.grho = dev::kG * d;
         sp.skip = skip ? 1 : 0;
-        sp.share = 0;
+        sp.pad = 0;
         tile[q] = sp;
     }
 }
 
-struct ExplicitSource {
-    const double *prisms, *density;
+struct ExplicitSource : dev::GzExplicit {
+    ExplicitSource(const double *p, const double *d) : dev::GzExplicit{p, d} {}
     __device__ void stage(StagedPrism *tile, int64_t t0, int cnt) const {
         stage_prisms(tile, prisms, density, t0, cnt);
     }
@@ -90,6 +89,19 @@ struct LayerSource {
         stage_layer(tile, ce, n_east, cn, n_north, bottom, top, density, threshold, t0, cnt);
     }
     static constexpr bool may_skip = true;
+    __device__ bool get(int64_t p, double (&b)[6], double &rho) const {
+        const unsigned j = (unsigned)p / (unsigned)n_north, k = (unsigned)p - j * (unsigned)n_north;
+        const int64_t idx = (int64_t)k * n_east + j;
+        const double half_e = (ce[1] - ce[0]) / 2, half_n = (cn[1] - cn[0]) / 2;
+        b[0] = ce[j] - half_e;
+        b[1] = ce[j] + half_e;
+        b[2] = cn[k] - half_n;
+        b[3] = cn[k] + half_n;
+        b[4] = bottom[idx];
+        b[5] = top[idx];
+        rho = density[idx];
+        return rho == 0.0 || rho != rho || (b[5] - b[4] < threshold) || b[5] != b[5] || b[4] != b[4];
+    }
 };
 
 static_assert(kTile <= 128, "tile_pairs marks at most 128 prisms");
@@ -118,21 +130,6 @@ __global__ __launch_bounds__(kObsPerBlock) void prism_forward_kernel(
         __syncthreads();
         src.stage(tile, t0, cnt);
         __syncthreads();
-        if constexpr (M == 0x8u) {  // edges shared with the previous prism (g_u reuse)
-            int sh[(kTile + kObsPerBlock - 1) / kObsPerBlock];
-#pragma unroll
-            for (int k = 0; k * kObsPerBlock < kTile; ++k) {
-                const int q = threadIdx.x + k * kObsPerBlock;
-                sh[k] = (q > 0 && q < cnt) ? dev::shared_edge(tile[q - 1], tile[q]) : 0;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int k = 0; k * kObsPerBlock < kTile; ++k) {
-                const int q = threadIdx.x + k * kObsPerBlock;
-                if (q < cnt) tile[q].share = sh[k];
-            }
-            __syncthreads();
-        }
         dev::tile_pairs<M, Src::may_skip>(tile, cnt, e, n, u, acc, sflags, tables);
     }
     if (valid) {
@@ -141,6 +138,36 @@ __global__ __launch_bounds__(kObsPerBlock) void prism_forward_kernel(
             partial[((int64_t)blockIdx.y * F::count + s) * n_obs + i] = acc[s];
         if (F::tensor && flags && sflags) atomicOr(flags, sflags);
     }
+}
+
+// g_u alone, each prism in the far form or the closed form (prism_far.h).
+template <class Src>
+__global__ __launch_bounds__(dev::kGzThreads, 4) void prism_gz_kernel(
+    const double *__restrict__ oe, const double *__restrict__ on, const double *__restrict__ ou,
+    int n_obs, Src src, int64_t n_src, int64_t chunk_len, double *__restrict__ partial) {
+    __shared__ dev::GzShared sh;
+    dm::load_tables(&sh.tables);
+    // Consecutive workgroups go to the 8 XCDs in turn: with a multiple of 8
+    // point blocks, rotate them from chunk to chunk, or the XCD of a block in
+    // the middle of the model gets its near prisms chunk after chunk.
+    const unsigned bx = (blockIdx.x + blockIdx.y) % gridDim.x;
+    const int64_t base = (int64_t)bx * dev::kGzThreads, i = base + threadIdx.x;
+    const bool valid = i < n_obs;
+    const int64_t ii = valid ? i : n_obs - 1;
+    dev::GzPoint pt{oe[ii], on[ii], ou[ii], 0.0, 0.0, oe[base], on[base]};
+    pt.x = pt.e - pt.xo;
+    pt.y = pt.n - pt.yo;
+    double acc = 0.0;
+    const int64_t c0 = (int64_t)blockIdx.y * chunk_len;
+    const int64_t c1 = c0 + chunk_len < n_src ? c0 + chunk_len : n_src;
+    if (c0 < c1) dev::gz_table(src, c0, sh);
+    dev::gz_box(pt, sh);
+    for (int64_t t0 = c0; t0 < c1; t0 += dev::kGzTile) {
+        const int cnt = (int)(c1 - t0 < dev::kGzTile ? c1 - t0 : dev::kGzTile);
+        dev::gz_stage(src, t0, cnt, pt.xo, pt.yo, sh);
+        dev::gz_tile(cnt, pt, acc, sh);
+    }
+    if (valid) partial[(int64_t)blockIdx.y * n_obs + i] = acc;
 }
 
 // Singular-point scan: bit f of *flags is set when some (point, prism)
@@ -183,17 +210,28 @@ __global__ __launch_bounds__(kObsPerBlock) void singular_scan_kernel(
     if (valid && found) atomicOr(flags, found);
 }
 
-// out[s][perm[i]] = units(sum over chunks in order of partial[c][s][i])
-// (perm NULL: the identity).
-__global__ void reduce_chunks_kernel(const double *__restrict__ partial, int64_t chunks, int nf,
-                                     int64_t n_obs, uint32_t mask, const int *__restrict__ perm,
-                                     double *__restrict__ out) {
-    int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)nf * n_obs) return;
-    int s = (int)(idx / n_obs);
-    int64_t i = idx - (int64_t)s * n_obs;
+// out[s][perm[i]] = units(sum over chunks of partial[c][s][i]) (perm NULL: the
+// identity).  Four waves per 64 outputs, a quarter of the chunks each, added
+// in order: a serial sum over all chunks is bound by the latency of its
+// loads (4096 points: 79 chunks took 11 us, 313 chunks take 9).
+__global__ __launch_bounds__(256) void reduce_chunks_kernel(
+    const double *__restrict__ partial, int64_t chunks, int nf, int64_t n_obs, uint32_t mask,
+    const int *__restrict__ perm, double *__restrict__ out) {
+    __shared__ double part[3][64];
+    const int lane = threadIdx.x & 63, quarter = threadIdx.x >> 6;
+    const int64_t total = (int64_t)nf * n_obs, idx = (int64_t)blockIdx.x * 64 + lane;
+    const int64_t c0 = chunks * quarter / 4, c1 = chunks * (quarter + 1) / 4;
     double sum = 0.0;
-    for (int64_t c = 0; c < chunks; ++c) sum += partial[(c * nf + s) * n_obs + i];
+    if (idx < total) {
+#pragma unroll 4
+        for (int64_t c = c0; c < c1; ++c) sum += partial[c * total + idx];
+    }
+    if (quarter) part[quarter - 1][lane] = sum;
+    __syncthreads();
+    if (quarter || idx >= total) return;
+    sum = ((sum + part[0][lane]) + part[1][lane]) + part[2][lane];
+    const int s = (int)(idx / n_obs);
+    const int64_t i = idx - (int64_t)s * n_obs;
     int f = 0, seen = -1;
     for (; f < 10; ++f)
         if ((mask >> f) & 1u)
@@ -213,16 +251,23 @@ int launch_forward(const double *oe, const double *on, const double *ou, int64_t
                    uint32_t *flags, hipStream_t stream) {
     const int64_t chunk_len = (n_src + chunks - 1) / chunks;
     dim3 grid((unsigned)((n_obs + kObsPerBlock - 1) / kObsPerBlock), (unsigned)chunks);
-    hipLaunchKernelGGL((prism_forward_kernel<M, Src>), grid, dim3(kObsPerBlock), 0, stream, oe, on,
-                       ou, (int)n_obs, src, n_src, chunk_len, partial, flags);
-    HMX_LAUNCHED("prism_forward_kernel");
+    if constexpr (M == 0x8u) {
+        grid.x = (unsigned)((n_obs + dev::kGzThreads - 1) / dev::kGzThreads);
+        hipLaunchKernelGGL((prism_gz_kernel<Src>), grid, dim3(dev::kGzThreads), 0, stream, oe, on,
+                           ou, (int)n_obs, src, n_src, chunk_len, partial);
+        HMX_LAUNCHED("prism_gz_kernel");
+    } else {
+        hipLaunchKernelGGL((prism_forward_kernel<M, Src>), grid, dim3(kObsPerBlock), 0, stream, oe,
+                           on, ou, (int)n_obs, src, n_src, chunk_len, partial, flags);
+        HMX_LAUNCHED("prism_forward_kernel");
+    }
     return HMX_OK;
 }
 
 int launch_reduce(const double *partial, int64_t chunks, int nf, int64_t n_obs, uint32_t mask,
                   const int *perm, double *out, hipStream_t stream) {
     int64_t total = (int64_t)nf * n_obs;
-    hipLaunchKernelGGL(reduce_chunks_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
+    hipLaunchKernelGGL(reduce_chunks_kernel, dim3((unsigned)((total + 63) / 64)), dim3(256), 0,
                        stream, partial, chunks, nf, n_obs, mask, perm, out);
     HMX_LAUNCHED("reduce_chunks_kernel");
     return HMX_OK;
@@ -264,7 +309,8 @@ bool has_kernel(uint32_t mask) {
 // Run the forward model for any field mask: one launch when the mask has
 // its own kernel, else one launch per field reusing the workspace.
 // chunk_cap > 0 limits the number of source chunks (so that the partial
-// sums fit a fixed scratch buffer).  With may_order, calls that pass
+// sums fit a fixed scratch buffer; the point order then depends on what is
+// left of it).  Calls that pass
 // use_point_order evaluate the points in wavefront-coherent order, sorted
 // into the workspace after the room for all fields' partial sums (the
 // layout hmx_forward_workspace_bytes sizes).
@@ -272,12 +318,12 @@ template <class Src>
 int run_forward(const double *oe, const double *on, const double *ou, int64_t n_obs,
                 const Src &src, int64_t n_src, uint32_t mask, double *out, uint32_t *flags,
                 void *workspace, size_t workspace_bytes, hipStream_t stream,
-                int64_t chunk_cap = 0, bool may_order = true) {
+                int64_t chunk_cap = 0) {
     if (n_obs <= 0) return HMX_OK;
     int cu = device_cu_count();
     if (cu < 0) return cu;
     const int nf = popcount10(mask);
-    int64_t chunks = forward_chunks(n_obs, n_src, cu);
+    int64_t chunks = prism_chunks(n_obs, n_src, cu);
     if (chunk_cap > 0 && chunks > chunk_cap) chunks = chunk_cap;
     if (n_src == 0) {
         // No sources: the reference returns zeros.
@@ -289,10 +335,12 @@ int run_forward(const double *oe, const double *on, const double *ou, int64_t n_
     }
     const size_t need_one = (size_t)chunks * (size_t)n_obs * sizeof(double);
     double *partial = static_cast<double *>(workspace);
-    const bool order = may_order && use_point_order(n_obs, n_src);
     const size_t order_at = point_order_offset(need_one * nf);
-    const size_t need = order ? order_at + point_order_bytes(n_obs)
-                              : (has_kernel(mask) ? need_one * nf : need_one);
+    const size_t with_order = order_at + point_order_bytes(n_obs);
+    const size_t need = chunk_cap == 0 && need_point_order(n_obs, n_src) ? with_order
+                        : has_kernel(mask)                          ? need_one * nf
+                                                                    : need_one;
+    const bool order = use_point_order(n_obs, n_src) && workspace_bytes >= with_order;
     if (!workspace || workspace_bytes < need)
         return fail(HMX_ERR_ARG, "workspace too small: %zu < %zu bytes", workspace_bytes, need);
     const int *perm = nullptr;
@@ -396,7 +444,7 @@ int hmx_prism_gravity_static(const double *easting, const double *northing,
     ExplicitSource src{prisms, density};
     return run_forward(easting, northing, upward, n_obs, src, n_prisms, field_mask, out,
                        singular_flags, ws, (size_t)kStaticScratchDoubles * sizeof(double),
-                       (hipStream_t)stream, kStaticScratchDoubles / per_chunk, false);
+                       (hipStream_t)stream, kStaticScratchDoubles / per_chunk);
 }
 
 int hmx_prism_gravity(const double *easting, const double *northing, const double *upward,

@@ -208,10 +208,9 @@ __device__ __forceinline__ bool any_lane(bool need) { return __any(need) != 0; }
 // two x-planes nor the two y-planes (no mixed quotient, no 2 pi branch);
 // kGenX lifts the first condition (the logarithms along x take their general
 // form; the face angles need the 2 pi branch only between both pairs).
-template <bool kTop, bool kGeneral, bool kShare = false, bool kGenX = kGeneral>
+template <bool kTop, bool kGeneral, bool kGenX = kGeneral>
 __device__ __forceinline__ double gu_sum(double x0, double x1, double y0, double y1, double z0,
-                                         double z1, const dm::Tables &tab, double *ftop,
-                                         int share = 0, double (*rb)[2] = nullptr) {
+                                         double z1, const dm::Tables &tab, double *ftop) {
     const double ys0 = y0 * y0, ys1 = y1 * y1;
     const double zs0 = z0 * z0, zs1 = z1 * z1;
     const double zt0 = z_tiny(zs0), zt1 = z_tiny(zs1);
@@ -224,33 +223,8 @@ __device__ __forceinline__ double gu_sum(double x0, double x1, double y0, double
         for (int j = 0; j < 2; ++j) {
             const double xy = fma(X[i], X[i], YS[j]);
             r[i][j][0] = vertex_r(xy, zt0);
-            if constexpr (!kShare) r[i][j][1] = vertex_r(xy, zt1);
+            r[i][j][1] = vertex_r(xy, zt1);
         }
-    if constexpr (kShare) {
-        // Bottom vertices (k = 1).  share 1: this prism's west edge is the
-        // previous prism's east edge (same S, N, B), so r[1][j][1] equals the
-        // previous r[0][j][1]; share 2: its south edge is the previous north
-        // edge (same W, E, B), so r[i][1][1] equals the previous r[i][0][1].
-        // rb holds the previous prism's bottom distances and receives these.
-        r[0][0][1] = vertex_r(fma(x0, x0, ys0), zt1);
-        if (share == 1) {
-            r[1][0][1] = rb[0][0];
-            r[1][1][1] = rb[0][1];
-            r[0][1][1] = vertex_r(fma(x0, x0, ys1), zt1);
-        } else if (share == 2) {
-            r[0][1][1] = rb[0][0];
-            r[1][1][1] = rb[1][0];
-            r[1][0][1] = vertex_r(fma(x1, x1, ys0), zt1);
-        } else {
-            r[0][1][1] = vertex_r(fma(x0, x0, ys1), zt1);
-            r[1][0][1] = vertex_r(fma(x1, x1, ys0), zt1);
-            r[1][1][1] = vertex_r(fma(x1, x1, ys1), zt1);
-        }
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) rb[i][j] = r[i][j][1];
-    }
     double sum = 0.0, top = 0.0;
     const unsigned flip_y = dm::sign_mask(y0 < 0.0), flip_x = dm::sign_mask(x0 < 0.0);
 #pragma unroll
@@ -623,7 +597,7 @@ __device__ __forceinline__ void prism_pair_path(double e, double n, double u, do
                                                 uint32_t &sflags, const dm::Tables &tab) {
     using F = FieldSet<M>;
     if constexpr (M == 0x8u) {  // g_u alone
-        acc[0] += grho * gu_sum<false, kGeneral, false, kGenX>(E - e, W - e, N - n, S - n, T - u,
+        acc[0] += grho * gu_sum<false, kGeneral, kGenX>(E - e, W - e, N - n, S - n, T - u,
                                                                B - u, tab, nullptr);
     } else if constexpr (M == 0x2u) {  // g_e alone: K_e is K_u with (x, y, z) -> (y, z, x)
         acc[0] += grho * gu_sum<false, kGeneral>(N - n, S - n, T - u, B - u, E - e, W - e, tab,
@@ -662,8 +636,7 @@ __device__ __forceinline__ void prism_pair(double e, double n, double u, double 
 }
 
 // Accumulate the prisms tile[0, cnt) (LDS, read as wave-uniform broadcasts;
-// P has w, e, s, n, b, t, grho, int share and, with kMaySkip, int skip) at
-// (e, n, u).
+// P has w, e, s, n, b, t, grho and, with kMaySkip, int skip) at (e, n, u).
 // Pass 1 evaluates the lean form for every prism that no lane of the wave
 // needs the general form for and marks the others in wave-uniform 128-bit
 // masks: those for which the x-planes alone made the lean form unusable
@@ -679,17 +652,10 @@ __device__ __forceinline__ void tile_pairs(const P *tile, int cnt, double e, dou
                                            double (&acc)[FieldSet<M>::count], uint32_t &sflags,
                                            const dm::Tables &tab) {
     uint64_t general_lo = 0, general_hi = 0, xonly_lo = 0, xonly_hi = 0;
-    // g_u alone: bottom vertex distances of the previous prism evaluated in
-    // this pass, reused where P::share says an edge is shared.
-    double rb[2][2];
-    bool prev_lean = false;
     for (int p = 0; p < cnt; ++p) {
         const P sp = tile[p];
         if constexpr (kMaySkip) {
-            if (sp.skip) {
-                prev_lean = false;
-                continue;
-            }
+            if (sp.skip) continue;
         }
         if (any_lane(needs_general<M>(e, n, u, sp.w, sp.e, sp.s, sp.n, sp.b, sp.t))) {
             bool full = true;
@@ -700,19 +666,10 @@ __device__ __forceinline__ void tile_pairs(const P *tile, int cnt, double e, dou
                 lo |= 1ull << p;
             else
                 hi |= 1ull << (p - 64);
-            prev_lean = false;
             continue;
         }
-        if constexpr (M == 0x8u) {
-            const int share = prev_lean ? __builtin_amdgcn_readfirstlane(sp.share) : 0;
-            acc[0] += sp.grho * gu_sum<false, false, true>(sp.e - e, sp.w - e, sp.n - n, sp.s - n,
-                                                          sp.t - u, sp.b - u, tab, nullptr,
-                                                          share, rb);
-            prev_lean = true;
-        } else {
-            prism_pair_path<M, false>(e, n, u, sp.w, sp.e, sp.s, sp.n, sp.b, sp.t, sp.grho, acc,
-                                      sflags, tab);
-        }
+        prism_pair_path<M, false>(e, n, u, sp.w, sp.e, sp.s, sp.n, sp.b, sp.t, sp.grho, acc,
+                                  sflags, tab);
     }
     if constexpr (has_x_only<M>()) {
         for (int half = 0; half < 2; ++half) {
@@ -736,16 +693,6 @@ __device__ __forceinline__ void tile_pairs(const P *tile, int cnt, double e, dou
                                      sflags, tab);
         }
     }
-}
-
-// Edge sharing between tile[q - 1] and tile[q] for the g_u bottom-vertex
-// reuse: 1 if q's west edge is q - 1's east edge (same S, N, B), 2 if q's
-// south edge is q - 1's north edge (same W, E, B), else 0.
-template <class P>
-__device__ __forceinline__ int shared_edge(const P &prev, const P &cur) {
-    if (cur.w == prev.e && cur.s == prev.s && cur.n == prev.n && cur.b == prev.b) return 1;
-    if (cur.s == prev.n && cur.w == prev.w && cur.e == prev.e && cur.b == prev.b) return 2;
-    return 0;
 }
 
 // Harmonica's sign flip and unit conversion of field f (gravity.py:228-235).

@@ -1,0 +1,503 @@
+// Far form of the prism g_u kernel: the vertical attraction of a prism whose
+// horizontal half-diagonal h is small next to its distance.
+//
+// The sum over the 8 vertices that gu_sum evaluates is
+//   S = int int [1/r_B - 1/r_T] dx dy   over the prism's rectangle,
+// with r_T, r_B the distances to the top and bottom faces (the integral over
+// z is exact, so tall prisms need no other treatment).  With (x, y, z) the
+// face centre seen from the point, s = x^2 + y^2, and a point of the face
+// displaced by d = (dx, dy), s becomes s + delta, delta = 2 (x dx + y dy) +
+// d^2, and Taylor's formula in delta averaged over the rectangle gives
+//   <1/r> = (1/r) [1 + sum_m C_m(x^2, y^2) u^m],  u = 1 / r^2,
+//   C_m = sum_{i + j = m} c_ij,
+//   c_ij = (-1)^m binom(2m, m) 4^(j-m) binom(m, 2j) <(x dx + y dy)^(2j) d^(2(i-j))>
+// where 2i is the order of a term in the size of the rectangle (only even
+// orders survive the average) and 0 <= j <= i.  Orders up to 2I need
+// C_1 .. C_2I.  The C_m are the same for both faces: a face then costs one
+// reciprocal square root and 2I + 2 multiply-adds.
+//
+// Truncation: the omitted order 2I + 2 is the average of |d|^(2I+2) P(cos)
+// / r^(2I+2), at most (h/r)^(2I+2) / (2I + 3) (a rectangle shrunk to a
+// line; 0.6 of that for a square).  far_ratio2 takes the distance from which
+// this is below 4e-15 of 1/r (measured against 40-digit quadrature of
+// squares and thin rectangles at that distance: 3e-16 to 3.6e-15, see the
+// tests).  gu_sum's own error there is larger: its terms are of size r, so
+// it is off by a few 2^-53 r where the face integral is below 4 h^2 / r.
+#pragma once
+
+#include "prism_device.h"
+
+namespace hmx {
+namespace dev {
+
+// Largest I staged and the number of constants c_ijk up to order 2I.
+constexpr int kFarMax = 5;
+constexpr int far_base(int i) {  // index of c_i00
+    int n = 0;
+    for (int t = 1; t < i; ++t) n += (t + 1) * (t + 2) / 2;
+    return n;
+}
+constexpr int far_index(int i, int j, int k) { return far_base(i) + j * (j + 1) / 2 + k; }
+constexpr int kFarConsts = far_base(kFarMax + 1);
+static_assert(kFarConsts == 55, "c_ijk up to i = 5");
+
+constexpr double far_binom(int n, int k) {
+    double b = 1.0;
+    for (int t = 0; t < k; ++t) b = b * (n - t) / (t + 1);
+    return b;
+}
+
+// Factor of X^k Y^(j-k) sum_p binom(i-j, p) mu_i[k+p] in c_ij.
+constexpr double far_factor(int i, int j, int k) {
+    const int m = i + j;
+    double f = far_binom(2 * m, m) * far_binom(m, 2 * j) * far_binom(2 * j, 2 * k);
+    for (int t = 0; t < m - j; ++t) f *= 0.25;
+    return m % 2 ? -f : f;
+}
+
+// The constants of order 2i of a rectangle with squared half-sides A (along
+// x) and B (along y): mu_i[q] = <dx^2q dy^(2i-2q)> = A^q B^(i-q) / ((2q + 1)
+// (2i - 2q + 1)), summed with binomial weights by repeated pairwise addition.
+template <int I>
+__device__ __forceinline__ void far_order_consts(double A, double B, double *c) {
+    double D[I + 1];
+    double pa[I + 1], pb[I + 1];
+    pa[0] = pb[0] = 1.0;
+#pragma unroll
+    for (int q = 1; q <= I; ++q) {
+        pa[q] = pa[q - 1] * A;
+        pb[q] = pb[q - 1] * B;
+    }
+#pragma unroll
+    for (int q = 0; q <= I; ++q)
+        D[q] = pa[q] * pb[I - q] * (1.0 / ((2 * q + 1) * (2 * I - 2 * q + 1)));
+#pragma unroll
+    for (int j = I; j >= 0; --j) {
+#pragma unroll
+        for (int k = 0; k <= j; ++k) c[far_index(I, j, k)] = far_factor(I, j, k) * D[k];
+#pragma unroll
+        for (int q = 0; q < j; ++q) D[q] = D[q] + D[q + 1];
+    }
+}
+
+// C_1 .. C_2I at X = x^2, Y = y^2; c(index) gives a constant.
+template <int I, class Consts>
+__device__ __forceinline__ void far_coefs(double X, double Y, const Consts &c,
+                                          double (&C)[2 * I + 1]) {
+    double mono[I + 1][I + 1];  // X^k Y^(j-k)
+    mono[0][0] = 1.0;
+#pragma unroll
+    for (int j = 1; j <= I; ++j) {
+        mono[j][0] = j == 1 ? Y : mono[j - 1][0] * Y;
+#pragma unroll
+        for (int k = 1; k <= j; ++k) mono[j][k] = j == 1 ? X : mono[j - 1][k - 1] * X;
+    }
+    // order by order, so that few constants are in registers at a time
+#pragma unroll
+    for (int i = 1; i <= I; ++i) {
+        C[2 * i] = C[2 * i - 1] = 0.0;
+#pragma unroll
+        for (int j = 0; j <= i; ++j) {
+            // the first order to reach C_m is i = ceil(m / 2), with j = m - i
+            const bool first = i == (i + j + 1) / 2;
+#pragma unroll
+            for (int k = 0; k <= j; ++k) {
+                const double ck = c(far_index(i, j, k));
+                if (j == 0)
+                    C[i] = first ? ck : C[i] + ck;
+                else if (first && k == 0)
+                    C[i + j] = ck * mono[j][k];
+                else
+                    C[i + j] = fma(ck, mono[j][k], C[i + j]);
+            }
+        }
+        if constexpr (I >= 4) __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// <1/r> over the face at height z, s = x^2 + y^2.
+template <int I>
+__device__ __forceinline__ double far_face(double s, double z, const double (&C)[2 * I + 1]) {
+    const double inv = dm::rsqrt_pos(fma(z, z, s));
+    const double u = inv * inv;
+    double p = C[2 * I];
+#pragma unroll
+    for (int m = 2 * I - 1; m >= 1; --m) p = fma(p, u, C[m]);
+    return fma(inv, p * u, inv);
+}
+
+// Square of the distance, in units of the half-diagonal h of the rectangle,
+// from which order 2I suffices: (1 / ((2I + 3) 4e-15))^(1 / (2I + 2)) =
+// 181, 48, 21.8, 12.9 for I = 2, 3, 4, 5.
+__device__ __forceinline__ constexpr double far_ratio2(int I) {
+    return I == 2 ? 181.0 * 181.0 : I == 3 ? 48.0 * 48.0 : I == 4 ? 21.8 * 21.8 : 12.9 * 12.9;
+}
+
+// A staged far prism: the rectangle's centre from the workgroup's origin, top,
+// bottom, weight times area, h^2 = A + B.  The centre is formed from bounds
+// already shifted to the origin, so its rounding is relative to its distance
+// from the workgroup's points and not to the coordinates' size.
+struct alignas(16) FarPrism {
+    double x, y, t, b, w, h2;
+};
+
+// Constants in LDS (kept per prism: stride kFarStride) or, for a tile of
+// equal rectangles, in scalar registers.
+constexpr int kFarStride = kFarConsts + 1;  // even: 16-byte aligned pairs
+struct FarLds {
+    const double *c;
+    __device__ __forceinline__ double operator()(int k) const { return c[k]; }
+};
+__device__ __forceinline__ double wave_uniform(double v) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+template <int I>
+struct FarScalar {
+    double c[far_base(I + 1)];
+    __device__ __forceinline__ explicit FarScalar(const double *lds) {
+#pragma unroll
+        for (int k = 0; k < far_base(I + 1); ++k) c[k] = wave_uniform(lds[k]);
+    }
+    __device__ __forceinline__ double operator()(int k) const { return c[k]; }
+};
+
+// weight * S of the staged prism at (x, y, u), x and y relative to the
+// workgroup's origin.
+template <int I, class Consts>
+__device__ __forceinline__ double far_gz(const FarPrism &rec, const Consts &c, double px, double py,
+                                         double pu) {
+    const double x = rec.x - px, y = rec.y - py;
+    const double X = x * x, Y = y * y, s = X + Y;
+    double C[2 * I + 1];
+    far_coefs<I>(X, Y, c, C);
+    return rec.w * (far_face<I>(s, rec.b - pu, C) - far_face<I>(s, rec.t - pu, C));
+}
+
+// Bounding box of the points of a wave (x and y relative to the origin).
+struct FarBox {
+    double x0, x1, y0, y1, u0, u1;
+};
+
+// Smallest squared distance from the box to the nearer face centre of a
+// staged prism; NaN (never far) if the prism or the whole box is NaN.
+__device__ __forceinline__ double far_distance2(const FarBox &b, const FarPrism &p) {
+    // fmax drops a NaN operand: keep it with the sum of the differences
+    const double nan_guard = ((p.x - b.x0) + (p.y - b.y0) + (p.t - b.u0) + (p.b - b.u0)) * 0.0;
+    const double dx = fmax(fmax(b.x0 - p.x, p.x - b.x1), 0.0);
+    const double dy = fmax(fmax(b.y0 - p.y, p.y - b.y1), 0.0);
+    const double dt = fmax(fmax(b.u0 - p.t, p.t - b.u1), 0.0);
+    const double db = fmax(fmax(b.u0 - p.b, p.b - b.u1), 0.0);
+    const double d = fmin(dt, db);
+    return fma(dx, dx, fma(dy, dy, d * d)) + nan_guard;
+}
+
+// Whether order 2I serves a prism at squared distance d2 (the upper bound
+// keeps the monomials of the constants finite).
+template <int I>
+__device__ __forceinline__ bool far_enough(double d2, double h2) {
+    return d2 >= far_ratio2(I) * h2 && d2 < 1e50;
+}
+
+// Prisms staged per pass of the g_u kernels, at most one per lane of a wave,
+// so that a wave sorts a tile into the forms with one comparison and one
+// ballot; with 32 a workgroup's LDS (27 KB) lets registers, not LDS, set the
+// waves per SIMD.
+constexpr int kGzTile = 32;
+constexpr int kGzWaves = 4;
+constexpr int kGzThreads = 64 * kGzWaves;
+constexpr int kGzList = 256;
+
+// One staged prism of the closed form: bounds and weight.
+struct alignas(16) GzPrism {
+    double w, e, s, n, b, t, grho, pad;
+};
+
+// Prisms given as (m, 6) rows [W, E, S, N, B, T] and densities, for gz_stage.
+struct GzExplicit {
+    const double *prisms, *density;
+    __device__ bool get(int64_t p, double (&b)[6], double &rho) const {
+#pragma unroll
+        for (int c = 0; c < 6; ++c) b[c] = prisms[6 * p + c];
+        rho = density[p];
+        return false;
+    }
+};
+
+// LDS of a g_u workgroup, one point per lane.
+struct GzShared {
+    GzPrism tile[kGzTile];
+    FarPrism far[kGzTile];
+    // constants per prism, if the rectangles differ; the last entry holds
+    // those of the workgroup's first prism
+    alignas(16) double consts[(kGzTile + 1) * kFarStride];
+    FarBox box[kGzWaves];
+    double A, B;        // squared half-sides of the last entry
+    unsigned live;      // prisms of the tile that are not left out
+    unsigned different; // 0: every live prism has the last entry's rectangle
+    // closed-form pairs of a wave and their values (gz_close)
+    uint16_t list[kGzWaves][kGzList];
+    double value[kGzWaves][64];
+    dm::Tables tables;
+};
+
+__device__ __forceinline__ double wave_min(double v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o));
+    return v;
+}
+__device__ __forceinline__ double wave_max(double v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o));
+    return v;
+}
+
+// A lane's point: as given, and relative to the workgroup's origin (xo, yo).
+struct GzPoint {
+    double e, n, u, x, y, xo, yo;
+};
+
+// Bounding box of the wave's points into sh.box (read after the next
+// barrier).
+__device__ __forceinline__ void gz_box(const GzPoint &pt, GzShared &sh) {
+    const FarBox b{wave_min(pt.x), wave_max(pt.x), wave_min(pt.y),
+                   wave_max(pt.y), wave_min(pt.u), wave_max(pt.u)};
+    if ((threadIdx.x & 63) == 0) sh.box[threadIdx.x >> 6] = b;
+}
+
+// All constants of a rectangle, in three parts of similar cost.
+__device__ __forceinline__ void far_consts(double A, double B, int part, double *c) {
+    if (part == 0) {
+        far_order_consts<1>(A, B, c);
+        far_order_consts<2>(A, B, c);
+        far_order_consts<3>(A, B, c);
+    } else if (part == 1) {
+        far_order_consts<4>(A, B, c);
+    } else {
+        far_order_consts<5>(A, B, c);
+    }
+}
+
+// Squared half-sides of a prism's rectangle.
+__device__ __forceinline__ void half_sides2(const double (&b)[6], double &A, double &B) {
+    const double width = b[1] - b[0], length = b[3] - b[2];
+    A = 0.25 * width * width;
+    B = 0.25 * length * length;
+}
+
+// The last entry of constants from prism p (the first of the workgroup's chunk).
+template <class Src>
+__device__ __forceinline__ void gz_table(const Src &src, int64_t p, GzShared &sh) {
+    if (threadIdx.x < 3) {
+        double b[6], rho, A, B;
+        src.get(p, b, rho);
+        half_sides2(b, A, B);
+        far_consts(A, B, threadIdx.x, sh.consts + kGzTile * kFarStride);
+        if (threadIdx.x == 0) {
+            sh.A = A;
+            sh.B = B;
+        }
+    }
+}
+
+// Stages prisms [t0, t0 + cnt), cnt <= kGzTile.  Src::get(p, bounds, rho)
+// returns whether the prism is left out.  Holds every barrier it needs before
+// and after.  Grids of equal cells, by far the most common layers, use the
+// last entry's constants (equal to 2^-36: they scale corrections below
+// (h/r)^2 / 3, so that is a relative 1e-14 at the shortest distance); a tile
+// with other rectangles gets its own constants, prism by prism.
+template <class Src>
+__device__ __forceinline__ void gz_stage(const Src &src, int64_t t0, int cnt, double xo, double yo,
+                                         GzShared &sh) {
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        const int q = threadIdx.x;
+        double b[6] = {}, rho = 0.0;
+        bool skip = true;
+        if (q < cnt) skip = src.get(t0 + q, b, rho);
+        double A, B;
+        half_sides2(b, A, B);
+        if (q < cnt) {
+            sh.tile[q] = GzPrism{b[0], b[1], b[2], b[3], b[4], b[5], kG * rho, 0.0};
+            sh.far[q] = FarPrism{0.5 * ((b[0] - xo) + (b[1] - xo)),
+                                 0.5 * ((b[2] - yo) + (b[3] - yo)), b[5], b[4],
+                                 kG * rho * ((b[1] - b[0]) * (b[3] - b[2])), A + B};
+        }
+        const bool same = fabs(A - sh.A) <= 0x1p-36 * sh.A && fabs(B - sh.B) <= 0x1p-36 * sh.B;
+        const uint64_t live = __ballot(!skip), different = __ballot(!skip && !same);
+        if (q == 0) {
+            sh.live = (unsigned)live;
+            sh.different = different ? 1u : 0u;
+        }
+    }
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(sh.different)) {
+        // one part per half wave
+        static_assert(kGzTile == 32 && kGzThreads >= 96, "room for three parts");
+        const int q = threadIdx.x & 31, part = threadIdx.x >> 5;
+        if (q < cnt && part < 3) {
+            double A, B;
+            const GzPrism &t = sh.tile[q];
+            const double b[6] = {t.w, t.e, t.s, t.n, 0.0, 0.0};
+            half_sides2(b, A, B);
+            far_consts(A, B, part, sh.consts + q * kFarStride);
+        }
+        __syncthreads();
+    }
+}
+
+// Whether order 10 serves the lane's own point.
+__device__ __forceinline__ bool lane_is_far(const FarPrism &p, double px, double py, double pu) {
+    const double x = p.x - px, y = p.y - py, t = p.t - pu, z = p.b - pu;
+    return far_enough<5>(fma(x, x, fma(y, y, fmin(t * t, z * z))), p.h2);
+}
+
+// Calls f(p) for the set bits p of a wave-uniform mask, in order.
+template <class F>
+__device__ __forceinline__ void for_bits(unsigned mask, const F &f) {
+    while (mask) {
+        const int p = __builtin_ctz(mask);
+        mask &= mask - 1;
+        f(p);
+    }
+}
+
+// Orders a wave's own LDS writes before its reads (the wave's LDS operations
+// complete in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The constants of prism p of the tile (different: 0 or 1).
+__device__ __forceinline__ const double *gz_consts(const double *consts, int p,
+                                                   unsigned different) {
+    return consts + (kGzTile + (p - kGzTile) * (int)different) * kFarStride;
+}
+
+// Adds the closed form of the pairs in `mask` (bit p: prism p of the tile at
+// the lane's point).  The wave's pairs are listed by lane and prism and
+// evaluated 64 at a time, one pair per lane whoever's it is, and each lane
+// adds the values of its own pairs in order.  Always the general closed
+// form: listed pairs lie between the prism's planes too often for 64 of them
+// to need the lean one.
+__device__ __forceinline__ void gz_close(GzShared &sh, unsigned mask, const GzPoint &pt,
+                                         double &acc) {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    uint16_t *list = sh.list[wave];
+    double *value = sh.value[wave];
+    while (any_lane(mask != 0)) {
+        const int count = __popc(mask);
+        int incl = count;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int v = __shfl_up(incl, o);
+            if (lane >= o) incl += v;
+        }
+        const int total = __builtin_amdgcn_readlane(incl, 63);
+        const int n = total < kGzList ? total : kGzList;
+        // the lane's entries [at, end); pairs past the list's end wait for the
+        // next round
+        const int at = incl - count < kGzList ? incl - count : kGzList;
+        int end = at;
+        while (mask && end < kGzList) {
+            list[end++] = (uint16_t)((unsigned)__builtin_ctz(mask) | lane << 5);
+            mask &= mask - 1;
+        }
+        wave_sync();
+        for (int b = 0; b < n; b += 64) {
+            const unsigned pair = list[b + lane < n ? b + lane : b];
+            const int from = pair >> 5;
+            const double e = __shfl(pt.e, from), nn = __shfl(pt.n, from), u = __shfl(pt.u, from);
+            const GzPrism sp = sh.tile[pair & 31u];
+            value[lane] = sp.grho * gu_sum<false, true>(sp.e - e, sp.w - e, sp.n - nn, sp.s - nn,
+                                                        sp.t - u, sp.b - u, sh.tables, nullptr);
+            wave_sync();
+            for (int k = at > b ? at : b; k < end && k < b + 64; ++k) acc += value[k - b];
+            wave_sync();
+        }
+    }
+}
+
+// Close lanes from which a wave evaluates the lean closed form for all its
+// lanes rather than list its pairs (about 300 against 400 issue slots).
+constexpr int kGzInline = 40;
+
+// Adds the prisms of `near`, which the bounding box does not show to be far
+// from all of the wave's points.  Each lane takes order 10 where its own
+// distance allows and the closed form elsewhere, so the form of a pair does
+// not depend on the points that share its wave (bar the orders of the far
+// form, which agree to 4e-15) and neither, to rounding, does the result on
+// their order.
+__device__ __forceinline__ void gz_near(GzShared &sh, unsigned near, unsigned different,
+                                        const GzPoint &pt, double &acc) {
+    unsigned mask = 0;
+    for_bits(near, [&](int p) {
+        const FarPrism rec = sh.far[p];
+        const bool close = !lane_is_far(rec, pt.x, pt.y, pt.u);
+        if (any_lane(!close)) {
+            const double v =
+                far_gz<5>(rec, FarLds{gz_consts(sh.consts, p, different)}, pt.x, pt.y, pt.u);
+            acc += close ? 0.0 : v;
+        }
+        const GzPrism sp = sh.tile[p];
+        if (__popcll(__ballot(close)) >= kGzInline &&
+            !any_lane(close && needs_general<0x8u>(pt.e, pt.n, pt.u, sp.w, sp.e, sp.s, sp.n, sp.b,
+                                                   sp.t))) {
+            const double v = sp.grho * gu_sum<false, false>(sp.e - pt.e, sp.w - pt.e, sp.n - pt.n,
+                                                            sp.s - pt.n, sp.t - pt.u, sp.b - pt.u,
+                                                            sh.tables, nullptr);
+            acc += close ? v : 0.0;
+        } else {
+            mask |= close ? 1u << p : 0u;
+        }
+    });
+    gz_close(sh, mask, pt, acc);
+}
+
+// One order of the far form, its constants in scalar registers where the
+// tile's rectangles are equal (up to order 6: 19 constants; the 34 of order 8
+// do not fit beside the rest).
+template <int I>
+__device__ __forceinline__ void gz_far(const GzShared &sh, unsigned different, unsigned mask,
+                                       const GzPoint &pt, double &acc) {
+    if (!mask) return;
+    if constexpr (I <= 3) {
+        if (!different) {
+            const FarScalar<I> c(sh.consts + kGzTile * kFarStride);
+            for_bits(mask, [&](int p) { acc += far_gz<I>(sh.far[p], c, pt.x, pt.y, pt.u); });
+            return;
+        }
+    }
+    for_bits(mask, [&](int p) {
+        acc += far_gz<I>(sh.far[p], FarLds{gz_consts(sh.consts, p, different)}, pt.x, pt.y, pt.u);
+    });
+}
+
+// Adds the g_u of the staged tile at the wave's points.  The forms are chosen
+// per prism and wave from the distance between the prism's face centres and
+// the bounding box of the wave's points: the lowest order that serves all of
+// them, uniform in the wave; then the prisms nearer than that, lane by lane.
+__device__ __forceinline__ void gz_tile(int cnt, const GzPoint &pt, double &acc, GzShared &sh) {
+    const int q = threadIdx.x & 63;
+    const unsigned live = __builtin_amdgcn_readfirstlane(sh.live);
+    const unsigned different = __builtin_amdgcn_readfirstlane(sh.different);
+    const FarPrism mine = sh.far[q < cnt ? q : 0];
+    const double d2 = far_distance2(sh.box[threadIdx.x >> 6], mine);
+    unsigned rest = live;
+    auto take = [&](bool far) {
+        const unsigned m = (unsigned)__ballot(far) & rest;
+        rest &= ~m;
+        return m;
+    };
+    const unsigned m2 = take(far_enough<2>(d2, mine.h2)), m3 = take(far_enough<3>(d2, mine.h2));
+    const unsigned m4 = take(far_enough<4>(d2, mine.h2)), m5 = take(far_enough<5>(d2, mine.h2));
+    gz_far<2>(sh, different, m2, pt, acc);
+    gz_far<3>(sh, different, m3, pt, acc);
+    gz_far<4>(sh, different, m4, pt, acc);
+    gz_far<5>(sh, different, m5, pt, acc);
+    if (rest) gz_near(sh, rest, different, pt, acc);
+}
+
+}  // namespace dev
+}  // namespace hmx

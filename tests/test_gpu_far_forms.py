@@ -1,0 +1,151 @@
+"""
+Far forms of the prism kernels (prism_far.h) against extended precision
+(numpy.longdouble, 2^-63; the closed form for near pairs, quadrature for far
+ones): models whose pairs fall on both
+sides of every order's distance, tiles of 1 to 65 prisms (a tile holds 32),
+equal and different rectangles, thin and zero-width rectangles, coordinates
+far from the origin, more close pairs per wave than its list holds, left-out
+layer cells and points with NaN.
+
+Tolerances, before the first run: a far pair is off by a few roundings of
+its two face terms w A / r (16 x 2^-53 of their sum; the truncation is below
+4e-15 = 36 x 2^-53 of each), a closed pair by a few roundings of its terms
+of size w r ln (64 x 2^-53 w r); the sums add the magnitudes (random signs
+only make the error smaller).
+"""
+
+import numpy as np
+import numpy.testing as npt
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+G = 6.6743e-11
+
+
+@pytest.fixture(scope="module")
+def hm():
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import harmonica_amd
+
+    return harmonica_amd
+
+
+def _gz_exact(coords, prisms, density):
+    """(g_z, error bound) in mGal."""
+    ld = np.longdouble
+    e, n, u = (np.asarray(c, dtype=ld)[:, None] for c in coords)
+    p = prisms.astype(ld)
+    total = np.zeros((e.shape[0], p.shape[0]), dtype=ld)
+    for i, x in enumerate((p[:, 1] - e, p[:, 0] - e)):
+        for j, y in enumerate((p[:, 3] - n, p[:, 2] - n)):
+            for k, z in enumerate((p[:, 5] - u, p[:, 4] - u)):
+                r = np.sqrt(x * x + y * y + z * z)
+                with np.errstate(all="ignore"):
+                    lx = np.where(x >= 0, np.log(r + x), np.log((y * y + z * z) / (r - x)))
+                    ly = np.where(y >= 0, np.log(r + y), np.log((x * x + z * z) / (r - y)))
+                    v = -(x * ly + y * lx - z * np.arctan2(x * y, z * r))
+                total += (-1) ** (i + j + k) * np.where(np.isfinite(v), v, 0)
+    # arctan2 above is the principal arctangent only for z r > 0: undo its
+    # branch for z < 0 (x y / (z r) is what the closed form takes)
+    for i, x in enumerate((p[:, 1] - e, p[:, 0] - e)):
+        for j, y in enumerate((p[:, 3] - n, p[:, 2] - n)):
+            for k, z in enumerate((p[:, 5] - u, p[:, 4] - u)):
+                branch = np.where(z < 0, np.where(x * y >= 0, 1, -1), 0)
+                total -= (-1) ** (i + j + k) * z * branch * np.arctan2(ld(0), ld(-1))
+    area = (p[:, 1] - p[:, 0]) * (p[:, 3] - p[:, 2])
+    half2 = ((p[:, 1] - p[:, 0]) ** 2 + (p[:, 3] - p[:, 2]) ** 2) / 4
+    dx, dy = (p[:, 0] + p[:, 1]) / 2 - e, (p[:, 2] + p[:, 3]) / 2 - n
+    rt, rb = (np.sqrt(dx * dx + dy * dy + (z - u) ** 2) for z in (p[:, 5], p[:, 4]))
+    far = np.minimum(rt, rb) ** 2 >= 12.0**2 * half2
+    # far pairs, where the closed form cancels even in extended precision: the
+    # integral over the faces by 10 x 10 Gauss-Legendre nodes ((1 / 12)^20)
+    x10, w10 = np.polynomial.legendre.leggauss(10)
+    quad = np.zeros_like(total)
+    for xa, wa in zip(x10.astype(ld), w10.astype(ld)):
+        for xb, wb in zip(x10.astype(ld), w10.astype(ld)):
+            s = (dx + xa * (p[:, 1] - p[:, 0]) / 2) ** 2 + (dy + xb * (p[:, 3] - p[:, 2]) / 2) ** 2
+            quad += wa * wb / 4 * (1 / np.sqrt(s + (p[:, 4] - u) ** 2)
+                                   - 1 / np.sqrt(s + (p[:, 5] - u) ** 2))
+    total = np.where(far, quad * area, total)  # upward component of the attraction
+    w = np.abs(1e5 * G * density)
+    area = np.abs(area)
+    # the kernels take the far form from 12.9 half-diagonals
+    far = np.minimum(rt, rb) ** 2 >= 12.9**2 * half2
+    bound = np.where(far, 52 * (area / rt + area / rb), 64 * (np.maximum(rt, rb) + np.sqrt(half2)))
+    eps = ld(2) ** -53
+    return ((total * (-1e5 * G * density)).sum(axis=1).astype(float),
+            (bound * w * eps).sum(axis=1).astype(float))
+
+
+def _model(kind, m, rng):
+    """(m, 6) prisms around the origin, sides about 100."""
+    if kind == "grid":
+        side = int(np.ceil(np.sqrt(m)))
+        k = np.arange(m)
+        x, y = 100.0 * (k % side), 100.0 * (k // side)
+        sx = sy = np.full(m, 100.0)
+    else:
+        x, y = rng.uniform(0, 3e3, m), rng.uniform(0, 3e3, m)
+        sx, sy = rng.uniform(20, 200, m), rng.uniform(20, 200, m)
+        if kind == "thin":
+            sx, sy[::3] = np.full(m, 1e-3), 300.0
+    t = rng.uniform(-400, 0, m)
+    return np.column_stack([x, x + sx, y, y + sy, t - rng.uniform(10, 3000, m), t])
+
+
+@pytest.mark.parametrize("kind", ["grid", "different", "thin"])
+@pytest.mark.parametrize("m", [1, 31, 32, 33, 65, 400])
+def test_gz_all_distances(hm, kind, m):
+    """Points at 30 m to 100 km from the model (all orders and the closed
+    form), in two orders: along the distance, and shuffled so that every wave
+    holds near and far points (its close pairs go through the list)."""
+    rng = np.random.default_rng(m)
+    prisms = _model(kind, m, rng)
+    density = rng.uniform(100, 500, m)
+    d, phi = np.geomspace(30.0, 1e5, 333), rng.uniform(0, 2 * np.pi, 333)
+    coords = (50.0 + d * np.cos(phi), 50.0 + d * np.sin(phi), rng.uniform(5.0, 300.0, 333))
+    expected, bound = _gz_exact(coords, prisms, density)
+    got = hm.prism_gravity(coords, prisms, density, field="g_z")
+    assert (np.abs(got - expected) <= bound).all()
+    order = rng.permutation(333)
+    mixed = hm.prism_gravity(tuple(c[order] for c in coords), prisms, density, field="g_z")
+    assert (np.abs(mixed - expected[order]) <= bound[order]).all()
+    npt.assert_allclose(mixed, got[order], rtol=0, atol=2.0 * bound.max())
+
+
+def test_gz_far_from_the_origin(hm):
+    """UTM-like coordinates: the far form's centre must not round to them."""
+    rng = np.random.default_rng(3)
+    prisms = _model("different", 300, rng)
+    density = rng.uniform(100, 500, 300)
+    coords = (rng.uniform(-2e4, 2e4, 200), rng.uniform(-2e4, 2e4, 200), rng.uniform(1, 900, 200))
+    shift = np.array([612345.678, 612345.678, 7123456.789, 7123456.789, 0, 0])
+    moved = prisms + shift  # rounds: take what the rounded bounds give
+    coords = (coords[0] + shift[0], coords[1] + shift[2], coords[2])
+    expected, bound = _gz_exact(coords, moved, density)
+    got = hm.prism_gravity(coords, moved, density, field="g_z")
+    assert (np.abs(got - expected) <= bound).all()
+
+
+def test_gz_layer_skips_and_nan_points(hm):
+    """A layer with NaN cells: the same as its remaining prisms; a NaN point
+    gives NaN at its own place only."""
+    rng = np.random.default_rng(4)
+    e, n = np.arange(40) * 100.0, np.arange(37) * 80.0
+    surface = rng.uniform(100, 900, (37, 40))
+    surface[rng.random(surface.shape) < 0.3] = np.nan
+    density = rng.uniform(2000, 3000, surface.shape)
+    layer = hm.prism_layer((e, n), surface, 0.0, properties={"density": density})
+    coords = [rng.uniform(-3e3, 7e3, 150), rng.uniform(-3e3, 7e3, 150), rng.uniform(950, 2e3, 150)]
+    coords[1][7] = np.nan
+    got = layer.prism_layer.gravity(coords, field="g_z")
+    prisms = layer.prism_layer._to_prisms()
+    keep = ~np.isnan(surface.ravel())
+    expected, bound = _gz_exact(coords, prisms[keep], density.ravel()[keep])
+    ok = np.arange(150) != 7
+    assert np.isnan(got[7])
+    assert (np.abs(got - expected) <= bound)[ok].all()
