@@ -126,6 +126,25 @@ __device__ __forceinline__ double far_face(double s, double z, const double (&C)
     return fma(inv, p * u, inv);
 }
 
+// <1/r> and its derivative -d<1/r>/dz / z = <1/r^3> (the sums over m with C_m
+// and (2m + 1) C_m: Horner's scheme for the polynomial and its derivative).
+template <int I>
+__device__ __forceinline__ void far_face_top(double s, double z, const double (&C)[2 * I + 1],
+                                             double &f, double &f3) {
+    const double inv = dm::rsqrt_pos(fma(z, z, s));
+    const double u = inv * inv;
+    double p = C[2 * I], d = C[2 * I];
+#pragma unroll
+    for (int m = 2 * I - 1; m >= 1; --m) {
+        p = fma(p, u, C[m]);
+        d = fma(d, u, p);
+    }
+    // p = sum C_m u^(m-1), d = its derivative's scheme: sum m C_m u^(m-1)
+    const double inv3 = inv * u;
+    f = fma(inv, p * u, inv);
+    f3 = fma(inv3, u * fma(2.0, d, p), inv3);
+}
+
 // Square of the distance, in units of the half-diagonal h of the rectangle,
 // from which order 2I suffices: (1 / ((2I + 3) 4e-15))^(1 / (2I + 2)) =
 // 181, 48, 21.8, 12.9 for I = 2, 3, 4, 5.
@@ -353,10 +372,10 @@ __device__ __forceinline__ bool lane_is_far(const FarPrism &p, double px, double
 }
 
 // Calls f(p) for the set bits p of a wave-uniform mask, in order.
-template <class F>
-__device__ __forceinline__ void for_bits(unsigned mask, const F &f) {
+template <class Mask, class F>
+__device__ __forceinline__ void for_bits(Mask mask, const F &f) {
     while (mask) {
-        const int p = __builtin_ctz(mask);
+        const int p = sizeof(Mask) == 8 ? __builtin_ctzll(mask) : __builtin_ctz((unsigned)mask);
         mask &= mask - 1;
         f(p);
     }
