@@ -71,6 +71,7 @@ SIGNATURES = {
     "hmx_lsq_svd_workspace_bytes": (_int, [_i64, _i64, _szp]),
     "hmx_lsq_svd": (_int, [_vp, _i64, _i64, _vp, _dbl, _int, _dbl, _vp, _vp,
                            ctypes.POINTER(ctypes.c_double), _vp, ctypes.c_size_t, _vp]),
+    "hmx_tesseroid_points_inside": (_int, [_vp, _vp, _vp, _vp, _i64, _vp, _i64, _vp, _vp]),
     "hmx_tesseroid_workspace_bytes": (_int, [_i64, _i64, _szp]),
     "hmx_tesseroid_gravity": (_int, [_vp, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _u32, _int, _vp,
                                      _vp, _vp, ctypes.c_size_t, _vp]),

@@ -187,6 +187,18 @@ int hmx_prism_magnetic(const double *easting, const double *northing, const doub
                        int64_t n_prisms, uint32_t component_mask, double *out, void *workspace,
                        size_t workspace_bytes, void *stream);
 
+/* Whether any point lies strictly inside a tesseroid (replaces
+ * check_points_outside_tesseroids, src/harmonica/_forward/_tesseroid_utils.py,
+ * for models without conflicts; the caller lists the conflicts otherwise).
+ *   longitude_180, longitude_360: the points' longitudes [deg] moved to
+ *     [-180, 180) and to [0, 360); latitude [deg], radius [m];
+ *   tesseroids: (n_tesseroids, 6) as hmx_tesseroid_gravity;
+ *   flag: device int, OR-ed with 1 if there is one; the caller clears it. */
+int hmx_tesseroid_points_inside(const double *longitude_180, const double *longitude_360,
+                                const double *latitude, const double *radius, int64_t n_obs,
+                                const double *tesseroids, int64_t n_tesseroids, int *flag,
+                                void *stream);
+
 /* Bytes of workspace needed by hmx_tesseroid_gravity. */
 int hmx_tesseroid_workspace_bytes(int64_t n_obs, int64_t n_tesseroids, size_t *bytes);
 

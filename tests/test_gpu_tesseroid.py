@@ -319,3 +319,45 @@ def test_tesseroid_layer_holes_and_threshold(hm):
     got = layer.tesseroid_layer.gravity(coordinates, field="g_z", thickness_threshold=100.0)
     tess = [layer.tesseroid_layer.get_tesseroid((i, j)) for i in range(1, 6) for j in range(5)]
     npt.assert_allclose(got, hm.tesseroid_gravity(coordinates, tess, [2670.0] * 25, field="g_z"))
+
+
+@pytest.mark.parametrize("field", ["potential", "g_z"])
+@pytest.mark.parametrize("m", [1, 31, 32, 33, 65])
+def test_divided_and_undivided_pairs(hm, field, m):
+    """Models of 1 to 65 tesseroids (a tile holds 32) of 0.02 to 3 degrees, at
+    points from 3 km above them to half a turn away: pairs that divide the
+    tesseroid (more than a wave's list of 256 holds), undivided ones nearer and
+    farther than 0.02 radii, in shuffled order.  Against the oracle at this
+    file's 1e-9: the far pairs' 1 - cos(psi) is at least 2e-4, where the
+    reference's form is good to 1e-12, and the others use that form."""
+    rng = np.random.default_rng(m)
+    w, s = rng.uniform(-4, 4, m), rng.uniform(-4, 4, m)
+    size = rng.choice([0.02, 0.3, 1.0, 3.0], (m, 2)) * rng.uniform(0.9, 1.1, (m, 2))
+    top = 6.371e6 + rng.uniform(-4e3, 2e3, m)
+    tess = np.column_stack([w, w + size[:, 0], s, s + size[:, 1], top - rng.uniform(1e3, 3e4, m),
+                            top])
+    density = rng.uniform(2000, 3000, m)
+    n = 300
+    coords = (np.r_[rng.uniform(-6, 7, 200), rng.uniform(-180, 180, 100)],
+              np.r_[rng.uniform(-6, 7, 200), rng.uniform(-90, 90, 100)],
+              6.371e6 + rng.uniform(5e3, 3e5, n))
+    order = rng.permutation(n)
+    coords = tuple(c[order] for c in coords)
+    got = hm.tesseroid_gravity(coords, tess, density, field)
+    expected = oracle.tesseroid_gravity(coords, tess, density, field)
+    npt.assert_allclose(got, expected, rtol=0, atol=TOL * np.abs(expected).max())
+
+
+@pytest.mark.parametrize("longitude", [10.5, 370.5 - 360.0, -349.5])
+def test_point_inside_found_on_the_device(hm, longitude):
+    """One point inside one of 200 tesseroids: the GPU check (enough pairs for
+    it) leads to the host's message; on a boundary it is outside."""
+    w = np.arange(200) * 0.5
+    tess = np.column_stack([w, w + 0.5, np.full(200, -1.0), np.full(200, 1.0),
+                            np.full(200, 6.3e6), np.full(200, 6.371e6)])
+    coords = [np.linspace(0, 99, 400), np.zeros(400), np.full(400, 6.4e6)]
+    coords[0][123], coords[2][123] = longitude + 0.25, 6.35e6
+    with pytest.raises(ValueError, match=r"Computation point '\(.*6350000.0\)'"):
+        hm.tesseroid_gravity(coords, tess, np.ones(200), "g_z")
+    coords[1][123] = 1.0  # on the northern boundary
+    assert np.isfinite(hm.tesseroid_gravity(coords, tess, np.ones(200), "g_z")).all()
