@@ -10,14 +10,12 @@
 // src/harmonica/_forward/prisms/magnetic.py:319-331 (field "b") and
 // :384-397 (one component) and the nT conversion of :195-197 and :271.
 //
-// Launch shape as the gravity forward kernel: 256 points per workgroup (one
-// per lane), prisms staged in LDS tiles of 128 and read as wave-uniform
-// broadcasts, each tile in two passes (lean closed form for the prisms no
-// lane of the wave needs the general form for, then the general form), one
-// chunk of the prism list per workgroup column, chunk partial sums reduced
-// in order by a second kernel (deterministic results).
+// Launch and forms as the gravity kernels (prism_fields_far.h): 256 points per
+// workgroup, one per lane, tiles of 32 prisms in LDS, far form or closed form
+// by distance, one chunk of the prism list per workgroup column, chunk
+// partial sums reduced in order by a second kernel (deterministic results).
 #include "hmx_internal.h"
-#include "prism_device.h"
+#include "prism_fields_far.h"
 
 namespace hmx {
 namespace {
@@ -28,14 +26,6 @@ constexpr double kPi = 3.141592653589793;
 // mu_0 / 4 / pi with mu_0 = 4 pi 1e-7, evaluated in that order.
 constexpr double kCm = 4.0 * kPi * 1e-7 / 4.0 / kPi;
 
-// One staged prism (80 bytes): bounds and c_m times the magnetisation.
-struct alignas(16) StagedMagPrism {
-    double w, e, s, n, b, t, me, mn, mu;
-    int pad0, pad1;
-};
-static_assert(sizeof(StagedMagPrism) == 80, "staged prism layout");
-static_assert(kTile <= 128, "the two-pass tile loop marks at most 128 prisms");
-
 // Components selected by bit c of C (0 = b_e, 1 = b_n, 2 = b_u) and the
 // tensor kernels (gravity field bits 4..9) they need.
 template <unsigned C>
@@ -45,37 +35,43 @@ struct MagSet {
     static constexpr int count = __builtin_popcount(C & 7u);
 };
 
-__device__ __forceinline__ void stage_mag(StagedMagPrism *tile, const double *__restrict__ prisms,
-                                          const double *__restrict__ me,
-                                          const double *__restrict__ mn,
-                                          const double *__restrict__ mu, int64_t t0, int cnt) {
-    double *flat = reinterpret_cast<double *>(tile);
-    const double *src = prisms + 6 * t0;
-    for (int idx = threadIdx.x; idx < 6 * cnt; idx += blockDim.x) {
-        const int p = idx / 6, c = idx - 6 * p;
-        flat[10 * p + c] = src[idx];
+// Prisms and magnetisations as given, for field_stage.
+struct MagSource {
+    const double *prisms, *me, *mn, *mu;
+    __device__ bool get(int64_t p, double (&b)[6], double (&weight)[3]) const {
+#pragma unroll
+        for (int c = 0; c < 6; ++c) b[c] = prisms[6 * p + c];
+        weight[0] = kCm * me[p];
+        weight[1] = kCm * mn[p];
+        weight[2] = kCm * mu[p];
+        return false;
     }
-    for (int p = threadIdx.x; p < cnt; p += blockDim.x) {
-        tile[p].me = kCm * me[t0 + p];
-        tile[p].mn = kCm * mn[t0 + p];
-        tile[p].mu = kCm * mu[t0 + p];
-    }
+};
+
+// The components' sums from K[f - 4] for gravity field bit f: ee 4, nn 5, uu
+// 6, en 7, eu 8, nu 9.
+template <unsigned C>
+__device__ __forceinline__ void magnetic_terms(const double *weight, const double (&K)[6],
+                                               double (&out)[MagSet<C>::count]) {
+    const double me = weight[0], mn = weight[1], mu = weight[2];
+    int s = 0;
+    if constexpr ((C & 1u) != 0) out[s++] = me * K[0] + mn * K[3] + mu * K[4];
+    if constexpr ((C & 2u) != 0) out[s++] = me * K[3] + mn * K[1] + mu * K[5];
+    if constexpr ((C & 4u) != 0) out[s++] = me * K[4] + mn * K[5] + mu * K[2];
 }
 
 // Add the selected components of one prism at (e, n, u) to acc[].  Without
 // kGeneral, dev::needs_general<MagSet<C>::tensor> must be false for the
-// point (it is then on no face plane, so on no edge), or with kXOnly
-// dev::needs_full_general (the point may lie between the x-planes).
-template <unsigned C, bool kGeneral, bool kXOnly = false>
-__device__ __forceinline__ void magnetic_pair(double e, double n, double u,
-                                              const StagedMagPrism &sp,
+// point (it is then on no face plane, so on no edge).
+template <unsigned C, bool kGeneral>
+__device__ __forceinline__ void magnetic_pair(double e, double n, double u, const double *b,
+                                              const double *weight,
                                               double (&acc)[MagSet<C>::count],
                                               const dm::Tables &tab) {
     constexpr unsigned M = MagSet<C>::tensor;
     using F = FieldSet<M>;
-    const double x0 = sp.e - e, x1 = sp.w - e, y0 = sp.n - n, y1 = sp.s - n;
-    const double z0 = sp.t - u, z1 = sp.b - u;
-    // K[f - 4] for gravity field bit f: ee 4, nn 5, uu 6, en 7, eu 8, nu 9.
+    const double x0 = b[1] - e, x1 = b[0] - e, y0 = b[3] - n, y1 = b[2] - n;
+    const double z0 = b[5] - u, z1 = b[4] - u;
     double K[6];
     if constexpr (kGeneral) {
         double vs[F::count];
@@ -84,15 +80,13 @@ __device__ __forceinline__ void magnetic_pair(double e, double n, double u,
 #pragma unroll
         for (int f = 4; f < 10; ++f)
             if ((M >> f) & 1u) K[f - 4] = vs[F::slot(f)];
-    } else if constexpr (kXOnly) {
-        dev::tensor_xonly<M>(x0, x1, y0, y1, z0, z1, K, tab);
     } else {
         dev::tensor_lean<M>(x0, x1, y0, y1, z0, z1, K, tab);
     }
-    int s = 0;
-    if constexpr ((C & 1u) != 0) acc[s++] += sp.me * K[0] + sp.mn * K[3] + sp.mu * K[4];
-    if constexpr ((C & 2u) != 0) acc[s++] += sp.me * K[3] + sp.mn * K[1] + sp.mu * K[5];
-    if constexpr ((C & 4u) != 0) acc[s++] += sp.me * K[4] + sp.mn * K[5] + sp.mu * K[2];
+    double terms[MagSet<C>::count];
+    magnetic_terms<C>(weight, K, terms);
+#pragma unroll
+    for (int c = 0; c < MagSet<C>::count; ++c) acc[c] += terms[c];
     if constexpr (kGeneral) {
         // On an edge: two coordinates on a bound of the prism, the third
         // between its bounds (vertices included).
@@ -108,76 +102,66 @@ __device__ __forceinline__ void magnetic_pair(double e, double n, double u,
     }
 }
 
-// The prisms tile[0, cnt) at (e, n, u), in three passes as dev::tile_pairs
-// (lean, x-only, general).
+// The sums of field_chunk: the selected components.
 template <unsigned C>
-__device__ __forceinline__ void magnetic_tile(const StagedMagPrism *tile, int cnt, double e,
-                                              double n, double u,
-                                              double (&acc)[MagSet<C>::count],
-                                              const dm::Tables &tab) {
-    constexpr unsigned M = MagSet<C>::tensor;
-    uint64_t general_lo = 0, general_hi = 0, xonly_lo = 0, xonly_hi = 0;
-    for (int p = 0; p < cnt; ++p) {
-        const StagedMagPrism sp = tile[p];
-        if (dev::any_lane(dev::needs_general<M>(e, n, u, sp.w, sp.e, sp.s, sp.n, sp.b, sp.t))) {
-            const bool full = dev::any_lane(
-                dev::needs_full_general<M>(e, n, u, sp.w, sp.e, sp.s, sp.n, sp.b, sp.t));
-            uint64_t &lo = full ? general_lo : xonly_lo, &hi = full ? general_hi : xonly_hi;
-            if (p < 64)
-                lo |= 1ull << p;
-            else
-                hi |= 1ull << (p - 64);
-            continue;
-        }
-        magnetic_pair<C, false>(e, n, u, sp, acc, tab);
+struct MagneticOp {
+    static constexpr unsigned fields = MagSet<C>::tensor;
+    static constexpr int weights = 3, values = MagSet<C>::count;
+    __device__ static void combine(const double *weight, const double (&vs)[FieldSet<fields>::count],
+                                   double (&out)[values]) {
+        double K[6];
+#pragma unroll
+        for (int f = 4; f < 10; ++f)
+            if ((fields >> f) & 1u) K[f - 4] = vs[FieldSet<fields>::slot(f)];
+        magnetic_terms<C>(weight, K, out);
     }
-    for (int half = 0; half < 2; ++half) {
-        uint64_t m = half ? xonly_hi : xonly_lo;
-        while (m) {
-            const int p = 64 * half + __builtin_ctzll(m);
-            m &= m - 1;
-            magnetic_pair<C, false, true>(e, n, u, tile[p], acc, tab);
-        }
+    template <bool kGeneral>
+    __device__ static void closed(double e, double n, double u, const double *b,
+                                  const double *weight, double (&acc)[values], uint32_t &,
+                                  const dm::Tables &tab) {
+        magnetic_pair<C, kGeneral>(e, n, u, b, weight, acc, tab);
     }
-    for (int half = 0; half < 2; ++half) {
-        uint64_t m = half ? general_hi : general_lo;
-        while (m) {
-            const int p = 64 * half + __builtin_ctzll(m);
-            m &= m - 1;
-            magnetic_pair<C, true>(e, n, u, tile[p], acc, tab);
-        }
+};
+
+// The far pairs into the partial sums.
+template <unsigned C>
+__global__ __launch_bounds__(dev::kGzThreads, 3) void magnetic_far_kernel(
+    const double *__restrict__ oe, const double *__restrict__ on, const double *__restrict__ ou,
+    int n_obs, MagSource src, int64_t n_src, int64_t chunk_len, double *__restrict__ partial) {
+    using Op = MagneticOp<C>;
+    __shared__ dev::FieldFarShared<Op> sh;
+    // rotated from chunk to chunk over the XCDs, as prism_gz_kernel
+    const unsigned bx = (blockIdx.x + blockIdx.y) % gridDim.x;
+    const int64_t base = (int64_t)bx * dev::kGzThreads, i = base + threadIdx.x;
+    const int64_t c0 = (int64_t)blockIdx.y * chunk_len;
+    const int64_t c1 = c0 + chunk_len < n_src ? c0 + chunk_len : n_src;
+    double acc[Op::values] = {};
+    dev::field_far_chunk<Op>(src, oe, on, ou, base, n_obs, c0, c1, acc, sh);
+    if (i < n_obs) {
+#pragma unroll
+        for (int s = 0; s < Op::values; ++s)
+            partial[((int64_t)blockIdx.y * Op::values + s) * n_obs + i] = acc[s];
     }
 }
 
+// The close pairs, added to the partial sums of magnetic_far_kernel.
 template <unsigned C>
-__global__ __launch_bounds__(kObsPerBlock) void prism_magnetic_kernel(
+__global__ __launch_bounds__(dev::kGzThreads, 3) void magnetic_close_kernel(
     const double *__restrict__ oe, const double *__restrict__ on, const double *__restrict__ ou,
-    int n_obs, const double *__restrict__ prisms, const double *__restrict__ me,
-    const double *__restrict__ mn, const double *__restrict__ mu, int64_t n_src,
-    int64_t chunk_len, double *__restrict__ partial) {
-    constexpr int NC = MagSet<C>::count;
-    __shared__ StagedMagPrism tile[kTile];
-    __shared__ dm::Tables tables;
-    dm::load_tables(&tables);
-    const int i = blockIdx.x * kObsPerBlock + threadIdx.x;
-    const bool valid = i < n_obs;
-    const int ii = valid ? i : n_obs - 1;
-    const double e = oe[ii], n = on[ii], u = ou[ii];
-    double acc[NC];
-#pragma unroll
-    for (int s = 0; s < NC; ++s) acc[s] = 0.0;
+    int n_obs, MagSource src, int64_t n_src, int64_t chunk_len, double *__restrict__ partial) {
+    using Op = MagneticOp<C>;
+    __shared__ dev::FieldCloseShared<Op> sh;
+    const unsigned bx = (blockIdx.x + blockIdx.y) % gridDim.x;
+    const int64_t base = (int64_t)bx * dev::kGzThreads, i = base + threadIdx.x;
     const int64_t c0 = (int64_t)blockIdx.y * chunk_len;
     const int64_t c1 = c0 + chunk_len < n_src ? c0 + chunk_len : n_src;
-    for (int64_t t0 = c0; t0 < c1; t0 += kTile) {
-        const int cnt = (int)(c1 - t0 < kTile ? c1 - t0 : kTile);
-        __syncthreads();
-        stage_mag(tile, prisms, me, mn, mu, t0, cnt);
-        __syncthreads();
-        magnetic_tile<C>(tile, cnt, e, n, u, acc, tables);
-    }
-    if (valid) {
+    double acc[Op::values] = {};
+    uint32_t flags = 0;
+    if (!dev::field_close_chunk<Op>(src, oe, on, ou, base, n_obs, c0, c1, acc, flags, sh)) return;
+    if (i < n_obs) {
 #pragma unroll
-        for (int s = 0; s < NC; ++s) partial[((int64_t)blockIdx.y * NC + s) * n_obs + i] = acc[s];
+        for (int s = 0; s < Op::values; ++s)
+            partial[((int64_t)blockIdx.y * Op::values + s) * n_obs + i] += acc[s];
     }
 }
 
@@ -205,10 +189,14 @@ int launch_magnetic(const double *oe, const double *on, const double *ou, int64_
                     const double *prisms, const double *me, const double *mn, const double *mu,
                     int64_t n_src, int64_t chunks, double *partial, hipStream_t stream) {
     const int64_t chunk_len = (n_src + chunks - 1) / chunks;
-    dim3 grid((unsigned)((n_obs + kObsPerBlock - 1) / kObsPerBlock), (unsigned)chunks);
-    hipLaunchKernelGGL((prism_magnetic_kernel<C>), grid, dim3(kObsPerBlock), 0, stream, oe, on, ou,
-                       (int)n_obs, prisms, me, mn, mu, n_src, chunk_len, partial);
-    HMX_LAUNCHED("prism_magnetic_kernel");
+    dim3 grid((unsigned)((n_obs + dev::kGzThreads - 1) / dev::kGzThreads), (unsigned)chunks);
+    const MagSource src{prisms, me, mn, mu};
+    hipLaunchKernelGGL((magnetic_far_kernel<C>), grid, dim3(dev::kGzThreads), 0, stream, oe, on, ou,
+                       (int)n_obs, src, n_src, chunk_len, partial);
+    HMX_LAUNCHED("magnetic_far_kernel");
+    hipLaunchKernelGGL((magnetic_close_kernel<C>), grid, dim3(dev::kGzThreads), 0, stream, oe, on,
+                       ou, (int)n_obs, src, n_src, chunk_len, partial);
+    HMX_LAUNCHED("magnetic_close_kernel");
     return HMX_OK;
 }
 
@@ -230,7 +218,7 @@ int hmx_prism_magnetic_workspace_bytes(int64_t n_obs, int64_t n_prisms, uint32_t
         return hmx::fail(HMX_ERR_ARG, "invalid component mask 0x%x", component_mask);
     const int cu = hmx::device_cu_count();
     if (cu < 0) return cu;
-    const int64_t chunks = hmx::forward_chunks(n_obs, n_prisms, cu);
+    const int64_t chunks = hmx::prism_chunks(n_obs, n_prisms, cu);
     *bytes = (size_t)chunks * (size_t)__builtin_popcount(component_mask) * (size_t)n_obs *
              sizeof(double);
     // the point order, after the partial sums
@@ -266,7 +254,7 @@ int hmx_prism_magnetic(const double *easting, const double *northing, const doub
         return hmx::fail(HMX_ERR_ARG, "NULL prism or magnetization array");
     const int cu = hmx::device_cu_count();
     if (cu < 0) return cu;
-    const int64_t chunks = hmx::forward_chunks(n_obs, n_prisms, cu);
+    const int64_t chunks = hmx::prism_chunks(n_obs, n_prisms, cu);
     const size_t partial_bytes = (size_t)chunks * (size_t)nc * (size_t)n_obs * sizeof(double);
     const size_t order_at = hmx::point_order_offset(partial_bytes);
     const size_t with_order = order_at + hmx::point_order_bytes(n_obs);

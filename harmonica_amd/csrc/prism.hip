@@ -2,93 +2,59 @@
 //
 // Launch shape: a workgroup owns 256 observation points (4 wavefronts, one
 // point per lane, FP64 accumulators in VGPRs) and one chunk of the prism
-// list.  Prisms are staged tile by tile into LDS with coalesced loads and
-// read back as wave-uniform broadcasts, so every lane of a wavefront
-// evaluates the same prism against its own point.  Each chunk writes its
+// list.  Prisms are staged tile by tile into LDS and read back as
+// wave-uniform broadcasts; each wavefront evaluates them in the far form or
+// the closed form (prism_far.h, prism_fields_far.h).  Each chunk writes its
 // partial sums to the workspace; a second kernel reduces the chunks in
 // order and applies harmonica's units, so results are deterministic.
 #include <mutex>
 
 #include "hmx_internal.h"
 #include "prism_device.h"
-#include "prism_far.h"
+#include "prism_fields_far.h"
 
 namespace hmx {
 namespace {
 
 using dev::FieldSet;
 
-// One staged prism (64 bytes): bounds, G * density and skip flag.
-struct alignas(16) StagedPrism {
-    double w, e, s, n, b, t, grho;
-    int skip, pad;
+// Sums the fields of FieldSet<M>, weight G * density.
+template <unsigned M>
+struct GravityOp {
+    static constexpr unsigned fields = M;
+    static constexpr int weights = 1, values = FieldSet<M>::count;
+    __device__ static void combine(const double *weight, const double (&vs)[values],
+                                   double (&out)[values]) {
+#pragma unroll
+        for (int s = 0; s < values; ++s) out[s] = weight[0] * vs[s];
+    }
+    template <bool kGeneral>
+    __device__ static void closed(double e, double n, double u, const double *b,
+                                  const double *weight, double (&acc)[values], uint32_t &flags,
+                                  const dm::Tables &tab) {
+        dev::prism_pair_path<M, kGeneral>(e, n, u, b[0], b[1], b[2], b[3], b[4], b[5], weight[0],
+                                          acc, flags, tab);
+    }
 };
-
-// Stage prisms [t0, t0 + cnt) of an (m, 6) row-major array.
-__device__ __forceinline__ void stage_prisms(StagedPrism *tile, const double *__restrict__ prisms,
-                                             const double *__restrict__ density, int64_t t0,
-                                             int cnt) {
-    double *flat = reinterpret_cast<double *>(tile);
-    const double *src = prisms + 6 * t0;
-    for (int idx = threadIdx.x; idx < 6 * cnt; idx += blockDim.x) {
-        int p = idx / 6, c = idx - 6 * p;
-        flat[8 * p + c] = src[idx];
-    }
-    for (int p = threadIdx.x; p < cnt; p += blockDim.x) {
-        tile[p].grho = dev::kG * density[t0 + p];
-        tile[p].skip = 0;
-    }
-}
-
-// Stage prisms [t0, t0 + cnt) of a layer, enumerated easting-major as the
-// reference loops (layer.py:590-594): p = j * n_north + k.  Bounds are
-// centre -/+ half the first spacing (layer.py:584-585,592-593,609-610);
-// skip rules of layer.py:595-607.
-__device__ __forceinline__ void stage_layer(StagedPrism *tile, const double *__restrict__ ce,
-                                            int n_east, const double *__restrict__ cn,
-                                            int n_north, const double *__restrict__ bottom,
-                                            const double *__restrict__ top,
-                                            const double *__restrict__ density, double threshold,
-                                            int64_t t0, int cnt) {
-    const double half_e = (ce[1] - ce[0]) / 2;
-    const double half_n = (cn[1] - cn[0]) / 2;
-    for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
-        int64_t p = t0 + q;
-        int j = (int)(p / n_north);
-        int k = (int)(p - (int64_t)j * n_north);
-        int64_t idx = (int64_t)k * n_east + j;
-        double d = density[idx], b = bottom[idx], t = top[idx];
-        bool skip = d == 0.0 || d != d || (t - b < threshold) || t != t || b != b;
-        StagedPrism sp;
-        sp.w = ce[j] - half_e;
-        sp.e = ce[j] + half_e;
-        sp.s = cn[k] - half_n;
-        sp.n = cn[k] + half_n;
-        sp.b = b;
-        sp.t = t;
-        sp.grho = dev::kG * d;
-        sp.skip = skip ? 1 : 0;
-        sp.pad = 0;
-        tile[q] = sp;
-    }
-}
 
 struct ExplicitSource : dev::GzExplicit {
     ExplicitSource(const double *p, const double *d) : dev::GzExplicit{p, d} {}
-    __device__ void stage(StagedPrism *tile, int64_t t0, int cnt) const {
-        stage_prisms(tile, prisms, density, t0, cnt);
+    using dev::GzExplicit::get;
+    __device__ bool get(int64_t p, double (&b)[6], double (&weight)[1]) const {
+        const bool skip = get(p, b, weight[0]);
+        weight[0] *= dev::kG;
+        return skip;
     }
-    static constexpr bool may_skip = false;
 };
 
+// Prisms of a layer, enumerated easting-major as the reference loops
+// (layer.py:590-594): p = j * n_north + k.  Bounds are centre -/+ half the
+// first spacing (layer.py:584-585,592-593,609-610); skip rules of
+// layer.py:595-607.
 struct LayerSource {
     const double *ce, *cn, *bottom, *top, *density;
     int n_east, n_north;
     double threshold;
-    __device__ void stage(StagedPrism *tile, int64_t t0, int cnt) const {
-        stage_layer(tile, ce, n_east, cn, n_north, bottom, top, density, threshold, t0, cnt);
-    }
-    static constexpr bool may_skip = true;
     __device__ bool get(int64_t p, double (&b)[6], double &rho) const {
         const unsigned j = (unsigned)p / (unsigned)n_north, k = (unsigned)p - j * (unsigned)n_north;
         const int64_t idx = (int64_t)k * n_east + j;
@@ -102,42 +68,57 @@ struct LayerSource {
         rho = density[idx];
         return rho == 0.0 || rho != rho || (b[5] - b[4] < threshold) || b[5] != b[5] || b[4] != b[4];
     }
+    __device__ bool get(int64_t p, double (&b)[6], double (&weight)[1]) const {
+        const bool skip = get(p, b, weight[0]);
+        weight[0] *= dev::kG;
+        return skip;
+    }
 };
 
-static_assert(kTile <= 128, "tile_pairs marks at most 128 prisms");
-
+// The far pairs of any field set into the partial sums.
 template <unsigned M, class Src>
-__global__ __launch_bounds__(kObsPerBlock) void prism_forward_kernel(
-    const double *__restrict__ oe, const double *__restrict__ on, const double *__restrict__ ou,
-    int n_obs, Src src, int64_t n_src, int64_t chunk_len, double *__restrict__ partial,
-    uint32_t *__restrict__ flags) {
-    using F = FieldSet<M>;
-    __shared__ StagedPrism tile[kTile];
-    __shared__ dm::Tables tables;
-    dm::load_tables(&tables);
-    const int i = blockIdx.x * kObsPerBlock + threadIdx.x;
-    const bool valid = i < n_obs;
-    const int ii = valid ? i : n_obs - 1;
-    const double e = oe[ii], n = on[ii], u = ou[ii];
-    double acc[F::count];
-#pragma unroll
-    for (int s = 0; s < F::count; ++s) acc[s] = 0.0;
-    uint32_t sflags = 0;
+__global__ __launch_bounds__(dev::kGzThreads, FieldSet<M>::count <= 3 ? 3 : 2) void
+prism_far_kernel(const double *__restrict__ oe, const double *__restrict__ on,
+                 const double *__restrict__ ou, int n_obs, Src src, int64_t n_src,
+                 int64_t chunk_len, double *__restrict__ partial) {
+    using Op = GravityOp<M>;
+    __shared__ dev::FieldFarShared<Op> sh;
+    // rotated from chunk to chunk over the XCDs, as prism_gz_kernel
+    const unsigned bx = (blockIdx.x + blockIdx.y) % gridDim.x;
+    const int64_t base = (int64_t)bx * dev::kGzThreads, i = base + threadIdx.x;
     const int64_t c0 = (int64_t)blockIdx.y * chunk_len;
     const int64_t c1 = c0 + chunk_len < n_src ? c0 + chunk_len : n_src;
-    for (int64_t t0 = c0; t0 < c1; t0 += kTile) {
-        const int cnt = (int)(c1 - t0 < kTile ? c1 - t0 : kTile);
-        __syncthreads();
-        src.stage(tile, t0, cnt);
-        __syncthreads();
-        dev::tile_pairs<M, Src::may_skip>(tile, cnt, e, n, u, acc, sflags, tables);
-    }
-    if (valid) {
+    double acc[Op::values] = {};
+    dev::field_far_chunk<Op>(src, oe, on, ou, base, n_obs, c0, c1, acc, sh);
+    if (i < n_obs) {
 #pragma unroll
-        for (int s = 0; s < F::count; ++s)
-            partial[((int64_t)blockIdx.y * F::count + s) * n_obs + i] = acc[s];
-        if (F::tensor && flags && sflags) atomicOr(flags, sflags);
+        for (int s = 0; s < Op::values; ++s)
+            partial[((int64_t)blockIdx.y * Op::values + s) * n_obs + i] = acc[s];
     }
+}
+
+// The close pairs, added to the partial sums of prism_far_kernel.
+template <unsigned M, class Src>
+__global__ __launch_bounds__(dev::kGzThreads, FieldSet<M>::count <= 3 ? 4 : 3) void
+prism_close_kernel(const double *__restrict__ oe, const double *__restrict__ on,
+                   const double *__restrict__ ou, int n_obs, Src src, int64_t n_src,
+                   int64_t chunk_len, double *__restrict__ partial,
+                   uint32_t *__restrict__ flags) {
+    using Op = GravityOp<M>;
+    __shared__ dev::FieldCloseShared<Op> sh;
+    const unsigned bx = (blockIdx.x + blockIdx.y) % gridDim.x;
+    const int64_t base = (int64_t)bx * dev::kGzThreads, i = base + threadIdx.x;
+    const int64_t c0 = (int64_t)blockIdx.y * chunk_len;
+    const int64_t c1 = c0 + chunk_len < n_src ? c0 + chunk_len : n_src;
+    double acc[Op::values] = {};
+    uint32_t found = 0;
+    if (!dev::field_close_chunk<Op>(src, oe, on, ou, base, n_obs, c0, c1, acc, found, sh)) return;
+    if (i < n_obs) {
+#pragma unroll
+        for (int s = 0; s < Op::values; ++s)
+            partial[((int64_t)blockIdx.y * Op::values + s) * n_obs + i] += acc[s];
+    }
+    if (FieldSet<M>::tensor && flags && found) atomicOr(flags, found);
 }
 
 // g_u alone, each prism in the far form or the closed form (prism_far.h).
@@ -172,26 +153,32 @@ __global__ __launch_bounds__(dev::kGzThreads, 4) void prism_gz_kernel(
 
 // Singular-point scan: bit f of *flags is set when some (point, prism)
 // pair is a singular point of tensor field f (replaces the serial scans
-// _any_singular_point_g_* of gravity.py:272-449).
+// _any_singular_point_g_* of gravity.py:272-449).  Singular points lie in the
+// prism's closed box: a lane tests a prism's box against the box of its
+// wave's points, and only prisms that pass are tested point by point (20,011
+// bodies below 2999 stations: 100 -> 9 us).
 __global__ __launch_bounds__(kObsPerBlock) void singular_scan_kernel(
     const double *__restrict__ oe, const double *__restrict__ on, const double *__restrict__ ou,
     int n_obs, const double *__restrict__ prisms, int64_t n_src, int64_t chunk_len,
     uint32_t mask, uint32_t *__restrict__ flags) {
-    __shared__ double tile[kTile * 6];
-    const int i = blockIdx.x * kObsPerBlock + threadIdx.x;
-    const bool valid = i < n_obs;
-    const int ii = valid ? i : n_obs - 1;
+    const int i = blockIdx.x * kObsPerBlock + threadIdx.x, lane = threadIdx.x & 63;
+    const int ii = i < n_obs ? i : n_obs - 1;
     const double e = oe[ii], n = on[ii], u = ou[ii];
+    const dev::FarBox box{dev::wave_min(e), dev::wave_max(e), dev::wave_min(n),
+                          dev::wave_max(n), dev::wave_min(u), dev::wave_max(u)};
     uint32_t found = 0;
     const int64_t c0 = (int64_t)blockIdx.y * chunk_len;
     const int64_t c1 = c0 + chunk_len < n_src ? c0 + chunk_len : n_src;
-    for (int64_t t0 = c0; t0 < c1; t0 += kTile) {
-        const int cnt = (int)(c1 - t0 < kTile ? c1 - t0 : kTile);
-        __syncthreads();
-        for (int idx = threadIdx.x; idx < 6 * cnt; idx += blockDim.x) tile[idx] = prisms[6 * t0 + idx];
-        __syncthreads();
-        for (int p = 0; p < cnt; ++p) {
-            const double *b = tile + 6 * p;
+    for (int64_t t0 = c0; t0 < c1; t0 += 64) {
+        bool meets = false;
+        if (t0 + lane < c1) {
+            const double *b = prisms + 6 * (t0 + lane);
+            meets = fmin(b[0], b[1]) <= box.x1 && box.x0 <= fmax(b[0], b[1]) &&
+                    fmin(b[2], b[3]) <= box.y1 && box.y0 <= fmax(b[2], b[3]) &&
+                    fmin(b[4], b[5]) <= box.u1 && box.u0 <= fmax(b[4], b[5]);
+        }
+        dev::for_bits((uint64_t)__ballot(meets), [&](int p) {
+            const double *b = prisms + 6 * (t0 + p);
             const bool in_e = b[0] <= e && e <= b[1], in_n = b[2] <= n && n <= b[3];
             const bool in_u = b[4] <= u && u <= b[5];
             const bool at_e = e == b[0] || e == b[1], at_n = n == b[2] || n == b[3];
@@ -204,10 +191,10 @@ __global__ __launch_bounds__(kObsPerBlock) void singular_scan_kernel(
             found |= edge_u ? 1u << 7 : 0u;
             found |= edge_n ? 1u << 8 : 0u;
             found |= edge_e ? 1u << 9 : 0u;
-        }
+        });
     }
     found &= mask;
-    if (valid && found) atomicOr(flags, found);
+    if (found) atomicOr(flags, found);
 }
 
 // out[s][perm[i]] = units(sum over chunks of partial[c][s][i]) (perm NULL: the
@@ -250,16 +237,18 @@ int launch_forward(const double *oe, const double *on, const double *ou, int64_t
                    const Src &src, int64_t n_src, int64_t chunks, double *partial,
                    uint32_t *flags, hipStream_t stream) {
     const int64_t chunk_len = (n_src + chunks - 1) / chunks;
-    dim3 grid((unsigned)((n_obs + kObsPerBlock - 1) / kObsPerBlock), (unsigned)chunks);
+    dim3 grid((unsigned)((n_obs + dev::kGzThreads - 1) / dev::kGzThreads), (unsigned)chunks);
     if constexpr (M == 0x8u) {
-        grid.x = (unsigned)((n_obs + dev::kGzThreads - 1) / dev::kGzThreads);
         hipLaunchKernelGGL((prism_gz_kernel<Src>), grid, dim3(dev::kGzThreads), 0, stream, oe, on,
                            ou, (int)n_obs, src, n_src, chunk_len, partial);
         HMX_LAUNCHED("prism_gz_kernel");
     } else {
-        hipLaunchKernelGGL((prism_forward_kernel<M, Src>), grid, dim3(kObsPerBlock), 0, stream, oe,
+        hipLaunchKernelGGL((prism_far_kernel<M, Src>), grid, dim3(dev::kGzThreads), 0, stream, oe,
+                           on, ou, (int)n_obs, src, n_src, chunk_len, partial);
+        HMX_LAUNCHED("prism_far_kernel");
+        hipLaunchKernelGGL((prism_close_kernel<M, Src>), grid, dim3(dev::kGzThreads), 0, stream, oe,
                            on, ou, (int)n_obs, src, n_src, chunk_len, partial, flags);
-        HMX_LAUNCHED("prism_forward_kernel");
+        HMX_LAUNCHED("prism_close_kernel");
     }
     return HMX_OK;
 }

@@ -205,10 +205,8 @@ __device__ __forceinline__ bool any_lane(bool need) { return __any(need) != 0; }
 // face_angle).  With kTop, *ftop receives the top-face sum
 // sum_{i,j} (-1)^(i+j) A_z(i, j, 0) (the derivative with respect to the top).
 // Without kGeneral the caller guarantees the point lies between neither the
-// two x-planes nor the two y-planes (no mixed quotient, no 2 pi branch);
-// kGenX lifts the first condition (the logarithms along x take their general
-// form; the face angles need the 2 pi branch only between both pairs).
-template <bool kTop, bool kGeneral, bool kGenX = kGeneral>
+// two x-planes nor the two y-planes (no mixed quotient, no 2 pi branch).
+template <bool kTop, bool kGeneral>
 __device__ __forceinline__ double gu_sum(double x0, double x1, double y0, double y1, double z0,
                                          double z1, const dm::Tables &tab, double *ftop) {
     const double ys0 = y0 * y0, ys1 = y1 * y1;
@@ -237,7 +235,7 @@ __device__ __forceinline__ double gu_sum(double x0, double x1, double y0, double
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const double c = j ? y1 : y0, cs = j ? ys1 : ys0;
-        const double l = log_quad<kGeneral || kGenX>(x0, x1, r[0][j][0], r[0][j][1], r[1][j][0],
+        const double l = log_quad<kGeneral>(x0, x1, r[0][j][0], r[0][j][1], r[1][j][0],
                                             r[1][j][1], cs, zt0, zt1, flip_x, tab);
         sum = fma(j ? -c : c, l, sum);
     }
@@ -277,10 +275,8 @@ __device__ __forceinline__ double gu_sum_paired(double x0, double x1, double y0,
 // x1 = W - e, y0 = N - n, y1 = S - n, z0 = T - u, z1 = B - u) into vs[],
 // singular-point bits into sflags.  Without kGeneral the caller guarantees
 // that the point is on no face plane of the prism and between the two
-// planes of no axis; kGenX lifts the last condition for the x-planes (the
-// logarithms along x take their general form; the face angles need theirs
-// only between two pairs of planes, the singular points lie on face planes).
-template <unsigned M, bool kGeneral, bool kGenX = kGeneral>
+// planes of no axis.
+template <unsigned M, bool kGeneral>
 __device__ __forceinline__ void prism_fields(double x0, double x1, double y0, double y1,
                                              double z0, double z1, double (&vs)[FieldSet<M>::count],
                                              uint32_t &sflags, const dm::Tables &tab) {
@@ -309,8 +305,7 @@ __device__ __forceinline__ void prism_fields(double x0, double x1, double y0, do
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
             if constexpr (F::Lx)
-                DLx[a][b] = log_diff<kGeneral || kGenX>(x0, x1, r[0][a][b], r[1][a][b],
-                                                        ys[a] + zs[b], fx,
+                DLx[a][b] = log_diff<kGeneral>(x0, x1, r[0][a][b], r[1][a][b], ys[a] + zs[b], fx,
                                                tab);
             if constexpr (F::Ly)
                 DLy[a][b] = log_diff<kGeneral>(y0, y1, r[a][0][b], r[a][1][b], xs[a] + zs[b], fy,
@@ -463,90 +458,6 @@ __device__ __forceinline__ void tensor_lean(double x0, double x1, double y0, dou
     (void)Z;
 }
 
-// tensor_lean for a point between the two x-planes of the prism but between
-// no other pair and on no face plane: the logarithms along x change branch
-// across the point, so K_nu is the sum of the four grouped x-logarithms of
-// prism_fields (general form), and the two x-face angles have opposite
-// signs, so K_ee is their difference taken angle by angle (neither face
-// is seen from inside: that needs the point between the y- and z-planes
-// too).  The other kernels keep the lean regrouping, which needs only their
-// own axis: K_en, K_eu one logarithm each, K_nn (and K_uu, or Laplace's
-// equation outside the prism) one arctangent each.
-template <unsigned TM>
-__device__ __forceinline__ void tensor_xonly(double x0, double x1, double y0, double y1,
-                                             double z0, double z1, double (&K)[6],
-                                             const dm::Tables &tab) {
-    using F = FieldSet<TM>;
-    const double xs[2] = {x0 * x0, x1 * x1}, ys[2] = {y0 * y0, y1 * y1};
-    const double zs[2] = {z0 * z0, z1 * z1};
-    const double Y[2] = {y0, y1}, Z[2] = {z0, z1};
-    double r[2][2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int k = 0; k < 2; ++k) r[i][j][k] = vertex_r(xs[i] + ys[j], z_tiny(zs[k]));
-    auto off = [&](auto coord, double a0) {
-        double num = 1.0, den = 1.0;
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int k = 0; k < 2; ++k) {
-                    const double t = r[i][j][k] + fabs(coord(i, j, k));
-                    if ((i + j + k) & 1)
-                        den *= t;
-                    else
-                        num *= t;
-                }
-        return dm::flip_sign(dm::log_pos(dm::div(num, den), tab), dm::sign_mask(a0 < 0.0));
-    };
-    if constexpr (F::en) K[3] = off([&](int, int, int k) { return Z[k]; }, z0);
-    if constexpr (F::eu) K[4] = off([&](int, int j, int) { return Y[j]; }, y0);
-    if constexpr (F::nu) {
-        const unsigned fx = dm::sign_mask(x0 < 0.0);
-        double s = 0.0;
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                const double d =
-                    log_diff<true>(x0, x1, r[0][j][k], r[1][j][k], ys[j] + zs[k], fx, tab);
-                s = (j + k) & 1 ? s - d : s + d;
-            }
-        K[5] = s;
-    }
-    auto diag = [&](double N0, double D0, double N1, double D1) {
-        return dm::atan2_full<false>(fma(N1, D0, -N0 * D1), fma(D0, D1, N0 * N1), tab);
-    };
-    constexpr bool kLaplace = F::ee && F::nn && F::uu;
-    if constexpr (F::ee) {
-        const double o0 = face_sum<false>(y0, y1, z0, z1, x0, r[0][0][0], r[0][0][1], r[0][1][0],
-                                          r[0][1][1], tab);
-        const double o1 = face_sum<false>(y0, y1, z0, z1, x1, r[1][0][0], r[1][0][1], r[1][1][0],
-                                          r[1][1][1], tab);
-        K[0] = -(o0 - o1);
-    }
-    if constexpr (F::nn) {
-        double N0, D0, N1, D1;
-        face_nd(z0, z1, x0, x1, y0, r[0][0][0], r[1][0][0], r[0][0][1], r[1][0][1], N0, D0);
-        face_nd(z0, z1, x0, x1, y1, r[0][1][0], r[1][1][0], r[0][1][1], r[1][1][1], N1, D1);
-        K[1] = diag(N0, D0, N1, D1);
-    }
-    if constexpr (F::uu) {
-        if constexpr (kLaplace) {
-            K[2] = -(K[0] + K[1]);
-        } else {
-            double N0, D0, N1, D1;
-            face_nd(x0, x1, y0, y1, z0, r[0][0][0], r[0][1][0], r[1][0][0], r[1][1][0], N0, D0);
-            face_nd(x0, x1, y0, y1, z1, r[0][0][1], r[0][1][1], r[1][0][1], r[1][1][1], N1, D1);
-            K[2] = diag(N0, D0, N1, D1);
-        }
-    }
-}
-
 // Whether the point (e, n, u) needs the general instantiation for this
 // prism: for g_u, g_e, g_n alone when it lies between the two planes of one
 // of the two axes the logarithms run along; for other field sets when it
@@ -565,40 +476,18 @@ __device__ __forceinline__ bool needs_general(double e, double n, double u, doub
     return bx || by || bz || x0 * x1 == 0.0 || y0 * y1 == 0.0 || z0 * z1 == 0.0;
 }
 
-// Field sets with an instantiation for points between the x-planes only (on
-// no face plane): g_u alone, those evaluated by prism_fields and the
-// tensor-only sets (tensor_xonly).
-template <unsigned M>
-__host__ __device__ constexpr bool has_x_only() {
-    return M != 0x2u && M != 0x4u;
-}
-
-// Whether the point needs the general instantiation for a reason other than
-// lying between the x-planes (has_x_only field sets): between the y-planes
-// (g_u alone), or between the y- or z-planes or on a face plane.
-template <unsigned M>
-__device__ __forceinline__ bool needs_full_general(double e, double n, double u, double W,
-                                                   double E, double S, double N, double B,
-                                                   double T) {
-    const double x0 = E - e, x1 = W - e, y0 = N - n, y1 = S - n, z0 = T - u, z1 = B - u;
-    const bool by = y0 >= 0.0 && y1 < 0.0, bz = z0 >= 0.0 && z1 < 0.0;
-    if constexpr (M == 0x8u) return by;
-    return by || bz || x0 * x1 == 0.0 || y0 * y1 == 0.0 || z0 * z1 == 0.0;
-}
-
 // Add the fields of one prism (bounds W, E, S, N, B, T; grho = G * density)
 // at (e, n, u) to acc[]; OR singular-point bits into sflags.  Without
-// kGeneral, needs_general<M> must be false for the point, or with kGenX
-// (has_x_only field sets) needs_full_general<M>.
-template <unsigned M, bool kGeneral, bool kGenX = kGeneral>
+// kGeneral, needs_general<M> must be false for the point.
+template <unsigned M, bool kGeneral>
 __device__ __forceinline__ void prism_pair_path(double e, double n, double u, double W, double E,
                                                 double S, double N, double B, double T,
                                                 double grho, double (&acc)[FieldSet<M>::count],
                                                 uint32_t &sflags, const dm::Tables &tab) {
     using F = FieldSet<M>;
     if constexpr (M == 0x8u) {  // g_u alone
-        acc[0] += grho * gu_sum<false, kGeneral, kGenX>(E - e, W - e, N - n, S - n, T - u,
-                                                               B - u, tab, nullptr);
+        acc[0] += grho * gu_sum<false, kGeneral>(E - e, W - e, N - n, S - n, T - u, B - u, tab,
+                                                 nullptr);
     } else if constexpr (M == 0x2u) {  // g_e alone: K_e is K_u with (x, y, z) -> (y, z, x)
         acc[0] += grho * gu_sum<false, kGeneral>(N - n, S - n, T - u, B - u, E - e, W - e, tab,
                                                  nullptr);
@@ -607,91 +496,15 @@ __device__ __forceinline__ void prism_pair_path(double e, double n, double u, do
                                                  nullptr);
     } else if constexpr ((M & 0xfu) == 0 && !kGeneral) {  // tensor terms only
         double K[6];
-        if constexpr (kGenX)
-            tensor_xonly<M>(E - e, W - e, N - n, S - n, T - u, B - u, K, tab);
-        else
-            tensor_lean<M>(E - e, W - e, N - n, S - n, T - u, B - u, K, tab);
+        tensor_lean<M>(E - e, W - e, N - n, S - n, T - u, B - u, K, tab);
 #pragma unroll
         for (int f = 4; f < 10; ++f)
             if ((M >> f) & 1u) acc[F::slot(f)] += grho * K[f - 4];
     } else {
         double vs[F::count];
-        prism_fields<M, kGeneral, kGenX>(E - e, W - e, N - n, S - n, T - u, B - u, vs, sflags,
-                                         tab);
+        prism_fields<M, kGeneral>(E - e, W - e, N - n, S - n, T - u, B - u, vs, sflags, tab);
 #pragma unroll
         for (int s = 0; s < F::count; ++s) acc[s] += grho * vs[s];
-    }
-}
-
-// prism_pair_path with the instantiation chosen per prism and wave.
-template <unsigned M>
-__device__ __forceinline__ void prism_pair(double e, double n, double u, double W, double E,
-                                           double S, double N, double B, double T, double grho,
-                                           double (&acc)[FieldSet<M>::count], uint32_t &sflags,
-                                           const dm::Tables &tab) {
-    if (any_lane(needs_general<M>(e, n, u, W, E, S, N, B, T)))
-        prism_pair_path<M, true>(e, n, u, W, E, S, N, B, T, grho, acc, sflags, tab);
-    else
-        prism_pair_path<M, false>(e, n, u, W, E, S, N, B, T, grho, acc, sflags, tab);
-}
-
-// Accumulate the prisms tile[0, cnt) (LDS, read as wave-uniform broadcasts;
-// P has w, e, s, n, b, t, grho and, with kMaySkip, int skip) at (e, n, u).
-// Pass 1 evaluates the lean form for every prism that no lane of the wave
-// needs the general form for and marks the others in wave-uniform 128-bit
-// masks: those for which the x-planes alone made the lean form unusable
-// (has_x_only field sets; for the 64 points of a wave along a grid row,
-// the prisms of the 64 columns the points fall in) and the rest.  Pass 2
-// evaluates the first with the x-only form, pass 3 the rest with the
-// general form.
-// Separate loops keep the forms' register allocations apart.  The order of
-// the additions is fixed by the prisms and the points, so results are
-// deterministic.
-template <unsigned M, bool kMaySkip, class P>
-__device__ __forceinline__ void tile_pairs(const P *tile, int cnt, double e, double n, double u,
-                                           double (&acc)[FieldSet<M>::count], uint32_t &sflags,
-                                           const dm::Tables &tab) {
-    uint64_t general_lo = 0, general_hi = 0, xonly_lo = 0, xonly_hi = 0;
-    for (int p = 0; p < cnt; ++p) {
-        const P sp = tile[p];
-        if constexpr (kMaySkip) {
-            if (sp.skip) continue;
-        }
-        if (any_lane(needs_general<M>(e, n, u, sp.w, sp.e, sp.s, sp.n, sp.b, sp.t))) {
-            bool full = true;
-            if constexpr (has_x_only<M>())
-                full = any_lane(needs_full_general<M>(e, n, u, sp.w, sp.e, sp.s, sp.n, sp.b, sp.t));
-            uint64_t &lo = full ? general_lo : xonly_lo, &hi = full ? general_hi : xonly_hi;
-            if (p < 64)
-                lo |= 1ull << p;
-            else
-                hi |= 1ull << (p - 64);
-            continue;
-        }
-        prism_pair_path<M, false>(e, n, u, sp.w, sp.e, sp.s, sp.n, sp.b, sp.t, sp.grho, acc,
-                                  sflags, tab);
-    }
-    if constexpr (has_x_only<M>()) {
-        for (int half = 0; half < 2; ++half) {
-            uint64_t m = half ? xonly_hi : xonly_lo;
-            while (m) {
-                const int p = 64 * half + __builtin_ctzll(m);
-                m &= m - 1;
-                const P sp = tile[p];
-                prism_pair_path<M, false, true>(e, n, u, sp.w, sp.e, sp.s, sp.n, sp.b, sp.t,
-                                                sp.grho, acc, sflags, tab);
-            }
-        }
-    }
-    for (int half = 0; half < 2; ++half) {
-        uint64_t m = half ? general_hi : general_lo;
-        while (m) {
-            const int p = 64 * half + __builtin_ctzll(m);
-            m &= m - 1;
-            const P sp = tile[p];
-            prism_pair_path<M, true>(e, n, u, sp.w, sp.e, sp.s, sp.n, sp.b, sp.t, sp.grho, acc,
-                                     sflags, tab);
-        }
     }
 }
 

@@ -199,8 +199,11 @@ struct FarBox {
 };
 
 // Smallest squared distance from the box to the nearer face centre of a
-// staged prism; NaN (never far) if the prism or the whole box is NaN.
+// staged prism; NaN (never far) if the prism or the whole box is NaN.  (No
+// contraction here and below: kernels that share the work of a pair have to
+// come to the same decision.)
 __device__ __forceinline__ double far_distance2(const FarBox &b, const FarPrism &p) {
+#pragma clang fp contract(off)
     // fmax drops a NaN operand: keep it with the sum of the differences
     const double nan_guard = ((p.x - b.x0) + (p.y - b.y0) + (p.t - b.u0) + (p.b - b.u0)) * 0.0;
     const double dx = fmax(fmax(b.x0 - p.x, p.x - b.x1), 0.0);
@@ -215,6 +218,7 @@ __device__ __forceinline__ double far_distance2(const FarBox &b, const FarPrism 
 // keeps the monomials of the constants finite).
 template <int I>
 __device__ __forceinline__ bool far_enough(double d2, double h2) {
+#pragma clang fp contract(off)
     return d2 >= far_ratio2(I) * h2 && d2 < 1e50;
 }
 
@@ -299,6 +303,7 @@ __device__ __forceinline__ void far_consts(double A, double B, int part, double 
 
 // Squared half-sides of a prism's rectangle.
 __device__ __forceinline__ void half_sides2(const double (&b)[6], double &A, double &B) {
+#pragma clang fp contract(off)
     const double width = b[1] - b[0], length = b[3] - b[2];
     A = 0.25 * width * width;
     B = 0.25 * length * length;
@@ -317,6 +322,18 @@ __device__ __forceinline__ void gz_table(const Src &src, int64_t p, GzShared &sh
             sh.B = B;
         }
     }
+}
+
+// The staged record of a prism (weight: of the far form, times the area).
+__device__ __forceinline__ FarPrism far_prism(const double (&b)[6], double xo, double yo,
+                                              double weight) {
+#pragma clang fp contract(off)
+    double A, B;
+    half_sides2(b, A, B);
+    const double area = (b[1] - b[0]) * (b[3] - b[2]);
+    return FarPrism{0.5 * ((b[0] - xo) + (b[1] - xo)), 0.5 * ((b[2] - yo) + (b[3] - yo)),
+                    b[5],                              b[4],
+                    weight * area,                     A + B};
 }
 
 // Stages prisms [t0, t0 + cnt), cnt <= kGzTile.  Src::get(p, bounds, rho)
@@ -338,9 +355,7 @@ __device__ __forceinline__ void gz_stage(const Src &src, int64_t t0, int cnt, do
         half_sides2(b, A, B);
         if (q < cnt) {
             sh.tile[q] = GzPrism{b[0], b[1], b[2], b[3], b[4], b[5], kG * rho, 0.0};
-            sh.far[q] = FarPrism{0.5 * ((b[0] - xo) + (b[1] - xo)),
-                                 0.5 * ((b[2] - yo) + (b[3] - yo)), b[5], b[4],
-                                 kG * rho * ((b[1] - b[0]) * (b[3] - b[2])), A + B};
+            sh.far[q] = far_prism(b, xo, yo, kG * rho);
         }
         const bool same = fabs(A - sh.A) <= 0x1p-36 * sh.A && fabs(B - sh.B) <= 0x1p-36 * sh.B;
         const uint64_t live = __ballot(!skip), different = __ballot(!skip && !same);

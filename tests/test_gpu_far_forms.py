@@ -181,3 +181,80 @@ def test_layer_gradient_is_the_adjoint(hm, shape, n_obs):
                 + (2000.0 + coords[2]) ** 2)
     weight = 1e5 * G * (np.abs(a).ravel() + 400.0 * np.abs(b).ravel())
     assert abs(left - right) <= 64 * 2.0**-53 * (weight[:, None] * (r + 1.0) * np.abs(v)).sum()
+
+
+TEN = ("potential", "g_e", "g_n", "g_z", "g_ee", "g_nn", "g_zz", "g_en", "g_ez", "g_nz")
+
+
+def _fields_exact(coords, prisms, weights):
+    """{field: (value, error bound)} of the ten fields (G, units and harmonica's
+    signs left out) in extended precision, closed form vertex by vertex; the
+    bound is 64 x 2^-53 of the terms' size r^2, r or 1 in sum over all pairs."""
+    ld = np.longdouble
+    e, n, u = (np.asarray(c, dtype=ld)[:, None] for c in coords)
+    p = prisms.astype(ld)
+    total = {f: 0 for f in TEN}
+    for i, x in enumerate((p[:, 1] - e, p[:, 0] - e)):
+        for j, y in enumerate((p[:, 3] - n, p[:, 2] - n)):
+            for k, z in enumerate((p[:, 5] - u, p[:, 4] - u)):
+                r = np.sqrt(x * x + y * y + z * z)
+                lx, ly, lz = (np.where(a >= 0, np.log(r + np.abs(a)),
+                                       np.log((b * b + c * c) / (r + np.abs(a))))
+                              for a, b, c in ((x, y, z), (y, x, z), (z, x, y)))
+                ax, ay, az = (np.arctan(b * c / (a * r)) for a, b, c in
+                              ((x, y, z), (y, x, z), (z, x, y)))
+                v = (x * y * lz + y * z * lx + z * x * ly
+                     - (x * x * ax + y * y * ay + z * z * az) / 2,
+                     -(y * lz + z * ly - x * ax), -(z * lx + x * lz - y * ay),
+                     -(x * ly + y * lx - z * az), -ax, -ay, -az, lz, ly, lx)
+                for f, value in zip(TEN, v):
+                    total[f] = total[f] + (-1) ** (i + j + k) * value
+    r = np.sqrt((np.abs((p[:, 0] + p[:, 1]) / 2 - e) + 300) ** 2
+                + (np.abs((p[:, 2] + p[:, 3]) / 2 - n) + 300) ** 2
+                + np.maximum(np.abs(p[:, 5] - u), np.abs(p[:, 4] - u)) ** 2)
+    w = np.abs(weights)
+    return {f: ((total[f] * weights).sum(axis=1).astype(float),
+                (64 * r ** (2 if k == 0 else 1 if k < 4 else 0) * w).sum(axis=1).astype(float)
+                * 2.0**-53) for k, f in enumerate(TEN)}
+
+
+_UNIT = dict(zip(TEN, (1.0, 1e5, 1e5, -1e5, 1e9, 1e9, 1e9, 1e9, -1e9, -1e9)))
+
+
+@pytest.mark.parametrize("kind", ["grid", "different"])
+@pytest.mark.parametrize("m", [1, 31, 33, 70])
+def test_all_fields_all_distances(hm, kind, m):
+    """Single fields, the fused sets and the magnetic components at points above
+    the model, below it, level with it and straight above one prism, from 40 m
+    to 100 km: every order, the closed form, and waves that mix them."""
+    from harmonica_amd._forward import prism_fields_device, to_device
+
+    rng = np.random.default_rng(m)
+    prisms = _model(kind, m, rng)
+    rho = rng.uniform(100, 500, m)
+    k = 200
+    d, phi = np.geomspace(40.0, 1e5, k), rng.uniform(0, 2 * np.pi, k)
+    up = np.r_[rng.uniform(5.0, 300.0, 80), rng.uniform(-4e3, -3.5e3, 60), rng.uniform(-300, -1, 60)]
+    coords = [53.0 + d * np.cos(phi), 47.0 + d * np.sin(phi), up]
+    up[::2] *= 5.0
+    centre = prisms[0, [0, 2]] + 0.37 * (prisms[0, [1, 3]] - prisms[0, [0, 2]])
+    coords = [np.r_[coords[0], np.full(20, centre[0])], np.r_[coords[1], np.full(20, centre[1])],
+              np.r_[coords[2], np.geomspace(500.0, 3e4, 20)]]
+    order = rng.permutation(k + 20)
+    coords = [c[order] for c in coords]
+    exact = _fields_exact(coords, prisms, G * rho)
+    dev = [to_device(np.ascontiguousarray(c)) for c in coords]
+    P, D = to_device(prisms), to_device(rho)
+    for fields in (*((f,) for f in TEN), TEN[1:4], TEN[4:], TEN):
+        got = prism_fields_device(*dev, P, D, fields).cpu().numpy()
+        for f, row in zip(fields, got):
+            value, bound = exact[f]
+            assert (np.abs(row / _UNIT[f] - value) <= bound).all(), (f, len(fields))
+    me, mn, mu = (rng.normal(size=m) for _ in range(3))
+    terms = {"b_e": ("g_ee", "g_en", "g_ez"), "b_n": ("g_en", "g_nn", "g_nz"),
+             "b_u": ("g_ez", "g_nz", "g_zz")}
+    for name, fields in terms.items():
+        parts = [_fields_exact(coords, prisms, w)[f] for w, f in zip((me, mn, mu), fields)]
+        value, bound = (sum(p[q] for p in parts) for q in (0, 1))
+        got = hm.prism_magnetic(coords, prisms, (me, mn, mu), name) / 100.0  # 1e-7 x 1e9
+        assert (np.abs(got - value) <= bound).all(), name
