@@ -524,122 +524,192 @@ int launch_gemm_tn(const double *A, int64_t lda, const double *B, int64_t ldb, i
 }
 
 // ---------------------------------------------------------------- Cholesky
-// v from another lane of the same group of 8 aligned lanes, by a DPP move
-// of its two 32-bit halves (kCtrl: quad_perm [1,0,3,2] = 0xb1 for lane ^ 1,
-// quad_perm [2,3,0,1] = 0x4e for lane ^ 2, row_half_mirror = 0x141 for
-// lane 7 - i of the group); a VALU operation, no trip through the LDS unit.
-template <int kCtrl>
-__device__ __forceinline__ double dpp_f64(double v) {
+// v of the given lane (a constant), the same in every lane.
+__device__ __forceinline__ double lane_f64(double v, int lane) {
     const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_mov_dpp((int)b, kCtrl, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), kCtrl, 0xf, 0xf, false);
+    const int lo = __builtin_amdgcn_readlane((int)b, lane);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
     return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
-// Sum over each group of 8 aligned lanes, in every lane of the group: the
-// pair and quad sums, then the other quad's sum (the same value in its four
-// lanes), so the result is the same as with xor shuffles 1, 2, 4.
-__device__ __forceinline__ double sum8_f64(double v) {
-    v += dpp_f64<0xb1>(v);
-    v += dpp_f64<0x4e>(v);
-    v += dpp_f64<0x141>(v);
-    return v;
+// Sizes of potrf_diag_kernel: tiles of 16 (the FP64 MFMA's), LDS row stride
+// 130 (rows of a tile start 4 banks apart, so an MFMA operand read along a
+// column of a tile, 16 rows x 4 columns, falls on distinct banks).
+constexpr int kDT = 16, kDTiles = kNB / kDT, kDS = kNB + 2;
+
+// c + sign * A B of two 16 x 16 tiles in LDS (row stride kDS); AT: A is
+// given transposed.
+template <bool AT>
+__device__ __forceinline__ double4_t tile_product(const double *A, const double *B, double sign,
+                                                  int lane, double4_t c) {
+    const int lo = lane & 15, hi = lane >> 4;
+#pragma unroll
+    for (int ks = 0; ks < kDT; ks += 4) {
+        const double a = AT ? A[(ks + hi) * kDS + lo] : A[lo * kDS + ks + hi];
+        c = Mfma<double>::step(sign * a, B[(ks + hi) * kDS + lo], c);
+    }
+    return c;
+}
+
+__device__ __forceinline__ void tile_store(double *C, double4_t c, int lane) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) C[Mfma<double>::row(lane, v) * kDS + (lane & 15)] = c[v];
 }
 
 // Factor the nb x nb diagonal block at D (upper, row-major, ld) in place as
 // U^T U and write U^-1 to Dinv (nb x nb, row-major, ld kNB) and its
-// transpose to DinvT.  One workgroup; the block lives in LDS.  On a
-// non-positive pivot, *info is set (once) to its 1-based global column and
-// the block is left unfinished.
+// transpose to DinvT.  One workgroup; the block lives in LDS, continued
+// past nb by the identity.  On a non-positive pivot, *info is set (once) to
+// its 1-based global column and the block is left unfinished.
+//
+// Bound by the chain through the 128 pivots, which one workgroup walks: the
+// work is 2 MFLOP.  So a step takes 16 pivots, not one: each of up to three
+// wavefronts eliminates the 16 x 16 diagonal tile in registers (lane c < 16
+// holds column c; the multipliers are broadcast by lane reads, no barrier
+// and no LDS between pivots) together with 48 further columns that ride in
+// its other lanes (the row panel, and the identity, whose columns become
+// the rows of the tile's inverse); then one barrier, and all wavefronts
+// update the trailing tiles by MFMA.  The inverse is put together from the
+// tiles' inverses by doubling, inv([A B; 0 C]) = [A^-1, -A^-1 B C^-1; 0,
+// C^-1], three levels with one MFMA tile per wavefront.  42 us per full
+// block, against 156 us for one pivot per barrier and an inverse by rows.
 __global__ __launch_bounds__(1024) void potrf_diag_kernel(double *__restrict__ D, int64_t ld,
                                                           int nb, int64_t col0,
                                                           double *__restrict__ Dinv,
                                                           double *__restrict__ DinvT,
                                                           int *__restrict__ info, int64_t bsd,
                                                           int64_t bsinv, int info_stride) {
-    constexpr int S = kNB + 1;
     // problem blockIdx.x of a strided batch
     D += (int64_t)blockIdx.x * bsd;
     Dinv += (int64_t)blockIdx.x * bsinv;
     DinvT += (int64_t)blockIdx.x * bsinv;
     info += (int64_t)blockIdx.x * info_stride;
-    __shared__ double L[kNB * S];
-    __shared__ double piv[kNB];
+    __shared__ double L[kNB * kDS];
+    __shared__ double Xd[kNB * (kDT + 1)];  // the tiles' inverses, one below the other
+    __shared__ int failed;
     const int tid = threadIdx.x, tx = tid & 31, ty = tid >> 5;  // 32 x 32 threads
-    // upper triangle of the block; the rest of L is zero (the inverse below
-    // multiplies it by zeros, and it may not hold finite values in D)
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tiles = (nb + kDT - 1) / kDT;
+    if (tid == 0) failed = 0;
+    // Upper triangle of the block (what lies below it in D may not be finite).
+#pragma unroll
     for (int r = ty; r < kNB; r += 32)
-        for (int c = tx; c < kNB; c += 32)
-            L[r * S + c] = (r < nb && c < nb && r <= c) ? D[r * ld + c] : 0.0;
-    __syncthreads();
-    // Right-looking factorisation, one barrier per column: every thread
-    // reads the pivot d (the same value, so the test is uniform) and updates
-    // its part of the trailing upper triangle by L[k][r] L[k][c] / d; row k
-    // itself is read only in step k and is scaled by its pivot at the end.
-    for (int k = 0; k < nb; ++k) {
-        const double d = L[k * S + k];
-        if (!(d > 0.0)) {
-            if (tid == 0) atomicCAS(info, 0, (int)(col0 + k + 1));
-            return;
+#pragma unroll
+        for (int c = tx; c < kNB; c += 32) {
+            const bool in = r <= c && c < nb;
+            const double v = D[in ? r * ld + c : 0];
+            L[r * kDS + c] = in ? v : (r == c ? 1.0 : 0.0);
         }
-        if (tid == 0) piv[k] = sqrt(d);
-        const double invd = 1.0 / d;
-        for (int r = k + 1 + ty; r < nb; r += 32) {
-            const double lr = L[k * S + r] * invd;
-            for (int c = r + tx; c < nb; c += 32) L[r * S + c] = fma(-lr, L[k * S + c], L[r * S + c]);
+    __syncthreads();
+    for (int b = 0; b < tiles; ++b) {
+        const int k0 = kDT * b;
+        // Columns beside the diagonal tile's: q = 0 .. 15 the identity's,
+        // q >= 16 column k0 + q of the block.
+        const int q = (64 - kDT) * wave + lane - kDT;
+        const bool diag = lane < kDT, unit = !diag && q < kDT;
+        const bool panel = !diag && !unit && q < kNB - k0;
+        const bool works = (64 - kDT) * wave < kNB - k0;  // uniform in the wavefront
+        double a[kDT];
+        if (works) {
+            const int col = diag ? k0 + lane : (panel ? k0 + q : k0);
+#pragma unroll
+            for (int r = 0; r < kDT; ++r) a[r] = L[(k0 + r) * kDS + col];
+            if (unit)
+#pragma unroll
+                for (int r = 0; r < kDT; ++r) a[r] = r == q ? 1.0 : 0.0;
+            int bad = 0;
+            double own = 1.0;  // lane k: pivot k
+#pragma unroll
+            for (int k = 0; k < kDT; ++k) {
+                const double d = lane_f64(a[k], k);
+                if (!(d > 0.0) && bad == 0) bad = k + 1;
+                if (lane == k) own = d;
+                const double t = a[k] * (1.0 / d);
+#pragma unroll
+                for (int r = k + 1; r < kDT; ++r) a[r] = fma(-lane_f64(a[k], r), t, a[r]);
+            }
+            const double root = sqrt(own), inv = 1.0 / root;
+#pragma unroll
+            for (int k = 0; k < kDT; ++k) {
+                a[k] *= lane_f64(inv, k);
+                if (lane == k) a[k] = root;
+            }
+            if (panel)
+#pragma unroll
+                for (int r = 0; r < kDT; ++r) L[(k0 + r) * kDS + k0 + q] = a[r];
+            if (unit)
+#pragma unroll
+                for (int r = 0; r < kDT; ++r) Xd[(k0 + q) * (kDT + 1) + r] = a[r];
+            if (tid == 0 && bad) {
+                atomicCAS(info, 0, (int)(col0 + k0 + bad));
+                failed = 1;
+            }
+        }
+        __syncthreads();
+        if (failed) return;
+        // The diagonal tile itself, which the other wavefronts read above.
+        if (wave == 0 && diag)
+#pragma unroll
+            for (int r = 0; r < kDT; ++r) L[(k0 + r) * kDS + k0 + lane] = r <= lane ? a[r] : 0.0;
+        const int m = tiles - 1 - b;
+        for (int t = wave; t < m * (m + 1) / 2; t += 16) {
+            int i = 0, j = t;  // tile t of the m x m upper triangle, by rows
+            while (j >= m - i) {
+                j -= m - i;
+                ++i;
+            }
+            const int ti = k0 + kDT * (1 + i), tj = ti + kDT * j;
+            double *C = L + ti * kDS + tj;
+            double4_t c;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) c[v] = C[Mfma<double>::row(lane, v) * kDS + (lane & 15)];
+            tile_store(C, tile_product<true>(L + k0 * kDS + ti, L + k0 * kDS + tj, -1.0, lane, c),
+                       lane);
         }
         __syncthreads();
     }
-    for (int r = ty; r < nb; r += 32) {
-        const double inv = 1.0 / piv[r];
-        for (int c = r + tx; c < nb; c += 32) L[r * S + c] = c == r ? piv[r] : L[r * S + c] * inv;
-    }
-    __syncthreads();
-    for (int r = ty; r < nb; r += 32)
-        for (int c = tx; c < nb; c += 32) D[r * ld + c] = r <= c ? L[r * S + c] : 0.0;
-    // reciprocals of the factor's diagonal, once (they multiply below)
-    if (tid < nb) piv[tid] = 1.0 / L[tid * S + tid];
-    __syncthreads();
-    // Inverse X = U^-1 row by row, from X U = I:
-    //   X[i][i] = 1 / U[i][i],  X[i][j] = -(sum_{k=i}^{j-1} X[i][k] U[k][j]) (1 / U[j][j]).
-    // Rows are independent, so there is no barrier: row i belongs to the 8
-    // adjacent lanes of its group, lane p keeping X[i][8 q + p] in xr[q]
-    // (zero until computed, and for k < i), each sum split over the lanes
-    // and combined by DPP moves.  Wavefront w holds rows 8 w .. 8 w + 7,
-    // whose terms start at k = 8 w, so its loops skip q < w uniformly.
-    {
-        const int i = tid >> 3, p = tid & 7, w = tid >> 6;
-        const bool live = i < nb;
-        double xr[16];
+    // The factor goes out; the diagonal tiles then hold their inverses.
 #pragma unroll
-        for (int q = 0; q < 16; ++q) xr[q] = (live && 8 * q + p == i) ? piv[i] : 0.0;
+    for (int r = ty; r < kNB; r += 32)
 #pragma unroll
-        for (int jb = 0; jb < 16; ++jb) {
-            if (jb < w) continue;  // uniform in the wavefront
-#pragma unroll
-            for (int jj = 0; jj < 8; ++jj) {
-                const int j = 8 * jb + jj;
-                double acc0 = 0.0, acc1 = 0.0;  // two chains of FMAs
-#pragma unroll
-                for (int q = 0; q <= jb; ++q) {
-                    if (q < w) continue;  // uniform in the wavefront
-                    if (q & 1)
-                        acc1 = fma(xr[q], L[(8 * q + p) * S + j], acc1);
-                    else
-                        acc0 = fma(xr[q], L[(8 * q + p) * S + j], acc0);
-                }
-                const double acc = sum8_f64(acc0 + acc1);
-                if (live && j > i && j < nb && p == jj) xr[jb] = -acc * piv[j];
-            }
+        for (int c = tx; c < kNB; c += 32) {
+            if (r < nb && c < nb) D[r * ld + c] = r <= c ? L[r * kDS + c] : 0.0;
+            if (r / kDT == c / kDT && r / kDT < tiles)
+                L[r * kDS + c] = r <= c ? Xd[r * (kDT + 1) + (c & (kDT - 1))] : 0.0;
         }
+    __syncthreads();
+    // Level h joins the inverses of h tiles to ones of 2 h: tile (i, j) of
+    // -A^-1 B C^-1 in place of B's, with A^-1 B kept where the tile (j, i)
+    // of the unused lower triangle lies.  4 h tiles in all, one per wavefront.
 #pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const int k = 8 * q + p;
-            const double v = (live && k < nb && k >= i) ? xr[q] : 0.0;
-            Dinv[i * kNB + k] = v;
-            DinvT[k * kNB + i] = v;
+    for (int h = 1; h < kDTiles; h *= 2) {
+        const int g = wave / (h * h), e = wave % (h * h);
+        const int first = 2 * g * h, mid = first + h, i = first + e / h, j = mid + e % h;
+        const bool works = wave < 4 * h && j < tiles;
+        if (works) {
+            double4_t c = {0.0, 0.0, 0.0, 0.0};
+            for (int k = i; k < mid; ++k)
+                c = tile_product<false>(L + kDT * (i * kDS + k), L + kDT * (k * kDS + j), 1.0,
+                                        lane, c);
+            tile_store(L + kDT * (j * kDS + i), c, lane);
         }
+        __syncthreads();
+        if (works) {
+            double4_t c = {0.0, 0.0, 0.0, 0.0};
+            for (int k = mid; k <= j; ++k)
+                c = tile_product<false>(L + kDT * (k * kDS + i), L + kDT * (k * kDS + j), -1.0,
+                                        lane, c);
+            tile_store(L + kDT * (i * kDS + j), c, lane);
+        }
+        __syncthreads();
     }
+#pragma unroll
+    for (int r = ty; r < kNB; r += 32)
+#pragma unroll
+        for (int c = tx; c < kNB; c += 32) {
+            Dinv[r * kNB + c] = r <= c && c < nb ? L[r * kDS + c] : 0.0;
+            DinvT[r * kNB + c] = c <= r && r < nb ? L[c * kDS + r] : 0.0;
+        }
 }
 
 // ------------------------------------------------------------------ solves

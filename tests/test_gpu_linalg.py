@@ -276,3 +276,49 @@ def test_lsq_svd_graded_and_rank_deficient(env):
     npt.assert_allclose(H @ coef, H @ expected, rtol=0, atol=1e-10 * np.abs(H @ expected).max())
     npt.assert_allclose(coef[:3], coef[40:], rtol=1e-8)
     npt.assert_allclose(coef, expected, rtol=1e-6, atol=1e-8 * np.abs(expected).max())
+
+
+def _factor(env, A, rhs):
+    """hmx_cholesky_solve of host arrays: (U, x, info)."""
+    torch, _lib, L = env
+    m = len(A)
+    nbytes = ctypes.c_size_t(0)
+    _lib.check(L.hmx_cholesky_workspace_bytes(m, ctypes.byref(nbytes)))
+    ws = torch.empty(nbytes.value, dtype=torch.uint8, device="cuda")
+    dA, dx = torch.tensor(A).cuda(), torch.tensor(rhs).cuda()
+    info = ctypes.c_int(-1)
+    _lib.check(L.hmx_cholesky_solve(_lib.ptr(dA), m, _lib.ptr(dx), ctypes.byref(info), _lib.ptr(ws),
+                                    nbytes.value, None))
+    return np.triu(dA.cpu().numpy()), dx.cpu().numpy(), info.value
+
+
+@pytest.mark.parametrize("m", [1, 2, 15, 16, 17, 31, 33, 48, 64, 79, 80, 81, 112, 113, 127, 144, 145])
+def test_diagonal_block_tiles(env, m):
+    """The diagonal block's 16 x 16 tiles: blocks that end inside, at and
+    just past a tile, with nothing finite below the diagonal.  Factor: the
+    backward error of a Cholesky factorisation, (m + 8) roundings (the 8 for
+    the reciprocals) of |U|^T |U|.  Solution: the spectrum lies in [m, 9 m]
+    or so, so 64 m roundings bound the error of x."""
+    rng = np.random.default_rng(m)
+    X = rng.normal(size=(2 * m, m))
+    A = X.T @ X + m * np.eye(m)
+    rhs = rng.normal(size=m)
+    given = A.copy()
+    given[np.tril_indices(m, -1)] = np.nan
+    U, x, info = _factor(env, given, rhs)
+    assert info == 0
+    ulp = 2.0**-52
+    wide = U.astype(np.longdouble)
+    bound = (m + 8) * ulp * (np.abs(U).T @ np.abs(U))
+    assert np.all(np.abs((wide.T @ wide).astype(float) - A) <= bound)
+    expected = np.linalg.solve(A, rhs)
+    npt.assert_allclose(x, expected, rtol=0, atol=64 * m * ulp * np.abs(expected).max())
+
+
+@pytest.mark.parametrize("m,bad", [(1, 0), (16, 15), (17, 16), (100, 15), (128, 0), (128, 127),
+                                   (144, 128), (145, 144)])
+@pytest.mark.parametrize("pivot", [-1.0, 0.0, np.nan])
+def test_diagonal_block_bad_pivot(env, m, bad, pivot):
+    A = np.eye(m)
+    A[bad, bad] = pivot
+    assert _factor(env, A, np.ones(m))[2] == bad + 1
