@@ -38,7 +38,6 @@ constexpr int kNB = 128;    // Cholesky block size
 constexpr int kOuter = 1024;  // Cholesky outer block (K of the big trailing updates)
 constexpr int kST = 128;    // SYRK block tile (kST x kST per workgroup of 256 threads)
 constexpr int kKC = 16;     // SYRK K chunk staged in LDS
-constexpr int kPad = 144;   // LDS row stride (doubles/floats) of the SYRK panels
 
 __device__ __forceinline__ double inv_dist(double ae, double an, double au, double be, double bn,
                                            double bu) {
@@ -183,62 +182,41 @@ struct Mfma<float> {
     static __device__ __forceinline__ int row(int lane, int v) { return 4 * (lane >> 4) + v; }
 };
 
-// Rows [k0, k0 + kKC) x columns [col0, col0 + kST) of a row-major K x cols
-// panel, fetched 8 consecutive columns per thread (16-byte loads when the
-// panel is aligned, zero outside the panel).
+// Rows [k0, k0 + kKC) x columns [col0, col0 + 16 W) of a row-major K x cols
+// panel, fetched W columns per thread (zero outside the panel) in pieces of
+// 16 bytes: piece i of slot c (0 .. 15) of a row starts at column
+// kVec (16 i + c), so the 16 slots of a row read 256 contiguous bytes and
+// write their LDS copies without bank conflicts.
 template <class T>
 struct Panel {
+    static constexpr int kVec = 16 / sizeof(T);
+    typedef T vec_t __attribute__((ext_vector_type(16 / sizeof(T))));
     const T *X;
     int64_t ld, rows, cols;
     bool vec;  // X and ld * sizeof(T) are multiples of 16 bytes
-    // Unchecked 16-byte loads: the caller guarantees the whole kKC x kST
+    // Unchecked 16-byte loads: the caller guarantees the whole kKC x 16 W
     // block is inside the panel and vec is set.
-    __device__ __forceinline__ void fetch_fast(int64_t k0, int64_t col0, int kk, int c8,
-                                               T (&v)[8]) const {
-        const T *p = X + (k0 + kk) * ld + col0 + 8 * c8;
-        if constexpr (sizeof(T) == 8) {
+    template <int P>
+    __device__ __forceinline__ void fetch_fast(int64_t k0, int64_t col0, int kk, int c,
+                                               vec_t (&v)[P]) const {
+        const T *p = X + (k0 + kk) * ld + col0;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const double2 d = reinterpret_cast<const double2 *>(p)[i];
-                v[2 * i] = d.x;
-                v[2 * i + 1] = d.y;
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const float4 f = reinterpret_cast<const float4 *>(p)[i];
-                v[4 * i] = f.x;
-                v[4 * i + 1] = f.y;
-                v[4 * i + 2] = f.z;
-                v[4 * i + 3] = f.w;
-            }
-        }
+        for (int i = 0; i < P; ++i) v[i] = *reinterpret_cast<const vec_t *>(p + kVec * (16 * i + c));
     }
-    __device__ __forceinline__ void fetch(int64_t k0, int64_t col0, int kk, int c8,
-                                          T (&v)[8]) const {
-        const int64_t k = k0 + kk, c = col0 + 8 * c8;
-        if (k < rows && c + 8 <= cols && vec) {
-            const T *p = X + k * ld + c;
-            if constexpr (sizeof(T) == 8) {
+    template <int P>
+    __device__ __forceinline__ void fetch(int64_t k0, int64_t col0, int kk, int cs,
+                                          vec_t (&v)[P]) const {
+        const int64_t k = k0 + kk;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const double2 d = reinterpret_cast<const double2 *>(p)[i];
-                    v[2 * i] = d.x;
-                    v[2 * i + 1] = d.y;
-                }
+        for (int i = 0; i < P; ++i) {
+            const int64_t c = col0 + kVec * (16 * i + cs);
+            if (k < rows && c + kVec <= cols && vec) {
+                v[i] = *reinterpret_cast<const vec_t *>(X + k * ld + c);
             } else {
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const float4 f = reinterpret_cast<const float4 *>(p)[i];
-                    v[4 * i] = f.x;
-                    v[4 * i + 1] = f.y;
-                    v[4 * i + 2] = f.z;
-                    v[4 * i + 3] = f.w;
-                }
+                for (int e = 0; e < kVec; ++e)
+                    v[i][e] = (k < rows && c + e < cols) ? X[k * ld + c + e] : T(0);
             }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = (k < rows && c + i < cols) ? X[k * ld + c + i] : T(0);
         }
     }
 };
@@ -249,56 +227,66 @@ Panel<T> make_panel(const T *X, int64_t ld, int64_t rows, int64_t cols) {
     return Panel<T>{X, ld, rows, cols, vec};
 }
 
-// The K loop of one kST x kST tile (see gemm_tn_kernel).  FAST: every chunk
+// The tile of a workgroup: 2 x 2 wavefronts of TR x TC MFMA tiles, whose
+// panels lie in LDS with 16 columns of padding (for doubles, rows then start
+// 32 banks apart, so an operand read's rows k and k + 1 share no bank).
+template <class T, int TR, int TC>
+struct alignas(16) GemmLds {
+    T a[kKC * (32 * TR + 16)], b[kKC * (32 * TC + 16)];
+};
+
+// The K loop of one 32 TR x 32 TC tile (see gemm_tn_kernel).  FAST: every chunk
 // is inside both panels and they are aligned, so the loads are unchecked
 // 16-byte loads; the loop body is straight-line code either way, which
 // keeps the accumulators in place across iterations.
-template <class T, bool FAST, bool UPPER>
+template <class T, bool FAST, bool UPPER, int TR, int TC>
 __device__ __forceinline__ void tile_k_loop(const Panel<T> &A, const Panel<T> &B, int64_t K,
-                                            int64_t r0, int64_t c0, T (*lds)[2][kKC * kPad],
+                                            int64_t r0, int64_t c0, GemmLds<T, TR, TC> *lds,
                                             int64_t M, int64_t N, double *C, int64_t ldc,
                                             double beta, double sign, double shift) {
     using acc_t = typename Mfma<T>::acc_t;
     constexpr bool kFold = !std::is_same<T, double>::value;
-    acc_t acc[4][4];
-    double4_t dacc[kFold ? 4 : 1][kFold ? 4 : 1];
+    constexpr int kPa = 32 * TR + 16, kPb = 32 * TC + 16;
+    acc_t acc[TR][TC];
+    double4_t dacc[kFold ? TR : 1][kFold ? TC : 1];
     // FP64 accumulators are carried across the whole K loop; their zeros
     // come out of the matrix unit itself so they live in the MFMA result
     // registers from the start (a plain zero would be a VGPR value and cost
     // a copy per iteration).  FP32 accumulators restart every chunk.
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < TR; ++a)
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
+        for (int c = 0; c < TC; ++c)
             acc[a][c] = kFold ? acc_t{0, 0, 0, 0}
                               : Mfma<T>::step(T(0), T(0), acc_t{0, 0, 0, 0});
     if constexpr (kFold) {
 #pragma unroll
-        for (int a = 0; a < 4; ++a)
+        for (int a = 0; a < TR; ++a)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) dacc[a][c] = double4_t{0, 0, 0, 0};
+            for (int c = 0; c < TC; ++c) dacc[a][c] = double4_t{0, 0, 0, 0};
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wr = wave >> 1, wc = wave & 1;
-    const int kk = threadIdx.x >> 4, c8 = threadIdx.x & 15;  // staging slot
-    T ra[8], rc[8];
+    const int kk = threadIdx.x >> 4, cs = threadIdx.x & 15;  // staging slot
+    constexpr int kVec = Panel<T>::kVec, kA = 2 * TR / kVec, kB = 2 * TC / kVec;
+    typename Panel<T>::vec_t ra[kA], rc[kB];
     auto fetch = [&](int64_t k0) {
         if constexpr (FAST) {
-            A.fetch_fast(k0, r0, kk, c8, ra);
-            B.fetch_fast(k0, c0, kk, c8, rc);
+            A.fetch_fast(k0, r0, kk, cs, ra);
+            B.fetch_fast(k0, c0, kk, cs, rc);
         } else {
-            A.fetch(k0, r0, kk, c8, ra);
-            B.fetch(k0, c0, kk, c8, rc);
+            A.fetch(k0, r0, kk, cs, ra);
+            B.fetch(k0, c0, kk, cs, rc);
         }
     };
     auto store = [&](int buf) {
-        T *pa = &lds[buf][0][kk * kPad + 8 * c8];
-        T *pb = &lds[buf][1][kk * kPad + 8 * c8];
+        T *pa = &lds[buf].a[kk * kPa + kVec * cs], *pb = &lds[buf].b[kk * kPb + kVec * cs];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            pa[i] = ra[i];
-            pb[i] = rc[i];
-        }
+        for (int i = 0; i < kA; ++i)
+            *reinterpret_cast<typename Panel<T>::vec_t *>(pa + kVec * 16 * i) = ra[i];
+#pragma unroll
+        for (int i = 0; i < kB; ++i)
+            *reinterpret_cast<typename Panel<T>::vec_t *>(pb + kVec * 16 * i) = rc[i];
     };
     // Chunk count as a wave-uniform 32-bit value (K < 2^31 * kKC), so the
     // loop control stays scalar.
@@ -312,28 +300,27 @@ __device__ __forceinline__ void tile_k_loop(const Panel<T> &A, const Panel<T> &B
         const int cur = ch & 1;
         const bool more = ch + 1 < chunks;
         if (more) fetch((int64_t)(ch + 1) * kKC);
-        const T *pr = lds[cur][0];
-        const T *pc = lds[cur][1];
+        const T *pr = lds[cur].a;
+        const T *pc = lds[cur].b;
 #pragma unroll
         for (int ks = 0; ks < kKC; ks += 4) {
             const int kr = ks + (lane >> 4);
-            T a[4], bb[4];
+            T a[TR], bb[TC];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                a[t] = pr[kr * kPad + 64 * wr + 16 * t + (lane & 15)];
-                bb[t] = pc[kr * kPad + 64 * wc + 16 * t + (lane & 15)];
-            }
+            for (int t = 0; t < TR; ++t) a[t] = pr[kr * kPa + 16 * (TR * wr + t) + (lane & 15)];
 #pragma unroll
-            for (int ti = 0; ti < 4; ++ti)
+            for (int t = 0; t < TC; ++t) bb[t] = pc[kr * kPb + 16 * (TC * wc + t) + (lane & 15)];
 #pragma unroll
-                for (int tj = 0; tj < 4; ++tj)
+            for (int ti = 0; ti < TR; ++ti)
+#pragma unroll
+                for (int tj = 0; tj < TC; ++tj)
                     acc[ti][tj] = Mfma<T>::step(a[ti], bb[tj], acc[ti][tj]);
         }
         if constexpr (kFold) {
 #pragma unroll
-            for (int ti = 0; ti < 4; ++ti)
+            for (int ti = 0; ti < TR; ++ti)
 #pragma unroll
-                for (int tj = 0; tj < 4; ++tj) {
+                for (int tj = 0; tj < TC; ++tj) {
 #pragma unroll
                     for (int v = 0; v < 4; ++v) dacc[ti][tj][v] += (double)acc[ti][tj][v];
                     acc[ti][tj] = acc_t{0, 0, 0, 0};
@@ -348,26 +335,26 @@ __device__ __forceinline__ void tile_k_loop(const Panel<T> &A, const Panel<T> &B
     // (clamped) addresses without branches, so their loads overlap, while
     // only a quarter of them is held at once.
 #pragma unroll
-    for (int ti = 0; ti < 4; ++ti) {
-        double old[4][4];
+    for (int ti = 0; ti < TR; ++ti) {
+        double old[TC][4];
         if (beta != 0.0) {
 #pragma unroll
-            for (int tj = 0; tj < 4; ++tj)
+            for (int tj = 0; tj < TC; ++tj)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    int64_t r = r0 + 64 * wr + 16 * ti + Mfma<T>::row(lane, v);
-                    int64_t c = c0 + 64 * wc + 16 * tj + (lane & 15);
+                    int64_t r = r0 + 16 * (TR * wr + ti) + Mfma<T>::row(lane, v);
+                    int64_t c = c0 + 16 * (TC * wc + tj) + (lane & 15);
                     r = r < M ? r : M - 1;
                     c = c < N ? c : N - 1;
                     old[tj][v] = C[r * ldc + c];
                 }
         }
 #pragma unroll
-        for (int tj = 0; tj < 4; ++tj)
+        for (int tj = 0; tj < TC; ++tj)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int64_t r = r0 + 64 * wr + 16 * ti + Mfma<T>::row(lane, v);
-                const int64_t c = c0 + 64 * wc + 16 * tj + (lane & 15);
+                const int64_t r = r0 + 16 * (TR * wr + ti) + Mfma<T>::row(lane, v);
+                const int64_t c = c0 + 16 * (TC * wc + tj) + (lane & 15);
                 if (r < M && c < N && (!UPPER || r <= c)) {
                     const double sum = kFold ? (double)dacc[kFold ? ti : 0][kFold ? tj : 0][v]
                                              : (double)acc[ti][tj][v];
@@ -427,43 +414,60 @@ inline unsigned upper_tile_xcd_blocks(int64_t tiles) {
 // (K x M) and B (K x N) row-major panels and C (M x N) row-major (ldc).
 // UPPER: M == N and only the upper triangle (r <= c) is computed (the
 // symmetric rank-K update A^T A when B == A).  A workgroup of 4 wavefronts
-// owns a kST x kST tile of C (2 x 2 waves of 64 x 64, each 4 x 4 MFMA
-// 16x16x4 tiles).  The K dimension goes through two LDS buffers in chunks
-// of kKC rows: the global loads of chunk c + 1 are issued before the MFMAs
-// of chunk c and written to the other buffer after them, so their latency
-// overlaps the matrix work and one barrier per chunk suffices.  Tiles fully
-// inside aligned panels (with K a multiple of kKC) run the unchecked loop.
-// FP32 MFMA accumulators are folded into FP64 after every chunk (FP32
-// inputs, FP64 sums).  Every workgroup reads all its inputs before it
-// writes its tile, and tiles are disjoint, so C may alias B when M <= kST
-// (used by the in-place panel solve of the Cholesky factorisation).
-template <class T, bool UPPER>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_tn_kernel(Panel<T> A, Panel<T> B, int64_t K,
-                                                      int64_t M, int64_t N, double *C, int64_t ldc,
-                                                      double beta, double sign, double shift,
-                                                      int64_t tiles_n, int64_t bsa, int64_t bsb,
-                                                      int64_t bsc,
-                                                      const int64_t *__restrict__ dims) {
-    __shared__ T lds[2][2][kKC * kPad];
+// owns a 32 TR x 32 TC tile of C (2 x 2 waves of TR x TC MFMA 16x16x4
+// tiles).  The K dimension goes through two LDS buffers in chunks of kKC
+// rows: the global loads of chunk c + 1 are issued before the MFMAs of chunk
+// c and written to the other buffer after them, so their latency overlaps
+// the matrix work and one barrier per chunk suffices.  Tiles fully inside
+// aligned panels (with K a multiple of kKC) run the unchecked loop.  FP32
+// MFMA accumulators are folded into FP64 after every chunk (FP32 inputs,
+// FP64 sums).  Every workgroup reads all its inputs before it writes its
+// tile, and tiles are disjoint, so C may alias B when M <= kST (used by the
+// in-place panel solve of the Cholesky factorisation; a tile then holds all
+// rows of its columns).
+// Whether a kernel's last tiles (those from `whole` on) are taken in four
+// quarters, by one workgroup each.
+template <class T, int TR, int TC>
+constexpr bool kQuarters = std::is_same<T, double>::value && TR == 4 && TC == 4;
+
+template <class T, bool UPPER, int TR, int TC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_tn_kernel(
+    Panel<T> A, Panel<T> B, int64_t K, int64_t M, int64_t N, double *C, int64_t ldc, double beta,
+    double sign, double shift, int64_t tiles_n, int64_t whole, int64_t bsa, int64_t bsb,
+    int64_t bsc, const int64_t *__restrict__ dims) {
+    constexpr int kRows = 32 * TR, kCols = 32 * TC;
+    static_assert(!UPPER || TR == TC, "the upper triangle of square tiles");
+    __shared__ GemmLds<T, TR, TC> lds[2];
+    int64_t t = blockIdx.x;
+    int quarter = -1;
+    if (kQuarters<T, TR, TC> && t >= whole) {
+        quarter = (int)((t - whole) & 3);
+        t = whole + (t - whole) / 4;
+    }
     // problem blockIdx.z of a strided batch (element strides of A, B, C)
     A.X += (int64_t)blockIdx.z * bsa;
     B.X += (int64_t)blockIdx.z * bsb;
     C += (int64_t)blockIdx.z * bsc;
     int64_t rb, cb;
     if (UPPER) {  // row-major over the upper triangle (FP64 MFMA is compute-bound)
-        int64_t bq = blockIdx.x, rem = tiles_n;
+        int64_t rem = tiles_n;
         rb = 0;
-        while (bq >= rem) {
-            bq -= rem;
+        while (t >= rem) {
+            t -= rem;
             ++rb;
             --rem;
         }
-        cb = rb + bq;
+        cb = rb + t;
     } else {
-        rb = blockIdx.x / tiles_n;
-        cb = blockIdx.x - rb * tiles_n;
+        rb = t / tiles_n;
+        cb = t - rb * tiles_n;
     }
-    const int64_t r0 = rb * kST, c0 = cb * kST;
+    int64_t r0 = rb * kRows, c0 = cb * kCols;
+    if (kQuarters<T, TR, TC> && quarter >= 0) {
+        r0 += (quarter >> 1) * (kRows / 2);
+        c0 += (quarter & 1) * (kCols / 2);
+        if (r0 >= M || c0 >= N || (UPPER && r0 > c0)) return;
+    }
     if (dims) {
         // Problem z uses only its first dims[2z] rows (the rest of its panels
         // are zero rows) and its first dims[2z + 1] rows and columns of C (the
@@ -473,16 +477,63 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         const int64_t kr = (kz + kKC - 1) / kKC * kKC;
         K = (r0 < mz && c0 < mz) ? (kr < K ? kr : K) : 0;
     }
-    const bool fast = A.vec && B.vec && r0 + kST <= M && c0 + kST <= N && K % kKC == 0;
-    if (fast)
-        tile_k_loop<T, true, UPPER>(A, B, K, r0, c0, lds, M, N, C, ldc, beta, sign, shift);
+    const bool aligned = A.vec && B.vec && K % kKC == 0;
+    if constexpr (kQuarters<T, TR, TC>) {
+        if (quarter >= 0) {
+            auto *half = reinterpret_cast<GemmLds<T, TR / 2, TC / 2> *>(lds);
+            if (aligned && r0 + kRows / 2 <= M && c0 + kCols / 2 <= N)
+                tile_k_loop<T, true, UPPER, TR / 2, TC / 2>(A, B, K, r0, c0, half, M, N, C, ldc,
+                                                            beta, sign, shift);
+            else
+                tile_k_loop<T, false, UPPER, TR / 2, TC / 2>(A, B, K, r0, c0, half, M, N, C, ldc,
+                                                             beta, sign, shift);
+            return;
+        }
+    }
+    if (aligned && r0 + kRows <= M && c0 + kCols <= N)
+        tile_k_loop<T, true, UPPER, TR, TC>(A, B, K, r0, c0, lds, M, N, C, ldc, beta, sign, shift);
     else
-        tile_k_loop<T, false, UPPER>(A, B, K, r0, c0, lds, M, N, C, ldc, beta, sign, shift);
+        tile_k_loop<T, false, UPPER, TR, TC>(A, B, K, r0, c0, lds, M, N, C, ldc, beta, sign, shift);
+}
+
+// The 128 x 128 tiles of doubles that the device holds at a time: two
+// workgroups (74 KB of LDS, 202 registers) on each of its 256 CUs.  The
+// 1128 tiles of a 6007 x 6007 upper triangle end in a round of 104, which
+// took as long as a full one on a part of the CUs: 4.75 ms, and 4.45 with
+// these 104 in quarters (3.25 at the matrix units' rate at the 2.1 GHz that
+// they hold; they are busy for 89% of the cycles of a busy CU).
+constexpr int64_t kRound = 512;
+
+template <class T, bool UPPER, int TR, int TC>
+int launch_gemm_tiles(const T *A, int64_t lda, const T *B, int64_t ldb, int64_t K, int64_t M,
+                      int64_t N, double *C, int64_t ldc, double beta, double sign, double shift,
+                      hipStream_t s, int batch, int64_t bsa, int64_t bsb, int64_t bsc,
+                      const int64_t *dims) {
+    const int64_t tm = (M + 32 * TR - 1) / (32 * TR), tn = (N + 32 * TC - 1) / (32 * TC);
+    const int64_t tiles = UPPER ? tn * (tn + 1) / 2 : tm * tn;
+    int64_t whole = tiles;
+    if (kQuarters<T, TR, TC> && batch == 1) whole = tiles / kRound * kRound;
+    const Panel<T> pa = make_panel(A, lda, K, M), pb = make_panel(B, ldb, K, N);
+    hipLaunchKernelGGL((gemm_tn_kernel<T, UPPER, TR, TC>),
+                       dim3((unsigned)(whole + 4 * (tiles - whole)), 1, (unsigned)batch),
+                       dim3(256), 0, s, pa, pb, K, M, N, C, ldc, beta, sign, shift, tn, whole, bsa,
+                       bsb, bsc, dims);
+    HMX_LAUNCHED("gemm_tn_kernel");
+    return HMX_OK;
 }
 
 // batch > 1: a strided batch of equal-shaped problems (element strides
 // bsa, bsb, bsc between consecutive A, B, C; multiples of 2 keep the
 // 16-byte loads aligned).
+// Tiles: 128 x 128 where they fill the device (kRound), because a wavefront
+// then reads 8 operands for 16 FP64 MFMAs; what is left after the last full
+// round goes in quarters.  Fewer tiles than a round leave CUs idle, and the
+// time is that of one tile: 64 x 64 tiles then, or 128 x 32 for M <= kST
+// (all rows in one workgroup, see gemm_tn_kernel on aliasing).  Measured
+// inside a factorisation of 6007 rows: row panel (128 x 5879, K = 128) 30 us
+// as 46 tiles, 14 us as 184; update of 896 x 5879 rows (K = 128) 61 and 43
+// us, of 128 x 4000 37 and 16 us; trailing update of 887 rows (K = 1024) 204
+// and 110 us.
 template <class T>
 int launch_gemm(const T *A, int64_t lda, const T *B, int64_t ldb, int64_t K, int64_t M,
                 int64_t N, double *C, int64_t ldc, double beta, double sign, double shift,
@@ -490,19 +541,24 @@ int launch_gemm(const T *A, int64_t lda, const T *B, int64_t ldb, int64_t K, int
                 int64_t bsc = 0, const int64_t *dims = nullptr) {
     if (M <= 0 || N <= 0 || batch <= 0) return HMX_OK;
     const int64_t tm = (M + kST - 1) / kST, tn = (N + kST - 1) / kST;
-    const Panel<T> pa = make_panel(A, lda, K, M), pb = make_panel(B, ldb, K, N);
-    if (upper) {
-        hipLaunchKernelGGL((gemm_tn_kernel<T, true>),
-                           dim3((unsigned)(tn * (tn + 1) / 2), 1, (unsigned)batch), dim3(256), 0,
-                           s, pa, pb, K, M, N, C, ldc, beta, sign, shift, tn, bsa, bsb, bsc, dims);
-        HMX_LAUNCHED("gemm_tn_kernel<upper>");
-    } else {
-        hipLaunchKernelGGL((gemm_tn_kernel<T, false>), dim3((unsigned)(tm * tn), 1, (unsigned)batch),
-                           dim3(256), 0, s, pa, pb, K, M, N, C, ldc, beta, sign, shift, tn, bsa,
-                           bsb, bsc, dims);
-        HMX_LAUNCHED("gemm_tn_kernel");
+    const int64_t tiles = (upper ? tn * (tn + 1) / 2 : tm * tn) * batch;
+    if constexpr (std::is_same<T, double>::value) {
+        if (tiles < kRound) {
+            if (upper)
+                return launch_gemm_tiles<T, true, 2, 2>(A, lda, B, ldb, K, M, N, C, ldc, beta, sign,
+                                                        shift, s, batch, bsa, bsb, bsc, dims);
+            if (M > kST)
+                return launch_gemm_tiles<T, false, 2, 2>(A, lda, B, ldb, K, M, N, C, ldc, beta,
+                                                         sign, shift, s, batch, bsa, bsb, bsc, dims);
+            return launch_gemm_tiles<T, false, 4, 1>(A, lda, B, ldb, K, M, N, C, ldc, beta, sign,
+                                                     shift, s, batch, bsa, bsb, bsc, dims);
+        }
     }
-    return HMX_OK;
+    if (upper)
+        return launch_gemm_tiles<T, true, 4, 4>(A, lda, B, ldb, K, M, N, C, ldc, beta, sign, shift,
+                                                s, batch, bsa, bsb, bsc, dims);
+    return launch_gemm_tiles<T, false, 4, 4>(A, lda, B, ldb, K, M, N, C, ldc, beta, sign, shift, s,
+                                             batch, bsa, bsb, bsc, dims);
 }
 
 // dims (device, 2 per problem, or NULL): the rows and the size each problem
@@ -1180,9 +1236,9 @@ __global__ __launch_bounds__(256) void colsumsq_kernel(const T *__restrict__ X, 
 }
 
 // A[j][j] += tau for j < m (row-major, leading dimension m).
-__global__ void add_diag_kernel(double *__restrict__ A, int64_t m, double tau) {
+__global__ void add_diag_kernel(double *__restrict__ A, int64_t ld, int64_t m, double tau) {
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j < m) A[j * m + j] += tau;
+    if (j < m) A[j * ld + j] += tau;
 }
 
 
@@ -1578,14 +1634,22 @@ inline bool svd_route_fits(int64_t n_data, int64_t n_src) {
     return n_src <= kSvdMaxSrc && n_data * n_src <= kSvdMaxElems;
 }
 
+// Row stride of a fit's normal matrix and scaled jacobian (rows start on
+// 128-byte lines, so the panel loads are 16 bytes wide whatever the number
+// of sources) and the jacobian's rows with their zero padding (whole kKC
+// chunks).  With the odd stride of 6007 sources every tile took the checked
+// 8-byte loads: 5.36 ms for their 6007 x 6007 product, 4.95 with this stride.
+inline int64_t fit_ld(int64_t n_src) { return (n_src + 15) / 16 * 16; }
+inline int64_t fit_rows(int64_t n_data) { return (n_data + kKC - 1) / kKC * kKC; }
+
 // Bytes of the scaled-jacobian region of the fit's workspace: the mode's
 // jacobian (FP64, FP32, or slices with their group scales), enlarged where
 // needed so that, with the copy of the normal matrix in front of it (mixed
 // modes), it holds the FP64 column-major jacobian of the SVD route.
 inline size_t fit_x_bytes(int64_t n_data, int64_t n_src, int mode) {
-    const size_t m = (size_t)n_src, n = (size_t)n_data;
-    size_t x_bytes = n * m * sizeof(double);  // X = W^1/2 J S
-    if (mode == HMX_FIT_FP32_MFMA) x_bytes = n * m * sizeof(float);
+    const size_t m = (size_t)n_src, n = (size_t)n_data, ld = (size_t)fit_ld(n_src);
+    size_t x_bytes = (size_t)fit_rows(n_data) * ld * sizeof(double);  // X = W^1/2 J S
+    if (mode == HMX_FIT_FP32_MFMA) x_bytes /= 2;
     if (mode == HMX_FIT_BF16_SPLIT || mode == HMX_FIT_INT8_SPLIT) {
         // slices (16-byte units of 8 or 16 rows, padded to whole chunks of
         // kSplitChunkUnits units) and the group scales
@@ -1596,7 +1660,7 @@ inline size_t fit_x_bytes(int64_t n_data, int64_t n_src, int mode) {
                   (n_units * rows + kFoldRows - 1) / kFoldRows * m * sizeof(double);
     }
     if (svd_route_fits(n_data, n_src)) {
-        const size_t avail = (mode == HMX_FIT_FP64 ? 0 : m * m * sizeof(double)) + x_bytes;
+        const size_t avail = (mode == HMX_FIT_FP64 ? 0 : m * ld * sizeof(double)) + x_bytes;
         const size_t g_bytes = n * m * sizeof(double);
         if (avail < g_bytes) x_bytes += g_bytes - avail;
     }
@@ -1730,6 +1794,9 @@ struct Fit {
     // Dimension of the factor (m unless padded; see the batched fits).
     int64_t mf = 0;
     int64_t fm() const { return mf ? mf : m; }
+    // Row stride of A (its dimension unless set).
+    int64_t lda = 0;
+    int64_t ld() const { return lda ? lda : fm(); }
 
     // The second stream of the factorisation's lookahead and its two
     // events; the stream is drained before it is destroyed.
@@ -1766,7 +1833,7 @@ struct Fit {
     // update of outer block P + kOuter, which waits for it.
     int cholesky(int *pivot, int batch = 1, int64_t bs_a = 0, int64_t bs_inv = 0,
                  int *infos = nullptr) {
-        const int64_t n = fm();
+        const int64_t n = fm(), ld = this->ld();
         int *dev_info = batch > 1 ? infos : dinfo;
         hipLaunchKernelGGL(fill_int_kernel, dim3(blocks_for(batch)), dim3(256), 0, s, dev_info,
                            (int64_t)batch, 0);
@@ -1792,25 +1859,25 @@ struct Fit {
             const int64_t Pend = P + kOuter < n ? P + kOuter : n;
             for (int64_t p = P; p < Pend; p += kNB) {
                 const int nb = (int)(n - p < kNB ? n - p : kNB);
-                double *D = A + p * n + p;
+                double *D = A + p * ld + p;
                 const int64_t blk = p / kNB;
-                hipLaunchKernelGGL(potrf_diag_kernel, dim3((unsigned)batch), dim3(1024), 0, s, D, n,
+                hipLaunchKernelGGL(potrf_diag_kernel, dim3((unsigned)batch), dim3(1024), 0, s, D, ld,
                                    nb, p, Dinv + blk * kNB * kNB, DinvT + blk * kNB * kNB,
                                    dev_info, bs_a, bs_inv, batch > 1 ? 1 : 0);
                 HMX_LAUNCHED("potrf_diag_kernel");
                 const int64_t rest = n - p - nb;
                 if (rest <= 0) break;
                 // U12 = U11^-T A12 = (U11^-1)^T A12, in place, up to column n.
-                int st = launch_gemm_tn(Dinv + blk * kNB * kNB, kNB, D + nb, n, nb, nb, rest,
-                                        D + nb, n, 0.0, 1.0, s, batch, bs_inv, bs_a, bs_a);
+                int st = launch_gemm_tn(Dinv + blk * kNB * kNB, kNB, D + nb, ld, nb, nb, rest,
+                                        D + nb, ld, 0.0, 1.0, s, batch, bs_inv, bs_a, bs_a);
                 if (st) return st;
                 // Rows [p + nb, Pend) of the outer block, columns [p + nb, n)
                 // (the few entries below the diagonal that this rectangle
                 // covers are never read).
                 const int64_t rows_in = Pend - p - nb;
                 if (rows_in > 0) {
-                    st = launch_gemm<double>(D + nb, n, D + nb, n, nb, rows_in, rest,
-                                             D + nb * n + nb, n, 1.0, -1.0, 0.0, false, s, batch,
+                    st = launch_gemm<double>(D + nb, ld, D + nb, ld, nb, rows_in, rest,
+                                             D + nb * ld + nb, ld, 1.0, -1.0, 0.0, false, s, batch,
                                              bs_a, bs_a, bs_a);
                     if (st) return st;
                 }
@@ -1822,13 +1889,13 @@ struct Fit {
             }
             if (Pend < n) {
                 const int64_t K = Pend - P, rest = n - Pend;
-                const double *panel = A + P * n + Pend;  // rows [P, Pend), columns [Pend, n)
-                double *T = A + Pend * n + Pend;
+                const double *panel = A + P * ld + Pend;  // rows [P, Pend), columns [Pend, n)
+                double *T = A + Pend * ld + Pend;
                 int st = HMX_OK;
                 if (!ahead || rest <= kOuter) {
                     st = join();
                     if (st) return st;
-                    st = launch_syrk<double>(panel, n, K, rest, T, n, 1.0, -1.0, 0.0, s, batch,
+                    st = launch_syrk<double>(panel, ld, K, rest, T, ld, 1.0, -1.0, 0.0, s, batch,
                                              bs_a, bs_a);
                     if (st) return st;
                 } else {
@@ -1839,14 +1906,14 @@ struct Fit {
                     st = join();  // the previous side update wrote the next outer block's rows
                     if (st) return st;
                     const int64_t top = kOuter, far = rest - kOuter;
-                    st = launch_syrk<double>(panel + top, n, K, far, T + top * n + top, n, 1.0,
+                    st = launch_syrk<double>(panel + top, ld, K, far, T + top * ld + top, ld, 1.0,
                                              -1.0, 0.0, side.s2);
                     if (st) return st;
                     HMX_HIP(hipEventRecord(side.rest, side.s2));
                     rest_pending = true;
                     // the next outer block's rows, all columns from Pend (the
                     // entries below the diagonal it covers are never read)
-                    st = launch_gemm<double>(panel, n, panel, n, K, top, rest, T, n, 1.0, -1.0,
+                    st = launch_gemm<double>(panel, ld, panel, ld, K, top, rest, T, ld, 1.0, -1.0,
                                              0.0, false, s);
                     if (st) return st;
                 }
@@ -1876,19 +1943,19 @@ struct Fit {
         hipLaunchKernelGGL(fill_sentinel_kernel, dim3(blocks_for(n)), dim3(256), 0, s, y, n);
         HMX_LAUNCHED("fill_sentinel_kernel");
         if (Ub)
-            hipLaunchKernelGGL(trsv_fwd_sync_kernel<true>, dim3(nb), dim3(1024), 0, s, A, Ub, n, n,
-                               Dinv, r, y, terr);
+            hipLaunchKernelGGL(trsv_fwd_sync_kernel<true>, dim3(nb), dim3(1024), 0, s, A, Ub, ld(),
+                               n, Dinv, r, y, terr);
         else
-            hipLaunchKernelGGL(trsv_fwd_sync_kernel<false>, dim3(nb), dim3(1024), 0, s, A, Ub, n,
+            hipLaunchKernelGGL(trsv_fwd_sync_kernel<false>, dim3(nb), dim3(1024), 0, s, A, Ub, ld(),
                                n, Dinv, r, y, terr);
         HMX_LAUNCHED("trsv_fwd_sync_kernel");
         hipLaunchKernelGGL(fill_sentinel_kernel, dim3(blocks_for(n)), dim3(256), 0, s, x, n);
         HMX_LAUNCHED("fill_sentinel_kernel");
         if (Ub)
-            hipLaunchKernelGGL(trsv_bwd_sync_kernel<true>, dim3(nb), dim3(1024), 0, s, A, Ub, n, n,
-                               DinvT, y, x, terr);
+            hipLaunchKernelGGL(trsv_bwd_sync_kernel<true>, dim3(nb), dim3(1024), 0, s, A, Ub, ld(),
+                               n, DinvT, y, x, terr);
         else
-            hipLaunchKernelGGL(trsv_bwd_sync_kernel<false>, dim3(nb), dim3(1024), 0, s, A, Ub, n,
+            hipLaunchKernelGGL(trsv_bwd_sync_kernel<false>, dim3(nb), dim3(1024), 0, s, A, Ub, ld(),
                                n, DinvT, y, x, terr);
         HMX_LAUNCHED("trsv_bwd_sync_kernel");
         return HMX_OK;
@@ -1908,7 +1975,7 @@ struct Fit {
         const int64_t n = fm();
         const int nb = (int)((n + kNB - 1) / kNB);
         if (nb > 1) {
-            hipLaunchKernelGGL(pack_upper_f32_kernel, dim3(nb, nb), dim3(256), 0, s, A, n, n, nb,
+            hipLaunchKernelGGL(pack_upper_f32_kernel, dim3(nb, nb), dim3(256), 0, s, A, ld(), n, nb,
                                dst);
             HMX_LAUNCHED("pack_upper_f32_kernel");
         }
@@ -2286,10 +2353,10 @@ int hmx_eqs_fit_workspace_bytes(int64_t n_data, int64_t n_src, int precision_mod
     if (mode != HMX_FIT_FP64 && mode != HMX_FIT_FP32_MFMA && mode != HMX_FIT_BF16_SPLIT &&
         mode != HMX_FIT_INT8_SPLIT)
         return fail(HMX_ERR_ARG, "invalid precision mode %d", precision_mode);
-    const size_t m = (size_t)n_src, n = (size_t)n_data;
+    const size_t m = (size_t)n_src, n = (size_t)n_data, ld = (size_t)fit_ld(n_src);
     const size_t nblk = (m + kNB - 1) / kNB;
     const size_t copies = mode == HMX_FIT_FP64 ? 1 : 2;
-    *bytes = copies * m * m * sizeof(double)             // A, then its factor U (+ a copy of A)
+    *bytes = copies * m * ld * sizeof(double)            // A, then its factor U (+ a copy of A)
              + fit_x_bytes(n_data, n_src, mode)        // the scaled jacobian (or its slices)
              + 2 * nblk * kNB * kNB * sizeof(double)  // inverses of diagonal blocks
              + (10 * m + n + 256) * sizeof(double)  // 10 m-vectors, n-vector, partials
@@ -2350,12 +2417,14 @@ int hmx_eqs_fit(const double *easting, const double *northing, const double *upw
     f.m = m;
     f.alpha = damping;
     f.s = s;
+    const int64_t ld = fit_ld(m), rows = fit_rows(nd);
     f.A = reinterpret_cast<double *>(ws);
-    ws += (size_t)m * m * sizeof(double);
+    f.lda = ld;
+    ws += (size_t)m * ld * sizeof(double);
     double *A_copy = nullptr;  // mixed mode: the unshifted normal matrix, for retries
     if (mixed) {
         A_copy = reinterpret_cast<double *>(ws);
-        ws += (size_t)m * m * sizeof(double);
+        ws += (size_t)m * ld * sizeof(double);
     }
     void *X = ws;
     double *fgroup = nullptr;  // split: (n_fold, m) power-of-2 column scales per row group
@@ -2406,13 +2475,23 @@ int hmx_eqs_fit(const double *easting, const double *northing, const double *upw
     } else if (mixed) {
         hipLaunchKernelGGL(scaled_jacobian_kernel<float>, dim3(gm, gy), dim3(256), 0, s, easting,
                            northing, upward, weights, nd, p_easting, p_northing, p_upward, f.scale,
-                           m, static_cast<float *>(X), m);
+                           m, static_cast<float *>(X), ld);
     } else {
         hipLaunchKernelGGL(scaled_jacobian_kernel<double>, dim3(gm, gy), dim3(256), 0, s, easting,
                            northing, upward, weights, nd, p_easting, p_northing, p_upward, f.scale,
-                           m, static_cast<double *>(X), m);
+                           m, static_cast<double *>(X), ld);
     }
-    if (!split) HMX_LAUNCHED("scaled_jacobian_kernel");
+    if (!split) {
+        HMX_LAUNCHED("scaled_jacobian_kernel");
+        const int64_t pad = (rows - nd) * ld / (mixed ? 2 : 1);  // in doubles (ld is even)
+        if (pad > 0) {
+            double *end = mixed ? reinterpret_cast<double *>(static_cast<float *>(X) + nd * ld)
+                                : static_cast<double *>(X) + nd * ld;
+            hipLaunchKernelGGL(fill_zero_f64_kernel, dim3(blocks_for(pad)), dim3(256), 0, s, end,
+                               pad);
+            HMX_LAUNCHED("fill_zero_f64_kernel");
+        }
+    }
 
     // The FP32-MFMA normal matrix differs from the FP64 one by about 2^-24
     // of its entries (input rounding and FP32 sums within each MFMA), the
@@ -2424,13 +2503,13 @@ int hmx_eqs_fit(const double *easting, const double *northing, const double *upw
     double tau = 0.0, dmax = 0.0;
     auto diag_max = [&](double *out) -> int {
         if (split)  // the diagonal of the saved normal matrix
-            return f.reduce(1, A_copy, nullptr, m, m + 1, out);
+            return f.reduce(1, A_copy, nullptr, m, ld + 1, out);
         if (mixed)
             hipLaunchKernelGGL(colsumsq_kernel<float>, dim3(gm), dim3(256), 0, s,
-                               static_cast<const float *>(X), m, nd, m, wk);
+                               static_cast<const float *>(X), ld, nd, m, wk);
         else
             hipLaunchKernelGGL(colsumsq_kernel<double>, dim3(gm), dim3(256), 0, s,
-                               static_cast<const double *>(X), m, nd, m, wk);
+                               static_cast<const double *>(X), ld, nd, m, wk);
         HMX_LAUNCHED("colsumsq_kernel");
         return f.reduce(1, wk, nullptr, m, 1, out);
     };
@@ -2440,9 +2519,9 @@ int hmx_eqs_fit(const double *easting, const double *northing, const double *upw
     bool use_svd = false;
     for (;;) {
         if (mixed && attempts > 0) {  // restore the normal matrix, add the shift
-            HMX_HIP(hipMemcpyAsync(f.A, A_copy, (size_t)m * m * sizeof(double),
+            HMX_HIP(hipMemcpyAsync(f.A, A_copy, (size_t)m * ld * sizeof(double),
                                    hipMemcpyDeviceToDevice, s));
-            hipLaunchKernelGGL(add_diag_kernel, dim3(gm), dim3(256), 0, s, f.A, m, tau);
+            hipLaunchKernelGGL(add_diag_kernel, dim3(gm), dim3(256), 0, s, f.A, ld, m, tau);
             HMX_LAUNCHED("add_diag_kernel");
         } else if (mixed) {
             if (split) {
@@ -2451,33 +2530,33 @@ int hmx_eqs_fit(const double *easting, const double *northing, const double *upw
                 if (int8) {
                     const int32x4_t *Sl = static_cast<const int32x4_t *>(X);
                     hipLaunchKernelGGL((gram_split_kernel<SplitInt8, 0, 1>), dim3(blocks),
-                                       dim3(512), 0, s, Sl, n_groups, m, fgroup, f.A, m, 0.0,
+                                       dim3(512), 0, s, Sl, n_groups, m, fgroup, f.A, ld, 0.0,
                                        damping, tiles);
                     HMX_LAUNCHED("gram_split_kernel<SplitInt8,0,1>");
                     hipLaunchKernelGGL((gram_split_kernel<SplitInt8, 2, 3>), dim3(blocks),
-                                       dim3(512), 0, s, Sl, n_groups, m, fgroup, f.A, m, 1.0, 0.0,
+                                       dim3(512), 0, s, Sl, n_groups, m, fgroup, f.A, ld, 1.0, 0.0,
                                        tiles);
                     HMX_LAUNCHED("gram_split_kernel<SplitInt8,2,3>");
                 } else {
                     const bf16x8_t *Sl = static_cast<const bf16x8_t *>(X);
                     hipLaunchKernelGGL((gram_split_kernel<SplitBf16, 0, 1>), dim3(blocks),
-                                       dim3(512), 0, s, Sl, n_groups, m, fgroup, f.A, m, 0.0,
+                                       dim3(512), 0, s, Sl, n_groups, m, fgroup, f.A, ld, 0.0,
                                        damping, tiles);
                     HMX_LAUNCHED("gram_split_kernel<SplitBf16,0,1>");
                     hipLaunchKernelGGL((gram_split_kernel<SplitBf16, 2, 3>), dim3(blocks),
-                                       dim3(512), 0, s, Sl, n_groups, m, fgroup, f.A, m, 1.0, 0.0,
+                                       dim3(512), 0, s, Sl, n_groups, m, fgroup, f.A, ld, 1.0, 0.0,
                                        tiles);
                     HMX_LAUNCHED("gram_split_kernel<SplitBf16,2,3>");
                 }
             } else {
-                st = launch_syrk<float>(static_cast<const float *>(X), m, nd, m, f.A, m, 0.0, 1.0,
+                st = launch_syrk<float>(static_cast<const float *>(X), ld, rows, m, f.A, ld, 0.0, 1.0,
                                         damping, s);
                 if (st) return st;
             }
-            HMX_HIP(hipMemcpyAsync(A_copy, f.A, (size_t)m * m * sizeof(double),
+            HMX_HIP(hipMemcpyAsync(A_copy, f.A, (size_t)m * ld * sizeof(double),
                                    hipMemcpyDeviceToDevice, s));
         } else {
-            st = launch_syrk<double>(static_cast<const double *>(X), m, nd, m, f.A, m, 0.0, 1.0,
+            st = launch_syrk<double>(static_cast<const double *>(X), ld, rows, m, f.A, ld, 0.0, 1.0,
                                      damping + tau, s);
             if (st) return st;
         }
@@ -2511,9 +2590,9 @@ int hmx_eqs_fit(const double *easting, const double *northing, const double *upw
     // singular values below lstsq's cut-off: SVD route.
     if (lstsq && svd_ok && !use_svd) {
         double umin = 0.0, umax = 0.0;
-        st = f.reduce(2, f.A, nullptr, m, m + 1, &umin);
+        st = f.reduce(2, f.A, nullptr, m, ld + 1, &umin);
         if (st) return st;
-        st = f.reduce(1, f.A, nullptr, m, m + 1, &umax);
+        st = f.reduce(1, f.A, nullptr, m, ld + 1, &umax);
         if (st) return st;
         if (!(umin * umin >= kLstsqPivotRatio * umax * umax)) use_svd = true;
     }
@@ -2529,7 +2608,7 @@ int hmx_eqs_fit(const double *easting, const double *northing, const double *upw
         // preconditioner only, and the substitutions read an FP32 blocked
         // copy of it, held where the saved normal matrix was (2 m^2 bytes
         // at most, against its 8 m^2).
-        if (mixed && allowed > 0 && f.upper_f32_bytes() <= (int64_t)(m * m * sizeof(double))) {
+        if (mixed && allowed > 0 && f.upper_f32_bytes() <= (int64_t)(m * ld * sizeof(double))) {
             st = f.use_upper_f32(reinterpret_cast<float *>(A_copy));
             if (st) return st;
         }
@@ -2555,7 +2634,7 @@ int hmx_eqs_fit(const double *easting, const double *northing, const double *upw
                                s, easting, northing, upward, weights, nd, p_easting, p_northing,
                                p_upward, f.scale, m, G);
             HMX_LAUNCHED("scaled_jacobian_cm_kernel");
-        } else if (mixed) {
+        } else if (mixed || ld != m) {
             hipLaunchKernelGGL(scaled_jacobian_kernel<double>, dim3(gm, gy), dim3(256), 0, s,
                                easting, northing, upward, weights, nd, p_easting, p_northing,
                                p_upward, f.scale, m, G, m);

@@ -402,3 +402,30 @@ def test_fit_more_sources_than_data(hm, damping):
         assert np.abs(pred - data).max() <= 1.5 * np.abs(ref - data).max() + 1e-9 * np.abs(data).max()
     else:
         npt.assert_allclose(pred, ref, rtol=0, atol=1e-7 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("n,m", [(49, 49), (64, 33), (49, 36), (36, 49), (33, 64)])
+@pytest.mark.parametrize("damping", [None, 1e-2])
+def test_fit_ragged_sizes(hm, n, m, damping):
+    """Numbers of data and sources off the 16 that the stored jacobian is
+    padded to, with more and with fewer data than sources.  Sources lie half
+    their spacing below the data, so the scaled jacobian's condition number
+    is below 1e3 (seen in the oracle's singular values) and the predictions
+    agree to 1e-10 of the data, 1e3^2 roundings."""
+    from harmonica_amd._eqs import fit_device
+
+    def grid(k, depth):
+        side = int(np.ceil(np.sqrt(k)))
+        e, nn = np.meshgrid(np.arange(side) * 100.0, np.arange(side) * 100.0)
+        return e.ravel()[:k] + depth, nn.ravel()[:k], np.full(k, -depth)
+
+    coords, pts = grid(n, 0.0), grid(m, 50.0)
+    rng = np.random.default_rng(n + m)
+    data = rng.normal(size=n)
+    J = oracle.eqs_jacobian(coords, pts)
+    scaled = J / J.std(axis=0)
+    sv = np.linalg.svd(scaled, compute_uv=False)
+    assert sv[0] < 1e3 * sv[min(n, m) - 1]
+    expected = oracle.eqs_fit_coefs_info(J, data, None, damping)[0]
+    coefs, _ = fit_device(coords, data, None, pts, damping)
+    npt.assert_allclose(J @ coefs, J @ expected, rtol=0, atol=1e-10 * np.abs(data).max())

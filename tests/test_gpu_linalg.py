@@ -322,3 +322,47 @@ def test_diagonal_block_bad_pivot(env, m, bad, pivot):
     A = np.eye(m)
     A[bad, bad] = pivot
     assert _factor(env, A, np.ones(m))[2] == bad + 1
+
+
+@pytest.mark.parametrize("shape,upper", [
+    ((16, 128, 64), False),     # 128 x 32 tiles, whole
+    ((33, 128, 33), False),     # and with a remainder in every direction
+    ((35, 127, 97), False),
+    ((48, 129, 191), False),    # 64 x 64 tiles
+    ((17, 192, 65), False),
+    ((32, 2944, 2944), False),  # 529 tiles of 128: one round, 17 in quarters
+    ((17, 2821, 2883), False),  # ragged, quarters past both edges
+    ((16, 128, 128), True),
+    ((19, 200, 200), True),
+    ((32, 4096, 4096), True),   # 528 tiles: 16 in quarters, some below the diagonal
+    ((18, 4035, 4035), True),
+])
+def test_gemm_tile_choice(env, shape, upper):
+    """Each tile shape at its edges; K + 3 roundings of |A|^T |B| + |C|."""
+    K, M, N = shape
+    rng = np.random.default_rng(K + M + N)
+    A = rng.normal(size=(K, M))
+    B = A if upper else rng.normal(size=(K, N))
+    C = rng.normal(size=(M, N))
+    got = _gemm(env, 0, A, B, C, 1.0, -1.0, 0.25, upper)
+    bound = (K + 3) * 2.0**-52 * (np.abs(A).T @ np.abs(B) + np.abs(C) + 0.25)
+    expected = C - A.T @ B
+    expected[np.arange(min(M, N)), np.arange(min(M, N))] += 0.25
+    if upper:
+        low = np.tril_indices(M, -1)
+        assert np.array_equal(got[low], C[low])
+        got, expected, bound = np.triu(got), np.triu(expected), np.triu(bound)
+    assert np.all(np.abs(got - expected) <= bound)
+
+
+@pytest.mark.parametrize("M,N", [(128, 100), (100, 300), (17, 33)])
+def test_gemm_in_place_on_b(env, M, N):
+    """C may be B where M <= 128 (here K = M)."""
+    torch, _lib, L = env
+    rng = np.random.default_rng(M + N)
+    A, B = rng.normal(size=(M, M)), rng.normal(size=(M, N))
+    dA, dB = torch.tensor(A).cuda(), torch.tensor(B).cuda()
+    _lib.check(L.hmx_gemm_tn(0, _lib.ptr(dA), M, _lib.ptr(dB), N, M, M, N, _lib.ptr(dB), N, 0.0,
+                             1.0, 0.0, 0, None))
+    bound = (M + 3) * 2.0**-52 * (np.abs(A).T @ np.abs(B))
+    assert np.all(np.abs(dB.cpu().numpy() - A.T @ B) <= bound)
