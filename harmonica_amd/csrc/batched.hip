@@ -197,8 +197,7 @@ int hmx_batched_prism_gz(const double *easting, const double *northing, const do
     hipLaunchKernelGGL(zero_counter_kernel, dim3(1), dim3(64), 0, s, counter);
     HMX_LAUNCHED("zero_counter_kernel");
     if (n_items > 0) {
-        // blocks_per_cu counts workgroups of four waves; these have two
-        const int64_t grid64 = std::min<int64_t>((int64_t)cu * blocks_per_cu * 2, n_items * kItemParts);
+        const int64_t grid64 = std::min<int64_t>((int64_t)cu * blocks_per_cu, n_items * kItemParts);
         hipLaunchKernelGGL(batched_gz_kernel, dim3((unsigned)grid64), dim3(dev::kGzThreads), 0, s,
                            easting, northing, upward, obs_offsets, prisms, density, items, n_items,
                            partial, counter);

@@ -30,16 +30,17 @@
 namespace hmx {
 namespace dev {
 
-// Largest I staged and the number of constants c_ijk up to order 2I.
-constexpr int kFarMax = 5;
+// Largest I, and up to which I the constants c_ijk are staged as such.
+constexpr int kFarMax = 6;
+constexpr int kFarPlain = 3;
 constexpr int far_base(int i) {  // index of c_i00
     int n = 0;
     for (int t = 1; t < i; ++t) n += (t + 1) * (t + 2) / 2;
     return n;
 }
 constexpr int far_index(int i, int j, int k) { return far_base(i) + j * (j + 1) / 2 + k; }
-constexpr int kFarConsts = far_base(kFarMax + 1);
-static_assert(kFarConsts == 55, "c_ijk up to i = 5");
+constexpr int kFarConsts = far_base(kFarPlain + 1);
+static_assert(kFarConsts == 19, "c_ijk up to i = 3");
 
 constexpr double far_binom(int n, int k) {
     double b = 1.0;
@@ -80,10 +81,118 @@ __device__ __forceinline__ void far_order_consts(double A, double B, double *c) 
     }
 }
 
+// The same averages in polar angles, d = |d| (cos th, sin th) and (x, y) =
+// s^(1/2) (cos ph, sin ph): with cos^2j a = sum_q w_jq cos 2qa,
+//   <(x dx + y dy)^(2j) d^(2(i-j))> = s^j sum_(q <= j) w_jq m_iq cos 2q ph,
+//   m_iq = <d^2i cos 2q th>
+// (the sines average to 0 over a rectangle), so the i + 1 moments m_iq of an
+// order take the place of its (i + 1)(i + 2)/2 constants, and what remains of
+// c_ij is a number far_polar(i, j, q).  Orders above 2 kFarPlain are formed
+// so: 27 numbers per prism in LDS up to order 12, where the c_ijk are 83 (35
+// KB of LDS, and registers that do not hold an order's 28), for about 40 more
+// operations a pair at order 10.  48 models of up to 200,000 prisms of
+// different rectangles: 119.5 ms with c_ijk up to order 10, 121.4 with the
+// moments up to order 10, 111.4 with the moments up to order 12, 112.5 with
+// c_ijk up to order 8 or 10 and the moments beyond (the arithmetic is then
+// less, the LDS traffic more); with the c_ijk of order 12 it spills (214 ms).
+constexpr int far_moment(int i, int q) { return (i - 1) * (i + 2) / 2 + q; }
+constexpr int kFarMoments = far_moment(kFarMax + 1, 0);
+static_assert(far_moment(1, 0) == 0 && far_moment(2, 0) == 2 && kFarMoments == 27, "m_iq");
+
+constexpr double far_polar(int i, int j, int q) {
+    const int m = i + j;
+    double f = far_binom(2 * m, m) * far_binom(m, 2 * j) * far_binom(2 * j, j - q);
+    for (int t = 0; t < m; ++t) f *= 0.25;
+    return (q ? 2.0 : 1.0) * (m % 2 ? -f : f);
+}
+
+// Coefficient of dx^2p dy^(2(i-p)) in d^2i cos 2q th.
+constexpr double far_angular(int i, int q, int p) {
+    double f = 0.0;
+    for (int k = 0; k <= q; ++k)
+        if (p >= k && p - k <= i - q) {
+            const double b = far_binom(2 * q, 2 * k) * far_binom(i - q, p - k);
+            f += (q - k) % 2 ? -b : b;
+        }
+    return f;
+}
+
+// The moments of order 2I of a rectangle (A, B as in far_order_consts).
+template <int I>
+__device__ __forceinline__ void far_order_moments(double A, double B, double *m) {
+    double pa[I + 1], pb[I + 1], mu[I + 1];
+    pa[0] = pb[0] = 1.0;
+#pragma unroll
+    for (int q = 1; q <= I; ++q) {
+        pa[q] = pa[q - 1] * A;
+        pb[q] = pb[q - 1] * B;
+    }
+#pragma unroll
+    for (int p = 0; p <= I; ++p)
+        mu[p] = pa[p] * pb[I - p] * (1.0 / ((2 * p + 1) * (2 * (I - p) + 1)));
+#pragma unroll
+    for (int q = 0; q <= I; ++q) {
+        double v = 0.0;
+#pragma unroll
+        for (int p = 0; p <= I; ++p) v = fma(far_angular(I, q, p), mu[p], v);
+        m[far_moment(I, q)] = v;
+    }
+}
+
+// far_polar(i, j, q) in scalar registers, set where it is used (83 of them
+// hoisted out of the loop over prisms would not fit the registers).
+template <int i, int j, int q>
+__device__ __forceinline__ double polar_const() {
+    constexpr unsigned long long bits = __builtin_bit_cast(unsigned long long, far_polar(i, j, q));
+    constexpr int low = (int)(bits & 0xffffffffull);
+    int hi, lo = 0;
+    asm volatile("s_mov_b32 %0, %1" : "=s"(hi) : "i"((int)(bits >> 32)));
+    if constexpr (low != 0) asm volatile("s_mov_b32 %0, %1" : "=s"(lo) : "i"(low));
+    return __hiloint2double(hi, lo);
+}
+
+// Adds the terms (i, j .. i, q) to C_(i+j), with h = m_iq s^j cos 2q ph.
+template <int I, int i, int q, int j>
+__device__ __forceinline__ void polar_terms(double s, double h, double (&C)[2 * I + 1]) {
+    // the first term to reach C_m: i = ceil(m / 2), q = 0
+    constexpr bool first = q == 0 && i == (i + j + 1) / 2;
+    const double f = polar_const<i, j, q>();
+    C[i + j] = first ? f * h : fma(f, h, C[i + j]);
+    if constexpr (j < i) polar_terms<I, i, q, j + 1>(s, h * s, C);
+}
+
+template <int I, int i, int q, class Consts>
+__device__ __forceinline__ void polar_order(double s, const double (&T)[I + 1], const Consts &c,
+                                            double (&C)[2 * I + 1]) {
+    const double m = c.moment(far_moment(i, q));
+    polar_terms<I, i, q, q>(s, q ? m * T[q] : m, C);
+    if constexpr (q < i)
+        polar_order<I, i, q + 1>(s, T, c, C);
+    else if constexpr (i < I)
+        polar_order<I, i + 1, 0>(s, T, c, C);
+}
+
+// C_1 .. C_2I from the moments.
+template <int I, class Consts>
+__device__ __forceinline__ void far_coefs_polar(double X, double Y, const Consts &c,
+                                                double (&C)[2 * I + 1]) {
+    const double s = X + Y, t1 = X - Y, t2 = 2.0 * t1, s2 = s * s;
+    double T[I + 1];  // s^q cos 2q ph
+    T[0] = 1.0;
+    T[1] = t1;
+#pragma unroll
+    for (int q = 2; q <= I; ++q) T[q] = fma(t2, T[q - 1], q == 2 ? -s2 : -s2 * T[q - 2]);
+    polar_order<I, 1, 0>(s, T, c, C);
+}
+
 // C_1 .. C_2I at X = x^2, Y = y^2; c(index) gives a constant.
 template <int I, class Consts>
 __device__ __forceinline__ void far_coefs(double X, double Y, const Consts &c,
                                           double (&C)[2 * I + 1]) {
+    if constexpr (I > kFarPlain) {
+        far_coefs_polar<I>(X, Y, c, C);
+        return;
+    }
     double mono[I + 1][I + 1];  // X^k Y^(j-k)
     mono[0][0] = 1.0;
 #pragma unroll
@@ -111,7 +220,6 @@ __device__ __forceinline__ void far_coefs(double X, double Y, const Consts &c,
                     C[i + j] = fma(ck, mono[j][k], C[i + j]);
             }
         }
-        if constexpr (I >= 4) __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -147,9 +255,13 @@ __device__ __forceinline__ void far_face_top(double s, double z, const double (&
 
 // Square of the distance, in units of the half-diagonal h of the rectangle,
 // from which order 2I suffices: (1 / ((2I + 3) 4e-15))^(1 / (2I + 2)) =
-// 181, 48, 21.8, 12.9 for I = 2, 3, 4, 5.
+// 181, 48, 21.8, 12.9, 8.8 for I = 2, 3, 4, 5, 6.
 __device__ __forceinline__ constexpr double far_ratio2(int I) {
-    return I == 2 ? 181.0 * 181.0 : I == 3 ? 48.0 * 48.0 : I == 4 ? 21.8 * 21.8 : 12.9 * 12.9;
+    return I == 2   ? 181.0 * 181.0
+           : I == 3 ? 48.0 * 48.0
+           : I == 4 ? 21.8 * 21.8
+           : I == 5 ? 12.9 * 12.9
+                    : 8.8 * 8.8;
 }
 
 // A staged far prism: the rectangle's centre from the workgroup's origin, top,
@@ -162,10 +274,13 @@ struct alignas(16) FarPrism {
 
 // Constants in LDS (kept per prism: stride kFarStride) or, for a tile of
 // equal rectangles, in scalar registers.
-constexpr int kFarStride = kFarConsts + 1;  // even: 16-byte aligned pairs
+// The c_ijk, then the moments, each 16-byte aligned.
+constexpr int kFarMomentsAt = (kFarConsts + 1) / 2 * 2;
+constexpr int kFarStride = (kFarMomentsAt + kFarMoments + 1) / 2 * 2;
 struct FarLds {
     const double *c;
     __device__ __forceinline__ double operator()(int k) const { return c[k]; }
+    __device__ __forceinline__ double moment(int k) const { return c[kFarMomentsAt + k]; }
 };
 __device__ __forceinline__ double wave_uniform(double v) {
     return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
@@ -295,9 +410,13 @@ __device__ __forceinline__ void far_consts(double A, double B, int part, double 
         far_order_consts<2>(A, B, c);
         far_order_consts<3>(A, B, c);
     } else if (part == 1) {
-        far_order_consts<4>(A, B, c);
+        far_order_moments<1>(A, B, c + kFarMomentsAt);
+        far_order_moments<2>(A, B, c + kFarMomentsAt);
+        far_order_moments<3>(A, B, c + kFarMomentsAt);
+        far_order_moments<4>(A, B, c + kFarMomentsAt);
     } else {
-        far_order_consts<5>(A, B, c);
+        far_order_moments<5>(A, B, c + kFarMomentsAt);
+        far_order_moments<6>(A, B, c + kFarMomentsAt);
     }
 }
 
@@ -380,10 +499,10 @@ __device__ __forceinline__ void gz_stage(const Src &src, int64_t t0, int cnt, do
     }
 }
 
-// Whether order 10 serves the lane's own point.
+// Whether order 2 kFarMax serves the lane's own point.
 __device__ __forceinline__ bool lane_is_far(const FarPrism &p, double px, double py, double pu) {
     const double x = p.x - px, y = p.y - py, t = p.t - pu, z = p.b - pu;
-    return far_enough<5>(fma(x, x, fma(y, y, fmin(t * t, z * z))), p.h2);
+    return far_enough<kFarMax>(fma(x, x, fma(y, y, fmin(t * t, z * z))), p.h2);
 }
 
 // Calls f(p) for the set bits p of a wave-uniform mask, in order.
@@ -458,7 +577,7 @@ __device__ __forceinline__ void gz_close(GzShared &sh, unsigned mask, const GzPo
 constexpr int kGzInline = 40;
 
 // Adds the prisms of `near`, which the bounding box does not show to be far
-// from all of the wave's points.  Each lane takes order 10 where its own
+// from all of the wave's points.  Each lane takes order 2 kFarMax where its own
 // distance allows and the closed form elsewhere, so the form of a pair does
 // not depend on the points that share its wave (bar the orders of the far
 // form, which agree to 4e-15) and neither, to rounding, does the result on
@@ -471,7 +590,7 @@ __device__ __forceinline__ void gz_near(GzShared &sh, unsigned near, unsigned di
         const bool close = !lane_is_far(rec, pt.x, pt.y, pt.u);
         if (any_lane(!close)) {
             const double v =
-                far_gz<5>(rec, FarLds{gz_consts(sh.consts, p, different)}, pt.x, pt.y, pt.u);
+                far_gz<kFarMax>(rec, FarLds{gz_consts(sh.consts, p, different)}, pt.x, pt.y, pt.u);
             acc += close ? 0.0 : v;
         }
         const GzPrism sp = sh.tile[p];
@@ -490,13 +609,12 @@ __device__ __forceinline__ void gz_near(GzShared &sh, unsigned near, unsigned di
 }
 
 // One order of the far form, its constants in scalar registers where the
-// tile's rectangles are equal (up to order 6: 19 constants; the 34 of order 8
-// do not fit beside the rest).
+// tile's rectangles are equal (up to order 6: 19 constants).
 template <int I>
 __device__ __forceinline__ void gz_far(const GzShared &sh, unsigned different, unsigned mask,
                                        const GzPoint &pt, double &acc) {
     if (!mask) return;
-    if constexpr (I <= 3) {
+    if constexpr (I <= kFarPlain) {
         if (!different) {
             const FarScalar<I> c(sh.consts + kGzTile * kFarStride);
             for_bits(mask, [&](int p) { acc += far_gz<I>(sh.far[p], c, pt.x, pt.y, pt.u); });
@@ -526,10 +644,12 @@ __device__ __forceinline__ void gz_tile(int cnt, const GzPoint &pt, double &acc,
     };
     const unsigned m2 = take(far_enough<2>(d2, mine.h2)), m3 = take(far_enough<3>(d2, mine.h2));
     const unsigned m4 = take(far_enough<4>(d2, mine.h2)), m5 = take(far_enough<5>(d2, mine.h2));
+    const unsigned m6 = take(far_enough<6>(d2, mine.h2));
     gz_far<2>(sh, different, m2, pt, acc);
     gz_far<3>(sh, different, m3, pt, acc);
     gz_far<4>(sh, different, m4, pt, acc);
     gz_far<5>(sh, different, m5, pt, acc);
+    gz_far<6>(sh, different, m6, pt, acc);
     if (rest) gz_near(sh, rest, different, pt, acc);
 }
 

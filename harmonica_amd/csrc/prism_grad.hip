@@ -202,7 +202,7 @@ __global__ __launch_bounds__(kObsPerBlock, 3) void gz_vjp_kernel(
         __syncthreads();
         if (!any_live) continue;
         uint64_t rest = cnt == 64 ? ~0ull : (1ull << cnt) - 1ull;
-        uint64_t m2 = 0, m3 = 0, m4 = 0, m5 = 0;
+        uint64_t m2 = 0, m3 = 0, m4 = 0, m5 = 0, m6 = 0;
         if (use_far) {
             const double4 o = tile[lane < cnt ? lane : 0];
             const double x = o.x - xo, y = o.y - yo;
@@ -222,6 +222,7 @@ __global__ __launch_bounds__(kObsPerBlock, 3) void gz_vjp_kernel(
             m3 = take(dev::far_enough<3>(d2, h2));
             m4 = take(dev::far_enough<4>(d2, h2));
             m5 = take(dev::far_enough<5>(d2, h2));
+            m6 = take(dev::far_enough<6>(d2, h2));
         }
         auto point = [&](int q) {
             const double4 o = tile[q];
@@ -238,16 +239,17 @@ __global__ __launch_bounds__(kObsPerBlock, 3) void gz_vjp_kernel(
         }
         dev::for_bits(m4, [&](int q) { vjp_far<4>(pr, lds, point(q), ga, gb); });
         dev::for_bits(m5, [&](int q) { vjp_far<5>(pr, lds, point(q), ga, gb); });
+        dev::for_bits(m6, [&](int q) { vjp_far<6>(pr, lds, point(q), ga, gb); });
         dev::for_bits(rest, [&](int q) {
             const double4 o = tile[q];
             bool close = true;
             if (use_far) {
                 const double x = pr.x - (o.x - xo), y = pr.y - (o.y - yo);
                 const double t = pr.b[5] - o.z, z = pr.b[4] - o.z;
-                close = !dev::far_enough<5>(fma(x, x, fma(y, y, fmin(t * t, z * z))), h2);
+                close = !dev::far_enough<dev::kFarMax>(fma(x, x, fma(y, y, fmin(t * t, z * z))), h2);
                 if (dev::any_lane(live && !close)) {
                     double sa = 0.0, sb = 0.0;
-                    vjp_far<5>(pr, lds, point(q), sa, sb);
+                    vjp_far<dev::kFarMax>(pr, lds, point(q), sa, sb);
                     ga += close ? 0.0 : sa;
                     gb += close ? 0.0 : sb;
                 }

@@ -258,3 +258,43 @@ def test_all_fields_all_distances(hm, kind, m):
         value, bound = (sum(p[q] for p in parts) for q in (0, 1))
         got = hm.prism_magnetic(coords, prisms, (me, mn, mu), name) / 100.0  # 1e-7 x 1e9
         assert (np.abs(got - value) <= bound).all(), name
+
+
+@pytest.mark.parametrize("others", [0, 1, 40], ids=["alone", "tile_different", "two_tiles"])
+@pytest.mark.parametrize("sides", [(100.0, 100.0), (100.0, 300.0), (1e-3, 300.0), (300.0, 1e-3)])
+def test_gz_orders_near_their_limit(hm, sides, others):
+    """One prism at 8.82 to 25 half-diagonals from its nearer face (the
+    shortest distances of orders 12, 10 and 8), straight above, below and to
+    the sides; `others` weightless prisms of other rectangles change what the
+    tile stages.  Bound as above, 52 x 2^-53 of the two face terms."""
+    ld = np.longdouble
+    rng = np.random.default_rng(int(sides[0]) + others)
+    a, b = sides
+    top, bottom = -50.0, -250.0
+    prism = np.array([[-a / 2, a / 2, -b / 2, b / 2, bottom, top]])
+    half = np.hypot(a, b) / 2
+    k = 300
+    r = half * np.geomspace(8.82, 25.0, k)
+    phi, mu = rng.uniform(0, 2 * np.pi, k), rng.uniform(0, 1, k)
+    phi[::5], mu[1::7], mu[2::7] = np.arctan2(b, a), 1.0, 0.0
+    s, z = r * np.sqrt(1 - mu * mu), r * mu
+    # above the top half of the time, below the bottom the other
+    up = np.where(np.arange(k) % 2 == 0, top + z, bottom - z)
+    coords = (s * np.cos(phi), s * np.sin(phi), up)
+    order = rng.permutation(k)
+    coords = tuple(c[order] for c in coords)
+    x10, w10 = np.polynomial.legendre.leggauss(10)  # error (1 / 8.8)^20
+    exact = np.zeros(k, dtype=ld)
+    e, n, u = (c.astype(ld) for c in coords)
+    for xa, wa in zip(x10.astype(ld), w10.astype(ld)):
+        for xb, wb in zip(x10.astype(ld), w10.astype(ld)):
+            q = (xa * a / 2 - e) ** 2 + (xb * b / 2 - n) ** 2
+            exact += wa * wb / 4 * (1 / np.sqrt(q + (bottom - u) ** 2)
+                                    - 1 / np.sqrt(q + (top - u) ** 2))
+    rt, rb = (np.sqrt(e * e + n * n + (f - u) ** 2) for f in (top, bottom))
+    scale = 1e5 * G * 300.0 * a * b
+    bound = 52 * ld(2) ** -53 * scale * (1 / rt + 1 / rb)
+    more = _model("different", max(others, 1), rng)[:others]
+    prisms, density = np.vstack([prism, more]), np.r_[300.0, np.zeros(others)]
+    got = hm.prism_gravity(coords, prisms, density, field="g_z")
+    assert (np.abs(got + scale * exact) <= bound).all()
