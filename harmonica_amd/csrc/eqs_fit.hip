@@ -1641,15 +1641,22 @@ inline bool svd_route_fits(int64_t n_data, int64_t n_src) {
 // 8-byte loads: 5.36 ms for their 6007 x 6007 product, 4.95 with this stride.
 inline int64_t fit_ld(int64_t n_src) { return (n_src + 15) / 16 * 16; }
 inline int64_t fit_rows(int64_t n_data) { return (n_data + kKC - 1) / kKC * kKC; }
+// Bytes of that padding: of the jacobian, and of one m x m matrix.
+inline size_t fit_x_padding(int64_t n_data, int64_t n_src) {
+    return (size_t)(fit_rows(n_data) * fit_ld(n_src) - n_data * n_src) * sizeof(double);
+}
+inline size_t fit_a_padding(int64_t n_src) {
+    return (size_t)n_src * (size_t)(fit_ld(n_src) - n_src) * sizeof(double);
+}
 
 // Bytes of the scaled-jacobian region of the fit's workspace: the mode's
 // jacobian (FP64, FP32, or slices with their group scales), enlarged where
 // needed so that, with the copy of the normal matrix in front of it (mixed
 // modes), it holds the FP64 column-major jacobian of the SVD route.
 inline size_t fit_x_bytes(int64_t n_data, int64_t n_src, int mode) {
-    const size_t m = (size_t)n_src, n = (size_t)n_data, ld = (size_t)fit_ld(n_src);
-    size_t x_bytes = (size_t)fit_rows(n_data) * ld * sizeof(double);  // X = W^1/2 J S
-    if (mode == HMX_FIT_FP32_MFMA) x_bytes /= 2;
+    const size_t m = (size_t)n_src, n = (size_t)n_data;
+    size_t x_bytes = n * m * sizeof(double);  // X = W^1/2 J S
+    if (mode == HMX_FIT_FP32_MFMA) x_bytes = n * m * sizeof(float);
     if (mode == HMX_FIT_BF16_SPLIT || mode == HMX_FIT_INT8_SPLIT) {
         // slices (16-byte units of 8 or 16 rows, padded to whole chunks of
         // kSplitChunkUnits units) and the group scales
@@ -1660,7 +1667,7 @@ inline size_t fit_x_bytes(int64_t n_data, int64_t n_src, int mode) {
                   (n_units * rows + kFoldRows - 1) / kFoldRows * m * sizeof(double);
     }
     if (svd_route_fits(n_data, n_src)) {
-        const size_t avail = (mode == HMX_FIT_FP64 ? 0 : m * ld * sizeof(double)) + x_bytes;
+        const size_t avail = (mode == HMX_FIT_FP64 ? 0 : m * m * sizeof(double)) + x_bytes;
         const size_t g_bytes = n * m * sizeof(double);
         if (avail < g_bytes) x_bytes += g_bytes - avail;
     }
@@ -2353,10 +2360,12 @@ int hmx_eqs_fit_workspace_bytes(int64_t n_data, int64_t n_src, int precision_mod
     if (mode != HMX_FIT_FP64 && mode != HMX_FIT_FP32_MFMA && mode != HMX_FIT_BF16_SPLIT &&
         mode != HMX_FIT_INT8_SPLIT)
         return fail(HMX_ERR_ARG, "invalid precision mode %d", precision_mode);
-    const size_t m = (size_t)n_src, n = (size_t)n_data, ld = (size_t)fit_ld(n_src);
+    const size_t m = (size_t)n_src, n = (size_t)n_data;
     const size_t nblk = (m + kNB - 1) / kNB;
     const size_t copies = mode == HMX_FIT_FP64 ? 1 : 2;
-    *bytes = copies * m * ld * sizeof(double)            // A, then its factor U (+ a copy of A)
+    // (the padding is counted alike in every mode: twice a matrix's)
+    *bytes = fit_x_padding(n_data, n_src) + 2 * fit_a_padding(n_src) +
+             copies * m * m * sizeof(double)             // A, then its factor U (+ a copy of A)
              + fit_x_bytes(n_data, n_src, mode)        // the scaled jacobian (or its slices)
              + 2 * nblk * kNB * kNB * sizeof(double)  // inverses of diagonal blocks
              + (10 * m + n + 256) * sizeof(double)  // 10 m-vectors, n-vector, partials
@@ -2429,7 +2438,7 @@ int hmx_eqs_fit(const double *easting, const double *northing, const double *upw
     void *X = ws;
     double *fgroup = nullptr;  // split: (n_fold, m) power-of-2 column scales per row group
     if (split) fgroup = reinterpret_cast<double *>(ws + (size_t)kSlices * n_groups * m * 16);
-    ws += fit_x_bytes(nd, m, precision_mode);
+    ws += fit_x_bytes(nd, m, precision_mode) + fit_x_padding(nd, m);
     f.Dinv = reinterpret_cast<double *>(ws);
     f.DinvT = f.Dinv + nblk * kNB * kNB;
     double *vec = f.DinvT + nblk * kNB * kNB;
