@@ -26,7 +26,7 @@ from sklearn.base import BaseEstimator
 from sklearn.utils.validation import check_is_fitted
 
 from . import _lib
-from ._forward import to_device
+from ._forward import to_device, to_device_together
 from ._layer import DataArrayLite
 from ._lib import check, lib, ptr, stream_handle
 
@@ -160,6 +160,13 @@ def _dev(a, dtype):
     return to_device(np.asarray(a), dtype=dtype)
 
 
+def _devs(arrays, dtype):
+    """_dev of several arrays; host arrays of float64 in one copy."""
+    if dtype == torch.float64 and not any(isinstance(a, torch.Tensor) for a in arrays):
+        return to_device_together(*(np.asarray(a) for a in arrays))
+    return [_dev(a, dtype) for a in arrays]
+
+
 def jacobian_device(coords, points, dtype=torch.float64):
     """(n_data, n_src) jacobian on the GPU (tensor)."""
     c = [_dev(x, dtype) for x in coords]
@@ -176,9 +183,8 @@ def predict_device(coords, points, coefs, dtype=torch.float64):
     """sum_j c_j / |x_i - p_j| on the GPU (tensor of the coordinates' size)."""
     import ctypes
 
-    c = [_dev(x, dtype) for x in coords]
-    p = [_dev(x, dtype) for x in points]
-    cf = _dev(coefs, dtype)
+    dev = _devs((*coords, *points, coefs), dtype)
+    c, p, cf = dev[:len(coords)], dev[len(coords):-1], dev[-1]
     n, m = c[0].numel(), p[0].numel()
     out = torch.empty(n, dtype=dtype, device=c[0].device)
     nbytes = ctypes.c_size_t(0)
@@ -271,10 +277,11 @@ def fit_device(coords, data, weights, points, damping, precision="float64", max_
         xy = coords[:2] if order_xy is None else order_xy
         order = spatial_order(*(np.asarray(v.cpu() if isinstance(v, torch.Tensor) else v)
                                 for v in xy[:2]))
-    c = [_dev(x, torch.float64) for x in coords]
-    p = [_dev(x, torch.float64) for x in points]
-    d = _dev(data, torch.float64)
-    w = None if weights is None else _dev(weights, torch.float64)
+    given = (*coords, *points, data) if weights is None else (*coords, *points, data, weights)
+    dev = _devs(given, torch.float64)
+    c, p = dev[:len(coords)], dev[len(coords):len(coords) + len(points)]
+    d = dev[len(coords) + len(points)]
+    w = None if weights is None else dev[-1]
     if split:
         idx = torch.as_tensor(order).to(c[0].device)
         c = [x[idx].contiguous() for x in c]

@@ -16,7 +16,7 @@ import warnings
 import numpy as np
 
 from . import _lib
-from ._forward import FIELDS, layer_fields_device, progressbar_context, to_device
+from ._forward import FIELDS, layer_fields_device, progressbar_context, to_device_together
 from ._grid_cells import all_cells, one_cell, top_and_bottom
 
 
@@ -239,12 +239,10 @@ class DatasetAccessorPrismLayer:
         with progressbar_context(coords[0].size, progressbar):
             if cast.size == 0:
                 return np.zeros(cast.shape, dtype=np.float64)
-            e, n, u = (to_device(c) for c in coords)
             out = layer_fields_device(
-                e, n, u,
-                to_device(self._obj.easting.values), to_device(self._obj.northing.values),
-                to_device(self._obj.bottom.values), to_device(self._obj.top.values),
-                to_device(density), (field,), thickness_threshold=thickness_threshold,
+                *to_device_together(*coords, self._obj.easting.values, self._obj.northing.values,
+                                    self._obj.bottom.values, self._obj.top.values, density),
+                (field,), thickness_threshold=thickness_threshold,
             )
             result = out[0].cpu().numpy()
         return result.reshape(cast.shape)
@@ -274,10 +272,11 @@ def layer_gravity_fields(layer, coordinates, fields, density_name="density",
     returns a (len(fields), n) float64 torch tensor on the GPU."""
     _lib.require_device()
     cast, coords = np.broadcast(*coordinates[:3]), coordinates
-    e, n, u = (to_device(np.broadcast_to(np.asarray(c, float), cast.shape).ravel()) for c in coords[:3])
+    coords = [np.broadcast_to(np.asarray(c, float), cast.shape).ravel() for c in coords[:3]]
     return layer_fields_device(
-        e, n, u, to_device(layer.easting.values), to_device(layer.northing.values),
-        to_device(layer.bottom.values), to_device(layer.top.values),
-        to_device(np.asarray(layer[density_name].values, float)), tuple(fields),
+        *to_device_together(*coords, layer.easting.values, layer.northing.values,
+                            layer.bottom.values, layer.top.values,
+                            np.asarray(layer[density_name].values, float)),
+        tuple(fields),
         thickness_threshold=0.0 if thickness_threshold is None else thickness_threshold,
     )

@@ -12,7 +12,7 @@ import numpy as np
 import torch
 
 from ._forward import (_prepare_coordinates, check_prisms, on_stream, progressbar_context,
-                       to_device)
+                       to_device_together)
 from ._lib import check, lib, ptr, stream_handle
 
 VALID_FIELDS = ("b", "b_e", "b_n", "b_u")
@@ -115,9 +115,7 @@ def prism_magnetic(
         if cast.size == 0:
             result = np.zeros((len(components), 0))
         else:
-            e, n, u = (to_device(c) for c in coords)
-            me, mn, mu = (to_device(m) for m in magnetization)
-            out = magnetic_fields_device(e, n, u, to_device(prisms.reshape(-1, 6)), me, mn, mu,
+            out = magnetic_fields_device(*to_device_together(*coords, prisms, *magnetization),
                                          components)
             result = out.cpu().numpy()
     arrays = tuple(r.astype(dtype, copy=False).reshape(cast.shape) for r in result)

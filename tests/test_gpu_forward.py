@@ -326,3 +326,28 @@ def test_point_fused_all_fields(hm):
     hp = [p.cpu().numpy() for p in pts]
     for k, f in enumerate(FIELDS):
         assert_parity(fused[k], oracle.point_gravity(coords, hp, m, f).ravel(), err_msg=f)
+
+
+@pytest.mark.parametrize("sizes", [(1,), (0, 3), (63, 64, 65), (5, 0, 0, 7), (1 << 18, 1), (1 << 17, 1 << 17)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32, np.int64])
+def test_arrays_uploaded_together(sizes, dtype):
+    """Every array arrives whole, in float64, aligned as an allocation: below
+    and above the size of one copy, empty, strided and two-dimensional."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from harmonica_amd._forward import to_device_together
+
+    rng = np.random.default_rng(len(sizes))
+    arrays = [rng.uniform(-9, 9, k).astype(np.float64) for k in sizes]
+    arrays[0] = arrays[0].astype(dtype)
+    arrays.append(rng.normal(size=(6, 11)).T)
+    arrays.append(rng.normal(size=50)[::3])
+    if dtype == np.float64:
+        arrays[-1][2] = np.nan
+    got = to_device_together(*arrays)
+    assert len(got) == len(arrays)
+    for g, a in zip(got, arrays):
+        assert g.dtype == torch.float64 and g.is_contiguous() and tuple(g.shape) == a.shape
+        assert g.data_ptr() % 256 == 0
+        npt.assert_array_equal(g.cpu().numpy(), a.astype(np.float64))
