@@ -573,7 +573,9 @@ __device__ __forceinline__ void gz_close(GzShared &sh, unsigned mask, const GzPo
 }
 
 // Close lanes from which a wave evaluates the lean closed form for all its
-// lanes rather than list its pairs (about 300 against 400 issue slots).
+// lanes rather than list its pairs (about 300 against 400 issue slots).  Lanes
+// that need the general form go to the list either way, and no longer take the
+// wave's other lanes along.
 constexpr int kGzInline = 40;
 
 // Adds the prisms of `near`, which the bounding box does not show to be far
@@ -594,13 +596,14 @@ __device__ __forceinline__ void gz_near(GzShared &sh, unsigned near, unsigned di
             acc += close ? 0.0 : v;
         }
         const GzPrism sp = sh.tile[p];
-        if (__popcll(__ballot(close)) >= kGzInline &&
-            !any_lane(close && needs_general<0x8u>(pt.e, pt.n, pt.u, sp.w, sp.e, sp.s, sp.n, sp.b,
-                                                   sp.t))) {
+        const bool lean = close && !needs_general<0x8u>(pt.e, pt.n, pt.u, sp.w, sp.e, sp.s, sp.n,
+                                                        sp.b, sp.t);
+        if (__popcll(__ballot(lean)) >= kGzInline) {
             const double v = sp.grho * gu_sum<false, false>(sp.e - pt.e, sp.w - pt.e, sp.n - pt.n,
                                                             sp.s - pt.n, sp.t - pt.u, sp.b - pt.u,
                                                             sh.tables, nullptr);
-            acc += close ? v : 0.0;
+            acc += lean ? v : 0.0;
+            mask |= close && !lean ? 1u << p : 0u;
         } else {
             mask |= close ? 1u << p : 0u;
         }

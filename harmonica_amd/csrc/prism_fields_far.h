@@ -478,6 +478,16 @@ __device__ __forceinline__ void field_close(FieldCloseWave<Op> &sh, const dm::Ta
     }
 }
 
+// Lanes from which a wave evaluates the lean closed form for all of them (as
+// kGzInline; the general form of a field set costs more beside the lean one,
+// and each field of a listed pair is added by itself).  Six tensor fields of
+// 147 x 133 cells of 903 m at 8008 points 870 m above the highest, this
+// kernel: 965 us with any lane that needs the general form sending all of the
+// wave's to the list, 707 with only such lanes listed and a limit of 40, 545
+// with 24, 530 with 16 or 10; ten fields of 317 x 290 cells, the call: 14.0,
+// 13.9, 13.6, 13.7 and 13.8 ms.
+constexpr int kFieldInline = 24;
+
 // The close pairs of 256 points and the prisms [c0, c1), added to acc.  Each
 // wave by itself: a lane reads a prism (the next one while this tile is
 // worked on), and only tiles with a prism near the wave's points go to LDS;
@@ -522,15 +532,16 @@ __device__ __forceinline__ bool field_close_chunk(const Src &src, const double *
         for_bits(near, [&](int p) {
             const bool close = !field_lane_far<M>(sh.far[p], pt);
             const double *t = sh.bounds[p];
-            if (__popcll(__ballot(close)) >= kGzInline &&
-                !any_lane(close &&
-                          needs_general<M>(pt.e, pt.n, pt.u, t[0], t[1], t[2], t[3], t[4], t[5]))) {
+            const bool lean = close && !needs_general<M>(pt.e, pt.n, pt.u, t[0], t[1], t[2], t[3],
+                                                         t[4], t[5]);
+            if (__popcll(__ballot(lean)) >= kFieldInline) {
                 double out[Op::values] = {};
                 uint32_t none = 0;
                 Op::template closed<false>(pt.e, pt.n, pt.u, t, sh.weight[p], out, none,
                                            shared.tables);
 #pragma unroll
-                for (int s = 0; s < Op::values; ++s) acc[s] += close ? out[s] : 0.0;
+                for (int s = 0; s < Op::values; ++s) acc[s] += lean ? out[s] : 0.0;
+                mask |= close && !lean ? 1ull << p : 0ull;
             } else {
                 mask |= close ? 1ull << p : 0ull;
             }

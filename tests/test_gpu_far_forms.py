@@ -298,3 +298,22 @@ def test_gz_orders_near_their_limit(hm, sides, others):
     prisms, density = np.vstack([prism, more]), np.r_[300.0, np.zeros(others)]
     got = hm.prism_gravity(coords, prisms, density, field="g_z")
     assert (np.abs(got + scale * exact) <= bound).all()
+
+
+@pytest.mark.parametrize("between", [0, 1, 23, 24, 25, 39, 40, 41, 63, 64])
+def test_close_waves_with_general_lanes(hm, between):
+    """A wave of 64 close points of which `between` lie between two planes of
+    the prisms (those pairs are listed, the rest evaluated in place or listed
+    by their number)."""
+    rng = np.random.default_rng(between)
+    prisms = np.array([[0.0, 100.0, 0.0, 80.0, -150.0, -50.0], [0.0, 100.0, 0.0, 80.0, -300.0, -160.0]])
+    density = np.array([300.0, -200.0])
+    e = np.r_[rng.uniform(5.0, 95.0, between), rng.uniform(110.0, 300.0, 64 - between)]
+    coords = [e, rng.uniform(90.0, 200.0, 64), rng.uniform(10.0, 60.0, 64)]
+    order = rng.permutation(64)
+    coords = [c[order] for c in coords]
+    exact = _fields_exact(coords, prisms, G * density)
+    for field in TEN:
+        got = hm.prism_gravity(tuple(coords), prisms, density, field=field) / _UNIT[field]
+        value, bound = exact[field]
+        assert (np.abs(got - value) <= bound).all(), field
