@@ -12,12 +12,9 @@ sequence in a HIP graph (torch.cuda.CUDAGraph) for replay.
 
 Each model's points are uploaded in boustrophedon strip order
 (``_eqs.strip_order``): a wavefront's 64 points then cover a compact patch,
-so that for most prisms no point of the wave lies between the prism's
-y-planes (or x-planes) and the wave takes the lean form of the g_z kernel
-instead of the general one.  On the 512-model workload (random points)
-unsorted waves needed the general form for 86% of the (wave, prism) pairs,
-sorted ones for 8%.  ``split()`` returns each model's values in the
-caller's order.
+so that most prisms are far from all of them and the wave takes a low order
+of the g_z kernel's far form.  ``split()`` returns each model's values in
+the caller's order.
 """
 
 import ctypes

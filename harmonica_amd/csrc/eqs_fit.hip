@@ -499,7 +499,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
 // The 128 x 128 tiles of doubles that the device holds at a time: two
 // workgroups (74 KB of LDS, 202 registers) on each of its 256 CUs.  The
 // 1128 tiles of a 6007 x 6007 upper triangle end in a round of 104, which
-// took as long as a full one on a part of the CUs: 4.75 ms, and 4.45 with
+// took as long as a full one on a part of the CUs: 4.47 ms, and 4.01 with
 // these 104 in quarters (3.25 at the matrix units' rate at the 2.1 GHz that
 // they hold; they are busy for 89% of the cycles of a busy CU).
 constexpr int64_t kRound = 512;

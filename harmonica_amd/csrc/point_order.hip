@@ -1,9 +1,9 @@
 // Wavefront-coherent order of the observation points of the pairwise prism
-// kernels.  A prism kernel picks, per wavefront and prism, the cheapest
-// closed form that is valid for all 64 points of the wavefront (lean, x-only
-// or general), so a wavefront whose points are spread over the survey area
-// pays for the general form on most prisms.  The points are therefore
-// evaluated in boustrophedon strip order: the bounding box of the points is
+// kernels.  A prism kernel picks, per wavefront and prism, the lowest order of
+// the far form that serves the bounding box of the wavefront's 64 points, and
+// the closed form where none does, so a wavefront whose points are spread over
+// the survey area pays for high orders and closed forms on most prisms.  The
+// points are therefore evaluated in boustrophedon strip order: the bounding box of the points is
 // cut into ns strips along northing and nc cells per strip along easting
 // (cells 4 times taller than wide, about n / 4 cells), strips are walked
 // alternately east- and westward, and a stable LSD radix sort of the cell

@@ -116,10 +116,10 @@ int hmx_forward_workspace_bytes(int64_t n_obs, int64_t n_sources, uint32_t field
  *             prism (gravity.py:239-269); that value is NaN.
  * Null prisms are NOT discarded here (the Python layer does it as
  * _discard_null_prisms, gravity.py:452-486, does).
- * Calls with at least 2048 points and 2^30 (point, prism) pairs evaluate the
- * points in a wavefront-coherent strip order sorted into the workspace
- * (also hmx_prism_layer_gravity and hmx_prism_magnetic); out is in the
- * caller's order either way. */
+ * Calls with at least 512 points and 2^25 (point, prism) pairs (2^28 beyond
+ * 8192 points) evaluate the points in a wavefront-coherent strip order sorted
+ * into the workspace (also hmx_prism_layer_gravity and hmx_prism_magnetic);
+ * out is in the caller's order either way. */
 int hmx_prism_gravity(const double *easting, const double *northing, const double *upward,
                       int64_t n_obs, const double *prisms, const double *density,
                       int64_t n_prisms, uint32_t field_mask, double *out,
@@ -134,8 +134,9 @@ int hmx_prism_gravity(const double *easting, const double *northing, const doubl
  * process ends.  n_obs times the fields of one launch (all of field_mask
  * for the masks with their own kernel: one field, g_e/g_n/g_z, the six
  * tensor terms, all ten; else 1) must not exceed 2^22, else HMX_ERR_ARG;
- * larger sums over prisms use fewer source chunks to fit.  Allocates
- * nothing.  Every call on one GPU shares its array: calls that overlap on
+ * larger sums over prisms use fewer source chunks to fit, and the points are
+ * sorted as in hmx_prism_gravity where the array has room for it beside the
+ * partial sums.  Allocates nothing.  Every call on one GPU shares its array: calls that overlap on
  * one GPU (several host threads or streams) race. */
 int hmx_prism_gravity_static(const double *easting, const double *northing,
                              const double *upward, int64_t n_obs, const double *prisms,
