@@ -100,9 +100,10 @@ constexpr int kSmallOrder = 8192;
 // one launch of 25-30 us up to kSmallOrder points, a dozen launches (0.1 ms)
 // beyond.  Scattered points over 20,000 bodies, g_z with and without the
 // sort: 1000 points 165 / 170 us, 3000 points 352 / 417 us, 8000 points 794 /
-// 992 us; over 2000 bodies 3000 points 73 / 57 us.
+// 992 us; over 2000 bodies 3000 points 73 / 57 us; six tensor fields of 58 x
+// 64 cells at 8085 points (3e7 pairs) 766 / 827 us.
 inline bool use_point_order(int64_t n_obs, int64_t n_src) {
-    const int64_t pairs = n_obs <= kSmallOrder ? (int64_t)1 << 25 : (int64_t)1 << 28;
+    const int64_t pairs = n_obs <= kSmallOrder ? (int64_t)1 << 24 : (int64_t)1 << 28;
     // n_obs * n_src >= pairs, without forming the product
     return n_obs >= 512 && n_src >= (pairs + n_obs - 1) / n_obs;
 }

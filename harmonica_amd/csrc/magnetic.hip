@@ -14,6 +14,7 @@
 // workgroup, one per lane, tiles of 32 prisms in LDS, far form or closed form
 // by distance, one chunk of the prism list per workgroup column, chunk
 // partial sums reduced in order by a second kernel (deterministic results).
+#include "chunk_sum.h"
 #include "hmx_internal.h"
 #include "prism_fields_far.h"
 
@@ -167,15 +168,14 @@ __global__ __launch_bounds__(dev::kGzThreads, 3) void magnetic_close_kernel(
 
 // out[s][perm[i]] = 1e9 * (sum over chunks in order of partial[c][s][i])
 // (T -> nT; perm NULL: the identity).
-__global__ void reduce_magnetic_kernel(const double *__restrict__ partial, int64_t chunks, int nc,
-                                       int64_t n_obs, const int *__restrict__ perm,
-                                       double *__restrict__ out) {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)nc * n_obs) return;
+__global__ __launch_bounds__(dev::kSumThreads) void reduce_magnetic_kernel(
+    const double *__restrict__ partial, int64_t chunks, int nc, int64_t n_obs,
+    const int *__restrict__ perm, double *__restrict__ out) {
+    const int64_t idx = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
+    double sum;
+    if (!dev::chunk_sum(partial, chunks, (int64_t)nc * n_obs, idx, sum)) return;
     const int s = (int)(idx / n_obs);
     const int64_t i = idx - (int64_t)s * n_obs;
-    double sum = 0.0;
-    for (int64_t c = 0; c < chunks; ++c) sum += partial[(c * nc + s) * n_obs + i];
     out[(int64_t)s * n_obs + (perm ? perm[i] : i)] = 1e9 * sum;
 }
 
@@ -297,8 +297,8 @@ int hmx_prism_magnetic(const double *easting, const double *northing, const doub
     }
     if (rc) return rc;
     const int64_t total = (int64_t)nc * n_obs;
-    hipLaunchKernelGGL(hmx::reduce_magnetic_kernel, dim3((unsigned)((total + 255) / 256)),
-                       dim3(256), 0, st, partial, chunks, nc, n_obs, perm, out);
+    hipLaunchKernelGGL(hmx::reduce_magnetic_kernel, dim3((unsigned)((total + 63) / 64)),
+                       dim3(hmx::dev::kSumThreads), 0, st, partial, chunks, nc, n_obs, perm, out);
     HMX_LAUNCHED("reduce_magnetic_kernel");
     return HMX_OK;
 }

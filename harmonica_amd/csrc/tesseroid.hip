@@ -24,6 +24,7 @@
 // tesseroids per pair (100000) set a flag the host turns into the
 // reference's OverflowError.
 #include "devmath.h"
+#include "chunk_sum.h"
 #include "hmx_internal.h"
 
 namespace hmx {
@@ -541,13 +542,12 @@ __global__ __launch_bounds__(256) void tess_inside_kernel(
 }
 
 // out[i] = scale * sum over chunks in order of partial[c][i].
-__global__ void reduce_tess_kernel(const double *__restrict__ partial, int64_t chunks,
-                                   int64_t n_obs, double scale, double *__restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_obs) return;
-    double sum = 0.0;
-    for (int64_t c = 0; c < chunks; ++c) sum += partial[c * n_obs + i];
-    out[i] = scale * sum;
+__global__ __launch_bounds__(dev::kSumThreads) void reduce_tess_kernel(
+    const double *__restrict__ partial, int64_t chunks, int64_t n_obs, double scale,
+    double *__restrict__ out) {
+    const int64_t i = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
+    double sum;
+    if (dev::chunk_sum(partial, chunks, n_obs, i, sum)) out[i] = scale * sum;
 }
 
 // Workspace: the chunk partials, then (256-byte aligned) one TessRoot and one
@@ -635,8 +635,8 @@ int hmx_tesseroid_gravity(const double *longitude, const double *latitude, const
     HMX_LAUNCHED("tesseroid_kernel");
     // g_z points down: the reference flips the sign of the upward kernel
     // and converts to mGal (tesseroid_gravity.py:207-211).
-    hipLaunchKernelGGL(reduce_tess_kernel, dim3((unsigned)((n_obs + 255) / 256)), dim3(256), 0,
-                       s, partial, chunks, n_obs, pot ? 1.0 : -1e5, out);
+    hipLaunchKernelGGL(reduce_tess_kernel, dim3((unsigned)((n_obs + 63) / 64)),
+                       dim3(dev::kSumThreads), 0, s, partial, chunks, n_obs, pot ? 1.0 : -1e5, out);
     HMX_LAUNCHED("reduce_tess_kernel");
     return HMX_OK;
 }
