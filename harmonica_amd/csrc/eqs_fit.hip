@@ -423,8 +423,8 @@ inline unsigned upper_tile_xcd_blocks(int64_t tiles) {
 // MFMA accumulators are folded into FP64 after every chunk (FP32 inputs,
 // FP64 sums).  Every workgroup reads all its inputs before it writes its
 // tile, and tiles are disjoint, so C may alias B when M <= kST (used by the
-// in-place panel solve of the Cholesky factorisation; a tile then holds all
-// rows of its columns).
+// in-place panel solve of the Cholesky factorisation; a workgroup then holds
+// all rows of its columns, see gemm_tiles).
 // Whether a kernel's last tiles (those from `whole` on) are taken in four
 // quarters, by one workgroup each.
 template <class T, int TR, int TC>
@@ -504,20 +504,46 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
 // they hold; they are busy for 89% of the cycles of a busy CU).
 constexpr int64_t kRound = 512;
 
+// How a product is cut: tiles of rows x cols, the first `whole` of `tiles`
+// taken by one workgroup each and the others in quarters.
+struct GemmTiles {
+    int64_t rows, cols, tiles, whole;
+};
+
+// Tiles: 128 x 128 where they fill the device (kRound), because a wavefront
+// then reads 8 operands for 16 FP64 MFMAs; what is left after the last full
+// round goes in quarters.  Fewer tiles than a round leave CUs idle, and the
+// time is that of one tile: 64 x 64 tiles then, or 128 x 32 for M <= kST.
+// With M <= kST every workgroup holds all rows of its columns (C may alias B,
+// see gemm_tn_kernel): no 64 x 64 tiles and no quarters, at any N.  Measured
+// inside a factorisation of 6007 rows: row panel (128 x 5879, K = 128) 30 us
+// as 46 tiles, 14 us as 184; update of 896 x 5879 rows (K = 128) 61 and 43
+// us, of 128 x 4000 37 and 16 us; trailing update of 887 rows (K = 1024) 204
+// and 110 us.
+inline GemmTiles gemm_tiles(bool f64, int64_t M, int64_t N, bool upper, int batch) {
+    auto cut = [&](int64_t rows, int64_t cols) {
+        const int64_t tm = (M + rows - 1) / rows, tn = (N + cols - 1) / cols;
+        const int64_t tiles = upper ? tn * (tn + 1) / 2 : tm * tn;
+        return GemmTiles{rows, cols, tiles, tiles};
+    };
+    GemmTiles t = cut(kST, kST);
+    if (!f64) return t;
+    if (t.tiles * batch < kRound) return upper || M > kST ? cut(kST / 2, kST / 2) : cut(kST, 32);
+    if (batch == 1 && M > kST) t.whole = t.tiles / kRound * kRound;
+    return t;
+}
+
 template <class T, bool UPPER, int TR, int TC>
-int launch_gemm_tiles(const T *A, int64_t lda, const T *B, int64_t ldb, int64_t K, int64_t M,
-                      int64_t N, double *C, int64_t ldc, double beta, double sign, double shift,
-                      hipStream_t s, int batch, int64_t bsa, int64_t bsb, int64_t bsc,
-                      const int64_t *dims) {
-    const int64_t tm = (M + 32 * TR - 1) / (32 * TR), tn = (N + 32 * TC - 1) / (32 * TC);
-    const int64_t tiles = UPPER ? tn * (tn + 1) / 2 : tm * tn;
-    int64_t whole = tiles;
-    if (kQuarters<T, TR, TC> && batch == 1) whole = tiles / kRound * kRound;
+int launch_gemm_tiles(const GemmTiles &t, const T *A, int64_t lda, const T *B, int64_t ldb,
+                      int64_t K, int64_t M, int64_t N, double *C, int64_t ldc, double beta,
+                      double sign, double shift, hipStream_t s, int batch, int64_t bsa, int64_t bsb,
+                      int64_t bsc, const int64_t *dims) {
+    const int64_t tn = (N + 32 * TC - 1) / (32 * TC);
     const Panel<T> pa = make_panel(A, lda, K, M), pb = make_panel(B, ldb, K, N);
     hipLaunchKernelGGL((gemm_tn_kernel<T, UPPER, TR, TC>),
-                       dim3((unsigned)(whole + 4 * (tiles - whole)), 1, (unsigned)batch),
-                       dim3(256), 0, s, pa, pb, K, M, N, C, ldc, beta, sign, shift, tn, whole, bsa,
-                       bsb, bsc, dims);
+                       dim3((unsigned)(t.whole + 4 * (t.tiles - t.whole)), 1, (unsigned)batch),
+                       dim3(256), 0, s, pa, pb, K, M, N, C, ldc, beta, sign, shift, tn, t.whole,
+                       bsa, bsb, bsc, dims);
     HMX_LAUNCHED("gemm_tn_kernel");
     return HMX_OK;
 }
@@ -525,40 +551,29 @@ int launch_gemm_tiles(const T *A, int64_t lda, const T *B, int64_t ldb, int64_t 
 // batch > 1: a strided batch of equal-shaped problems (element strides
 // bsa, bsb, bsc between consecutive A, B, C; multiples of 2 keep the
 // 16-byte loads aligned).
-// Tiles: 128 x 128 where they fill the device (kRound), because a wavefront
-// then reads 8 operands for 16 FP64 MFMAs; what is left after the last full
-// round goes in quarters.  Fewer tiles than a round leave CUs idle, and the
-// time is that of one tile: 64 x 64 tiles then, or 128 x 32 for M <= kST
-// (all rows in one workgroup, see gemm_tn_kernel on aliasing).  Measured
-// inside a factorisation of 6007 rows: row panel (128 x 5879, K = 128) 30 us
-// as 46 tiles, 14 us as 184; update of 896 x 5879 rows (K = 128) 61 and 43
-// us, of 128 x 4000 37 and 16 us; trailing update of 887 rows (K = 1024) 204
-// and 110 us.
 template <class T>
 int launch_gemm(const T *A, int64_t lda, const T *B, int64_t ldb, int64_t K, int64_t M,
                 int64_t N, double *C, int64_t ldc, double beta, double sign, double shift,
                 bool upper, hipStream_t s, int batch = 1, int64_t bsa = 0, int64_t bsb = 0,
                 int64_t bsc = 0, const int64_t *dims = nullptr) {
     if (M <= 0 || N <= 0 || batch <= 0) return HMX_OK;
-    const int64_t tm = (M + kST - 1) / kST, tn = (N + kST - 1) / kST;
-    const int64_t tiles = (upper ? tn * (tn + 1) / 2 : tm * tn) * batch;
+    const GemmTiles t = gemm_tiles(std::is_same<T, double>::value, M, N, upper, batch);
     if constexpr (std::is_same<T, double>::value) {
-        if (tiles < kRound) {
-            if (upper)
-                return launch_gemm_tiles<T, true, 2, 2>(A, lda, B, ldb, K, M, N, C, ldc, beta, sign,
-                                                        shift, s, batch, bsa, bsb, bsc, dims);
-            if (M > kST)
-                return launch_gemm_tiles<T, false, 2, 2>(A, lda, B, ldb, K, M, N, C, ldc, beta,
-                                                         sign, shift, s, batch, bsa, bsb, bsc, dims);
-            return launch_gemm_tiles<T, false, 4, 1>(A, lda, B, ldb, K, M, N, C, ldc, beta, sign,
+        if (t.rows == kST / 2 && upper)
+            return launch_gemm_tiles<T, true, 2, 2>(t, A, lda, B, ldb, K, M, N, C, ldc, beta, sign,
+                                                    shift, s, batch, bsa, bsb, bsc, dims);
+        if (t.rows == kST / 2)
+            return launch_gemm_tiles<T, false, 2, 2>(t, A, lda, B, ldb, K, M, N, C, ldc, beta, sign,
                                                      shift, s, batch, bsa, bsb, bsc, dims);
-        }
+        if (t.cols == 32)
+            return launch_gemm_tiles<T, false, 4, 1>(t, A, lda, B, ldb, K, M, N, C, ldc, beta, sign,
+                                                     shift, s, batch, bsa, bsb, bsc, dims);
     }
     if (upper)
-        return launch_gemm_tiles<T, true, 4, 4>(A, lda, B, ldb, K, M, N, C, ldc, beta, sign, shift,
-                                                s, batch, bsa, bsb, bsc, dims);
-    return launch_gemm_tiles<T, false, 4, 4>(A, lda, B, ldb, K, M, N, C, ldc, beta, sign, shift, s,
-                                             batch, bsa, bsb, bsc, dims);
+        return launch_gemm_tiles<T, true, 4, 4>(t, A, lda, B, ldb, K, M, N, C, ldc, beta, sign,
+                                                shift, s, batch, bsa, bsb, bsc, dims);
+    return launch_gemm_tiles<T, false, 4, 4>(t, A, lda, B, ldb, K, M, N, C, ldc, beta, sign, shift,
+                                             s, batch, bsa, bsb, bsc, dims);
 }
 
 // dims (device, 2 per problem, or NULL): the rows and the size each problem
@@ -2305,6 +2320,21 @@ int hmx_gemm_tn(int dtype, const void *A, int64_t lda, const void *B, int64_t ld
         return launch_gemm<float>((const float *)A, lda, (const float *)B, ldb, K, M, N, C, ldc,
                                   beta, sign, shift, upper != 0, s);
     return fail(HMX_ERR_ARG, "invalid dtype %d", dtype);
+}
+
+int hmx_gemm_tn_tiles(int dtype, int64_t M, int64_t N, int upper, int64_t *tiles) {
+    using namespace hmx;
+    clear_error();
+    if (!tiles) return fail(HMX_ERR_ARG, "tiles is NULL");
+    if (M < 0 || N < 0) return fail(HMX_ERR_ARG, "negative size");
+    if (upper && M != N) return fail(HMX_ERR_ARG, "upper requires M == N");
+    if (dtype != HMX_F64 && dtype != HMX_F32) return fail(HMX_ERR_ARG, "invalid dtype %d", dtype);
+    const GemmTiles t = gemm_tiles(dtype == HMX_F64, M, N, upper != 0, 1);
+    tiles[0] = t.rows;
+    tiles[1] = t.cols;
+    tiles[2] = t.tiles;
+    tiles[3] = t.whole;
+    return HMX_OK;
 }
 
 int hmx_cholesky_workspace_bytes(int64_t m, size_t *bytes) {

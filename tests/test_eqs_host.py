@@ -159,3 +159,22 @@ def test_fit_workspace_bytes_per_mode():
     assert st == 0 and bi == common + m * m * 8 + 4 * (20096 // 16) * 16 * m + 20 * m * 8
     assert nbytes(n, m, 4)[0] == _lib.HMX_ERR_ARG
     assert nbytes(0, m, _lib.HMX_FIT_FP64)[0] == _lib.HMX_ERR_ARG
+
+
+@pytest.mark.parametrize("M", [1, 16, 63, 64, 65, 100, 127, 128])
+def test_products_in_place_have_all_rows_in_a_workgroup(M):
+    """hmx_gemm_tn and the panel solve of the factorisation write C over B
+    where M <= 128: at no width may two workgroups share a column."""
+    import ctypes
+
+    from harmonica_amd import _lib
+
+    L = _lib.lib()
+    tiles = (ctypes.c_int64 * 4)()
+    widths = {1, 31, 127, 128, 6007, 60000, 70000, 10**6}
+    for rounds in (1, 2, 3):
+        widths |= {128 * (512 * rounds + k) + d for k in (-1, 0, 1, 5) for d in (-1, 0, 1, 64)}
+    for N in sorted(widths):
+        _lib.check(L.hmx_gemm_tn_tiles(_lib.HMX_F64, M, N, 0, tiles))
+        rows, cols, count, whole = tiles
+        assert rows >= M and whole == count == -(-N // cols), N

@@ -366,3 +366,27 @@ def test_gemm_in_place_on_b(env, M, N):
                              1.0, 0.0, 0, None))
     bound = (M + 3) * 2.0**-52 * (np.abs(A).T @ np.abs(B))
     assert np.all(np.abs(dB.cpu().numpy() - A.T @ B) <= bound)
+
+
+@pytest.mark.parametrize("M", [100, 128])
+@pytest.mark.parametrize("N", [65537, 66001, 131300])
+def test_gemm_in_place_wide(env, M, N):
+    """C over B at widths of more than 512 tiles, as in the panel solve of a
+    factorisation of as many rows: bit by bit the product out of place, and
+    that to K + 3 roundings at columns all over the width."""
+    torch, _lib, L = env
+    gen = torch.Generator(device="cuda").manual_seed(M + N)
+    make = lambda *s: torch.randn(*s, dtype=torch.float64, device="cuda", generator=gen)
+    dA, dB, dC = make(M, M), make(M, N), torch.empty(M, N, dtype=torch.float64, device="cuda")
+
+    def product(C):
+        _lib.check(L.hmx_gemm_tn(_lib.HMX_F64, _lib.ptr(dA), M, _lib.ptr(dB), N, M, M, N,
+                                 _lib.ptr(C), N, 0.0, 1.0, 0.0, 0, None))
+
+    columns = torch.arange(0, N, 97, device="cuda")
+    A, B = dA.cpu().numpy(), dB[:, columns].cpu().numpy()
+    product(dC)
+    bound = (M + 3) * 2.0**-52 * (np.abs(A).T @ np.abs(B))
+    assert np.all(np.abs(dC[:, columns].cpu().numpy() - A.T @ B) <= bound)
+    product(dB)
+    assert torch.equal(dB, dC)
