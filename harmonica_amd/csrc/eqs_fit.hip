@@ -1688,6 +1688,13 @@ inline size_t fit_x_bytes(int64_t n_data, int64_t n_src, int mode) {
     }
     return x_bytes;
 }
+// The region with its padding, in whole 16 bytes: doubles follow it (the
+// substitutions poll them 8 bytes at a time, the products load them 16 at a
+// time), and an FP32 jacobian with odd numbers of data and sources ends 4
+// bytes past one.
+inline size_t fit_x_region(int64_t n_data, int64_t n_src, int mode) {
+    return (fit_x_bytes(n_data, n_src, mode) + fit_x_padding(n_data, n_src) + 15) / 16 * 16;
+}
 
 // Stream events at the phase boundaries of a fit (destroyed on every
 // return path); elapsed times in seconds.
@@ -2394,9 +2401,9 @@ int hmx_eqs_fit_workspace_bytes(int64_t n_data, int64_t n_src, int precision_mod
     const size_t nblk = (m + kNB - 1) / kNB;
     const size_t copies = mode == HMX_FIT_FP64 ? 1 : 2;
     // (the padding is counted alike in every mode: twice a matrix's)
-    *bytes = fit_x_padding(n_data, n_src) + 2 * fit_a_padding(n_src) +
+    *bytes = 2 * fit_a_padding(n_src) +
              copies * m * m * sizeof(double)             // A, then its factor U (+ a copy of A)
-             + fit_x_bytes(n_data, n_src, mode)        // the scaled jacobian (or its slices)
+             + fit_x_region(n_data, n_src, mode)       // the scaled jacobian (or its slices)
              + 2 * nblk * kNB * kNB * sizeof(double)  // inverses of diagonal blocks
              + (10 * m + n + 256) * sizeof(double)  // 10 m-vectors, n-vector, partials
              + split_doubles(m > n ? m : n) * sizeof(double) + 256  // split sums, info
@@ -2468,7 +2475,7 @@ int hmx_eqs_fit(const double *easting, const double *northing, const double *upw
     void *X = ws;
     double *fgroup = nullptr;  // split: (n_fold, m) power-of-2 column scales per row group
     if (split) fgroup = reinterpret_cast<double *>(ws + (size_t)kSlices * n_groups * m * 16);
-    ws += fit_x_bytes(nd, m, precision_mode) + fit_x_padding(nd, m);
+    ws += fit_x_region(nd, m, precision_mode);
     f.Dinv = reinterpret_cast<double *>(ws);
     f.DinvT = f.Dinv + nblk * kNB * kNB;
     double *vec = f.DinvT + nblk * kNB * kNB;

@@ -178,3 +178,22 @@ def test_products_in_place_have_all_rows_in_a_workgroup(M):
         _lib.check(L.hmx_gemm_tn_tiles(_lib.HMX_F64, M, N, 0, tiles))
         rows, cols, count, whole = tiles
         assert rows >= M and whole == count == -(-N // cols), N
+
+
+@pytest.mark.parametrize("n,m", [(33, 21), (6007, 6007), (20001, 8209), (1023, 15)])
+def test_fit_workspace_regions_are_aligned(n, m):
+    """What follows the scaled jacobian in a fit's workspace are doubles that
+    are read 16 bytes at a time: with odd numbers of data and sources its region
+    still ends on a multiple of 16 bytes, so the modes' workspaces differ by
+    such multiples (up to one m x m matrix, which may be odd)."""
+    import ctypes
+
+    from harmonica_amd import _lib
+
+    sizes = []
+    for mode in (_lib.HMX_FIT_FP64, _lib.HMX_FIT_FP32_MFMA, _lib.HMX_FIT_BF16_SPLIT,
+                 _lib.HMX_FIT_INT8_SPLIT):
+        b = ctypes.c_size_t(0)
+        _lib.check(_lib.lib().hmx_eqs_fit_workspace_bytes(n, m, mode, ctypes.byref(b)))
+        sizes.append(b.value - (0 if mode == _lib.HMX_FIT_FP64 else 8 * m * m))
+    assert all((b - sizes[0]) % 16 == 0 for b in sizes)

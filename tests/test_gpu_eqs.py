@@ -429,3 +429,25 @@ def test_fit_ragged_sizes(hm, n, m, damping):
     expected = oracle.eqs_fit_coefs_info(J, data, None, damping)[0]
     coefs, _ = fit_device(coords, data, None, pts, damping)
     npt.assert_allclose(J @ coefs, J @ expected, rtol=0, atol=1e-10 * np.abs(data).max())
+
+
+@pytest.mark.parametrize("precision", ["mixed", "mixed-bf16", "mixed-fp32"])
+@pytest.mark.parametrize("n,m", [(49, 49), (63, 33), (301, 169)])
+def test_mixed_fit_ragged_sizes(hm, n, m, precision):
+    """Odd numbers of data and sources, so the stored low-precision jacobian
+    ends off the alignment of the doubles behind it.  Sources lie half their
+    spacing below the data; the bound is the mixed fits' bar for
+    predictions, 1e-6 of the data."""
+    from harmonica_amd._eqs import fit_device
+
+    def grid(k, depth):
+        side = int(np.ceil(np.sqrt(k)))
+        e, nn = np.meshgrid(np.arange(side) * 100.0, np.arange(side) * 100.0)
+        return e.ravel()[:k] + depth, nn.ravel()[:k], np.full(k, -depth)
+
+    coords, pts = grid(n, 0.0), grid(m, 50.0)
+    data = np.random.default_rng(n + m).normal(size=n)
+    J = oracle.eqs_jacobian(coords, pts)
+    expected = oracle.eqs_fit_coefs_info(J, data, None, 1e-2)[0]
+    coefs, _ = fit_device(coords, data, None, pts, 1e-2, precision=precision)
+    npt.assert_allclose(J @ coefs, J @ expected, rtol=0, atol=1e-6 * np.abs(data).max())
