@@ -5,8 +5,8 @@
 // l_T - l_B, l = ln(z + r); with q = |z| and lambda = ln(q + r), l = lambda
 // for z >= 0 and ln(x^2 + y^2) - lambda for z < 0, so for a point above the
 // top or below the bottom V = sg (lambda_T - lambda_B), sg the sign of z (the
-// logarithm of x^2 + y^2 cancels; points between the two take the closed
-// form).  g_u is the average of phi_B - phi_T, phi = 1/r, and the other fields
+// logarithm of x^2 + y^2 cancels; points between the two, whichever of them
+// is higher, take the closed form).  g_u is the average of phi_B - phi_T, phi = 1/r, and the other fields
 // are derivatives of these two.  With f^(m) the m-th derivative with respect
 // to s = x^2 + y^2, the average of f over the rectangle is sum_m K_m f^(m), K_m
 // the polynomials C_m of prism_far.h without phi's factor, and
@@ -253,7 +253,8 @@ __device__ __forceinline__ bool field_lane_far(const FarPrism &p, const GzPoint 
     const double x = p.x - pt.x, y = p.y - pt.y, t = p.t - pt.u, z = p.b - pt.u;
     const double s = fma(x, x, y * y), d2 = s + fmin(t * t, z * z);
     const bool far = far_enough<FarNeeds<M>::orders>(d2, p.h2);
-    if constexpr (FarNeeds<M>::lambda) return far && s >= 4.0 * p.h2 && (t <= 0.0 || z >= 0.0);
+    if constexpr (FarNeeds<M>::lambda)
+        return far && s >= 4.0 * p.h2 && (fmax(t, z) <= 0.0 || fmin(t, z) >= 0.0);
     return far;
 }
 
@@ -264,7 +265,9 @@ __device__ __forceinline__ bool field_box_far(double d2, const FarPrism &p, cons
     if constexpr (FarNeeds<M>::lambda) {
         const double dx = fmax(fmax(b.x0 - p.x, p.x - b.x1), 0.0);
         const double dy = fmax(fmax(b.y0 - p.y, p.y - b.y1), 0.0);
-        if (!(fma(dx, dx, dy * dy) >= 4.0 * p.h2 && (p.t <= b.u0 || p.b >= b.u1))) return false;
+        if (!(fma(dx, dx, dy * dy) >= 4.0 * p.h2 &&
+              (fmax(p.t, p.b) <= b.u0 || fmin(p.t, p.b) >= b.u1)))
+            return false;
     }
     return far_enough<I>(d2, p.h2);
 }

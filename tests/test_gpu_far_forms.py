@@ -317,3 +317,54 @@ def test_close_waves_with_general_lanes(hm, between):
         got = hm.prism_gravity(tuple(coords), prisms, density, field=field) / _UNIT[field]
         value, bound = exact[field]
         assert (np.abs(got - value) <= bound).all(), field
+
+
+def _device_fields(coords, prisms, density, fields):
+    from harmonica_amd._forward import prism_fields_device, to_device
+
+    dev = [to_device(np.ascontiguousarray(c)) for c in coords]
+    return prism_fields_device(*dev, to_device(prisms), to_device(density), fields).cpu().numpy()
+
+
+def test_bottom_above_top(hm):
+    """Prisms given with bottom and top exchanged, as the calls without checks
+    take them, are prisms of the opposite sign: for points above both planes
+    and below both in every field, for points between them in the fields whose
+    closed form needs no logarithm along z, beside the model (the branches of
+    the logarithms and of the angles in front of a face are chosen for bottom
+    <= top)."""
+    from harmonica_amd._forward import to_device
+    from harmonica_amd._magnetic import magnetic_fields_device
+
+    rng = np.random.default_rng(8)
+    prisms = _model("different", 40, rng)
+    prisms[:, 4], prisms[:, 5] = -2000.0 - rng.uniform(0, 50, 40), -1000.0 + rng.uniform(0, 50, 40)
+    density = rng.uniform(100, 500, 40)
+    swapped = prisms[:, [0, 1, 2, 3, 5, 4]]
+    n = 300
+    d, phi = np.geomspace(50.0, 5e4, n), rng.uniform(0.05, 1.5, n)
+    flat = (3300.0 + d * np.cos(phi), 3300.0 + d * np.sin(phi))
+    for low, high, fields in ((-900.0, 500.0, TEN), (-4000.0, -2100.0, TEN),
+                              (-1900.0, -1100.0, ("g_z", "g_ee", "g_nn", "g_zz", "g_ez", "g_nz"))):
+        coords = [*flat, rng.uniform(low, high, n)]
+        exact = _fields_exact(coords, prisms, -G * density)
+        for chosen in ((f,) for f in fields):
+            row = _device_fields(coords, swapped, density, chosen)[0]
+            value, bound = exact[chosen[0]]
+            assert (np.abs(row / _UNIT[chosen[0]] - value) <= bound).all(), (chosen, low)
+        for chosen in (TEN[4:], TEN):
+            rows = _device_fields(coords, swapped, density, chosen)
+            for f, row in zip(chosen, rows):
+                if f in fields:
+                    value, bound = exact[f]
+                    assert (np.abs(row / _UNIT[f] - value) <= bound).all(), (f, low)
+        # magnetisations along e and u (b_e) and along n and u (b_n)
+        dev = [to_device(np.ascontiguousarray(c)) for c in coords]
+        me, mu, zero = density, density[::-1].copy(), np.zeros(40)
+        for name, m, terms in (("b_e", (me, zero, mu), ("g_ee", "g_ez")),
+                               ("b_n", (zero, me, mu), ("g_nn", "g_nz"))):
+            parts = [_fields_exact(coords, prisms, -w)[f] for w, f in zip((me, mu), terms)]
+            value, bound = (sum(p[q] for p in parts) for q in (0, 1))
+            got = magnetic_fields_device(*dev, to_device(swapped), *(to_device(x) for x in m),
+                                         (name,)).cpu().numpy()[0] / 100.0
+            assert (np.abs(got - value) <= bound).all(), (name, low)
