@@ -264,8 +264,16 @@ __device__ __forceinline__ constexpr double far_ratio2(int I) {
                     : 8.8 * 8.8;
 }
 
+// The squared half-diagonal that decides on the far form, NaN (never far) for a
+// prism without area: its far form is 0 times a sum that is not finite at the
+// points of its axis, the closed form is 0.
+__device__ __forceinline__ double far_half2(double A, double B) {
+    const double h2 = A + B;
+    return h2 > 0.0 ? h2 : __builtin_nan("");
+}
+
 // A staged far prism: the rectangle's centre from the workgroup's origin, top,
-// bottom, weight times area, h^2 = A + B.  The centre is formed from bounds
+// bottom, weight times area, far_half2.  The centre is formed from bounds
 // already shifted to the origin, so its rounding is relative to its distance
 // from the workgroup's points and not to the coordinates' size.
 struct alignas(16) FarPrism {
@@ -452,7 +460,7 @@ __device__ __forceinline__ FarPrism far_prism(const double (&b)[6], double xo, d
     const double area = (b[1] - b[0]) * (b[3] - b[2]);
     return FarPrism{0.5 * ((b[0] - xo) + (b[1] - xo)), 0.5 * ((b[2] - yo) + (b[3] - yo)),
                     b[5],                              b[4],
-                    weight * area,                     A + B};
+                    weight * area,                     far_half2(A, B)};
 }
 
 // Stages prisms [t0, t0 + cnt), cnt <= kGzTile.  Src::get(p, bounds, rho)

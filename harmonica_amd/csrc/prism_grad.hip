@@ -186,7 +186,7 @@ __global__ __launch_bounds__(kObsPerBlock, 3) void gz_vjp_kernel(
     const double b0 = dev::wave_min(live ? pr.b[4] : inf);
     const double b1 = dev::wave_max(live ? pr.b[4] : -inf);
     const bool any_live = dev::any_lane(live);
-    const double h2 = A0 + B0;
+    const double h2 = dev::far_half2(A0, B0);
     __syncthreads();
     bool use_far = true;
 #pragma unroll

@@ -368,3 +368,45 @@ def test_bottom_above_top(hm):
             got = magnetic_fields_device(*dev, to_device(swapped), *(to_device(x) for x in m),
                                          (name,)).cpu().numpy()[0] / 100.0
             assert (np.abs(got - value) <= bound).all(), (name, low)
+
+
+def test_prisms_without_area(hm):
+    """A prism of zero width in both directions, which the device-level calls
+    do not leave out, adds 0 at every point off its edges, to the rounding of
+    the closed form's terms (64 x 2^-53 of w r^2, w r or w): straight above
+    and below it, level with it and at its own height range.  So do its
+    derivatives."""
+    import ctypes
+
+    import torch
+
+    from harmonica_amd import _lib
+    from harmonica_amd._forward import to_device
+    from harmonica_amd._magnetic import magnetic_fields_device
+
+    prisms = np.array([[10.0, 10.0, 20.0, 20.0, -300.0, -100.0]])
+    e = np.r_[np.full(40, 10.0), np.full(20, 10.0), np.linspace(-50, 500, 40)]
+    n = np.r_[np.full(40, 20.0), np.full(20, 25.0), np.linspace(-50, 500, 40)]
+    u = np.r_[np.geomspace(0.5, 1e5, 20) - 100.0, -300.0 - np.geomspace(0.5, 1e5, 20),
+              np.linspace(-400, 0, 20), np.linspace(-500, 500, 40)]
+    coords = [e, n, u]
+    ulp, r = 64 * 2.0**-53, np.hypot(np.hypot(e - 10, n - 20), np.abs(u + 200) + 100)
+    for fields in (*((f,) for f in TEN), TEN[1:4], TEN[4:], TEN):
+        for f, row in zip(fields, _device_fields(coords, prisms, np.array([300.0]), fields)):
+            power = 2 if f == "potential" else 1 if f in TEN[1:4] else 0
+            assert (np.abs(row / _UNIT[f]) <= ulp * G * 300.0 * r**power).all(), (f, fields)
+    dev = [to_device(c) for c in coords]
+    one = to_device(np.ones(1))
+    for names in (("b_e",), ("b_n",), ("b_u",), ("b_e", "b_n", "b_u")):
+        got = magnetic_fields_device(*dev, to_device(prisms), one, one, one, names)
+        assert (np.abs(got.cpu().numpy()) <= 3 * 100.0 * ulp).all(), names
+    v, grads = to_device(np.ones(e.size)), torch.full((2, 1), 7.0, dtype=torch.float64).cuda()
+    nbytes = ctypes.c_size_t(0)
+    _lib.check(_lib.lib().hmx_gz_grad_workspace_bytes(e.size, 1, ctypes.byref(nbytes)))
+    ws = torch.empty(nbytes.value, dtype=torch.uint8, device="cuda")
+    p = to_device(prisms)
+    _lib.check(_lib.lib().hmx_prism_gz_vjp(*(_lib.ptr(c) for c in dev), _lib.ptr(v), e.size,
+                                           _lib.ptr(p), 1, _lib.ptr(grads[0]), _lib.ptr(grads[1]),
+                                           _lib.ptr(ws), nbytes.value, None))
+    ga, gb = grads.cpu().numpy()[:, 0]
+    assert abs(ga) <= ulp * r.sum() and abs(gb) <= ulp * e.size
