@@ -265,11 +265,13 @@ __device__ __forceinline__ constexpr double far_ratio2(int I) {
 }
 
 // The squared half-diagonal that decides on the far form, NaN (never far) for a
-// prism without area: its far form is 0 times a sum that is not finite at the
-// points of its axis, the closed form is 0.
+// prism without area, whose far form is 0 times a sum that is not finite at the
+// points of its axis, and for sizes whose powers could leave the range of
+// doubles: with 1e-10 < h < 1e10 and distances below 1e14 the largest, (h r)^12
+// and r^-25, stay below 1e290.
 __device__ __forceinline__ double far_half2(double A, double B) {
     const double h2 = A + B;
-    return h2 > 0.0 ? h2 : __builtin_nan("");
+    return h2 > 1e-20 && h2 < 1e20 ? h2 : __builtin_nan("");
 }
 
 // A staged far prism: the rectangle's centre from the workgroup's origin, top,
@@ -337,12 +339,12 @@ __device__ __forceinline__ double far_distance2(const FarBox &b, const FarPrism 
     return fma(dx, dx, fma(dy, dy, d * d)) + nan_guard;
 }
 
-// Whether order 2I serves a prism at squared distance d2 (the upper bound
-// keeps the monomials of the constants finite).
+// Whether order 2I serves a prism at squared distance d2 (see far_half2 on the
+// upper bound).
 template <int I>
 __device__ __forceinline__ bool far_enough(double d2, double h2) {
 #pragma clang fp contract(off)
-    return d2 >= far_ratio2(I) * h2 && d2 < 1e50;
+    return d2 >= far_ratio2(I) * h2 && d2 < 1e28;
 }
 
 // Prisms staged per pass of the g_u kernels, at most one per lane of a wave,

@@ -410,3 +410,26 @@ def test_prisms_without_area(hm):
                                            _lib.ptr(ws), nbytes.value, None))
     ga, gb = grads.cpu().numpy()[:, 0]
     assert abs(ga) <= ulp * r.sum() and abs(gb) <= ulp * e.size
+
+
+@pytest.mark.parametrize("power", [45, -55])
+def test_sizes_far_from_a_metre(hm, power):
+    """A model scaled by 2^45 and by 2^-55: the potential scales by the
+    square, accelerations by the first power, the tensor not at all.  The
+    powers of the expansion would overflow there (the half-diagonal times the
+    distance, and the inverse distance, to the twelfth)."""
+    rng = np.random.default_rng(12)
+    prisms = _model("different", 20, rng)
+    density = rng.uniform(100, 500, 20)
+    n = 130
+    d, phi = np.geomspace(300.0, 2e4, n), rng.uniform(0, 2 * np.pi, n)
+    coords = [1500.0 + d * np.cos(phi), 1500.0 + d * np.sin(phi), rng.uniform(5.0, 3e3, n)]
+    exact = _fields_exact(coords, prisms, G * density)
+    scale = 2.0**power
+    scaled = [c * scale for c in coords]
+    for fields in (*((f,) for f in TEN), TEN[1:4], TEN[4:], TEN):
+        rows = _device_fields(scaled, prisms * scale, density, fields)
+        for f, row in zip(fields, rows):
+            value, bound = exact[f]
+            size = scale ** (2 if f == "potential" else 1 if f in TEN[1:4] else 0)
+            assert (np.abs(row / size / _UNIT[f] - value) <= bound).all(), (f, fields)
