@@ -321,10 +321,29 @@ __device__ __forceinline__ double far_gz(const FarPrism &rec, const Consts &c, d
 // Bounding box of the points of a wave (x and y relative to the origin).
 struct FarBox {
     double x0, x1, y0, y1, u0, u1;
+    // squared distance of its farthest corner from the origin
+    __device__ __forceinline__ double reach2() const {
+#pragma clang fp contract(off)
+        return fmax(x0 * x0, x1 * x1) + fmax(y0 * y0, y1 * y1);
+    }
 };
 
+// Whether the coordinates relative to the origin are good enough for a prism
+// at squared distance d2 of points up to reach2 (squared) from the origin.
+// Point and prism round to about 2^-53 of their distance R from it, 2 R / r
+// roundings of the distance r between them; the closed form, which takes their
+// difference from the coordinates as given, is off by 4 to 16 (r/h)^2
+// roundings.  So points of a workgroup may be spread widely (r^3 >= 4 R h^2: R
+// up to 170 h at the shortest r, 8.8 h), but one that lies a continent away, or
+// at a placeholder's 1e20 m, does not spoil the others.
+__device__ __forceinline__ bool far_resolved(double d2, double h2, double reach2) {
+#pragma clang fp contract(off)
+    return d2 * d2 * d2 >= 16.0 * reach2 * (h2 * h2);
+}
+
 // Smallest squared distance from the box to the nearer face centre of a
-// staged prism; NaN (never far) if the prism or the whole box is NaN.  (No
+// staged prism; -1 (never far) if the coordinates do not resolve it, NaN
+// (neither) if the prism or the whole box is NaN.  (No
 // contraction here and below: kernels that share the work of a pair have to
 // come to the same decision.)
 __device__ __forceinline__ double far_distance2(const FarBox &b, const FarPrism &p) {
@@ -336,7 +355,8 @@ __device__ __forceinline__ double far_distance2(const FarBox &b, const FarPrism 
     const double dt = fmax(fmax(b.u0 - p.t, p.t - b.u1), 0.0);
     const double db = fmax(fmax(b.u0 - p.b, p.b - b.u1), 0.0);
     const double d = fmin(dt, db);
-    return fma(dx, dx, fma(dy, dy, d * d)) + nan_guard;
+    const double d2 = fma(dx, dx, fma(dy, dy, d * d)) + nan_guard;
+    return far_resolved(d2, p.h2, b.reach2()) ? d2 : -1.0;
 }
 
 // Whether order 2I serves a prism at squared distance d2 (see far_half2 on the
@@ -512,7 +532,8 @@ __device__ __forceinline__ void gz_stage(const Src &src, int64_t t0, int cnt, do
 // Whether order 2 kFarMax serves the lane's own point.
 __device__ __forceinline__ bool lane_is_far(const FarPrism &p, double px, double py, double pu) {
     const double x = p.x - px, y = p.y - py, t = p.t - pu, z = p.b - pu;
-    return far_enough<kFarMax>(fma(x, x, fma(y, y, fmin(t * t, z * z))), p.h2);
+    const double d2 = fma(x, x, fma(y, y, fmin(t * t, z * z)));
+    return far_enough<kFarMax>(d2, p.h2) && far_resolved(d2, p.h2, fma(px, px, py * py));
 }
 
 // Calls f(p) for the set bits p of a wave-uniform mask, in order.

@@ -252,7 +252,8 @@ __device__ __forceinline__ bool field_lane_far(const FarPrism &p, const GzPoint 
 #pragma clang fp contract(off)
     const double x = p.x - pt.x, y = p.y - pt.y, t = p.t - pt.u, z = p.b - pt.u;
     const double s = fma(x, x, y * y), d2 = s + fmin(t * t, z * z);
-    const bool far = far_enough<FarNeeds<M>::orders>(d2, p.h2);
+    const bool far = far_enough<FarNeeds<M>::orders>(d2, p.h2) &&
+                     far_resolved(d2, p.h2, fma(pt.x, pt.x, pt.y * pt.y));
     if constexpr (FarNeeds<M>::lambda)
         return far && s >= 4.0 * p.h2 && (fmax(t, z) <= 0.0 || fmin(t, z) >= 0.0);
     return far;

@@ -212,7 +212,8 @@ __global__ __launch_bounds__(kObsPerBlock, 3) void gz_vjp_kernel(
             const double dt = fmax(fmax(box.u0 - o.z, o.z - box.u1), 0.0);
             const double db = fmax(fmax(b0 - o.z, o.z - b1), 0.0);
             const double d = fmin(dt, db);
-            const double d2 = fma(dx, dx, fma(dy, dy, d * d)) + guard;
+            double d2 = fma(dx, dx, fma(dy, dy, d * d)) + guard;
+            if (!dev::far_resolved(d2, h2, fma(x, x, y * y))) d2 = -1.0;
             auto take = [&](bool far) {
                 const uint64_t m = __ballot(far) & rest;
                 rest &= ~m;
@@ -244,9 +245,11 @@ __global__ __launch_bounds__(kObsPerBlock, 3) void gz_vjp_kernel(
             const double4 o = tile[q];
             bool close = true;
             if (use_far) {
-                const double x = pr.x - (o.x - xo), y = pr.y - (o.y - yo);
+                const double px = o.x - xo, py = o.y - yo, x = pr.x - px, y = pr.y - py;
                 const double t = pr.b[5] - o.z, z = pr.b[4] - o.z;
-                close = !dev::far_enough<dev::kFarMax>(fma(x, x, fma(y, y, fmin(t * t, z * z))), h2);
+                const double d2 = fma(x, x, fma(y, y, fmin(t * t, z * z)));
+                close = !(dev::far_enough<dev::kFarMax>(d2, h2) &&
+                          dev::far_resolved(d2, h2, fma(px, px, py * py)));
                 if (dev::any_lane(live && !close)) {
                     double sa = 0.0, sb = 0.0;
                     vjp_far<dev::kFarMax>(pr, lds, point(q), sa, sb);
