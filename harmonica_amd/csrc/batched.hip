@@ -55,7 +55,7 @@ __global__ __launch_bounds__(dev::kGzThreads, 4) void batched_gz_kernel(
         pt.x = pt.e - pt.xo;
         pt.y = pt.n - pt.yo;
         if (p0 < p1) dev::gz_table(src, p0, sh);
-        dev::gz_box(pt, sh);
+        dev::point_box(pt, sh.box);
         double acc = 0.0;
         for (int64_t t0 = p0; t0 < p1; t0 += dev::kGzTile) {
             const int cnt = (int)(p1 - t0 < dev::kGzTile ? p1 - t0 : dev::kGzTile);

@@ -142,7 +142,7 @@ __global__ __launch_bounds__(dev::kGzThreads, 4) void prism_gz_kernel(
     const int64_t c0 = (int64_t)blockIdx.y * chunk_len;
     const int64_t c1 = c0 + chunk_len < n_src ? c0 + chunk_len : n_src;
     if (c0 < c1) dev::gz_table(src, c0, sh);
-    dev::gz_box(pt, sh);
+    dev::point_box(pt, sh.box);
     for (int64_t t0 = c0; t0 < c1; t0 += dev::kGzTile) {
         const int cnt = (int)(c1 - t0 < dev::kGzTile ? c1 - t0 : dev::kGzTile);
         dev::gz_stage(src, t0, cnt, pt.xo, pt.yo, sh);
@@ -165,7 +165,8 @@ __global__ __launch_bounds__(kObsPerBlock) void singular_scan_kernel(
     const int ii = i < n_obs ? i : n_obs - 1;
     const double e = oe[ii], n = on[ii], u = ou[ii];
     const dev::FarBox box{dev::wave_min(e), dev::wave_max(e), dev::wave_min(n),
-                          dev::wave_max(n), dev::wave_min(u), dev::wave_max(u)};
+                          dev::wave_max(n), dev::wave_min(u), dev::wave_max(u),
+                          0.0};
     uint32_t found = 0;
     const int64_t c0 = (int64_t)blockIdx.y * chunk_len;
     const int64_t c1 = c0 + chunk_len < n_src ? c0 + chunk_len : n_src;

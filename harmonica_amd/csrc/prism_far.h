@@ -318,14 +318,10 @@ __device__ __forceinline__ double far_gz(const FarPrism &rec, const Consts &c, d
     return rec.w * (far_face<I>(s, rec.b - pu, C) - far_face<I>(s, rec.t - pu, C));
 }
 
-// Bounding box of the points of a wave (x and y relative to the origin).
+// Bounding box of the points of a wave (x and y relative to the origin), and
+// the squared distance of its farthest corner from the origin.
 struct FarBox {
-    double x0, x1, y0, y1, u0, u1;
-    // squared distance of its farthest corner from the origin
-    __device__ __forceinline__ double reach2() const {
-#pragma clang fp contract(off)
-        return fmax(x0 * x0, x1 * x1) + fmax(y0 * y0, y1 * y1);
-    }
+    double x0, x1, y0, y1, u0, u1, reach2;
 };
 
 // Whether the coordinates relative to the origin are good enough for a prism
@@ -356,7 +352,7 @@ __device__ __forceinline__ double far_distance2(const FarBox &b, const FarPrism 
     const double db = fmax(fmax(b.u0 - p.b, p.b - b.u1), 0.0);
     const double d = fmin(dt, db);
     const double d2 = fma(dx, dx, fma(dy, dy, d * d)) + nan_guard;
-    return far_resolved(d2, p.h2, b.reach2()) ? d2 : -1.0;
+    return far_resolved(d2, p.h2, b.reach2) ? d2 : -1.0;
 }
 
 // Whether order 2I serves a prism at squared distance d2 (see far_half2 on the
@@ -425,12 +421,14 @@ struct GzPoint {
     double e, n, u, x, y, xo, yo;
 };
 
-// Bounding box of the wave's points into sh.box (read after the next
+// Bounding box of the wave's points into box[wave] (read after the next
 // barrier).
-__device__ __forceinline__ void gz_box(const GzPoint &pt, GzShared &sh) {
-    const FarBox b{wave_min(pt.x), wave_max(pt.x), wave_min(pt.y),
-                   wave_max(pt.y), wave_min(pt.u), wave_max(pt.u)};
-    if ((threadIdx.x & 63) == 0) sh.box[threadIdx.x >> 6] = b;
+__device__ __forceinline__ void point_box(const GzPoint &pt, FarBox *box) {
+#pragma clang fp contract(off)
+    FarBox b{wave_min(pt.x), wave_max(pt.x), wave_min(pt.y),
+             wave_max(pt.y), wave_min(pt.u), wave_max(pt.u), 0.0};
+    b.reach2 = fmax(b.x0 * b.x0, b.x1 * b.x1) + fmax(b.y0 * b.y0, b.y1 * b.y1);
+    if ((threadIdx.x & 63) == 0) box[threadIdx.x >> 6] = b;
 }
 
 // All constants of a rectangle, in three parts of similar cost.
@@ -529,11 +527,24 @@ __device__ __forceinline__ void gz_stage(const Src &src, int64_t t0, int cnt, do
     }
 }
 
-// Whether order 2 kFarMax serves the lane's own point.
-__device__ __forceinline__ bool lane_is_far(const FarPrism &p, double px, double py, double pu) {
+// Whether a prism is small enough next to a wave's reach that far_resolved
+// can fail at the distances of the far form, 8.8 h and more.  Asked once per
+// wave and prism: in the lanes' own tests far_resolved cost 1 to 2% of calls
+// with many near prisms.
+__device__ __forceinline__ bool far_unsure(const FarBox &b, double h2) {
+#pragma clang fp contract(off)
+    return !(b.reach2 <= 29000.0 * h2);
+}
+
+// Whether order 2 kFarMax serves the lane's own point (unsure: uniform in the
+// wave).
+__device__ __forceinline__ bool lane_is_far(const FarPrism &p, bool unsure, double px, double py,
+                                            double pu) {
     const double x = p.x - px, y = p.y - py, t = p.t - pu, z = p.b - pu;
     const double d2 = fma(x, x, fma(y, y, fmin(t * t, z * z)));
-    return far_enough<kFarMax>(d2, p.h2) && far_resolved(d2, p.h2, fma(px, px, py * py));
+    bool far = far_enough<kFarMax>(d2, p.h2);
+    if (unsure) far = far && far_resolved(d2, p.h2, fma(px, px, py * py));
+    return far;
 }
 
 // Calls f(p) for the set bits p of a wave-uniform mask, in order.
@@ -615,12 +626,12 @@ constexpr int kGzInline = 40;
 // not depend on the points that share its wave (bar the orders of the far
 // form, which agree to 4e-15) and neither, to rounding, does the result on
 // their order.
-__device__ __forceinline__ void gz_near(GzShared &sh, unsigned near, unsigned different,
-                                        const GzPoint &pt, double &acc) {
+__device__ __forceinline__ void gz_near(GzShared &sh, unsigned near, unsigned unsure,
+                                        unsigned different, const GzPoint &pt, double &acc) {
     unsigned mask = 0;
     for_bits(near, [&](int p) {
         const FarPrism rec = sh.far[p];
-        const bool close = !lane_is_far(rec, pt.x, pt.y, pt.u);
+        const bool close = !lane_is_far(rec, (unsure >> p) & 1u, pt.x, pt.y, pt.u);
         if (any_lane(!close)) {
             const double v =
                 far_gz<kFarMax>(rec, FarLds{gz_consts(sh.consts, p, different)}, pt.x, pt.y, pt.u);
@@ -669,7 +680,9 @@ __device__ __forceinline__ void gz_tile(int cnt, const GzPoint &pt, double &acc,
     const unsigned live = __builtin_amdgcn_readfirstlane(sh.live);
     const unsigned different = __builtin_amdgcn_readfirstlane(sh.different);
     const FarPrism mine = sh.far[q < cnt ? q : 0];
-    const double d2 = far_distance2(sh.box[threadIdx.x >> 6], mine);
+    const FarBox &box = sh.box[threadIdx.x >> 6];
+    const double d2 = far_distance2(box, mine);
+    const unsigned unsure = (unsigned)__ballot(far_unsure(box, mine.h2));
     unsigned rest = live;
     auto take = [&](bool far) {
         const unsigned m = (unsigned)__ballot(far) & rest;
@@ -684,7 +697,7 @@ __device__ __forceinline__ void gz_tile(int cnt, const GzPoint &pt, double &acc,
     gz_far<4>(sh, different, m4, pt, acc);
     gz_far<5>(sh, different, m5, pt, acc);
     gz_far<6>(sh, different, m6, pt, acc);
-    if (rest) gz_near(sh, rest, different, pt, acc);
+    if (rest) gz_near(sh, rest, unsure, different, pt, acc);
 }
 
 }  // namespace dev

@@ -246,14 +246,15 @@ __device__ __forceinline__ void far_fields(double x, double y, double zt, double
     if constexpr (F::nn && !Q::nn_direct) vs[F::slot(5)] = -(vs[F::slot(4)] + vs[F::slot(6)]);
 }
 
-// Whether the far form of the highest order serves the lane's own point.
+// Whether the far form of the highest order serves the lane's own point
+// (unsure: far_unsure of the wave's box).
 template <unsigned M>
-__device__ __forceinline__ bool field_lane_far(const FarPrism &p, const GzPoint &pt) {
+__device__ __forceinline__ bool field_lane_far(const FarPrism &p, bool unsure, const GzPoint &pt) {
 #pragma clang fp contract(off)
     const double x = p.x - pt.x, y = p.y - pt.y, t = p.t - pt.u, z = p.b - pt.u;
     const double s = fma(x, x, y * y), d2 = s + fmin(t * t, z * z);
-    const bool far = far_enough<FarNeeds<M>::orders>(d2, p.h2) &&
-                     far_resolved(d2, p.h2, fma(pt.x, pt.x, pt.y * pt.y));
+    bool far = far_enough<FarNeeds<M>::orders>(d2, p.h2);
+    if (unsure) far = far && far_resolved(d2, p.h2, fma(pt.x, pt.x, pt.y * pt.y));
     if constexpr (FarNeeds<M>::lambda)
         return far && s >= 4.0 * p.h2 && (fmax(t, z) <= 0.0 || fmin(t, z) >= 0.0);
     return far;
@@ -301,9 +302,7 @@ __device__ __forceinline__ GzPoint field_point(const double *__restrict__ oe,
     GzPoint pt{oe[ii], on[ii], ou[ii], 0.0, 0.0, oe[base], on[base]};
     pt.x = pt.e - pt.xo;
     pt.y = pt.n - pt.yo;
-    const FarBox b{wave_min(pt.x), wave_max(pt.x), wave_min(pt.y),
-                   wave_max(pt.y), wave_min(pt.u), wave_max(pt.u)};
-    if ((threadIdx.x & 63) == 0) box[threadIdx.x >> 6] = b;
+    point_box(pt, box);
     return pt;
 }
 
@@ -395,7 +394,7 @@ __device__ __forceinline__ void field_far_chunk(const Src &src, const double *__
         }
         const int q = threadIdx.x & 63;
         const FarPrism mine = sh.far[q < cnt ? q : 0];
-        const FarBox box = sh.box[threadIdx.x >> 6];
+        const FarBox &box = sh.box[threadIdx.x >> 6];
         const double d2 = far_distance2(box, mine);
         unsigned rest = live;
         auto take = [&](bool far) {
@@ -412,8 +411,9 @@ __device__ __forceinline__ void field_far_chunk(const Src &src, const double *__
         if constexpr (Q::orders >= 5)
             field_far<5>(sh, different, take(field_box_far<5, M>(d2, mine, box)), pt, acc);
         // prisms that are far from some of the wave's points only
+        const unsigned unsure = (unsigned)__ballot(far_unsure(box, mine.h2));
         for_bits(rest, [&](int p) {
-            const bool far = field_lane_far<M>(sh.far[p], pt);
+            const bool far = field_lane_far<M>(sh.far[p], (unsure >> p) & 1u, pt);
             if (!any_lane(far)) return;
             double v[Op::values] = {};
             field_far<Q::orders>(sh, different, 1u << p, pt, v);
@@ -511,7 +511,8 @@ __device__ __forceinline__ bool field_close_chunk(const Src &src, const double *
     const GzPoint pt = field_point(oe, on, ou, base, n_obs, shared.box);
     __syncthreads();
     const int q = threadIdx.x & 63;
-    const FarBox box = shared.box[threadIdx.x >> 6];
+    // (read again for every tile: in registers it costs the closed forms spills)
+    const FarBox &box = shared.box[threadIdx.x >> 6];
     FieldCloseWave<Op> &sh = shared.wave[threadIdx.x >> 6];
     bool any = false, skip = true;
     double b[6] = {}, weight[Op::weights] = {};
@@ -520,6 +521,7 @@ __device__ __forceinline__ bool field_close_chunk(const Src &src, const double *
         const FarPrism rec = far_prism(b, pt.xo, pt.yo, 1.0);
         const uint64_t near = __ballot(
             !skip && !field_box_far<Q::orders, M>(far_distance2(box, rec), rec, box));
+        const uint64_t unsure = __ballot(far_unsure(box, rec.h2));
         if (near) {
             sh.far[q] = rec;
 #pragma unroll
@@ -534,7 +536,7 @@ __device__ __forceinline__ bool field_close_chunk(const Src &src, const double *
         wave_sync();
         uint64_t mask = 0;
         for_bits(near, [&](int p) {
-            const bool close = !field_lane_far<M>(sh.far[p], pt);
+            const bool close = !field_lane_far<M>(sh.far[p], (unsure >> p) & 1u, pt);
             const double *t = sh.bounds[p];
             const bool lean = close && !needs_general<M>(pt.e, pt.n, pt.u, t[0], t[1], t[2], t[3],
                                                          t[4], t[5]);

@@ -182,7 +182,8 @@ __global__ __launch_bounds__(kObsPerBlock, 3) void gz_vjp_kernel(
     const double inf = __builtin_inf();
     const dev::FarBox box{dev::wave_min(live ? pr.x : inf),    dev::wave_max(live ? pr.x : -inf),
                           dev::wave_min(live ? pr.y : inf),    dev::wave_max(live ? pr.y : -inf),
-                          dev::wave_min(live ? pr.b[5] : inf), dev::wave_max(live ? pr.b[5] : -inf)};
+                          dev::wave_min(live ? pr.b[5] : inf), dev::wave_max(live ? pr.b[5] : -inf),
+                          0.0};
     const double b0 = dev::wave_min(live ? pr.b[4] : inf);
     const double b1 = dev::wave_max(live ? pr.b[4] : -inf);
     const bool any_live = dev::any_lane(live);
