@@ -483,12 +483,23 @@ __device__ __forceinline__ FarPrism far_prism(const double (&b)[6], double xo, d
                     weight * area,                     far_half2(A, B)};
 }
 
+// Whether squared half-sides are equal enough to share constants: to 2^-36, as
+// the sides of equal cells of some metres round at coordinates of some 1e6 m.
+// The constants scale corrections of up to (h/r)^2 / 3, so sharing them is off
+// by up to that part of 2^-36: 6e-14 of <1/r> at the shortest distance, 8.8
+// half-diagonals, 1e-14 at 21.8 (order 8), 2e-15 at 48 (order 6).  The closed
+// form is off by up to 16 (r/h)^2 2^-53 = 1.4e-13 at 8.8.  (The two constants of
+// order 2 from each prism itself leave 1e-15, but cost g_zz of 20,011 bodies
+// 10%, a layer of 100 x 100 cells 3%.)
+__device__ __forceinline__ bool far_alike(double A, double B, double A0, double B0) {
+    return fabs(A - A0) <= 0x1p-36 * A0 && fabs(B - B0) <= 0x1p-36 * B0;
+}
+
 // Stages prisms [t0, t0 + cnt), cnt <= kGzTile.  Src::get(p, bounds, rho)
 // returns whether the prism is left out.  Holds every barrier it needs before
 // and after.  Grids of equal cells, by far the most common layers, use the
-// last entry's constants (equal to 2^-36: they scale corrections below
-// (h/r)^2 / 3, so that is a relative 1e-14 at the shortest distance); a tile
-// with other rectangles gets its own constants, prism by prism.
+// last entry's constants; a tile with other rectangles gets its own, prism by
+// prism.
 template <class Src>
 __device__ __forceinline__ void gz_stage(const Src &src, int64_t t0, int cnt, double xo, double yo,
                                          GzShared &sh) {
@@ -504,7 +515,7 @@ __device__ __forceinline__ void gz_stage(const Src &src, int64_t t0, int cnt, do
             sh.tile[q] = GzPrism{b[0], b[1], b[2], b[3], b[4], b[5], kG * rho, 0.0};
             sh.far[q] = far_prism(b, xo, yo, kG * rho);
         }
-        const bool same = fabs(A - sh.A) <= 0x1p-36 * sh.A && fabs(B - sh.B) <= 0x1p-36 * sh.B;
+        const bool same = far_alike(A, B, sh.A, sh.B);
         const uint64_t live = __ballot(!skip), different = __ballot(!skip && !same);
         if (q == 0) {
             sh.live = (unsigned)live;

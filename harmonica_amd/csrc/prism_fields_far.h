@@ -370,8 +370,7 @@ __device__ __forceinline__ void field_far_chunk(const Src &src, const double *__
 #pragma unroll
                 for (int k = 0; k < Op::weights; ++k) sh.weight[q][k] = weight[k];
             }
-            const bool same =
-                fabs(A - sh.A) <= 0x1p-36 * sh.A && fabs(B - sh.B) <= 0x1p-36 * sh.B;
+            const bool same = far_alike(A, B, sh.A, sh.B);
             const uint64_t live = __ballot(!skip), other = __ballot(!skip && !same);
             if (q == 0) {
                 sh.live = (unsigned)live;

@@ -174,7 +174,7 @@ __global__ __launch_bounds__(kObsPerBlock, 3) void gz_vjp_kernel(
     double A, B, A0, B0;
     dev::half_sides2(pr.b, A, B);
     dev::half_sides2(first, A0, B0);
-    const bool like = fabs(A - A0) <= 0x1p-36 * A0 && fabs(B - B0) <= 0x1p-36 * B0;
+    const bool like = dev::far_alike(A, B, A0, B0);
     const bool all_like = !dev::any_lane(live && !like);
     if (lane == 0) same[threadIdx.x >> 6] = all_like;
     if (threadIdx.x < 3) dev::far_consts(A0, B0, threadIdx.x, consts);

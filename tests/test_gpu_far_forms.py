@@ -453,3 +453,42 @@ def test_one_point_far_away(hm, where):
         for f, row in zip(fields, rows):
             value, bound = exact[f]
             assert (np.abs(row[1:] / _UNIT[f] - value) <= bound).all(), (f, fields)
+
+
+@pytest.mark.parametrize("sides", [(100.0, 100.0), (100.0, 300.0)])
+def test_gz_rectangles_nearly_equal(hm, sides):
+    """Rectangles that share the constants of the chunk's first one though
+    their sides differ by just under the tolerance, at 8.82 to 60
+    half-diagonals: 52 x 2^-53 of the two face terms as above, and 2^-36 of
+    the correction of order 2, at most (h/r)^2 / 3 of each."""
+    ld = np.longdouble
+    rng = np.random.default_rng(int(sides[1]))
+    a, b = sides
+    near = 1.0 + 2.0**-37.05  # of a side: just under 2^-36 of its square
+    top, bottom = -50.0, -250.0
+    first = np.array([-a / 2, a / 2, -b / 2, b / 2, bottom, top])
+    a, b = a * near, b * near
+    prism = np.array([-a / 2, a / 2, -b / 2, b / 2, bottom, top])
+    a, b = prism[1] - prism[0], prism[3] - prism[2]
+    half = np.hypot(a, b) / 2
+    k = 400
+    r = half * np.geomspace(8.82, 60.0, k)
+    phi, mu = rng.uniform(0, 2 * np.pi, k), rng.uniform(0, 1, k)
+    phi[::5], mu[1::7], mu[2::7] = np.arctan2(b, a), 1.0, 0.0
+    s, z = r * np.sqrt(1 - mu * mu), r * mu
+    up = np.where(np.arange(k) % 2 == 0, top + z, bottom - z)
+    coords = (s * np.cos(phi), s * np.sin(phi), up)
+    x10, w10 = np.polynomial.legendre.leggauss(10)
+    exact = np.zeros(k, dtype=ld)
+    e, n, u = (c.astype(ld) for c in coords)
+    for xa, wa in zip(x10.astype(ld), w10.astype(ld)):
+        for xb, wb in zip(x10.astype(ld), w10.astype(ld)):
+            q = (xa * a / 2 - e) ** 2 + (xb * b / 2 - n) ** 2
+            exact += wa * wb / 4 * (1 / np.sqrt(q + (bottom - u) ** 2)
+                                    - 1 / np.sqrt(q + (top - u) ** 2))
+    rt, rb = (np.sqrt(e * e + n * n + (f - u) ** 2) for f in (top, bottom))
+    scale = 1e5 * G * 300.0 * a * b
+    bound = scale * sum((52 * ld(2) ** -53 + ld(2) ** -36 * (half / x) ** 2 / 3) / x
+                        for x in (rt, rb))
+    got = _device_fields(coords, np.vstack([first, prism]), np.array([0.0, 300.0]), ("g_z",))[0]
+    assert (np.abs(got + scale * exact) <= bound).all()
