@@ -36,7 +36,7 @@ struct MagSet {
     static constexpr int count = __builtin_popcount(C & 7u);
 };
 
-// Prisms and magnetisations as given, for field_stage.
+// Prisms and magnetisations as given, for the field chunks.
 struct MagSource {
     const double *prisms, *me, *mn, *mu;
     __device__ bool get(int64_t p, double (&b)[6], double (&weight)[3]) const {
@@ -103,7 +103,7 @@ __device__ __forceinline__ void magnetic_pair(double e, double n, double u, cons
     }
 }
 
-// The sums of field_chunk: the selected components.
+// The sums of field_far_chunk and field_close_chunk: the selected components.
 template <unsigned C>
 struct MagneticOp {
     static constexpr unsigned fields = MagSet<C>::tensor;

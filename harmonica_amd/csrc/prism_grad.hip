@@ -146,7 +146,7 @@ __device__ __forceinline__ void vjp_far(const VjpPrism &p, const Consts &c, cons
 // rectangles (every layer) take the far form wherever it serves all prisms of
 // a wave (by the bounding boxes of their centres, tops and bottoms), its
 // constants in scalar registers up to order 6; nearer points go lane by lane
-// as in the forward kernel, order 10 or the closed form by the lane's own
+// as in the forward kernel, order 12 or the closed form by the lane's own
 // distance.  200 x 200 layer and 128 x 128
 // points: 7.06 -> 2.2 ms (every pair in the closed form before), bound by FP64
 // issue (85% of the issue cycles while the CUs are busy).

@@ -492,3 +492,28 @@ def test_gz_rectangles_nearly_equal(hm, sides):
                         for x in (rt, rb))
     got = _device_fields(coords, np.vstack([first, prism]), np.array([0.0, 300.0]), ("g_z",))[0]
     assert (np.abs(got + scale * exact) <= bound).all()
+
+
+@pytest.mark.parametrize("kind", ["grid", "different"])
+@pytest.mark.parametrize("m", [1, 33, 65])
+def test_gz_order_12_in_tiles(hm, kind, m):
+    """Points 250 m to 2 km from the model, where most pairs take the highest
+    orders: pairs from 8.81 half-diagonals on to the far form's bound (52 x
+    2^-53 of the two face terms), nearer ones to the closed form's."""
+    rng = np.random.default_rng(100 + m)
+    prisms = _model(kind, m, rng)
+    density = rng.uniform(100, 500, m)
+    d, phi = np.geomspace(250.0, 2e3, 256), rng.uniform(0, 2 * np.pi, 256)
+    coords = (50.0 + d * np.cos(phi), 50.0 + d * np.sin(phi), rng.uniform(5.0, 1500.0, 256))
+    expected, _ = _gz_exact(coords, prisms, density)
+    e, n, u = (c[:, None] for c in coords)
+    area = (prisms[:, 1] - prisms[:, 0]) * (prisms[:, 3] - prisms[:, 2])
+    half = np.hypot(prisms[:, 1] - prisms[:, 0], prisms[:, 3] - prisms[:, 2]) / 2
+    s = np.hypot((prisms[:, 0] + prisms[:, 1]) / 2 - e, (prisms[:, 2] + prisms[:, 3]) / 2 - n)
+    rt, rb = (np.hypot(s, z - u) for z in (prisms[:, 5], prisms[:, 4]))
+    far = np.minimum(rt, rb) >= 8.81 * half
+    bound = np.where(far, 52 * area * (1 / rt + 1 / rb), 64 * (np.maximum(rt, rb) + half))
+    bound = 2.0**-53 * (bound * 1e5 * G * density).sum(axis=1)
+    for order in (np.arange(256), rng.permutation(256)):
+        got = hm.prism_gravity(tuple(c[order] for c in coords), prisms, density, field="g_z")
+        assert (np.abs(got - expected[order]) <= bound[order]).all()
