@@ -98,7 +98,7 @@ SIGNATURES = {
     "hmx_mfma_probe": (_int, [_int, _vp, _vp, _vp, _vp]),
     "hmx_gemm_tn": (_int, [_int, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _vp, _i64, _dbl, _dbl,
                            _dbl, _int, _vp]),
-    "hmx_gemm_tn_tiles": (_int, [_int, _i64, _i64, _int, ctypes.POINTER(_i64)]),
+    "hmx_gemm_tn_tiles": (_int, [_int, _i64, _i64, _int, _int, ctypes.POINTER(_i64)]),
     "hmx_cholesky_workspace_bytes": (_int, [_i64, _szp]),
     "hmx_cholesky_solve": (_int, [_vp, _i64, _vp, ctypes.POINTER(ctypes.c_int), _vp,
                                   ctypes.c_size_t, _vp]),

@@ -496,13 +496,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         tile_k_loop<T, false, UPPER, TR, TC>(A, B, K, r0, c0, lds, M, N, C, ldc, beta, sign, shift);
 }
 
-// The 128 x 128 tiles of doubles that the device holds at a time: two
-// workgroups (74 KB of LDS, 202 registers) on each of its 256 CUs.  The
-// 1128 tiles of a 6007 x 6007 upper triangle end in a round of 104, which
-// took as long as a full one on a part of the CUs: 4.47 ms, and 4.01 with
+// The 128 x 128 tiles of doubles that a device holds at a time: two
+// workgroups (74 KB of LDS, 202 registers) on each of its CUs.  With 256 of
+// them, the 1128 tiles of a 6007 x 6007 upper triangle end in a round of 104,
+// which took as long as a full one on a part of the CUs: 4.47 ms, and 4.01 with
 // these 104 in quarters (3.25 at the matrix units' rate at the 2.1 GHz that
 // they hold; they are busy for 89% of the cycles of a busy CU).
-constexpr int64_t kRound = 512;
+inline int64_t tile_round(int n_cu) { return 2 * (int64_t)n_cu; }
 
 // How a product is cut: tiles of rows x cols, the first `whole` of `tiles`
 // taken by one workgroup each and the others in quarters.
@@ -510,7 +510,7 @@ struct GemmTiles {
     int64_t rows, cols, tiles, whole;
 };
 
-// Tiles: 128 x 128 where they fill the device (kRound), because a wavefront
+// Tiles: 128 x 128 where they fill the device (tile_round), because a wavefront
 // then reads 8 operands for 16 FP64 MFMAs; what is left after the last full
 // round goes in quarters.  Fewer tiles than a round leave CUs idle, and the
 // time is that of one tile: 64 x 64 tiles then, or 128 x 32 for M <= kST.
@@ -520,7 +520,7 @@ struct GemmTiles {
 // as 46 tiles, 14 us as 184; update of 896 x 5879 rows (K = 128) 61 and 43
 // us, of 128 x 4000 37 and 16 us; trailing update of 887 rows (K = 1024) 204
 // and 110 us.
-inline GemmTiles gemm_tiles(bool f64, int64_t M, int64_t N, bool upper, int batch) {
+inline GemmTiles gemm_tiles(bool f64, int64_t M, int64_t N, bool upper, int batch, int n_cu) {
     auto cut = [&](int64_t rows, int64_t cols) {
         const int64_t tm = (M + rows - 1) / rows, tn = (N + cols - 1) / cols;
         const int64_t tiles = upper ? tn * (tn + 1) / 2 : tm * tn;
@@ -528,8 +528,9 @@ inline GemmTiles gemm_tiles(bool f64, int64_t M, int64_t N, bool upper, int batc
     };
     GemmTiles t = cut(kST, kST);
     if (!f64) return t;
-    if (t.tiles * batch < kRound) return upper || M > kST ? cut(kST / 2, kST / 2) : cut(kST, 32);
-    if (batch == 1 && M > kST) t.whole = t.tiles / kRound * kRound;
+    const int64_t round = tile_round(n_cu);
+    if (t.tiles * batch < round) return upper || M > kST ? cut(kST / 2, kST / 2) : cut(kST, 32);
+    if (batch == 1 && M > kST) t.whole = t.tiles / round * round;
     return t;
 }
 
@@ -557,7 +558,9 @@ int launch_gemm(const T *A, int64_t lda, const T *B, int64_t ldb, int64_t K, int
                 bool upper, hipStream_t s, int batch = 1, int64_t bsa = 0, int64_t bsb = 0,
                 int64_t bsc = 0, const int64_t *dims = nullptr) {
     if (M <= 0 || N <= 0 || batch <= 0) return HMX_OK;
-    const GemmTiles t = gemm_tiles(std::is_same<T, double>::value, M, N, upper, batch);
+    const int cu = device_cu_count();
+    if (cu < 0) return cu;
+    const GemmTiles t = gemm_tiles(std::is_same<T, double>::value, M, N, upper, batch, cu);
     if constexpr (std::is_same<T, double>::value) {
         if (t.rows == kST / 2 && upper)
             return launch_gemm_tiles<T, true, 2, 2>(t, A, lda, B, ldb, K, M, N, C, ldc, beta, sign,
@@ -2329,14 +2332,14 @@ int hmx_gemm_tn(int dtype, const void *A, int64_t lda, const void *B, int64_t ld
     return fail(HMX_ERR_ARG, "invalid dtype %d", dtype);
 }
 
-int hmx_gemm_tn_tiles(int dtype, int64_t M, int64_t N, int upper, int64_t *tiles) {
+int hmx_gemm_tn_tiles(int dtype, int64_t M, int64_t N, int upper, int n_cu, int64_t *tiles) {
     using namespace hmx;
     clear_error();
     if (!tiles) return fail(HMX_ERR_ARG, "tiles is NULL");
-    if (M < 0 || N < 0) return fail(HMX_ERR_ARG, "negative size");
+    if (M < 0 || N < 0 || n_cu <= 0) return fail(HMX_ERR_ARG, "invalid sizes");
     if (upper && M != N) return fail(HMX_ERR_ARG, "upper requires M == N");
     if (dtype != HMX_F64 && dtype != HMX_F32) return fail(HMX_ERR_ARG, "invalid dtype %d", dtype);
-    const GemmTiles t = gemm_tiles(dtype == HMX_F64, M, N, upper != 0, 1);
+    const GemmTiles t = gemm_tiles(dtype == HMX_F64, M, N, upper != 0, 1, n_cu);
     tiles[0] = t.rows;
     tiles[1] = t.cols;
     tiles[2] = t.tiles;

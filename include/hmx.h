@@ -479,9 +479,10 @@ int hmx_eqs_gb_fit(const double *easting, const double *northing, const double *
  *   B (K x N, ldb) row-major in dtype, C (M x N, ldc) FP64; upper != 0
  *   computes only the upper triangle (M == N).  C may be B (HMX_F64,
  *   upper == 0) where M <= 128.
- * hmx_gemm_tn_tiles: how hmx_gemm_tn cuts C (host arithmetic): tiles[0] rows
- *   and tiles[1] columns of a tile, tiles[2] tiles, of which one workgroup
- *   takes each of the first tiles[3] and four a quarter each of the others.
+ * hmx_gemm_tn_tiles: how hmx_gemm_tn cuts C on a device of n_cu compute units
+ *   (host arithmetic): tiles[0] rows and tiles[1] columns of a tile, tiles[2]
+ *   tiles, of which one workgroup takes each of the first tiles[3] and four a
+ *   quarter each of the others.
  * hmx_cholesky_solve: factor the SPD matrix A (m x m, row-major, upper
  *   triangle read) in place as U^T U (FP64, blocked) and overwrite x with
  *   A^-1 x; *info (host) = 0 or the 1-based column of a failed pivot. */
@@ -489,7 +490,7 @@ int hmx_mfma_probe(int dtype, const double *a, const double *b, double *out, voi
 int hmx_gemm_tn(int dtype, const void *A, int64_t lda, const void *B, int64_t ldb, int64_t K,
                 int64_t M, int64_t N, double *C, int64_t ldc, double beta, double sign,
                 double shift, int upper, void *stream);
-int hmx_gemm_tn_tiles(int dtype, int64_t M, int64_t N, int upper, int64_t *tiles);
+int hmx_gemm_tn_tiles(int dtype, int64_t M, int64_t N, int upper, int n_cu, int64_t *tiles);
 int hmx_cholesky_workspace_bytes(int64_t m, size_t *bytes);
 int hmx_cholesky_solve(double *A, int64_t m, double *x, int *info, void *workspace,
                        size_t workspace_bytes, void *stream);

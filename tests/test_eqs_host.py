@@ -161,8 +161,9 @@ def test_fit_workspace_bytes_per_mode():
     assert nbytes(0, m, _lib.HMX_FIT_FP64)[0] == _lib.HMX_ERR_ARG
 
 
+@pytest.mark.parametrize("n_cu", [64, 256, 304])
 @pytest.mark.parametrize("M", [1, 16, 63, 64, 65, 100, 127, 128])
-def test_products_in_place_have_all_rows_in_a_workgroup(M):
+def test_products_in_place_have_all_rows_in_a_workgroup(M, n_cu):
     """hmx_gemm_tn and the panel solve of the factorisation write C over B
     where M <= 128: at no width may two workgroups share a column."""
     import ctypes
@@ -173,9 +174,9 @@ def test_products_in_place_have_all_rows_in_a_workgroup(M):
     tiles = (ctypes.c_int64 * 4)()
     widths = {1, 31, 127, 128, 6007, 60000, 70000, 10**6}
     for rounds in (1, 2, 3):
-        widths |= {128 * (512 * rounds + k) + d for k in (-1, 0, 1, 5) for d in (-1, 0, 1, 64)}
+        widths |= {128 * (2 * n_cu * rounds + k) + d for k in (-1, 0, 1, 5) for d in (-1, 0, 1, 64)}
     for N in sorted(widths):
-        _lib.check(L.hmx_gemm_tn_tiles(_lib.HMX_F64, M, N, 0, tiles))
+        _lib.check(L.hmx_gemm_tn_tiles(_lib.HMX_F64, M, N, 0, n_cu, tiles))
         rows, cols, count, whole = tiles
         assert rows >= M and whole == count == -(-N // cols), N
 
@@ -197,3 +198,20 @@ def test_fit_workspace_regions_are_aligned(n, m):
         _lib.check(_lib.lib().hmx_eqs_fit_workspace_bytes(n, m, mode, ctypes.byref(b)))
         sizes.append(b.value - (0 if mode == _lib.HMX_FIT_FP64 else 8 * m * m))
     assert all((b - sizes[0]) % 16 == 0 for b in sizes)
+
+
+@pytest.mark.parametrize("n_cu,expected", [(304, (64, 64, 46**2, 46**2)),
+                                           (256, (128, 128, 529, 512)),
+                                           (64, (128, 128, 529, 512)),
+                                           (100, (128, 128, 529, 400))])
+def test_products_are_cut_for_the_device(n_cu, expected):
+    """2944 x 2944 in 529 tiles of 128 x 128: in whole rounds of two per
+    compute unit and the rest in quarters, or, where they do not fill the
+    device once, in smaller tiles."""
+    import ctypes
+
+    from harmonica_amd import _lib
+
+    tiles = (ctypes.c_int64 * 4)()
+    _lib.check(_lib.lib().hmx_gemm_tn_tiles(_lib.HMX_F64, 2944, 2944, 0, n_cu, tiles))
+    assert tuple(tiles) == expected
