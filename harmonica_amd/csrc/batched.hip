@@ -27,9 +27,7 @@ namespace {
 
 constexpr int kItemWords = 5;  // model, tile, p0, p1, slot
 
-// Workgroups (of kGzThreads, one point per lane) that share an item.
-constexpr int kItemParts = kObsPerBlock / dev::kGzThreads;
-static_assert(kItemParts * dev::kGzThreads == kObsPerBlock, "parts cover an item");
+static_assert(dev::kGzThreads == kObsPerBlock, "a workgroup covers an item's points");
 
 __global__ __launch_bounds__(dev::kGzThreads, 4) void batched_gz_kernel(
     const double *__restrict__ oe, const double *__restrict__ on, const double *__restrict__ ou,
@@ -44,9 +42,9 @@ __global__ __launch_bounds__(dev::kGzThreads, 4) void batched_gz_kernel(
         __syncthreads();
         if (threadIdx.x == 0) item_id = (long long)atomicAdd(counter, 1ull);
         __syncthreads();
-        const long long k = item_id / kItemParts;
+        const long long k = item_id;
         if (k >= n_items) break;
-        const int local = (int)(item_id % kItemParts) * dev::kGzThreads + threadIdx.x;
+        const int local = threadIdx.x;
         const int64_t *it = items + kItemWords * k;
         const int64_t b = it[0], T = it[1], p0 = it[2], p1 = it[3], slot = it[4];
         const int64_t first = obs_off[b] + T * kObsPerBlock, end = obs_off[b + 1];
@@ -197,7 +195,7 @@ int hmx_batched_prism_gz(const double *easting, const double *northing, const do
     hipLaunchKernelGGL(zero_counter_kernel, dim3(1), dim3(64), 0, s, counter);
     HMX_LAUNCHED("zero_counter_kernel");
     if (n_items > 0) {
-        const int64_t grid64 = std::min<int64_t>((int64_t)cu * blocks_per_cu, n_items * kItemParts);
+        const int64_t grid64 = std::min<int64_t>((int64_t)cu * blocks_per_cu, n_items);
         hipLaunchKernelGGL(batched_gz_kernel, dim3((unsigned)grid64), dim3(dev::kGzThreads), 0, s,
                            easting, northing, upward, obs_offsets, prisms, density, items, n_items,
                            partial, counter);
