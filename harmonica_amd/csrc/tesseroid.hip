@@ -494,7 +494,8 @@ __global__ __launch_bounds__(kObsPerBlock, 3) void tesseroid_kernel(
             const TessFar &F = sh.tile[p];
             const double dx = X.x[0] - F.c[0], dy = X.x[1] - F.c[1], dz = X.x[2] - F.c[2];
             const double d2 = fma(dx, dx, fma(dy, dy, dz * dz));
-            const bool far = d2 >= F.far2, near = d2 < F.near2;
+            // (a point at infinity is neither: its terms are 1 / inf)
+            const bool far = d2 >= F.far2 && d2 < 1e300, near = d2 < F.near2;
             if (__any(far)) {
                 const double v = tess_glq_far<kPot>(X, F);
                 acc += far ? v : 0.0;

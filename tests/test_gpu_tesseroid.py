@@ -361,3 +361,11 @@ def test_point_inside_found_on_the_device(hm, longitude):
         hm.tesseroid_gravity(coords, tess, np.ones(200), "g_z")
     coords[1][123] = 1.0  # on the northern boundary
     assert np.isfinite(hm.tesseroid_gravity(coords, tess, np.ones(200), "g_z")).all()
+
+
+def test_point_at_infinity(hm):
+    """The potential at infinite radius, a sum of 1 / distance, is 0."""
+    tess = [[-10.0, -9.0, 20.0, 21.0, 6.36e6, 6.371e6], [5.0, 8.0, -3.0, 1.0, 6.3e6, 6.37e6]]
+    coords = (np.array([50.0, 50.0]), np.array([30.0, 30.0]), np.array([np.inf, 6.6e6]))
+    got = hm.tesseroid_gravity(coords, tess, [2670.0, 300.0], "potential")
+    assert got[0] == 0.0 and np.isfinite(got[1]) and got[1] > 0
