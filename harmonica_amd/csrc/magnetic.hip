@@ -168,12 +168,13 @@ __global__ __launch_bounds__(dev::kGzThreads, 3) void magnetic_close_kernel(
 
 // out[s][perm[i]] = 1e9 * (sum over chunks in order of partial[c][s][i])
 // (T -> nT; perm NULL: the identity).
-__global__ __launch_bounds__(dev::kSumThreads) void reduce_magnetic_kernel(
+template <int P>
+__global__ __launch_bounds__(dev::SumShape<P>::threads) void reduce_magnetic_kernel(
     const double *__restrict__ partial, int64_t chunks, int nc, int64_t n_obs,
     const int *__restrict__ perm, double *__restrict__ out) {
-    const int64_t idx = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
+    int64_t idx;
     double sum;
-    if (!dev::chunk_sum(partial, chunks, (int64_t)nc * n_obs, idx, sum)) return;
+    if (!dev::chunk_sum<P>(partial, chunks, (int64_t)nc * n_obs, idx, sum)) return;
     const int s = (int)(idx / n_obs);
     const int64_t i = idx - (int64_t)s * n_obs;
     out[(int64_t)s * n_obs + (perm ? perm[i] : i)] = 1e9 * sum;
@@ -198,6 +199,24 @@ int launch_magnetic(const double *oe, const double *on, const double *ou, int64_
                        ou, (int)n_obs, src, n_src, chunk_len, partial);
     HMX_LAUNCHED("magnetic_close_kernel");
     return HMX_OK;
+}
+
+template <int P>
+int launch_reduce_parts(const double *partial, int64_t chunks, int nc, int64_t n_obs,
+                        const int *perm, double *out, hipStream_t stream) {
+    using S = dev::SumShape<P>;
+    const int64_t blocks = ((int64_t)nc * n_obs + S::outputs - 1) / S::outputs;
+    hipLaunchKernelGGL((reduce_magnetic_kernel<P>), dim3((unsigned)blocks), dim3(S::threads), 0,
+                       stream, partial, chunks, nc, n_obs, perm, out);
+    HMX_LAUNCHED("reduce_magnetic_kernel");
+    return HMX_OK;
+}
+
+int launch_reduce(const double *partial, int64_t chunks, int nc, int64_t n_obs, const int *perm,
+                  double *out, hipStream_t stream) {
+    return dev::sum_parts(chunks, (int64_t)nc * n_obs, 16) == 1
+               ? launch_reduce_parts<1>(partial, chunks, nc, n_obs, perm, out, stream)
+               : launch_reduce_parts<16>(partial, chunks, nc, n_obs, perm, out, stream);
 }
 
 bool valid_components(uint32_t mask) { return mask != 0 && (mask & ~7u) == 0; }
@@ -296,11 +315,7 @@ int hmx_prism_magnetic(const double *easting, const double *northing, const doub
         return hmx::fail(HMX_ERR_ARG, "invalid component mask 0x%x", component_mask);
     }
     if (rc) return rc;
-    const int64_t total = (int64_t)nc * n_obs;
-    hipLaunchKernelGGL(hmx::reduce_magnetic_kernel, dim3((unsigned)((total + 63) / 64)),
-                       dim3(hmx::dev::kSumThreads), 0, st, partial, chunks, nc, n_obs, perm, out);
-    HMX_LAUNCHED("reduce_magnetic_kernel");
-    return HMX_OK;
+    return hmx::launch_reduce(partial, chunks, nc, n_obs, perm, out, st);
 }
 
 }  // extern "C"

@@ -9,6 +9,7 @@
 // order and applies harmonica's units, so results are deterministic.
 #include <mutex>
 
+#include "chunk_sum.h"
 #include "hmx_internal.h"
 #include "prism_device.h"
 #include "prism_fields_far.h"
@@ -199,25 +200,15 @@ __global__ __launch_bounds__(kObsPerBlock) void singular_scan_kernel(
 }
 
 // out[s][perm[i]] = units(sum over chunks of partial[c][s][i]) (perm NULL: the
-// identity).  Four waves per 64 outputs, a quarter of the chunks each, added
-// in order: a serial sum over all chunks is bound by the latency of its
-// loads (4096 points: 79 chunks took 11 us, 313 chunks take 9).
-__global__ __launch_bounds__(256) void reduce_chunks_kernel(
+// identity), four waves per 64 outputs (4096 points: 79 chunks took 11 us with a
+// thread per output, 313 chunks take 9) or a thread each (sum_parts).
+template <int P>
+__global__ __launch_bounds__(dev::SumShape<P>::threads) void reduce_chunks_kernel(
     const double *__restrict__ partial, int64_t chunks, int nf, int64_t n_obs, uint32_t mask,
     const int *__restrict__ perm, double *__restrict__ out) {
-    __shared__ double part[3][64];
-    const int lane = threadIdx.x & 63, quarter = threadIdx.x >> 6;
-    const int64_t total = (int64_t)nf * n_obs, idx = (int64_t)blockIdx.x * 64 + lane;
-    const int64_t c0 = chunks * quarter / 4, c1 = chunks * (quarter + 1) / 4;
-    double sum = 0.0;
-    if (idx < total) {
-#pragma unroll 4
-        for (int64_t c = c0; c < c1; ++c) sum += partial[c * total + idx];
-    }
-    if (quarter) part[quarter - 1][lane] = sum;
-    __syncthreads();
-    if (quarter || idx >= total) return;
-    sum = ((sum + part[0][lane]) + part[1][lane]) + part[2][lane];
+    int64_t idx;
+    double sum;
+    if (!dev::chunk_sum<P>(partial, chunks, (int64_t)nf * n_obs, idx, sum)) return;
     const int s = (int)(idx / n_obs);
     const int64_t i = idx - (int64_t)s * n_obs;
     int f = 0, seen = -1;
@@ -254,13 +245,22 @@ int launch_forward(const double *oe, const double *on, const double *ou, int64_t
     return HMX_OK;
 }
 
-int launch_reduce(const double *partial, int64_t chunks, int nf, int64_t n_obs, uint32_t mask,
-                  const int *perm, double *out, hipStream_t stream) {
-    int64_t total = (int64_t)nf * n_obs;
-    hipLaunchKernelGGL(reduce_chunks_kernel, dim3((unsigned)((total + 63) / 64)), dim3(256), 0,
+template <int P>
+int launch_reduce_parts(const double *partial, int64_t chunks, int nf, int64_t n_obs, uint32_t mask,
+                        const int *perm, double *out, hipStream_t stream) {
+    using S = dev::SumShape<P>;
+    const int64_t blocks = ((int64_t)nf * n_obs + S::outputs - 1) / S::outputs;
+    hipLaunchKernelGGL((reduce_chunks_kernel<P>), dim3((unsigned)blocks), dim3(S::threads), 0,
                        stream, partial, chunks, nf, n_obs, mask, perm, out);
     HMX_LAUNCHED("reduce_chunks_kernel");
     return HMX_OK;
+}
+
+int launch_reduce(const double *partial, int64_t chunks, int nf, int64_t n_obs, uint32_t mask,
+                  const int *perm, double *out, hipStream_t stream) {
+    return dev::sum_parts(chunks, (int64_t)nf * n_obs, 4) == 1
+               ? launch_reduce_parts<1>(partial, chunks, nf, n_obs, mask, perm, out, stream)
+               : launch_reduce_parts<4>(partial, chunks, nf, n_obs, mask, perm, out, stream);
 }
 
 // Field sets with their own kernel instantiation: each single field, the

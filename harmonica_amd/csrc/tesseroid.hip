@@ -543,12 +543,23 @@ __global__ __launch_bounds__(256) void tess_inside_kernel(
 }
 
 // out[i] = scale * sum over chunks in order of partial[c][i].
-__global__ __launch_bounds__(dev::kSumThreads) void reduce_tess_kernel(
+template <int P>
+__global__ __launch_bounds__(dev::SumShape<P>::threads) void reduce_tess_kernel(
     const double *__restrict__ partial, int64_t chunks, int64_t n_obs, double scale,
     double *__restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
+    int64_t i;
     double sum;
-    if (dev::chunk_sum(partial, chunks, n_obs, i, sum)) out[i] = scale * sum;
+    if (dev::chunk_sum<P>(partial, chunks, n_obs, i, sum)) out[i] = scale * sum;
+}
+
+template <int P>
+int launch_reduce(const double *partial, int64_t chunks, int64_t n_obs, double scale, double *out,
+                  hipStream_t stream) {
+    using S = dev::SumShape<P>;
+    hipLaunchKernelGGL((reduce_tess_kernel<P>), dim3((unsigned)((n_obs + S::outputs - 1) / S::outputs)),
+                       dim3(S::threads), 0, stream, partial, chunks, n_obs, scale, out);
+    HMX_LAUNCHED("reduce_tess_kernel");
+    return HMX_OK;
 }
 
 // Workspace: the chunk partials, then (256-byte aligned) one TessRoot and one
@@ -636,10 +647,10 @@ int hmx_tesseroid_gravity(const double *longitude, const double *latitude, const
     HMX_LAUNCHED("tesseroid_kernel");
     // g_z points down: the reference flips the sign of the upward kernel
     // and converts to mGal (tesseroid_gravity.py:207-211).
-    hipLaunchKernelGGL(reduce_tess_kernel, dim3((unsigned)((n_obs + 63) / 64)),
-                       dim3(dev::kSumThreads), 0, s, partial, chunks, n_obs, pot ? 1.0 : -1e5, out);
-    HMX_LAUNCHED("reduce_tess_kernel");
-    return HMX_OK;
+    const double scale = pot ? 1.0 : -1e5;
+    return dev::sum_parts(chunks, n_obs, 16) == 1
+               ? launch_reduce<1>(partial, chunks, n_obs, scale, out, s)
+               : launch_reduce<16>(partial, chunks, n_obs, scale, out, s);
 }
 
 int hmx_tesseroid_points_inside(const double *longitude_180, const double *longitude_360,

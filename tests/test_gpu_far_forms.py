@@ -517,3 +517,32 @@ def test_gz_order_12_in_tiles(hm, kind, m):
     for order in (np.arange(256), rng.permutation(256)):
         got = hm.prism_gravity(tuple(c[order] for c in coords), prisms, density, field="g_z")
         assert (np.abs(got - expected[order]) <= bound[order]).all()
+
+
+def test_more_outputs_than_a_launch_has_threads(hm):
+    """A reduction of 2^28 + 30 outputs (b_e, b_n, b_u of one prism at 2^28 / 3 +
+    10 points): 16 waves per 64 outputs would pass the 2^32 threads of a
+    launch.  The points repeat, and so do the values."""
+    import torch
+
+    from harmonica_amd._magnetic import magnetic_fields_device
+
+    if torch.cuda.get_device_properties(0).total_memory < 32 << 30:
+        pytest.skip("needs 10 GB")
+    n, k = (1 << 28) // 3 + 11, 1009
+    rng = np.random.default_rng(5)
+    base = [torch.as_tensor(rng.uniform(lo, hi, k)).cuda() for lo, hi in
+            ((-500, 500), (-500, 500), (10, 90))]
+    coords = [b.repeat(n // k + 1)[:n].contiguous() for b in base]
+    prism = torch.tensor([[-30.0, 40.0, -20.0, 60.0, -200.0, -50.0]], dtype=torch.float64).cuda()
+    mag = [torch.tensor([v], dtype=torch.float64).cuda() for v in (1.0, -2.0, 0.5)]
+    names = ("b_e", "b_n", "b_u")
+    few = magnetic_fields_device(*base, prism, *mag, names)
+    many = magnetic_fields_device(*coords, prism, *mag, names)
+    # the far form's offsets have another origin in each workgroup: 2^-40 of
+    # the largest value, 2^13 roundings
+    assert torch.isfinite(few).all()
+    tolerance = 2.0**-40 * few.abs().max()
+    for start in (0, k, (n // k - 1) * k):
+        assert (many[:, start:start + k] - few).abs().max() <= tolerance
+    assert (many[:, (n // k) * k:] - few[:, :n % k]).abs().max() <= tolerance
