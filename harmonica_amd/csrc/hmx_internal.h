@@ -96,13 +96,19 @@ struct PointOrder {
 constexpr int kSmallOrder = 8192;
 
 // Whether a prism call sorts its points: enough points for the strips to
-// matter and enough pairs that the sort costs little next to the pair loop:
-// one launch of 25-30 us up to kSmallOrder points, a dozen launches (0.1 ms)
-// beyond.  Scattered points over 20,000 bodies, g_z with and without the
-// sort: 1000 points 165 / 170 us, 3000 points 352 / 417 us, 8000 points 794 /
-// 992 us; over 2000 bodies 3000 points 73 / 57 us; six tensor fields of 58 x
-// 64 cells at 8085 points (3e7 pairs) 766 / 827 us.
+// matter and enough pairs that the sort costs little next to the pair loop.
+// Up to kSmallOrder points it is one launch of 25-30 us.  Scattered points
+// over 20,000 bodies, g_z with and without the sort: 1000 points 165 / 170 us,
+// 3000 points 352 / 417 us, 8000 points 794 / 992 us; over 2000 bodies 3000
+// points 73 / 57 us; six tensor fields of 58 x 64 cells at 8085 points (3e7
+// pairs) 766 / 827 us.  Beyond, it is a dozen launches (0.1 ms) and 1.2 ns a
+// point, which scattered points get back from a few hundred prisms on and a
+// raster's hardly ever: 1e6 points, g_z, 128 prisms 1.55 / 1.17 ms scattered
+// and 1.50 / 0.35 as a raster, 512 prisms 2.5 / 4.4 and 2.4 / 1.2 ms; 200,000
+// points, 1024 prisms 0.67 / 1.82 and 0.66 / 0.51 ms.  (1e7 points over 28
+// prisms spent 15 of 17 ms in it.)
 inline bool use_point_order(int64_t n_obs, int64_t n_src) {
+    if (n_obs > kSmallOrder && n_src < 512) return false;
     const int64_t pairs = n_obs <= kSmallOrder ? (int64_t)1 << 24 : (int64_t)1 << 28;
     // n_obs * n_src >= pairs, without forming the product
     return n_obs >= 512 && n_src >= (pairs + n_obs - 1) / n_obs;
@@ -111,7 +117,8 @@ inline bool use_point_order(int64_t n_obs, int64_t n_src) {
 // Whether a call with a workspace too small for the order is refused; below
 // this it evaluates the points in the caller's order.
 inline bool need_point_order(int64_t n_obs, int64_t n_src) {
-    return n_obs >= 2048 && n_src >= (((int64_t)1 << 30) + n_obs - 1) / n_obs;
+    return use_point_order(n_obs, n_src) && n_obs >= 2048 &&
+           n_src >= (((int64_t)1 << 30) + n_obs - 1) / n_obs;
 }
 
 // Bytes of the order's workspace region for n_obs points.

@@ -116,8 +116,8 @@ int hmx_forward_workspace_bytes(int64_t n_obs, int64_t n_sources, uint32_t field
  *             prism (gravity.py:239-269); that value is NaN.
  * Null prisms are NOT discarded here (the Python layer does it as
  * _discard_null_prisms, gravity.py:452-486, does).
- * Calls with at least 512 points and 2^24 (point, prism) pairs (2^28 beyond
- * 8192 points) evaluate the points in a wavefront-coherent strip order sorted
+ * Calls with at least 512 points and 2^24 (point, prism) pairs (beyond 8192
+ * points 2^28 pairs and 512 prisms) evaluate the points in a wavefront-coherent strip order sorted
  * into the workspace (also hmx_prism_layer_gravity and hmx_prism_magnetic);
  * out is in the caller's order either way. */
 int hmx_prism_gravity(const double *easting, const double *northing, const double *upward,

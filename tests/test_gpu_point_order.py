@@ -194,3 +194,36 @@ def test_sorted_with_nan_coordinates(hm, model):
         assert np.isnan(got[k][bad]).all()
         assert np.isfinite(got[k][~bad]).all()
         assert_close(got[k], ref[k], 1e-13)
+
+
+def test_many_points_over_few_prisms_are_not_sorted():
+    """Beyond 8192 points a call sorts from 512 prisms on: sorting costs as much
+    as a few hundred prisms.  Below, the workspace has no room for the order and
+    the call none of its launches."""
+    import ctypes
+
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from harmonica_amd import _lib
+    from harmonica_amd._forward import prism_fields_device
+
+    L, n = _lib.lib(), 1 << 20
+    sizes = []
+    for m in (511, 512):
+        b = ctypes.c_size_t(0)
+        _lib.check(L.hmx_forward_workspace_bytes(n, m, _lib.FIELD_BIT["g_z"], ctypes.byref(b)))
+        sizes.append(b.value)
+    assert sizes[1] - sizes[0] >= 3 * 8 * n  # the ordered coordinates at least
+    rng = np.random.default_rng(1)
+    w = rng.uniform(0, 3e4, (512, 2))
+    p = torch.as_tensor(np.column_stack([w[:, 0], w[:, 0] + 90, w[:, 1], w[:, 1] + 70,
+                                         np.full(512, -900.0), np.full(512, -100.0)])).cuda()
+    rho = torch.full((512,), 300.0, dtype=torch.float64).cuda()
+    c = [torch.as_tensor(v).cuda() for v in (*rng.uniform(0, 3e4, (2, n)), np.full(n, 50.0))]
+    rho[511] = 0.0
+    sorted_, plain = (prism_fields_device(*c, p[:m].contiguous(), rho[:m].contiguous(), ("g_z",))
+                      for m in (512, 511))
+    # every pair to 64 x 2^-53 of w r (the closed form's bound), r < 5e4
+    assert (sorted_ - plain).abs().max() <= 2 * 512 * 64 * 2.0**-53 * 1e5 * 6.6743e-11 * 300 * 5e4
