@@ -121,6 +121,32 @@ inline bool need_point_order(int64_t n_obs, int64_t n_src) {
            n_src >= (((int64_t)1 << 30) + n_obs - 1) / n_obs;
 }
 
+// Whether a call of many points in the caller's order takes the closed form for
+// every pair.  Over few prisms: one kernel with little to prepare, where the far form stages constants
+// for each workgroup and, but for g_z, runs a second kernel for the close pairs.
+// `sorted`: the points are in wavefront-coherent order.  Times per call (us, far
+// / closed), points scattered over 40 km, and as a raster:
+//                         scattered                      raster
+//   20,000 points, 16     g_z 23 / 18,    b 33 / 26      19 / 18,   28 / 27
+//   1e6, 1                g_z 42 / 24,    b 128 / 46     32 / 23,   83 / 38
+//   1e6, 7                g_z 98 / 85,    b 230 / 151    47 / 82,   134 / 114
+//   1e6, 16               g_z 176 / 180,  b 364 / 316    65 / 175,  204 / 234
+//   1e6, 32               g_zz 300 / 217, b 613 / 627    130 / 194, 321 / 444
+// The line depends on what the closed form costs, most with the potential or g_z
+// among the fields.  And g_ee, g_nn or g_en alone, whose closed form is the
+// cheapest and whose far form the dearest of a single field: 1e6 points, 256
+// prisms, g_ee 2.83 / 1.57 ms scattered and 1.43 / 1.39 as a raster.  Otherwise
+// the far form stays, for a tenth of the closed form's error and less: in calls
+// of fewer points, which it costs a few us (256 points, 3 prisms: 22 / 21), and
+// over more prisms also where scattered points mix far and close lanes (1e6
+// points, 256 prisms: g_zz 2.03 / 1.57 ms; as a raster 0.80 / 1.40).
+inline bool use_closed(uint32_t mask, int64_t n_obs, int64_t n_src, bool sorted) {
+    if (sorted || n_obs <= kSmallOrder) return false;
+    if (mask == HMX_G_EE || mask == HMX_G_NN || mask == HMX_G_EN) return true;
+    if (!(mask & (HMX_POTENTIAL | HMX_G_Z))) return n_src < 32;
+    return n_src < (n_obs > ((int64_t)1 << 17) ? 4 : 16);
+}
+
 // Bytes of the order's workspace region for n_obs points.
 size_t point_order_bytes(int64_t n_obs);
 

@@ -166,6 +166,26 @@ __global__ __launch_bounds__(dev::kGzThreads, 3) void magnetic_close_kernel(
     }
 }
 
+// Every pair by the closed form (use_closed says for which calls).
+template <unsigned C>
+__global__ __launch_bounds__(dev::kGzThreads) void magnetic_closed_kernel(
+    const double *__restrict__ oe, const double *__restrict__ on, const double *__restrict__ ou,
+    int n_obs, MagSource src, int64_t n_src, int64_t chunk_len, double *__restrict__ partial) {
+    using Op = MagneticOp<C>;
+    __shared__ dev::FieldClosedShared<Op> sh;
+    const int64_t base = (int64_t)blockIdx.x * dev::kGzThreads, i = base + threadIdx.x;
+    const int64_t c0 = (int64_t)blockIdx.y * chunk_len;
+    const int64_t c1 = c0 + chunk_len < n_src ? c0 + chunk_len : n_src;
+    double acc[Op::values] = {};
+    uint32_t flags = 0;
+    dev::field_closed_chunk<Op>(src, oe, on, ou, base, n_obs, c0, c1, acc, flags, sh);
+    if (i < n_obs) {
+#pragma unroll
+        for (int s = 0; s < Op::values; ++s)
+            partial[((int64_t)blockIdx.y * Op::values + s) * n_obs + i] = acc[s];
+    }
+}
+
 // out[s][perm[i]] = 1e9 * (sum over chunks in order of partial[c][s][i])
 // (T -> nT; perm NULL: the identity).
 template <int P>
@@ -188,10 +208,17 @@ __global__ void fill_zero_mag_kernel(double *__restrict__ out, int64_t n) {
 template <unsigned C>
 int launch_magnetic(const double *oe, const double *on, const double *ou, int64_t n_obs,
                     const double *prisms, const double *me, const double *mn, const double *mu,
-                    int64_t n_src, int64_t chunks, double *partial, hipStream_t stream) {
+                    int64_t n_src, int64_t chunks, bool sorted, double *partial,
+                    hipStream_t stream) {
     const int64_t chunk_len = (n_src + chunks - 1) / chunks;
     dim3 grid((unsigned)((n_obs + dev::kGzThreads - 1) / dev::kGzThreads), (unsigned)chunks);
     const MagSource src{prisms, me, mn, mu};
+    if (use_closed(MagSet<C>::tensor, n_obs, n_src, sorted)) {
+        hipLaunchKernelGGL((magnetic_closed_kernel<C>), grid, dim3(dev::kGzThreads), 0, stream, oe,
+                           on, ou, (int)n_obs, src, n_src, chunk_len, partial);
+        HMX_LAUNCHED("magnetic_closed_kernel");
+        return HMX_OK;
+    }
     hipLaunchKernelGGL((magnetic_far_kernel<C>), grid, dim3(dev::kGzThreads), 0, stream, oe, on, ou,
                        (int)n_obs, src, n_src, chunk_len, partial);
     HMX_LAUNCHED("magnetic_far_kernel");
@@ -301,7 +328,7 @@ int hmx_prism_magnetic(const double *easting, const double *northing, const doub
     case C:                                                                                   \
         rc = hmx::launch_magnetic<C>(easting, northing, upward, n_obs, prisms,                \
                                      magnetization_e, magnetization_n, magnetization_u,       \
-                                     n_prisms, chunks, partial, st);                          \
+                                     n_prisms, chunks, order, partial, st);                   \
         break;
         HMX_MAG_CASE(1u)
         HMX_MAG_CASE(2u)

@@ -122,6 +122,28 @@ prism_close_kernel(const double *__restrict__ oe, const double *__restrict__ on,
     if (FieldSet<M>::tensor && flags && found) atomicOr(flags, found);
 }
 
+// Every pair by the closed form (use_closed says for which calls).
+template <unsigned M, class Src>
+__global__ __launch_bounds__(dev::kGzThreads) void prism_closed_kernel(
+    const double *__restrict__ oe, const double *__restrict__ on, const double *__restrict__ ou,
+    int n_obs, Src src, int64_t n_src, int64_t chunk_len, double *__restrict__ partial,
+    uint32_t *__restrict__ flags) {
+    using Op = GravityOp<M>;
+    __shared__ dev::FieldClosedShared<Op> sh;
+    const int64_t base = (int64_t)blockIdx.x * dev::kGzThreads, i = base + threadIdx.x;
+    const int64_t c0 = (int64_t)blockIdx.y * chunk_len;
+    const int64_t c1 = c0 + chunk_len < n_src ? c0 + chunk_len : n_src;
+    double acc[Op::values] = {};
+    uint32_t found = 0;
+    dev::field_closed_chunk<Op>(src, oe, on, ou, base, n_obs, c0, c1, acc, found, sh);
+    if (i < n_obs) {
+#pragma unroll
+        for (int s = 0; s < Op::values; ++s)
+            partial[((int64_t)blockIdx.y * Op::values + s) * n_obs + i] = acc[s];
+    }
+    if (FieldSet<M>::tensor && flags && found) atomicOr(flags, found);
+}
+
 // g_u alone, each prism in the far form or the closed form (prism_far.h).
 template <class Src>
 __global__ __launch_bounds__(dev::kGzThreads, 4) void prism_gz_kernel(
@@ -226,10 +248,16 @@ __global__ void fill_zero_kernel(double *__restrict__ out, int64_t n) {
 
 template <unsigned M, class Src>
 int launch_forward(const double *oe, const double *on, const double *ou, int64_t n_obs,
-                   const Src &src, int64_t n_src, int64_t chunks, double *partial,
+                   const Src &src, int64_t n_src, int64_t chunks, bool sorted, double *partial,
                    uint32_t *flags, hipStream_t stream) {
     const int64_t chunk_len = (n_src + chunks - 1) / chunks;
     dim3 grid((unsigned)((n_obs + dev::kGzThreads - 1) / dev::kGzThreads), (unsigned)chunks);
+    if (use_closed(M, n_obs, n_src, sorted)) {
+        hipLaunchKernelGGL((prism_closed_kernel<M, Src>), grid, dim3(dev::kGzThreads), 0, stream,
+                           oe, on, ou, (int)n_obs, src, n_src, chunk_len, partial, flags);
+        HMX_LAUNCHED("prism_closed_kernel");
+        return HMX_OK;
+    }
     if constexpr (M == 0x8u) {
         hipLaunchKernelGGL((prism_gz_kernel<Src>), grid, dim3(dev::kGzThreads), 0, stream, oe, on,
                            ou, (int)n_obs, src, n_src, chunk_len, partial);
@@ -267,12 +295,12 @@ int launch_reduce(const double *partial, int64_t chunks, int nf, int64_t n_obs, 
 // three accelerations, the six tensor terms and all ten.
 template <class Src>
 int dispatch_mask(uint32_t mask, const double *oe, const double *on, const double *ou,
-                  int64_t n_obs, const Src &src, int64_t n_src, int64_t chunks, double *partial,
-                  uint32_t *flags, hipStream_t stream) {
+                  int64_t n_obs, const Src &src, int64_t n_src, int64_t chunks, bool sorted,
+                  double *partial, uint32_t *flags, hipStream_t stream) {
 #define HMX_CASE(MASK)                                                                          \
     case MASK:                                                                                  \
-        return launch_forward<MASK, Src>(oe, on, ou, n_obs, src, n_src, chunks, partial, flags, \
-                                         stream);
+        return launch_forward<MASK, Src>(oe, on, ou, n_obs, src, n_src, chunks, sorted, partial, \
+                                         flags, stream);
     switch (mask) {
         HMX_CASE(0x001u)
         HMX_CASE(0x002u)
@@ -345,8 +373,8 @@ int run_forward(const double *oe, const double *on, const double *ou, int64_t n_
         perm = po.perm;
     }
     if (has_kernel(mask)) {
-        int st = dispatch_mask<Src>(mask, oe, on, ou, n_obs, src, n_src, chunks, partial, flags,
-                                    stream);
+        int st = dispatch_mask<Src>(mask, oe, on, ou, n_obs, src, n_src, chunks, order, partial,
+                                    flags, stream);
         if (st) return st;
         return launch_reduce(partial, chunks, nf, n_obs, mask, perm, out, stream);
     }
@@ -354,8 +382,8 @@ int run_forward(const double *oe, const double *on, const double *ou, int64_t n_
     for (int f = 0; f < 10; ++f) {
         if (!((mask >> f) & 1u)) continue;
         uint32_t m = 1u << f;
-        int st = dispatch_mask<Src>(m, oe, on, ou, n_obs, src, n_src, chunks, partial, flags,
-                                    stream);
+        int st = dispatch_mask<Src>(m, oe, on, ou, n_obs, src, n_src, chunks, order, partial,
+                                    flags, stream);
         if (st) return st;
         st = launch_reduce(partial, chunks, 1, n_obs, m, perm, out + (int64_t)s * n_obs, stream);
         if (st) return st;

@@ -296,6 +296,11 @@ __device__ __forceinline__ double wave_uniform(double v) {
     return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
                             __builtin_amdgcn_readfirstlane(__double2loint(v)));
 }
+__device__ __forceinline__ uint64_t wave_uniform(unsigned long long v) {
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+    return (uint64_t)hi << 32 | lo;
+}
 template <int I>
 struct FarScalar {
     double c[far_base(I + 1)];

@@ -557,5 +557,60 @@ __device__ __forceinline__ bool field_close_chunk(const Src &src, const double *
     return any;
 }
 
+// LDS of a workgroup that evaluates every pair by the closed form.
+template <class Op>
+struct FieldClosedShared {
+    double bounds[64][6];
+    double weight[64][Op::weights];
+    unsigned long long live;
+    dm::Tables tables;
+};
+
+// All pairs of 256 points and the prisms [c0, c1) by the closed form, added to
+// acc: per wave first the prisms that no lane needs the general form for, then
+// the others, in two loops, which keep the forms' registers apart.
+template <class Op, class Src>
+__device__ __forceinline__ void field_closed_chunk(const Src &src, const double *__restrict__ oe,
+                                                   const double *__restrict__ on,
+                                                   const double *__restrict__ ou, int64_t base,
+                                                   int64_t n_obs, int64_t c0, int64_t c1,
+                                                   double (&acc)[Op::values], uint32_t &flags,
+                                                   FieldClosedShared<Op> &sh) {
+    dm::load_tables(&sh.tables);
+    const int64_t i = base + threadIdx.x, ii = i < n_obs ? i : n_obs - 1;
+    const double e = oe[ii], n = on[ii], u = ou[ii];
+    for (int64_t t0 = c0; t0 < c1; t0 += 64) {
+        __syncthreads();
+        if (threadIdx.x < 64) {
+            const int q = threadIdx.x;
+            double b[6], weight[Op::weights];
+            bool skip = true;
+            if (t0 + q < c1) {
+                skip = src.get(t0 + q, b, weight);
+#pragma unroll
+                for (int k = 0; k < 6; ++k) sh.bounds[q][k] = b[k];
+#pragma unroll
+                for (int k = 0; k < Op::weights; ++k) sh.weight[q][k] = weight[k];
+            }
+            const uint64_t live = __ballot(!skip);
+            if (q == 0) sh.live = live;
+        }
+        __syncthreads();
+        const uint64_t live = wave_uniform(sh.live);
+        uint64_t general = 0;
+        for_bits(live, [&](int p) {
+            const double *t = sh.bounds[p];
+            if (any_lane(needs_general<Op::fields>(e, n, u, t[0], t[1], t[2], t[3], t[4], t[5]))) {
+                general |= 1ull << p;
+                return;
+            }
+            Op::template closed<false>(e, n, u, t, sh.weight[p], acc, flags, sh.tables);
+        });
+        for_bits(general, [&](int p) {
+            Op::template closed<true>(e, n, u, sh.bounds[p], sh.weight[p], acc, flags, sh.tables);
+        });
+    }
+}
+
 }  // namespace dev
 }  // namespace hmx

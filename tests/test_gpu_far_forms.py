@@ -546,3 +546,75 @@ def test_more_outputs_than_a_launch_has_threads(hm):
     for start in (0, k, (n // k - 1) * k):
         assert (many[:, start:start + k] - few).abs().max() <= tolerance
     assert (many[:, (n // k) * k:] - few[:, :n % k]).abs().max() <= tolerance
+
+
+@pytest.mark.parametrize("n,m", [(8192, 8), (8193, 16), (8193, 31), (8193, 32), (131072, 15),
+                                 (131073, 3), (131073, 4)])
+def test_few_prisms(hm, n, m):
+    """Calls on both sides of the lines below which every pair takes the closed
+    form (beyond 8192 points: 32 prisms, with the potential or g_z 16, and 4
+    beyond 131,072 points; g_ee, g_nn and g_en alone at any number), explicit prisms, a layer and the magnetic field, to
+    the closed form's bound."""
+    import torch
+
+    from harmonica_amd._forward import layer_fields_device, prism_fields_device, to_device
+    from harmonica_amd._magnetic import magnetic_fields_device
+
+    rng = np.random.default_rng(n + m)
+    prisms = _model("different", m, rng)
+    rho = rng.uniform(100, 500, m)
+    coords = [rng.uniform(-3e3, 6e3, n), rng.uniform(-3e3, 6e3, n), rng.uniform(5.0, 900.0, n)]
+    pick = np.unique(np.r_[0, n - 1, rng.integers(0, n, 250)])
+    some = [c[pick] for c in coords]
+    exact = _fields_exact(some, prisms, G * rho)
+    dev, P, D = [to_device(c) for c in coords], to_device(prisms), to_device(rho)
+    index = torch.as_tensor(pick).cuda()
+    for fields in (*((f,) for f in TEN), TEN[1:4], TEN[4:], TEN, ("g_z", "g_zz")):
+        got = prism_fields_device(*dev, P, D, fields)[:, index].cpu().numpy()
+        for f, row in zip(fields, got):
+            value, bound = exact[f]
+            assert (np.abs(row / _UNIT[f] - value) <= bound).all(), (f, len(fields))
+    mag = [rng.normal(size=m) for _ in range(3)]
+    terms = {"b_e": ("g_ee", "g_en", "g_ez"), "b_n": ("g_en", "g_nn", "g_nz"),
+             "b_u": ("g_ez", "g_nz", "g_zz")}
+    got = magnetic_fields_device(*dev, P, *(to_device(x) for x in mag), tuple(terms))
+    for row, (name, fields) in zip(got[:, index].cpu().numpy() / 100.0, terms.items()):
+        parts = [_fields_exact(some, prisms, w)[f] for w, f in zip(mag, fields)]
+        value, bound = (sum(p[q] for p in parts) for q in (0, 1))
+        assert (np.abs(row - value) <= bound).all(), name
+    # a layer of 2 x 3 cells, one of them left out
+    e, nn = np.array([0.0, 200.0]), np.array([0.0, 150.0, 300.0])
+    top = rng.uniform(-300, -10, (3, 2))
+    density = rng.uniform(100, 500, (3, 2))
+    density[1, 0] = np.nan
+    cells = np.array([[x - 100, x + 100, y - 75, y + 75, -900.0, top[j, i]]
+                      for i, x in enumerate(e) for j, y in enumerate(nn) if (j, i) != (1, 0)])
+    weights = np.array([density[j, i] for i in range(2) for j in range(3) if (j, i) != (1, 0)])
+    got = layer_fields_device(*dev, to_device(e), to_device(nn), to_device(np.full((3, 2), -900.0)),
+                              to_device(top), to_device(density), TEN)[:, index].cpu().numpy()
+    for f, row in zip(TEN, got):
+        value, bound = _fields_exact(some, cells, G * weights)[f]
+        assert (np.abs(row / _UNIT[f] - value) <= bound).all(), f
+
+
+def test_few_prisms_at_their_edges(hm):
+    """Singular points and points on faces in a call that takes the closed
+    form: NaN exactly for the fields that are singular there, and the flags."""
+    k = 2500  # 10,000 points
+    import torch
+
+    from harmonica_amd._forward import prism_fields_device, to_device
+
+    prism = np.array([[0.0, 100.0, 0.0, 80.0, -150.0, -50.0]])
+    # on an easting-parallel edge, a northing-parallel one, an upward one, a face
+    coords = [np.tile(c, k) for c in ([50.0, 0.0, 100.0, 50.0], [0.0, 40.0, 80.0, 40.0],
+                                      [-50.0, -50.0, -100.0, -50.0])]
+    flags = torch.zeros(1, dtype=torch.int32).cuda()
+    got = prism_fields_device(*(to_device(c) for c in coords), to_device(prism),
+                              to_device(np.ones(1)), TEN, flags=flags).cpu().numpy()
+    nan = np.isnan(got)
+    expected = {"g_ee": (0, 1, 1, 0), "g_nn": (1, 0, 1, 0), "g_zz": (1, 1, 0, 0),
+                "g_en": (0, 0, 1, 0), "g_ez": (0, 1, 0, 0), "g_nz": (1, 0, 0, 0)}
+    for f, row in zip(TEN, nan):
+        assert (row.reshape(k, 4) == np.array(expected.get(f, (0, 0, 0, 0)), bool)).all(), f
+    assert int(flags.item()) == 0x3f0
