@@ -56,6 +56,8 @@ struct FarNeeds {
     static constexpr bool phi = F::gu || phi1;
     static constexpr bool kx = F::ge || F::ee || F::en || F::eu;
     static constexpr bool ky = F::gn || nn_direct || F::en || F::nu;
+    // logarithms along horizontal edges without a coefficient (on_edge_line)
+    static constexpr bool edges = F::eu || F::nu;
     // Highest order 2I.  317 x 290 cells, ten fields at 13,320 points: up to
     // order 6 19.4 ms (close pairs 6.5), up to order 8 14.4 ms (1.9).
     static constexpr int orders = lambda ? 4 : 5;
@@ -246,15 +248,45 @@ __device__ __forceinline__ void far_fields(double x, double y, double zt, double
     if constexpr (F::nn && !Q::nn_direct) vs[F::slot(5)] = -(vs[F::slot(4)] + vs[F::slot(6)]);
 }
 
-// Whether the far form of the highest order serves the lane's own point
-// (unsure: far_unsure of the wave's box).
+// Horizontal bounds W, E, S, N of a prism from the workgroup's origin, rounded
+// as the points are.
+struct FarEdges {
+    double w, e, s, n;
+    __device__ __forceinline__ FarEdges() = default;
+    __device__ __forceinline__ FarEdges(const double (&b)[6], const GzPoint &pt)
+        : w(b[0] - pt.xo), e(b[1] - pt.xo), s(b[2] - pt.yo), n(b[3] - pt.yo) {}
+};
+
+// Whether a point of the box may lie on the line of a horizontal edge of the
+// prism, level with its top or bottom and in one of its vertical planes.
+// There the logarithm along the edge, of ln(x + r) for x < 0, has the argument
+// 0 and counts as 0 (the convention of the closed form, prism_device.h), in
+// g_ez along northing and in g_nz along easting: by that, and not by the
+// field's limit, which the far form gives, they take the closed form.
 template <unsigned M>
-__device__ __forceinline__ bool field_lane_far(const FarPrism &p, bool unsure, const GzPoint &pt) {
+__device__ __forceinline__ bool near_edge_line(const FarBox &b, const FarPrism &p,
+                                               const FarEdges &g) {
+    auto in = [](double v, double lo, double hi) { return lo <= v && v <= hi; };
+    const bool level = in(p.t, b.u0, b.u1) || in(p.b, b.u0, b.u1);
+    const bool x = FieldSet<M>::eu && (in(g.w, b.x0, b.x1) || in(g.e, b.x0, b.x1));
+    const bool y = FieldSet<M>::nu && (in(g.s, b.y0, b.y1) || in(g.n, b.y0, b.y1));
+    return level && (x || y);
+}
+
+// Whether the far form of the highest order serves the lane's own point
+// (special: far_unsure or near_edge_line of the wave's box; of the latter's
+// prisms, all points level with the top or bottom are left to the closed form).
+template <unsigned M>
+__device__ __forceinline__ bool field_lane_far(const FarPrism &p, bool special,
+                                               const GzPoint &pt) {
 #pragma clang fp contract(off)
     const double x = p.x - pt.x, y = p.y - pt.y, t = p.t - pt.u, z = p.b - pt.u;
     const double s = fma(x, x, y * y), d2 = s + fmin(t * t, z * z);
     bool far = far_enough<FarNeeds<M>::orders>(d2, p.h2);
-    if (unsure) far = far && far_resolved(d2, p.h2, fma(pt.x, pt.x, pt.y * pt.y));
+    if (special) {
+        far = far && far_resolved(d2, p.h2, fma(pt.x, pt.x, pt.y * pt.y));
+        if constexpr (FarNeeds<M>::edges) far = far && t != 0.0 && z != 0.0;
+    }
     if constexpr (FarNeeds<M>::lambda)
         return far && s >= 4.0 * p.h2 && (fmax(t, z) <= 0.0 || fmin(t, z) >= 0.0);
     return far;
@@ -286,6 +318,7 @@ struct FieldFarShared {
     // constants per prism, if the rectangles differ; the last entry holds
     // those of the workgroup's first prism
     alignas(16) double consts[(kGzTile + 1) * Q::stride];
+    FarEdges edges[Q::edges ? kGzTile : 1];
     FarBox box[kGzWaves];
     double A, B;
     unsigned live, different;
@@ -367,6 +400,7 @@ __device__ __forceinline__ void field_far_chunk(const Src &src, const double *__
             half_sides2(b, A, B);
             if (q < cnt) {
                 sh.far[q] = far_prism(b, pt.xo, pt.yo, 1.0);
+                if constexpr (Q::edges) sh.edges[q] = FarEdges(b, pt);
 #pragma unroll
                 for (int k = 0; k < Op::weights; ++k) sh.weight[q][k] = weight[k];
             }
@@ -394,7 +428,13 @@ __device__ __forceinline__ void field_far_chunk(const Src &src, const double *__
         const int q = threadIdx.x & 63;
         const FarPrism mine = sh.far[q < cnt ? q : 0];
         const FarBox &box = sh.box[threadIdx.x >> 6];
-        const double d2 = far_distance2(box, mine);
+        double d2 = far_distance2(box, mine);
+        bool special = far_unsure(box, mine.h2);
+        if constexpr (Q::edges)
+            if (near_edge_line<M>(box, mine, sh.edges[q < cnt ? q : 0])) {
+                special = true;
+                d2 = -1.0;
+            }
         unsigned rest = live;
         auto take = [&](bool far) {
             const unsigned m = (unsigned)__ballot(far) & rest;
@@ -410,9 +450,9 @@ __device__ __forceinline__ void field_far_chunk(const Src &src, const double *__
         if constexpr (Q::orders >= 5)
             field_far<5>(sh, different, take(field_box_far<5, M>(d2, mine, box)), pt, acc);
         // prisms that are far from some of the wave's points only
-        const unsigned unsure = (unsigned)__ballot(far_unsure(box, mine.h2));
+        const unsigned specials = (unsigned)__ballot(special);
         for_bits(rest, [&](int p) {
-            const bool far = field_lane_far<M>(sh.far[p], (unsure >> p) & 1u, pt);
+            const bool far = field_lane_far<M>(sh.far[p], (specials >> p) & 1u, pt);
             if (!any_lane(far)) return;
             double v[Op::values] = {};
             field_far<Q::orders>(sh, different, 1u << p, pt, v);
@@ -518,9 +558,12 @@ __device__ __forceinline__ bool field_close_chunk(const Src &src, const double *
     if (c0 + q < c1) skip = src.get(c0 + q, b, weight);
     for (int64_t t0 = c0; t0 < c1; t0 += 64) {
         const FarPrism rec = far_prism(b, pt.xo, pt.yo, 1.0);
-        const uint64_t near = __ballot(
-            !skip && !field_box_far<Q::orders, M>(far_distance2(box, rec), rec, box));
-        const uint64_t unsure = __ballot(far_unsure(box, rec.h2));
+        bool edge_line = false;
+        if constexpr (Q::edges) edge_line = near_edge_line<M>(box, rec, FarEdges(b, pt));
+        const uint64_t near =
+            __ballot(!skip && (edge_line || !field_box_far<Q::orders, M>(far_distance2(box, rec),
+                                                                         rec, box)));
+        const uint64_t specials = __ballot(edge_line || far_unsure(box, rec.h2));
         if (near) {
             sh.far[q] = rec;
 #pragma unroll
@@ -535,7 +578,7 @@ __device__ __forceinline__ bool field_close_chunk(const Src &src, const double *
         wave_sync();
         uint64_t mask = 0;
         for_bits(near, [&](int p) {
-            const bool close = !field_lane_far<M>(sh.far[p], (unsure >> p) & 1u, pt);
+            const bool close = !field_lane_far<M>(sh.far[p], (specials >> p) & 1u, pt);
             const double *t = sh.bounds[p];
             const bool lean = close && !needs_general<M>(pt.e, pt.n, pt.u, t[0], t[1], t[2], t[3],
                                                          t[4], t[5]);

@@ -618,3 +618,49 @@ def test_few_prisms_at_their_edges(hm):
     for f, row in zip(TEN, nan):
         assert (row.reshape(k, 4) == np.array(expected.get(f, (0, 0, 0, 0)), bool)).all(), f
     assert int(flags.item()) == 0x3f0
+
+
+@pytest.mark.parametrize("others", [0, 50])
+def test_points_on_the_lines_of_edges(hm, others):
+    """Points exactly on the lines of a prism's edges, from its corners to 10,000
+    half-diagonals away: where an edge points away from them, ln(x + r) along
+    it has the argument 0 and counts as 0, as in the oracle.  Alone, and as
+    some points of waves that lie elsewhere; over one prism, and over others
+    around it.  To 64 roundings of the oracle's terms, logarithms below 32 in
+    magnitude and angles, in sum over all pairs."""
+    import oracle
+
+    rng = np.random.default_rng(others)
+    prisms = np.vstack([[[0.0, 100.0, 0.0, 80.0, -150.0, -50.0]],
+                        _model("different", max(others, 1), rng)[:others]])
+    prisms[1:, 4:] -= 500.0
+    density = rng.uniform(100, 500, len(prisms))
+    d = np.geomspace(30.0, 6e5, 40)
+    lines = []
+    for low, high, axis in ((0, 100, 0), (0, 80, 1), (-150, -50, 2)):
+        along = np.r_[high + d, low - d]
+        corners = [c for a, c in enumerate(((0.0, 100.0), (0.0, 80.0), (-150.0, -50.0))) if a != axis]
+        for first in corners[0]:
+            for second in corners[1]:
+                rest = [np.full(80, first), np.full(80, second)]
+                rest.insert(axis, along)
+                lines.append(np.array(rest))
+    lines = np.concatenate(lines, axis=1)
+    k = lines.shape[1]
+    elsewhere = np.array([rng.uniform(-3e3, 3e3, k), rng.uniform(-3e3, 3e3, k),
+                          rng.uniform(-50.0, 900.0, k)])
+    mixed = np.concatenate([lines, elsewhere], axis=1)[:, rng.permutation(2 * k)]
+    ulp = 64 * 2.0**-53 * 8 * 32
+    for coords in (lines, mixed):
+        expected = {f: oracle.prism_gravity(tuple(coords), prisms, density, f) for f in TEN[4:]}
+        for chosen in (*((f,) for f in TEN[4:]), TEN[4:], TEN):
+            rows = _device_fields(coords, prisms, density, chosen)
+            for f, row in zip(chosen, rows):
+                if f in expected:
+                    error = np.abs(row - expected[f]).max()
+                    assert error <= ulp * G * 1e9 * density.sum(), (f, len(chosen))
+        mag = tuple(rng.normal(size=len(prisms)) for _ in range(3))
+        for f in ("b_e", "b_n", "b_u"):
+            error = np.abs(hm.prism_magnetic(tuple(coords), prisms, mag, f)
+                           - oracle.prism_magnetic(tuple(coords), prisms, mag, f)).max()
+            assert error <= ulp * 100.0 * np.abs(mag).sum(), f
