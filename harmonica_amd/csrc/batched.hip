@@ -55,10 +55,12 @@ __global__ __launch_bounds__(dev::kGzThreads, 4) void batched_gz_kernel(
         if (p0 < p1) dev::gz_table(src, p0, sh);
         dev::point_box(pt, sh.box);
         double acc = 0.0;
+        bool sure = false;
         for (int64_t t0 = p0; t0 < p1; t0 += dev::kGzTile) {
             const int cnt = (int)(p1 - t0 < dev::kGzTile ? p1 - t0 : dev::kGzTile);
             dev::gz_stage(src, t0, cnt, pt.xo, pt.yo, sh);
-            dev::gz_tile(cnt, pt, acc, sh);
+            if (t0 == p0) sure = dev::gz_sure(sh);
+            dev::gz_tile(cnt, sure, pt, acc, sh);
         }
         partial[slot * kObsPerBlock + local] = i < end ? acc : 0.0;
     }

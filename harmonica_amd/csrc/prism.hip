@@ -162,6 +162,7 @@ __global__ __launch_bounds__(dev::kGzThreads, 4) void prism_gz_kernel(
     pt.x = pt.e - pt.xo;
     pt.y = pt.n - pt.yo;
     double acc = 0.0;
+    bool sure = false;
     const int64_t c0 = (int64_t)blockIdx.y * chunk_len;
     const int64_t c1 = c0 + chunk_len < n_src ? c0 + chunk_len : n_src;
     if (c0 < c1) dev::gz_table(src, c0, sh);
@@ -169,7 +170,8 @@ __global__ __launch_bounds__(dev::kGzThreads, 4) void prism_gz_kernel(
     for (int64_t t0 = c0; t0 < c1; t0 += dev::kGzTile) {
         const int cnt = (int)(c1 - t0 < dev::kGzTile ? c1 - t0 : dev::kGzTile);
         dev::gz_stage(src, t0, cnt, pt.xo, pt.yo, sh);
-        dev::gz_tile(cnt, pt, acc, sh);
+        if (t0 == c0) sure = dev::gz_sure(sh);
+        dev::gz_tile(cnt, sure, pt, acc, sh);
     }
     if (valid) partial[(int64_t)blockIdx.y * n_obs + i] = acc;
 }

@@ -334,17 +334,45 @@ struct FarBox {
 // Point and prism round to about 2^-53 of their distance R from it, 2 R / r
 // roundings of the distance r between them; the closed form, which takes their
 // difference from the coordinates as given, is off by 4 to 16 (r/h)^2
-// roundings.  So points of a workgroup may be spread widely (r^3 >= 4 R h^2: R
-// up to 170 h at the shortest r, 8.8 h), but one that lies a continent away, or
-// at a placeholder's 1e20 m, does not spoil the others.
+// roundings.  So points of a workgroup may be spread widely (2 R / r <= 4
+// (r/h)^2: R up to 1360 h at the shortest r, 8.8 h), but one that lies a
+// continent away, or at a placeholder's 1e20 m, does not spoil the others.
 __device__ __forceinline__ bool far_resolved(double d2, double h2, double reach2) {
 #pragma clang fp contract(off)
-    return d2 * d2 * d2 >= 16.0 * reach2 * (h2 * h2);
+    return d2 * d2 * d2 >= 0.25 * reach2 * (h2 * h2);
+}
+
+// Whether far_resolved can fail at the distances of the far form, 8.8 h and
+// more.  Asked once per wave and prism: in all lanes' own tests far_resolved
+// cost 1 to 4% of calls with many near prisms.
+__device__ __forceinline__ bool far_unsure(double h2, double reach2) {
+#pragma clang fp contract(off)
+    return !(reach2 <= 1.85e6 * h2);
+}
+
+// The same rule as a larger h2: order 2I and lower ones by it start where
+// far_resolved holds.  For kernels that have no registers for a test beside the
+// distance's: the six tensor fields' and ten fields' close pairs took 13% longer
+// with one.  By FP32 logarithm and exponential, 1e-4 on the far side.
+__device__ __forceinline__ float far_reach(double reach2) {  // log2(R^2 / 4)
+    return __builtin_amdgcn_logf((float)reach2) - 2.0f;
+}
+template <int I>
+__device__ __forceinline__ double far_sure_half2(double h2, float reach) {
+    const float log_h2 = __builtin_amdgcn_logf((float)h2);
+    const float log_r2 = fmaf(2.0f, log_h2, reach) * (1.0f / 3.0f);
+    const double least = (double)__builtin_amdgcn_exp2f(log_r2) * (1.0001 / far_ratio2(I));
+    return h2 < least ? least : h2;
+}
+
+// A lane's value, the same for all lanes (lane uniform in the wave).
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
 }
 
 // Smallest squared distance from the box to the nearer face centre of a
-// staged prism; -1 (never far) if the coordinates do not resolve it, NaN
-// (neither) if the prism or the whole box is NaN.  (No
+// staged prism; NaN (never far) if the prism or the whole box is NaN.  (No
 // contraction here and below: kernels that share the work of a pair have to
 // come to the same decision.)
 __device__ __forceinline__ double far_distance2(const FarBox &b, const FarPrism &p) {
@@ -356,8 +384,7 @@ __device__ __forceinline__ double far_distance2(const FarBox &b, const FarPrism 
     const double dt = fmax(fmax(b.u0 - p.t, p.t - b.u1), 0.0);
     const double db = fmax(fmax(b.u0 - p.b, p.b - b.u1), 0.0);
     const double d = fmin(dt, db);
-    const double d2 = fma(dx, dx, fma(dy, dy, d * d)) + nan_guard;
-    return far_resolved(d2, p.h2, b.reach2) ? d2 : -1.0;
+    return fma(dx, dx, fma(dy, dy, d * d)) + nan_guard;
 }
 
 // Whether order 2I serves a prism at squared distance d2 (see far_half2 on the
@@ -543,24 +570,11 @@ __device__ __forceinline__ void gz_stage(const Src &src, int64_t t0, int cnt, do
     }
 }
 
-// Whether a prism is small enough next to a wave's reach that far_resolved
-// can fail at the distances of the far form, 8.8 h and more.  Asked once per
-// wave and prism: in the lanes' own tests far_resolved cost 1 to 2% of calls
-// with many near prisms.
-__device__ __forceinline__ bool far_unsure(const FarBox &b, double h2) {
-#pragma clang fp contract(off)
-    return !(b.reach2 <= 29000.0 * h2);
-}
-
-// Whether order 2 kFarMax serves the lane's own point (unsure: uniform in the
-// wave).
-__device__ __forceinline__ bool lane_is_far(const FarPrism &p, bool unsure, double px, double py,
-                                            double pu) {
+// Squared distance of the lane's own point from the nearer face centre.
+__device__ __forceinline__ double lane_distance2(const FarPrism &p, double px, double py,
+                                                 double pu) {
     const double x = p.x - px, y = p.y - py, t = p.t - pu, z = p.b - pu;
-    const double d2 = fma(x, x, fma(y, y, fmin(t * t, z * z)));
-    bool far = far_enough<kFarMax>(d2, p.h2);
-    if (unsure) far = far && far_resolved(d2, p.h2, fma(px, px, py * py));
-    return far;
+    return fma(x, x, fma(y, y, fmin(t * t, z * z)));
 }
 
 // Calls f(p) for the set bits p of a wave-uniform mask, in order.
@@ -644,10 +658,19 @@ constexpr int kGzInline = 40;
 // their order.
 __device__ __forceinline__ void gz_near(GzShared &sh, unsigned near, unsigned unsure,
                                         unsigned different, const GzPoint &pt, double &acc) {
-    unsigned mask = 0;
+    // the lane's pairs that its offset from the origin does not resolve
+    unsigned mask = 0, coarse = 0;
+    for_bits(near & unsure, [&](int p) {
+        const double d2 = lane_distance2(sh.far[p], pt.x, pt.y, pt.u);
+        double px = pt.x, py = pt.y;  // their squares only here, not held in registers
+        asm volatile("" : "+v"(px), "+v"(py));
+        const bool fine = far_resolved(d2, sh.far[p].h2, fma(px, px, py * py));
+        coarse |= fine ? 0u : 1u << p;
+    });
     for_bits(near, [&](int p) {
         const FarPrism rec = sh.far[p];
-        const bool close = !lane_is_far(rec, (unsure >> p) & 1u, pt.x, pt.y, pt.u);
+        const double d2 = lane_distance2(rec, pt.x, pt.y, pt.u);
+        const bool close = !far_enough<kFarMax>(d2, rec.h2) || ((coarse >> p) & 1u);
         if (any_lane(!close)) {
             const double v =
                 far_gz<kFarMax>(rec, FarLds{gz_consts(sh.consts, p, different)}, pt.x, pt.y, pt.u);
@@ -687,18 +710,30 @@ __device__ __forceinline__ void gz_far(const GzShared &sh, unsigned different, u
     });
 }
 
-// Adds the g_u of the staged tile at the wave's points.  The forms are chosen
+// Whether no prism like the chunk's first one is unsure for the wave (uniform;
+// after the first gz_stage).  Per prism of every tile this cost 1% of a model of
+// 1,000,000 prisms.
+__device__ __forceinline__ bool gz_sure(const GzShared &sh) {
+    return !any_lane(far_unsure(0.999 * (sh.A + sh.B), sh.box[threadIdx.x >> 6].reach2));
+}
+
+// Adds the g_u of the staged tile at the wave's points (sure: gz_sure).  The forms are chosen
 // per prism and wave from the distance between the prism's face centres and
 // the bounding box of the wave's points: the lowest order that serves all of
 // them, uniform in the wave; then the prisms nearer than that, lane by lane.
-__device__ __forceinline__ void gz_tile(int cnt, const GzPoint &pt, double &acc, GzShared &sh) {
+__device__ __forceinline__ void gz_tile(int cnt, bool sure, const GzPoint &pt, double &acc,
+                                        GzShared &sh) {
     const int q = threadIdx.x & 63;
     const unsigned live = __builtin_amdgcn_readfirstlane(sh.live);
     const unsigned different = __builtin_amdgcn_readfirstlane(sh.different);
     const FarPrism mine = sh.far[q < cnt ? q : 0];
     const FarBox &box = sh.box[threadIdx.x >> 6];
-    const double d2 = far_distance2(box, mine);
-    const unsigned unsure = (unsigned)__ballot(far_unsure(box, mine.h2));
+    double d2 = far_distance2(box, mine);
+    unsigned unsure = 0;
+    if (different || !sure) {
+        unsure = (unsigned)__ballot(far_unsure(mine.h2, box.reach2));
+        if (unsure && !far_resolved(d2, mine.h2, box.reach2)) d2 = -1.0;
+    }
     unsigned rest = live;
     auto take = [&](bool far) {
         const unsigned m = (unsigned)__ballot(far) & rest;

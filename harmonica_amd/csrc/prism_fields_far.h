@@ -248,62 +248,53 @@ __device__ __forceinline__ void far_fields(double x, double y, double zt, double
     if constexpr (F::nn && !Q::nn_direct) vs[F::slot(5)] = -(vs[F::slot(4)] + vs[F::slot(6)]);
 }
 
-// Horizontal bounds W, E, S, N of a prism from the workgroup's origin, rounded
-// as the points are.
-struct FarEdges {
-    double w, e, s, n;
-    __device__ __forceinline__ FarEdges() = default;
-    __device__ __forceinline__ FarEdges(const double (&b)[6], const GzPoint &pt)
-        : w(b[0] - pt.xo), e(b[1] - pt.xo), s(b[2] - pt.yo), n(b[3] - pt.yo) {}
-};
-
-// Whether a point of the box may lie on the line of a horizontal edge of the
-// prism, level with its top or bottom and in one of its vertical planes.
-// There the logarithm along the edge, of ln(x + r) for x < 0, has the argument
-// 0 and counts as 0 (the convention of the closed form, prism_device.h), in
-// g_ez along northing and in g_nz along easting: by that, and not by the
-// field's limit, which the far form gives, they take the closed form.
-template <unsigned M>
-__device__ __forceinline__ bool near_edge_line(const FarBox &b, const FarPrism &p,
-                                               const FarEdges &g) {
-    auto in = [](double v, double lo, double hi) { return lo <= v && v <= hi; };
-    const bool level = in(p.t, b.u0, b.u1) || in(p.b, b.u0, b.u1);
-    const bool x = FieldSet<M>::eu && (in(g.w, b.x0, b.x1) || in(g.e, b.x0, b.x1));
-    const bool y = FieldSet<M>::nu && (in(g.s, b.y0, b.y1) || in(g.n, b.y0, b.y1));
-    return level && (x || y);
+// The staged record of a prism per unit weight; one with its bottom above its
+// top as the prism between them, of the opposite sign (point above or below
+// both is asked by these heights).
+__device__ __forceinline__ FarPrism field_prism(const double (&b)[6], const GzPoint &pt) {
+    FarPrism p = far_prism(b, pt.xo, pt.yo, 1.0);
+    if (p.t < p.b) p = FarPrism{p.x, p.y, p.b, p.t, -p.w, p.h2};
+    return p;
 }
 
-// Whether the far form of the highest order serves the lane's own point
-// (special: far_unsure or near_edge_line of the wave's box; of the latter's
-// prisms, all points level with the top or bottom are left to the closed form).
+// Points level with a prism's top or bottom: where such a point lies on the line
+// of a horizontal edge, the logarithm along the edge, of ln(x + r) for x < 0,
+// has the argument 0 and counts as 0 (the convention of the closed form,
+// prism_device.h), in g_ez along northing and in g_nz along easting.  By that,
+// and not by the field's limit, which the far form gives, field sets with these
+// two leave level points to the closed form.
+
+// Whether the far form of the highest order serves the lane's own point (h2:
+// far_sure_half2).
 template <unsigned M>
-__device__ __forceinline__ bool field_lane_far(const FarPrism &p, bool special,
-                                               const GzPoint &pt) {
+__device__ __forceinline__ bool field_lane_far(const FarPrism &p, double h2, const GzPoint &pt) {
 #pragma clang fp contract(off)
     const double x = p.x - pt.x, y = p.y - pt.y, t = p.t - pt.u, z = p.b - pt.u;
     const double s = fma(x, x, y * y), d2 = s + fmin(t * t, z * z);
-    bool far = far_enough<FarNeeds<M>::orders>(d2, p.h2);
-    if (special) {
-        far = far && far_resolved(d2, p.h2, fma(pt.x, pt.x, pt.y * pt.y));
-        if constexpr (FarNeeds<M>::edges) far = far && t != 0.0 && z != 0.0;
+    const bool far = far_enough<FarNeeds<M>::orders>(d2, h2);
+    if constexpr (FarNeeds<M>::lambda) {
+        const bool outside = FarNeeds<M>::edges ? t < 0.0 || z > 0.0 : t <= 0.0 || z >= 0.0;
+        return far && s >= 4.0 * h2 && outside;
     }
-    if constexpr (FarNeeds<M>::lambda)
-        return far && s >= 4.0 * p.h2 && (fmax(t, z) <= 0.0 || fmin(t, z) >= 0.0);
-    return far;
+    return FarNeeds<M>::edges ? far && t != 0.0 && z != 0.0 : far;
 }
 
 // Whether order 2I serves every point in the box.
 template <int I, unsigned M>
-__device__ __forceinline__ bool field_box_far(double d2, const FarPrism &p, const FarBox &b) {
+__device__ __forceinline__ bool field_box_far(double d2, double h2, const FarPrism &p,
+                                              const FarBox &b) {
 #pragma clang fp contract(off)
     if constexpr (FarNeeds<M>::lambda) {
         const double dx = fmax(fmax(b.x0 - p.x, p.x - b.x1), 0.0);
         const double dy = fmax(fmax(b.y0 - p.y, p.y - b.y1), 0.0);
-        if (!(fma(dx, dx, dy * dy) >= 4.0 * p.h2 &&
-              (fmax(p.t, p.b) <= b.u0 || fmin(p.t, p.b) >= b.u1)))
-            return false;
+        const bool outside = FarNeeds<M>::edges ? p.t < b.u0 || p.b > b.u1
+                                                : p.t <= b.u0 || p.b >= b.u1;
+        if (!(fma(dx, dx, dy * dy) >= 4.0 * h2 && outside)) return false;
+    } else if constexpr (FarNeeds<M>::edges) {
+        const bool level = (b.u0 <= p.t && p.t <= b.u1) || (b.u0 <= p.b && p.b <= b.u1);
+        if (level) return false;
     }
-    return far_enough<I>(d2, p.h2);
+    return far_enough<I>(d2, h2);
 }
 
 // What a call sums: Op::fields the field set, Op::weights per prism, Op::values
@@ -318,7 +309,6 @@ struct FieldFarShared {
     // constants per prism, if the rectangles differ; the last entry holds
     // those of the workgroup's first prism
     alignas(16) double consts[(kGzTile + 1) * Q::stride];
-    FarEdges edges[Q::edges ? kGzTile : 1];
     FarBox box[kGzWaves];
     double A, B;
     unsigned live, different;
@@ -399,8 +389,7 @@ __device__ __forceinline__ void field_far_chunk(const Src &src, const double *__
             if (q < cnt) skip = src.get(t0 + q, b, weight);
             half_sides2(b, A, B);
             if (q < cnt) {
-                sh.far[q] = far_prism(b, pt.xo, pt.yo, 1.0);
-                if constexpr (Q::edges) sh.edges[q] = FarEdges(b, pt);
+                sh.far[q] = field_prism(b, pt);
 #pragma unroll
                 for (int k = 0; k < Op::weights; ++k) sh.weight[q][k] = weight[k];
             }
@@ -428,31 +417,25 @@ __device__ __forceinline__ void field_far_chunk(const Src &src, const double *__
         const int q = threadIdx.x & 63;
         const FarPrism mine = sh.far[q < cnt ? q : 0];
         const FarBox &box = sh.box[threadIdx.x >> 6];
-        double d2 = far_distance2(box, mine);
-        bool special = far_unsure(box, mine.h2);
-        if constexpr (Q::edges)
-            if (near_edge_line<M>(box, mine, sh.edges[q < cnt ? q : 0])) {
-                special = true;
-                d2 = -1.0;
-            }
+        const double d2 = far_distance2(box, mine);
+        const double h2 = far_sure_half2<Q::orders>(mine.h2, far_reach(box.reach2));
         unsigned rest = live;
         auto take = [&](bool far) {
             const unsigned m = (unsigned)__ballot(far) & rest;
             rest &= ~m;
             return m;
         };
-        const unsigned m2 = take(field_box_far<2, M>(d2, mine, box));
-        const unsigned m3 = take(field_box_far<3, M>(d2, mine, box));
+        const unsigned m2 = take(field_box_far<2, M>(d2, h2, mine, box));
+        const unsigned m3 = take(field_box_far<3, M>(d2, h2, mine, box));
         field_far<2>(sh, different, m2, pt, acc);
         field_far<3>(sh, different, m3, pt, acc);
         if constexpr (Q::orders >= 4)
-            field_far<4>(sh, different, take(field_box_far<4, M>(d2, mine, box)), pt, acc);
+            field_far<4>(sh, different, take(field_box_far<4, M>(d2, h2, mine, box)), pt, acc);
         if constexpr (Q::orders >= 5)
-            field_far<5>(sh, different, take(field_box_far<5, M>(d2, mine, box)), pt, acc);
+            field_far<5>(sh, different, take(field_box_far<5, M>(d2, h2, mine, box)), pt, acc);
         // prisms that are far from some of the wave's points only
-        const unsigned specials = (unsigned)__ballot(special);
         for_bits(rest, [&](int p) {
-            const bool far = field_lane_far<M>(sh.far[p], (specials >> p) & 1u, pt);
+            const bool far = field_lane_far<M>(sh.far[p], lane_value(h2, p), pt);
             if (!any_lane(far)) return;
             double v[Op::values] = {};
             field_far<Q::orders>(sh, different, 1u << p, pt, v);
@@ -550,20 +533,17 @@ __device__ __forceinline__ bool field_close_chunk(const Src &src, const double *
     const GzPoint pt = field_point(oe, on, ou, base, n_obs, shared.box);
     __syncthreads();
     const int q = threadIdx.x & 63;
-    // (read again for every tile: in registers it costs the closed forms spills)
-    const FarBox &box = shared.box[threadIdx.x >> 6];
+    const FarBox box = shared.box[threadIdx.x >> 6];
+    const float reach = far_reach(box.reach2);
     FieldCloseWave<Op> &sh = shared.wave[threadIdx.x >> 6];
     bool any = false, skip = true;
     double b[6] = {}, weight[Op::weights] = {};
     if (c0 + q < c1) skip = src.get(c0 + q, b, weight);
     for (int64_t t0 = c0; t0 < c1; t0 += 64) {
-        const FarPrism rec = far_prism(b, pt.xo, pt.yo, 1.0);
-        bool edge_line = false;
-        if constexpr (Q::edges) edge_line = near_edge_line<M>(box, rec, FarEdges(b, pt));
-        const uint64_t near =
-            __ballot(!skip && (edge_line || !field_box_far<Q::orders, M>(far_distance2(box, rec),
-                                                                         rec, box)));
-        const uint64_t specials = __ballot(edge_line || far_unsure(box, rec.h2));
+        FarPrism rec = field_prism(b, pt);
+        rec.h2 = far_sure_half2<Q::orders>(rec.h2, reach);
+        const uint64_t near = __ballot(
+            !skip && !field_box_far<Q::orders, M>(far_distance2(box, rec), rec.h2, rec, box));
         if (near) {
             sh.far[q] = rec;
 #pragma unroll
@@ -578,7 +558,7 @@ __device__ __forceinline__ bool field_close_chunk(const Src &src, const double *
         wave_sync();
         uint64_t mask = 0;
         for_bits(near, [&](int p) {
-            const bool close = !field_lane_far<M>(sh.far[p], (specials >> p) & 1u, pt);
+            const bool close = !field_lane_far<M>(sh.far[p], sh.far[p].h2, pt);
             const double *t = sh.bounds[p];
             const bool lean = close && !needs_general<M>(pt.e, pt.n, pt.u, t[0], t[1], t[2], t[3],
                                                          t[4], t[5]);

@@ -203,6 +203,7 @@ __global__ __launch_bounds__(kObsPerBlock, 3) void gz_vjp_kernel(
         __syncthreads();
         if (!any_live) continue;
         uint64_t rest = cnt == 64 ? ~0ull : (1ull << cnt) - 1ull;
+        double point_h2 = h2;  // of the lane's point
         uint64_t m2 = 0, m3 = 0, m4 = 0, m5 = 0, m6 = 0;
         if (use_far) {
             const double4 o = tile[lane < cnt ? lane : 0];
@@ -213,18 +214,18 @@ __global__ __launch_bounds__(kObsPerBlock, 3) void gz_vjp_kernel(
             const double dt = fmax(fmax(box.u0 - o.z, o.z - box.u1), 0.0);
             const double db = fmax(fmax(b0 - o.z, o.z - b1), 0.0);
             const double d = fmin(dt, db);
-            double d2 = fma(dx, dx, fma(dy, dy, d * d)) + guard;
-            if (!dev::far_resolved(d2, h2, fma(x, x, y * y))) d2 = -1.0;
+            const double d2 = fma(dx, dx, fma(dy, dy, d * d)) + guard;
+            point_h2 = dev::far_sure_half2<dev::kFarMax>(h2, dev::far_reach(fma(x, x, y * y)));
             auto take = [&](bool far) {
                 const uint64_t m = __ballot(far) & rest;
                 rest &= ~m;
                 return m;
             };
-            m2 = take(dev::far_enough<2>(d2, h2));
-            m3 = take(dev::far_enough<3>(d2, h2));
-            m4 = take(dev::far_enough<4>(d2, h2));
-            m5 = take(dev::far_enough<5>(d2, h2));
-            m6 = take(dev::far_enough<6>(d2, h2));
+            m2 = take(dev::far_enough<2>(d2, point_h2));
+            m3 = take(dev::far_enough<3>(d2, point_h2));
+            m4 = take(dev::far_enough<4>(d2, point_h2));
+            m5 = take(dev::far_enough<5>(d2, point_h2));
+            m6 = take(dev::far_enough<6>(d2, point_h2));
         }
         auto point = [&](int q) {
             const double4 o = tile[q];
@@ -246,11 +247,10 @@ __global__ __launch_bounds__(kObsPerBlock, 3) void gz_vjp_kernel(
             const double4 o = tile[q];
             bool close = true;
             if (use_far) {
-                const double px = o.x - xo, py = o.y - yo, x = pr.x - px, y = pr.y - py;
+                const double x = pr.x - (o.x - xo), y = pr.y - (o.y - yo);
                 const double t = pr.b[5] - o.z, z = pr.b[4] - o.z;
-                const double d2 = fma(x, x, fma(y, y, fmin(t * t, z * z)));
-                close = !(dev::far_enough<dev::kFarMax>(d2, h2) &&
-                          dev::far_resolved(d2, h2, fma(px, px, py * py)));
+                close = !dev::far_enough<dev::kFarMax>(fma(x, x, fma(y, y, fmin(t * t, z * z))),
+                                                       dev::lane_value(point_h2, q));
                 if (dev::any_lane(live && !close)) {
                     double sa = 0.0, sb = 0.0;
                     vjp_far<dev::kFarMax>(pr, lds, point(q), sa, sb);
