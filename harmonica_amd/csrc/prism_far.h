@@ -270,6 +270,7 @@ __device__ __forceinline__ constexpr double far_ratio2(int I) {
 // doubles: with 1e-10 < h < 1e10 and distances below 1e14 the largest, (h r)^12
 // and r^-25, stay below 1e290.
 __device__ __forceinline__ double far_half2(double A, double B) {
+#pragma clang fp contract(off)
     const double h2 = A + B;
     return h2 > 1e-20 && h2 < 1e20 ? h2 : __builtin_nan("");
 }
@@ -355,10 +356,12 @@ __device__ __forceinline__ bool far_unsure(double h2, double reach2) {
 // distance's: the six tensor fields' and ten fields' close pairs took 13% longer
 // with one.  By FP32 logarithm and exponential, 1e-4 on the far side.
 __device__ __forceinline__ float far_reach(double reach2) {  // log2(R^2 / 4)
+#pragma clang fp contract(off)
     return __builtin_amdgcn_logf((float)reach2) - 2.0f;
 }
 template <int I>
 __device__ __forceinline__ double far_sure_half2(double h2, float reach) {
+#pragma clang fp contract(off)
     const float log_h2 = __builtin_amdgcn_logf((float)h2);
     const float log_r2 = fmaf(2.0f, log_h2, reach) * (1.0f / 3.0f);
     const double least = (double)__builtin_amdgcn_exp2f(log_r2) * (1.0001 / far_ratio2(I));
