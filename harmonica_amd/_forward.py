@@ -261,7 +261,8 @@ def prism_gravity(
     with progressbar_context(coords[0].size, progressbar):
         if cast.size == 0:
             return np.zeros(cast.shape, dtype=dtype)
-        e, n, u, dev_prisms, dev_density = to_device_together(*coords, prisms, density)
+        e, n, u = coords
+        e, n, u, dev_prisms, dev_density = to_device_together(e, n, u, prisms, density)
         out = prism_fields_device(e, n, u, dev_prisms, dev_density, (field,))
         if singular_check:
             # The reference scans every prism, null ones included, before

@@ -239,8 +239,9 @@ class DatasetAccessorPrismLayer:
         with progressbar_context(coords[0].size, progressbar):
             if cast.size == 0:
                 return np.zeros(cast.shape, dtype=np.float64)
+            e, n, u = coords
             out = layer_fields_device(
-                *to_device_together(*coords, self._obj.easting.values, self._obj.northing.values,
+                *to_device_together(e, n, u, self._obj.easting.values, self._obj.northing.values,
                                     self._obj.bottom.values, self._obj.top.values, density),
                 (field,), thickness_threshold=thickness_threshold,
             )
@@ -272,9 +273,9 @@ def layer_gravity_fields(layer, coordinates, fields, density_name="density",
     returns a (len(fields), n) float64 torch tensor on the GPU."""
     _lib.require_device()
     cast, coords = np.broadcast(*coordinates[:3]), coordinates
-    coords = [np.broadcast_to(np.asarray(c, float), cast.shape).ravel() for c in coords[:3]]
+    e, n, u = (np.broadcast_to(np.asarray(c, float), cast.shape).ravel() for c in coords[:3])
     return layer_fields_device(
-        *to_device_together(*coords, layer.easting.values, layer.northing.values,
+        *to_device_together(e, n, u, layer.easting.values, layer.northing.values,
                             layer.bottom.values, layer.top.values,
                             np.asarray(layer[density_name].values, float)),
         tuple(fields),

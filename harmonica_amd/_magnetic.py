@@ -115,7 +115,9 @@ def prism_magnetic(
         if cast.size == 0:
             result = np.zeros((len(components), 0))
         else:
-            out = magnetic_fields_device(*to_device_together(*coords, prisms, *magnetization),
+            e, n, u = coords
+            me, mn, mu = magnetization
+            out = magnetic_fields_device(*to_device_together(e, n, u, prisms, me, mn, mu),
                                          components)
             result = out.cpu().numpy()
     arrays = tuple(r.astype(dtype, copy=False).reshape(cast.shape) for r in result)

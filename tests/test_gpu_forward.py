@@ -351,3 +351,21 @@ def test_arrays_uploaded_together(sizes, dtype):
         assert g.dtype == torch.float64 and g.is_contiguous() and tuple(g.shape) == a.shape
         assert g.data_ptr() % 256 == 0
         npt.assert_array_equal(g.cpu().numpy(), a.astype(np.float64))
+
+
+def test_two_coordinates_or_magnetizations_are_refused(hm):
+    """Too few arrays are refused before any of them takes another's place."""
+    from harmonica_amd._layer import layer_gravity_fields
+
+    two, three = (np.zeros(3), np.ones(3)), (np.zeros(3), np.ones(3), np.ones(3))
+    prisms, one = [[0.0, 1.0, 0.0, 1.0, -2.0, -1.0]], np.ones(1)
+    layer = hm.prism_layer((np.arange(3.0), np.arange(2.0)), np.zeros((2, 3)), -1.0,
+                           properties={"density": np.ones((2, 3))})
+    calls = (lambda: hm.prism_gravity(two, prisms, one, "g_z"),
+             lambda: hm.prism_magnetic(two, prisms, (one, one, one), "b"),
+             lambda: hm.prism_magnetic(three, prisms, (one, one), "b", disable_checks=True),
+             lambda: layer.prism_layer.gravity(two, "g_z"),
+             lambda: layer_gravity_fields(layer, two, ("g_z",)))
+    for call in calls:
+        with pytest.raises(ValueError, match="expected 3, got 2"):
+            call()
